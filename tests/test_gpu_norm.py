@@ -91,7 +91,8 @@ def test_rmsnorm_plain_gamma_and_errors(gpu):
                     torch.zeros(8192, dtype=torch.bfloat16, device=gpu), 1e-6)
 
 
-@pytest.mark.parametrize("rows,cols", [(7, 520), (333, 2560), (4099, 2560), (64, 4096)])
+@pytest.mark.parametrize("rows,cols", [(7, 520), (333, 2560), (4099, 2560), (64, 4096), (2, 8),
+                                       (253, 24), (2049, 1000)])
 def test_rmsnorm_backward_matches_autograd(gpu, rows, cols):
     """dx and the weight gradient of the fused norm against fp64 autograd of the HF formula
     on the same bf16 inputs: each within one bf16 ulp (plus 1e-5 of the RMS for the fp32
