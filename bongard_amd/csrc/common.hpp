@@ -227,17 +227,8 @@ __device__ __forceinline__ float mx_multiplier(uint32_t e) {
 constexpr int kWaveTilePitch = 17;  // dwords per staged row (odd: conflict-free row writes)
 constexpr int kWaveTileDwords = 64 * kWaveTilePitch;
 
-// Transpose of a 64 x 64 byte tile that one wave has staged in its own LDS region (row r
-// at lds + r * kWaveTilePitch dwords, kWaveTileDwords in all): lane l gets columns
-// 4 (l & 15) + c, c < 4, over rows 16 (l >> 4) .. +15 as t[c] (byte i of t[c] = row
-// 16 (l >> 4) + i). No barrier is needed between the wave's staging stores and these
-// reads: a wave's LDS accesses complete in order.
-__device__ __forceinline__ void wave_transpose64_staged(const uint32_t* lds, int lane,
-                                                        uint4 (&t)[4]) {
-  const int row0 = (lane >> 4) * 16, cg = lane & 15;
-  uint32_t d[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) d[i] = lds[(row0 + i) * kWaveTilePitch + cg];
+// Dword i of d holds 4 columns of row i: t[c] becomes column c of the 16 rows (byte i = row i).
+__device__ __forceinline__ void transpose_4x16(const uint32_t (&d)[16], uint4 (&t)[4]) {
   uint32_t c[4][4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {  // 4 x 4 byte transpose of rows 4k .. 4k+3
@@ -252,6 +243,20 @@ __device__ __forceinline__ void wave_transpose64_staged(const uint32_t* lds, int
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) t[k] = make_uint4(c[k][0], c[k][1], c[k][2], c[k][3]);
+}
+
+// Transpose of a 64 x 64 byte tile that one wave has staged in its own LDS region (row r
+// at lds + r * kWaveTilePitch dwords, kWaveTileDwords in all): lane l gets columns
+// 4 (l & 15) + c, c < 4, over rows 16 (l >> 4) .. +15 as t[c] (byte i of t[c] = row
+// 16 (l >> 4) + i). No barrier is needed between the wave's staging stores and these
+// reads: a wave's LDS accesses complete in order.
+__device__ __forceinline__ void wave_transpose64_staged(const uint32_t* lds, int lane,
+                                                        uint4 (&t)[4]) {
+  const int row0 = (lane >> 4) * 16, cg = lane & 15;
+  uint32_t d[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) d[i] = lds[(row0 + i) * kWaveTilePitch + cg];
+  transpose_4x16(d, t);
 }
 
 // Tile t of a grid of tile rows x tiles_c tile columns, in tile-row-pair order: tiles 2j

@@ -23,8 +23,7 @@ namespace {
 
 constexpr int kMxNT = 256;
 constexpr int kMxMaxRowBlocks = 8192;
-constexpr int kMT = 64;                // columnwise tile (rows x cols)
-constexpr int kMPitch = kMT + 4;
+constexpr int kMT = 128;               // tile of the two-copy kernel (rows x cols)
 constexpr int kMaxMxTileBlocks = 2048;
 // Rowwise: a 16-lane group handles 128 consecutive elements of a row (4 blocks, 4 lanes
 // each, 8 elements per lane) and writes the dword of their 4 scale bytes. Grid-stride over
@@ -113,104 +112,199 @@ int64_t mx_row_blocks(int64_t rows, int64_t ld_sc) {
                                                 kMxMaxRowBlocks));
 }
 
-// Columnwise, transposed: 64 x 64 tiles of x; each column's two 32-row blocks get their
-// scales from an LDS pass over |x|; q_t [cols, rows], scales [cols, ld_sc_t].
+// Exponents (mx_exponent) of two packed |x| maxima given as finite bf16 keys: fp8_max is
+// 1.75 x 2^S, so amax / fp8_max rounds up to a power of two with exponent E - S where the
+// mantissa is at most 1.75 (96 / 128 above 1) and E - S + 1 past it, i.e. ((key + 31) >> 7) - S,
+// at least 0 (equal to mx_exponent on every finite key).
 template <int FMT>
-__global__ __launch_bounds__(kMxNT) void mx_col_kernel(const uint16_t* __restrict__ x,
-                                                       int64_t rows, int64_t cols,
-                                                       uint8_t* __restrict__ out_t,
-                                                       uint8_t* __restrict__ sc_t,
-                                                       int64_t ld_sc_t) {
-  __shared__ uint16_t keys[kMT][kMT + 2];       // |x| bf16 keys, [row][col]
-  __shared__ float mult[2][kMT];                // per (row block, column)
-  __shared__ uint32_t tile[kMT * kMPitch / 4];  // fp8 bytes, [row][col]
-  uint8_t* tb = reinterpret_cast<uint8_t*>(tile);
-  const int64_t tiles_c = (cols + kMT - 1) / kMT;
-  const int64_t ntiles = tiles_c * ((rows + kMT - 1) / kMT);
-  const int64_t nblk_rows = rows / 32;
-  const int t = threadIdx.x;
-  for (int64_t tile_id = blockIdx.x; tile_id < ntiles; tile_id += gridDim.x) {
-    const int64_t r0 = (tile_id / tiles_c) * kMT, c0 = (tile_id % tiles_c) * kMT;
-    const int lr = t >> 2, lc = (t & 3) * 16;
-    const int64_t r = r0 + lr, c = c0 + lc;
-    const bool valid = r < rows && c < cols;
-    uint4 a0 = make_uint4(0u, 0u, 0u, 0u), a1 = a0;
-    if (valid) {
-      const uint4* src4 = reinterpret_cast<const uint4*>(x + r * cols + c);
-      a0 = src4[0];
-      a1 = src4[1];
-    }
-    {
-      const uint32_t w[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+__device__ __forceinline__ uint32_t mx_exponent_finite_pk(uint32_t keys) {
+  constexpr unsigned short S = FMT == BF8_E4M3 ? 8 : 15;
+  const u16x2 lim = {S, S};
+  u16x2 k = __builtin_bit_cast(u16x2, keys);
+  k = (u16x2)((u16x2)(k + (u16x2){31, 31}) >> 7);
+  k = (u16x2)(__builtin_elementwise_max(k, lim) - lim);
+  return __builtin_bit_cast(uint32_t, k);
+}
+
+// Quantizes 8 bf16 values with their own multipliers. FINITE: none of the values is inf or
+// NaN, so no product leaves +-fp8_max.
+template <int FMT, bool FINITE>
+__device__ __forceinline__ uint2 mx_quant8_vs(uint4 v, const float* s) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  uint32_t q[2];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        keys[lr][lc + 2 * i] = (uint16_t)(w[i] & 0x7FFFu);
-        keys[lr][lc + 2 * i + 1] = (uint16_t)((w[i] >> 16) & 0x7FFFu);
+  for (int k = 0; k < 2; ++k) {
+    const float x0 = bf16_lo(w[2 * k]), x1 = bf16_hi(w[2 * k]);
+    const float x2 = bf16_lo(w[2 * k + 1]), x3 = bf16_hi(w[2 * k + 1]);
+    const float* t = s + 4 * k;
+    if constexpr (FINITE) {
+      q[k] = quant4_finite<FMT, false>(x0 * t[0], x1 * t[1], x2 * t[2], x3 * t[3]);
+    } else {
+      q[k] = quant4<FMT>(x0 * t[0], x1 * t[1], x2 * t[2], x3 * t[3], x0, x1, x2, x3, t[0]);
+      // quant4 signs a NaN product by one scale: redo those by their own column's
+      const float xs[4] = {x0, x1, x2, x3};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float pr = xs[e] * t[e];
+        if (__builtin_expect(pr != pr, 0))
+          q[k] = (q[k] & ~(0xFFu << (8 * e))) | (nan_byte(xs[e], t[e]) << (8 * e));
       }
     }
+  }
+  return make_uint2(q[0], q[1]);
+}
+
+// Both copies of x in one pass (or the columnwise one alone). A block takes 128 x 128 tiles,
+// each wave 32 rows of all 128 columns: lane l holds columns 8 (l & 15) .. +7 of the rows
+// 4 k + l / 16, k < 8, so a row block of 32 is four neighbouring lanes (two DPP exchanges) and a
+// column block of 32 rows is the wave's eight pieces and the four lanes of a column group (two
+// lane exchanges of packed 16-bit maxima). The columnwise bytes meet in LDS; each wave then
+// turns 32 columns of all 128 rows. Every store instruction of either output writes whole
+// 128-byte lines, and every scale store a whole dword of four blocks.
+// HBM-bound: 2 B read, 1 B (+ 1/32) written per element and copy; x is read once for the two
+// copies, where a rowwise and a columnwise pass read it twice. Both copies, inputs rotated past
+// the MALL: [4096, 20480] 133.1 us in two passes, 78.4 us in one (4.3 TB/s); [20480, 2560]
+// 72.9 -> 45.4 us (4.7 TB/s); one pass over 64 x 64 tiles per wave, whose stores are half
+// lines, 99.7 and 56.3 us.
+struct MxTile {
+  int64_t rows, cols;
+  uint8_t* out;
+  uint8_t* sc;
+  int64_t ld_sc;
+  uint8_t* out_t;
+  uint8_t* sc_t;
+  int64_t ld_sc_t;
+};
+
+constexpr int kMPitch = kMT / 4 + 1;  // dwords per staged row (odd)
+
+template <int FMT, bool FINITE>
+__device__ __forceinline__ void mx_tile_body(const MxTile& p, int64_t r0, int64_t c0,
+                                             const uint4 (&v)[8], const uint32_t (&rk)[8],
+                                             const uint32_t (&cm)[4], uint32_t* stage,
+                                             uint8_t* ecol, int wid, int lane) {
+  const int cl = lane & 15, lr = lane >> 4;
+  const int64_t c = c0 + 8 * cl;
+  const int64_t wr0 = r0 + 32 * wid;
+  if (p.out) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t r = wr0 + 4 * k + lr;
+      uint32_t e;
+      if constexpr (FINITE)
+        e = mx_exponent_finite_pk<FMT>(rk[k]) & 0xFFFFu;
+      else
+        e = mx_exponent<FMT>(rk[k] << 16);
+      if (r < p.rows && c < p.cols) {
+        const float mult = mx_multiplier(e);
+        *reinterpret_cast<uint2*>(p.out + r * p.cols + c) =
+            FINITE ? quant8_bf16_finite<FMT, false>(v[k], mult) : quant8_bf16<FMT>(v[k], mult);
+      }
+      if (c >= p.cols) e = kMxPadScale;  // blocks past the row pad its last dword of scales
+      // lanes 0, 4, 8, 12 of the 16 hold the four blocks: gather into lane 0
+      e |= (uint32_t)__shfl_down((int)e, 4, 64) << 8;
+      e |= (uint32_t)__shfl_down((int)e, 8, 64) << 16;
+      if (cl == 0 && r < p.rows)
+        *reinterpret_cast<uint32_t*>(p.sc + r * p.ld_sc + (c0 >> 5)) = e;
+    }
+  }
+  if (!p.out_t) return;
+  float s[8];
+  uint32_t ex[4];  // packed pairs of the lane's column exponents
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (FINITE)
+      ex[i] = mx_exponent_finite_pk<FMT>(cm[i]);
+    else
+      ex[i] = mx_exponent<FMT>(cm[i] << 16) | (mx_exponent<FMT>(cm[i] & 0xFFFF0000u) << 16);
+    s[2 * i] = mx_multiplier(ex[i] & 0xFFFFu);
+    s[2 * i + 1] = mx_multiplier(ex[i] >> 16);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint2 q = mx_quant8_vs<FMT, FINITE>(v[k], s);
+    uint32_t* d = stage + (32 * wid + 4 * k + lr) * kMPitch + 2 * cl;
+    d[0] = q.x;
+    d[1] = q.y;
+  }
+  if (lr == 0) {
+    const bool valid = wr0 < p.rows;  // rows % 32 == 0: the wave's block is whole or absent
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ecol[(8 * cl + 2 * i) * 4 + wid] = valid ? (uint8_t)ex[i] : (uint8_t)kMxPadScale;
+      ecol[(8 * cl + 2 * i + 1) * 4 + wid] = valid ? (uint8_t)(ex[i] >> 16) : (uint8_t)kMxPadScale;
+    }
+  }
+}
+
+template <int FMT>
+__global__ __launch_bounds__(kMxNT) void mx_tile_kernel(const uint16_t* __restrict__ x, MxTile p) {
+  __shared__ uint32_t stage[kMT * kMPitch];
+  __shared__ __attribute__((aligned(4))) uint8_t ecol[kMT * 4];  // [column][row block]
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int64_t tiles_c = (p.cols + kMT - 1) / kMT, tiles_r = (p.rows + kMT - 1) / kMT;
+  const int64_t ntiles = tiles_c * tiles_r;
+  const int cl = lane & 15, lr = lane >> 4;
+  const bool sc_dwords = ((uintptr_t)p.sc_t & 3) == 0;
+  for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int64_t r0 = (t / tiles_c) * kMT, c0 = (t % tiles_c) * kMT;
+    const int64_t c = c0 + 8 * cl;
+    uint4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int64_t r = r0 + 32 * wid + 4 * k + lr;
+      v[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (r < p.rows && c < p.cols)
+        v[k] = *reinterpret_cast<const uint4*>(x + r * p.cols + c);
+    }
+    uint32_t rk[8], cm[4] = {};
+    uint32_t top = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t a[4] = {v[k].x & 0x7FFF7FFFu, v[k].y & 0x7FFF7FFFu, v[k].z & 0x7FFF7FFFu,
+                             v[k].w & 0x7FFF7FFFu};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cm[i] = pk_max_u16(cm[i], a[i]);
+      uint32_t m = pk_max_u16(pk_max_u16(a[0], a[1]), pk_max_u16(a[2], a[3]));
+      m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true));
+      m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, true));
+      rk[k] = max(m & 0xFFFFu, m >> 16);
+      top = max(top, rk[k]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 16, 64));
+      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 32, 64));
+    }
+    if (__builtin_expect(__any(top >= 0x7F80u), 0))
+      mx_tile_body<FMT, false>(p, r0, c0, v, rk, cm, stage, ecol, wid, lane);
+    else
+      mx_tile_body<FMT, true>(p, r0, c0, v, rk, cm, stage, ecol, wid, lane);
     __syncthreads();
-    if (t < 2 * kMT) {
-      const int col = t & (kMT - 1), blk = t >> 6;
-      uint32_t m = 0;
-#pragma unroll 8
-      for (int i = 0; i < 32; ++i) m = max(m, (uint32_t)keys[blk * 32 + i][col]);
-      const uint32_t e = mx_exponent<FMT>(m << 16);
-      mult[blk][col] = mx_multiplier(e);
-      const int64_t gc = c0 + col, gb = r0 / 32 + blk;
-      if (gc < cols) {
-        uint8_t* srow = sc_t + gc * ld_sc_t;
-        if (gb < nblk_rows) srow[gb] = (uint8_t)e;
-        // the last tile row also pads the column's scale row to whole dwords
-        if (blk == 1 && r0 + kMT >= rows)
-          for (int64_t pb = nblk_rows; pb < ld_sc_t; ++pb) srow[pb] = (uint8_t)kMxPadScale;
+    // lane: 16 rows (lane & 7) x 4 columns (lane >> 3) of the wave's 32 columns
+    const int rg = (lane & 7) * 16, cg = 8 * wid + (lane >> 3);
+    uint32_t d[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) d[i] = stage[(rg + i) * kMPitch + cg];
+    uint4 tq[4];
+    transpose_4x16(d, tq);
+    const int64_t tc = r0 + rg;  // column of out_t (a row of x)
+    if (tc < p.rows) {
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) {
+        const int64_t tr = c0 + 4 * cg + cc;  // row of out_t (a column of x)
+        if (tr < p.cols) *reinterpret_cast<uint4*>(p.out_t + tr * p.rows + tc) = tq[cc];
       }
     }
-    __syncthreads();
-    {
-      uint32_t q[4] = {0u, 0u, 0u, 0u};
-      if (valid) {
-        float s[16];
+    if (threadIdx.x < kMT && c0 + threadIdx.x < p.cols) {
+      // four blocks of one column; the last tile row's absent blocks pad the scale row
+      const uint32_t e4 = *reinterpret_cast<const uint32_t*>(ecol + 4 * threadIdx.x);
+      uint8_t* dst = p.sc_t + (c0 + threadIdx.x) * p.ld_sc_t + (r0 >> 5);
+      if (sc_dwords) {
+        *reinterpret_cast<uint32_t*>(dst) = e4;
+      } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = mult[lr >> 5][lc + i];
-        const uint4 w0 = a0, w1 = a1;
-        // per-element multipliers: quantize in groups of 4 with their own factors
-        const float xs[16] = {bf16_lo(w0.x), bf16_hi(w0.x), bf16_lo(w0.y), bf16_hi(w0.y),
-                              bf16_lo(w0.z), bf16_hi(w0.z), bf16_lo(w0.w), bf16_hi(w0.w),
-                              bf16_lo(w1.x), bf16_hi(w1.x), bf16_lo(w1.y), bf16_hi(w1.y),
-                              bf16_lo(w1.z), bf16_hi(w1.z), bf16_lo(w1.w), bf16_hi(w1.w)};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          uint32_t wq = quant4<FMT>(xs[4 * k] * s[4 * k], xs[4 * k + 1] * s[4 * k + 1],
-                                    xs[4 * k + 2] * s[4 * k + 2], xs[4 * k + 3] * s[4 * k + 3],
-                                    xs[4 * k], xs[4 * k + 1], xs[4 * k + 2], xs[4 * k + 3],
-                                    s[4 * k]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float pr = xs[4 * k + e] * s[4 * k + e];
-            if (__builtin_expect(pr != pr, 0))
-              wq = (wq & ~(0xFFu << (8 * e))) | (nan_byte(xs[4 * k + e], s[4 * k + e]) << (8 * e));
-          }
-          q[k] = wq;
-        }
-      }
-      uint32_t* dst = reinterpret_cast<uint32_t*>(tb + lr * kMPitch + lc);
-      dst[0] = q[0]; dst[1] = q[1]; dst[2] = q[2]; dst[3] = q[3];
-    }
-    __syncthreads();
-    {
-      const int oc = t >> 2, orow = (t & 3) * 16;
-      const int64_t tr = c0 + oc, tc = r0 + orow;
-      if (tr < cols && tc < rows) {
-        uint32_t w[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t b0 = tb[(orow + 4 * j + 0) * kMPitch + oc];
-          const uint32_t b1 = tb[(orow + 4 * j + 1) * kMPitch + oc];
-          const uint32_t b2 = tb[(orow + 4 * j + 2) * kMPitch + oc];
-          const uint32_t b3 = tb[(orow + 4 * j + 3) * kMPitch + oc];
-          w[j] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
-        }
-        *reinterpret_cast<uint4*>(out_t + tr * rows + tc) = make_uint4(w[0], w[1], w[2], w[3]);
+        for (int b = 0; b < 4; ++b) dst[b] = (uint8_t)(e4 >> (8 * b));
       }
     }
     __syncthreads();
@@ -244,7 +338,7 @@ int bf8_quantize_mx_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uin
             "bf8_quantize_mx_bf16: x, out_t 16-byte, out 8-byte, out_scales 4-byte aligned");
   hipStream_t s = as_stream(stream);
   const uint16_t* xs = (const uint16_t*)x;
-  if (out) {
+  if (!out_t) {
     const int64_t ld = bf8_mx_scale_ld(cols);
     const unsigned grid = (unsigned)mx_row_blocks(rows, ld);
     if (fmt == BF8_E4M3)
@@ -253,22 +347,24 @@ int bf8_quantize_mx_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uin
     else
       hipLaunchKernelGGL(mx_row_kernel<BF8_E5M2>, dim3(grid), dim3(kMxNT), 0, s, xs, rows, cols,
                          out, out_scales, ld);
-    const int rc = launch_status("mx_row_kernel");
-    if (rc != BF8_OK) return rc;
+    return launch_status("mx_row_kernel");
   }
-  if (out_t) {
-    const int64_t ld = bf8_mx_scale_ld(rows);
-    const int64_t tiles = ((rows + kMT - 1) / kMT) * ((cols + kMT - 1) / kMT);
-    const unsigned grid = (unsigned)std::min<int64_t>(tiles, kMaxMxTileBlocks);
-    if (fmt == BF8_E4M3)
-      hipLaunchKernelGGL(mx_col_kernel<BF8_E4M3>, dim3(grid), dim3(kMxNT), 0, s, xs, rows, cols,
-                         out_t, out_t_scales, ld);
-    else
-      hipLaunchKernelGGL(mx_col_kernel<BF8_E5M2>, dim3(grid), dim3(kMxNT), 0, s, xs, rows, cols,
-                         out_t, out_t_scales, ld);
-    return launch_status("mx_col_kernel");
-  }
-  return BF8_OK;
+  MxTile p{};
+  p.rows = rows;
+  p.cols = cols;
+  p.out = out;
+  p.sc = out_scales;
+  p.ld_sc = out ? bf8_mx_scale_ld(cols) : 0;
+  p.out_t = out_t;
+  p.sc_t = out_t_scales;
+  p.ld_sc_t = bf8_mx_scale_ld(rows);
+  const int64_t tiles = ((rows + kMT - 1) / kMT) * ((cols + kMT - 1) / kMT);
+  const unsigned grid = (unsigned)std::min<int64_t>(tiles, kMaxMxTileBlocks);
+  if (fmt == BF8_E4M3)
+    hipLaunchKernelGGL(mx_tile_kernel<BF8_E4M3>, dim3(grid), dim3(kMxNT), 0, s, xs, p);
+  else
+    hipLaunchKernelGGL(mx_tile_kernel<BF8_E5M2>, dim3(grid), dim3(kMxNT), 0, s, xs, p);
+  return launch_status("mx_tile_kernel");
 }
 
 int bf8_quantize_mx_many_bf16(int count, const void* const* x, const int64_t* rows,

@@ -52,6 +52,30 @@ def test_quantize_mx_bit_exact(gpu, rows, cols, fmt):
     assert same_q and same_s
 
 
+@pytest.mark.parametrize("rows,cols", [(32, 32), (128, 128), (160, 96), (288, 416), (64, 144)])
+def test_quantize_mx_two_copies_edges(gpu, rows, cols):
+    """Both copies from one pass over 128 x 128 tiles: whole and partial tiles in either
+    direction (scale padding included), blocks holding inf, NaN and the largest and smallest
+    magnitudes, and the columnwise copy alone."""
+    x = _x(rows, cols, 3 * rows + cols, spread=False).float()
+    x[1, 3], x[rows - 1, cols - 1], x[rows // 2, cols // 2] = float("inf"), float("nan"), -float("inf")
+    x[2, :16] = 3.38e38
+    x[3, 16:32] = 1e-39
+    x = x.to(torch.bfloat16)
+    rowwise = cols % 32 == 0
+    q = ops.quantize_mx(x.to(gpu), rowwise=rowwise, colwise=True)
+    only = ops.quantize_mx(x.to(gpu), rowwise=False, colwise=True)
+    torch.cuda.synchronize()
+    cq, ce = orc.quantize_mx(x, ops.E4M3, 0)
+    for t in (q, only):
+        assert torch.equal(t.data_t.view(torch.uint8).cpu(), cq)
+        assert torch.equal(t.scales_t.cpu(), orc.mx_scale_rows(ce))
+    if rowwise:
+        rq, re = orc.quantize_mx(x, ops.E4M3, -1)
+        assert torch.equal(q.data.view(torch.uint8).cpu(), rq)
+        assert torch.equal(q.scales.cpu(), orc.mx_scale_rows(re))
+
+
 def test_quantize_mx_errors(gpu):
     with pytest.raises(Exception, match="cols"):
         ops.quantize_mx(torch.zeros(32, 48, dtype=torch.bfloat16, device=gpu))
