@@ -280,14 +280,15 @@ class Fp8LinearNvfp4Function(_Fp8Function):
         x4t, xst, x_meta, w4t, wst, w_meta = ctx.saved_tensors
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dyq = ops.quantize_nvfp4(dy.contiguous(), rowwise=need_dx, colwise=need_dw,
-                                 dequant_rows=True)
+                                 dequant_rows=True, dequant_cols=True)
         dx = dw = None
         if need_dx:
             wdt = ops.nvfp4_dequant(ctx.wq, transpose=True) if ctx.wq is not None else None
             dx = ops.gemm_nvfp4(None, None, dyq.meta, w4t, wst, w_meta,
                                 a_deq=ops.nvfp4_dequant(dyq), b_deq=wdt)
         if need_dw:
-            dw = ops.gemm_nvfp4(dyq.data_t, dyq.scales_t, dyq.meta, x4t, xst, x_meta)
+            dw = ops.gemm_nvfp4(None, None, dyq.meta, x4t, xst, x_meta,
+                                a_deq=ops.nvfp4_dequant(dyq, transpose=True))
         return dx, dw, None, None
 
 
@@ -356,14 +357,15 @@ class GegluGateUpNvfp4Function(_Fp8Function):
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dGU, dparts = ops.geglu_bwd(dH.contiguous(), GU)
         dq = ops.quantize_nvfp4(dGU, rowwise=need_dx, colwise=need_dw, partials=dparts,
-                                dequant_rows=True)
+                                dequant_rows=True, dequant_cols=True)
         dx = dw = None
         if need_dx:
             wdt = ops.nvfp4_dequant(ctx.wq, transpose=True) if ctx.wq is not None else None
             dx = ops.gemm_nvfp4(None, None, dq.meta, w4t, wst, w_meta,
                                 a_deq=ops.nvfp4_dequant(dq), b_deq=wdt)
         if need_dw:
-            dw = ops.gemm_nvfp4(dq.data_t, dq.scales_t, dq.meta, x4t, xst, x_meta)
+            dw = ops.gemm_nvfp4(None, None, dq.meta, x4t, xst, x_meta,
+                                a_deq=ops.nvfp4_dequant(dq, transpose=True))
         return dx, dw, None, None, None
 
 

@@ -1008,7 +1008,8 @@ def nvfp4_dequant(q, *, transpose=False):
     return d
 
 
-def quantize_nvfp4(x, *, rowwise=True, colwise=False, partials=None, dequant_rows=False):
+def quantize_nvfp4(x, *, rowwise=True, colwise=False, partials=None, dequant_rows=False,
+                   dequant_cols=False):
     """NVFP4 quantization of a bf16 tensor (flattened to 2-D): an amax pass and the block
     quantization (rowwise needs cols % 16 == 0, columnwise rows % 16 == 0). ``partials``:
     the amax partials of |x| its producer wrote (int32 / uint32 fp32 bits: ``geglu_bwd``'s,
@@ -1016,7 +1017,8 @@ def quantize_nvfp4(x, *, rowwise=True, colwise=False, partials=None, dequant_row
     (bf8_quantize_nvfp4_partials_bf16, the same outputs bit for bit). ``dequant_rows``: the
     rowwise copy is kept only as its exact bf16 dequantization (``nvfp4_dequant(q)``; data
     and scales None), for a tensor whose rowwise copy only feeds the next GEMM
-    (bf8_quantize_nvfp4_dequant_bf16)."""
+    (bf8_quantize_nvfp4_dequant_bf16); ``dequant_cols``: the columnwise copy likewise
+    (``nvfp4_dequant(q, transpose=True)``; cols % 8 == 0)."""
     _require_gpu(x, partials)
     x = _bf16_2d(x)
     rows, cols = x.shape
@@ -1024,24 +1026,29 @@ def quantize_nvfp4(x, *, rowwise=True, colwise=False, partials=None, dequant_row
     meta = new_meta(dev)
     u8 = torch.uint8
     codes = rowwise and not dequant_rows
+    codes_t = colwise and not dequant_cols
     out = torch.empty((rows, cols // 2), dtype=u8, device=dev) if codes else None
     sc = torch.empty((rows, cols // 16), dtype=u8, device=dev) if codes else None
-    out_t = torch.empty((cols, rows // 2), dtype=u8, device=dev) if colwise else None
-    sc_t = torch.empty((cols, rows // 16), dtype=u8, device=dev) if colwise else None
+    out_t = torch.empty((cols, rows // 2), dtype=u8, device=dev) if codes_t else None
+    sc_t = torch.empty((cols, rows // 16), dtype=u8, device=dev) if codes_t else None
     L = _lib.lib()
     if partials is not None:
         if partials.dtype != torch.int32 or partials.dim() != 1 or partials.numel() < 1:
             raise ValueError("quantize_nvfp4: partials must be a non-empty 1-D int32 tensor")
-    if dequant_rows and rowwise:
-        deq = torch.empty((rows, cols), dtype=torch.bfloat16, device=dev)
+    if (dequant_rows and rowwise) or (dequant_cols and colwise):
+        if codes:
+            raise ValueError("quantize_nvfp4: dequant_cols with rowwise codes is not supported")
+        deq = torch.empty((rows, cols), dtype=torch.bfloat16, device=dev) if rowwise else None
+        deq_t = (torch.empty((cols, rows), dtype=torch.bfloat16, device=dev)
+                 if colwise and dequant_cols else None)
         if partials is not None:
             parts, n_parts = partials.contiguous(), partials.numel()
         else:
-            parts, n_parts = partials_buffer(max(1, int(L.bf8_amax_partials(rows * cols))), dev), 0
-        _lib.check(L.bf8_quantize_nvfp4_dequant_bf16(
-            _ptr(x), rows, cols, _ptr(parts), n_parts, _ptr(deq), _ptr(out_t), _ptr(sc_t),
-            _ptr(meta), _stream(dev)), "bf8_quantize_nvfp4_dequant_bf16")
-        return NvFp4Tensor(None, None, out_t, sc_t, meta, rows, cols, _deq=deq)
+            parts, n_parts = partials_buffer(max(1, _amax_partials_cached(rows * cols)), dev), 0
+        _lib.check(L.bf8_quantize_nvfp4_dequant2_bf16(
+            _ptr(x), rows, cols, _ptr(parts), n_parts, _ptr(deq), _ptr(deq_t), _ptr(out_t),
+            _ptr(sc_t), _ptr(meta), _stream(dev)), "bf8_quantize_nvfp4_dequant2_bf16")
+        return NvFp4Tensor(None, None, out_t, sc_t, meta, rows, cols, _deq=deq, _deq_t=deq_t)
     if partials is not None:
         _lib.check(L.bf8_quantize_nvfp4_partials_bf16(
             _ptr(x), rows, cols, _ptr(partials.contiguous()), partials.numel(), _ptr(out),

@@ -400,6 +400,15 @@ int bf8_quantize_nvfp4_dequant_bf16(const void* x, int64_t rows, int64_t cols,
                                     uint32_t* partials, int64_t n_partials, void* deq,
                                     uint8_t* out_t, uint8_t* out_t_scales, float* meta,
                                     void* stream);
+/* bf8_quantize_nvfp4_dequant_bf16 whose columnwise copy may also be written as its exact bf16
+ * dequantization deq_t [cols, rows] (bf8_dequant_nvfp4 of out_t, bit for bit; rows % 16 == 0,
+ * cols % 8 == 0), for a gradient whose two copies each feed one GEMM (dY and dGU under
+ * NVFP4BlockScaling: bongard/te_linear.py:17,38). At least one of deq and deq_t; deq_t or
+ * out_t. */
+int bf8_quantize_nvfp4_dequant2_bf16(const void* x, int64_t rows, int64_t cols,
+                                     uint32_t* partials, int64_t n_partials, void* deq,
+                                     void* deq_t, uint8_t* out_t, uint8_t* out_t_scales,
+                                     float* meta, void* stream);
 int bf8_dequant_nvfp4(const uint8_t* q, const uint8_t* scales, int64_t rows, int64_t cols,
                       void* out, void* stream);
 size_t bf8_gemm_bf16_workspace(int64_t M, int64_t N, int64_t K);

@@ -68,6 +68,47 @@ def test_quantize_nvfp4_bit_exact(gpu, rows, cols):
     assert torch.equal(deq.cpu().float(), ref)        # e2m1 x e4m3 is exact in bf16
 
 
+@pytest.mark.parametrize("rows,cols", [(16, 128), (128, 128), (144, 272), (272, 48), (400, 2560)])
+def test_quantize_nvfp4_tile_edges(gpu, rows, cols):
+    """Whole and partial 128 x 128 tiles in either direction: codes and scales of both copies
+    against the oracle, and both copies written as their bf16 dequantization."""
+    x = _inputs(rows, cols, 7 * rows + cols)
+    q = ops.quantize_nvfp4(x.to(gpu), rowwise=True, colwise=True)
+    d = ops.quantize_nvfp4(x.to(gpu), rowwise=True, colwise=True, dequant_rows=True,
+                           dequant_cols=True)
+    dt = ops.quantize_nvfp4(x.to(gpu), rowwise=False, colwise=True, dequant_cols=True)
+    torch.cuda.synchronize()
+    p, sb, _, _, _ = orc.quantize_nvfp4(x)
+    pt, st, _, _, _ = orc.quantize_nvfp4(x, axis=0)
+    assert torch.equal(q.data.cpu(), p) and torch.equal(q.scales.cpu(), sb)
+    assert torch.equal(q.data_t.cpu(), pt) and torch.equal(q.scales_t.cpu(), st)
+    assert torch.equal(ops.nvfp4_dequant(d).cpu().float(), orc.dequant_nvfp4(p, sb))
+    for t in (d, dt):
+        assert t.data_t is None and torch.equal(t.meta, q.meta)
+        assert torch.equal(ops.nvfp4_dequant(t, transpose=True).cpu().float(),
+                           orc.dequant_nvfp4(pt, st))
+
+
+@pytest.mark.parametrize("special", [None, float("inf"), float("nan")])
+def test_quantize_nvfp4_broken_rows_and_non_finite(gpu, special):
+    """Columns that do not fill 16-byte vectors take the per-column kernel: the same bytes as the
+    tile kernel gives for those columns of a padded tensor under the same tensor amax, also
+    where the tensor or some of its blocks hold inf or NaN."""
+    x = _inputs(160, 24, 5)
+    if special is not None:
+        x[3, 4], x[100, 7] = special, -special
+    x = x.to(gpu)
+    parts = ops.amax(x)
+    finite = ops.amax(torch.full((16, 8), 3.0, dtype=torch.bfloat16, device=gpu))
+    for pr in (parts, finite):   # the tensor's own amax, and a finite scale for its blocks
+        a = ops.quantize_nvfp4(x, rowwise=False, colwise=True, partials=pr)
+        b = ops.quantize_nvfp4(x[:, :20].contiguous(), rowwise=False, colwise=True, partials=pr)
+        torch.cuda.synchronize()
+        assert torch.equal(a.data_t[:20], b.data_t) and torch.equal(a.scales_t[:20], b.scales_t)
+    with pytest.raises(Exception, match="cols"):
+        ops.quantize_nvfp4(x[:, :20].contiguous(), rowwise=False, colwise=True, dequant_cols=True)
+
+
 def test_quantize_nvfp4_zero_tensor_and_columnwise_only(gpu):
     x = torch.zeros(32, 64, dtype=torch.bfloat16)
     q = ops.quantize_nvfp4(x.to(gpu), rowwise=False, colwise=True)
