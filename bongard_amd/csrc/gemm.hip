@@ -65,7 +65,7 @@ constexpr TileInfo kTiles[NUM_TILES] = {
     {128, 64, 1, 0.1, 0.0, "128x64k2", false},
     {64, 128, 1, 0.1, 0.0, "64x128k2", false},
     {128, 128, 1, 0.1, 0.0, "128x128k2", false},
-    {256, 256, 1, 10.0, 9.2, "256x256w8", false},
+    {256, 256, 1, 10.0, 9.2, "256x256w8", true},
     {256, 256, 1, 10.0, 0.0, "256x256w8x", false},
 };
 // Whether `tile` has a gated-GELU variant for I = N / 2: tiles of 128 or 64 H columns take
@@ -240,8 +240,8 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
     // K-major operands: the eight-wave 256x256 tiles only
     if (kmajor && tile != TILE_256x256w8) continue;
     // the eight-wave 256x256 tile replaces the four-wave one wherever it has a variant
-    // (measured faster on every large shape, same bits); MX keeps the four-wave tile
-    if (!mx && tile == TILE_256x256) continue;
+    // (measured faster on every large shape, same bits)
+    if (tile == TILE_256x256) continue;
     // the extra-B-slot twin of the eight-wave tile is substituted below, by K
     if (tile == TILE_256x256w8x) continue;
     for (int s = 1; s <= (geglu ? 1 : kMaxSplits); ++s) {
@@ -830,31 +830,52 @@ static int check_mx_operand(const char* who, const char* what, const uint8_t* q,
   return BF8_OK;
 }
 
-int bf8_gemm_mx(const uint8_t* A, int64_t lda, const uint8_t* A_scales, int64_t lda_sc,
-                const uint8_t* B, int64_t ldb, const uint8_t* B_scales, int64_t ldb_sc,
-                int64_t M, int64_t N, int64_t K, const void* bias, void* C, int out_dtype,
-                int64_t ldc, void* ws, size_t ws_bytes, void* stream) {
-  BF8_CHECK(out_dtype == BF8_OUT_BF16 || out_dtype == BF8_OUT_F32, "bf8_gemm_mx: bad out_dtype");
-  BF8_CHECK(M >= 0 && N >= 0 && K >= 0, "bf8_gemm_mx: negative shape");
-  BF8_CHECK(K % 32 == 0, "bf8_gemm_mx: K must be a multiple of the 32-element block (got %lld)",
+// One plane of scale dwords per 128 K-values: [(K + 127) / 128][rows], 4-byte aligned.
+static int check_mx_planes(const char* who, const char* what, const uint8_t* q, int64_t ld,
+                           const uint32_t* planes, int64_t rows, int64_t K) {
+  BF8_CHECK(q && planes, "%s: %s or its scale planes are NULL", who, what);
+  BF8_CHECK(ld % 16 == 0 && ld >= K && ((uintptr_t)q & 15) == 0,
+            "%s: %s needs a 16-byte aligned base and row stride >= K", who, what);
+  BF8_CHECK(((uintptr_t)planes & 3) == 0, "%s: %s scale planes need 4-byte alignment", who, what);
+  BF8_CHECK(rows * ld < (1LL << 31) && rows * bf8_mx_scale_ld(K) < (1LL << 31),
+            "%s: %s larger than 2 GiB", who, what);
+  return BF8_OK;
+}
+
+static MxScales row_scales(const uint8_t* sc, int64_t ld) {
+  return MxScales{const_cast<uint8_t*>(sc), ld, 4};
+}
+static MxScales plane_scales(const uint32_t* planes, int64_t rows) {
+  return MxScales{(uint8_t*)const_cast<uint32_t*>(planes), 4, 4 * rows};
+}
+
+static int gemm_mx_args(const char* who, int64_t M, int64_t N, int64_t K, const void* bias,
+                        const void* C, int out_dtype, int64_t ldc, const void* ws,
+                        size_t ws_bytes) {
+  BF8_CHECK(out_dtype == BF8_OUT_BF16 || out_dtype == BF8_OUT_F32, "%s: bad out_dtype", who);
+  BF8_CHECK(M >= 0 && N >= 0 && K >= 0, "%s: negative shape", who);
+  BF8_CHECK(K % 32 == 0, "%s: K must be a multiple of the 32-element block (got %lld)", who,
             (long long)K);
-  BF8_CHECK(N % 8 == 0 && ldc >= N && ldc % 4 == 0,
-            "bf8_gemm_mx: need N %% 8 == 0, ldc >= N, ldc %% 4 == 0");
+  BF8_CHECK(N % 8 == 0 && ldc >= N && ldc % 4 == 0, "%s: need N %% 8 == 0, ldc >= N, ldc %% 4 == 0",
+            who);
   BF8_CHECK(((uintptr_t)C & 15) == 0 && ((uintptr_t)bias & 7) == 0,
-            "bf8_gemm_mx: C must be 16-byte, bias 8-byte aligned");
+            "%s: C must be 16-byte, bias 8-byte aligned", who);
   BF8_CHECK(ws_bytes == 0 || (ws && ((uintptr_t)ws & 255) == 0),
-            "bf8_gemm_mx: workspace must be 256-byte aligned");
+            "%s: workspace must be 256-byte aligned", who);
   if (M == 0 || N == 0) return BF8_OK;
-  BF8_CHECK(K > 0, "bf8_gemm_mx: K == 0 is not supported");
-  BF8_CHECK(C != nullptr, "bf8_gemm_mx: C is NULL");
-  int rc = check_mx_operand("bf8_gemm_mx", "A", A, lda, A_scales, lda_sc, M, K);
-  if (rc) return rc;
-  rc = check_mx_operand("bf8_gemm_mx", "B", B, ldb, B_scales, ldb_sc, N, K);
-  if (rc) return rc;
+  BF8_CHECK(K > 0, "%s: K == 0 is not supported", who);
+  BF8_CHECK(C != nullptr, "%s: C is NULL", who);
+  return BF8_OK;
+}
+
+static int gemm_mx_launch(const uint8_t* A, int64_t lda, MxScales a_sc, const uint8_t* B,
+                          int64_t ldb, MxScales b_sc, int64_t M, int64_t N, int64_t K,
+                          const void* bias, void* C, int out_dtype, int64_t ldc, void* ws,
+                          size_t ws_bytes, void* stream) {
   GemmParams p{};
   p.A = A; p.B = B; p.lda = lda; p.ldb = ldb;
   p.M = (int)M; p.N = (int)N; p.K = (int)K; p.I = 0;
-  p.a_sc = A_scales; p.b_sc = B_scales; p.a_sc_ld = lda_sc; p.b_sc_ld = ldb_sc;
+  p.a_sc = a_sc; p.b_sc = b_sc;
   p.n_seg = 1;
   for (int s = 0; s < 4; ++s) p.seg_end[s] = (int)N;
   p.bias = (const uint16_t*)bias; p.C = C; p.ldc = ldc;
@@ -863,12 +884,39 @@ int bf8_gemm_mx(const uint8_t* A, int64_t lda, const uint8_t* A_scales, int64_t 
                      true);
 }
 
+int bf8_gemm_mx(const uint8_t* A, int64_t lda, const uint8_t* A_scales, int64_t lda_sc,
+                const uint8_t* B, int64_t ldb, const uint8_t* B_scales, int64_t ldb_sc,
+                int64_t M, int64_t N, int64_t K, const void* bias, void* C, int out_dtype,
+                int64_t ldc, void* ws, size_t ws_bytes, void* stream) {
+  const char* who = "bf8_gemm_mx";
+  int rc = gemm_mx_args(who, M, N, K, bias, C, out_dtype, ldc, ws, ws_bytes);
+  if (rc || M == 0 || N == 0) return rc;
+  rc = check_mx_operand(who, "A", A, lda, A_scales, lda_sc, M, K);
+  if (rc) return rc;
+  rc = check_mx_operand(who, "B", B, ldb, B_scales, ldb_sc, N, K);
+  if (rc) return rc;
+  return gemm_mx_launch(A, lda, row_scales(A_scales, lda_sc), B, ldb, row_scales(B_scales, ldb_sc),
+                        M, N, K, bias, C, out_dtype, ldc, ws, ws_bytes, stream);
+}
+
+int bf8_gemm_mx_planes(const uint8_t* A, int64_t lda, const uint32_t* A_planes, const uint8_t* B,
+                       int64_t ldb, const uint32_t* B_planes, int64_t M, int64_t N, int64_t K,
+                       const void* bias, void* C, int out_dtype, int64_t ldc, void* ws,
+                       size_t ws_bytes, void* stream) {
+  const char* who = "bf8_gemm_mx_planes";
+  int rc = gemm_mx_args(who, M, N, K, bias, C, out_dtype, ldc, ws, ws_bytes);
+  if (rc || M == 0 || N == 0) return rc;
+  rc = check_mx_planes(who, "A", A, lda, A_planes, M, K);
+  if (rc) return rc;
+  rc = check_mx_planes(who, "B", B, ldb, B_planes, N, K);
+  if (rc) return rc;
+  return gemm_mx_launch(A, lda, plane_scales(A_planes, M), B, ldb, plane_scales(B_planes, N), M, N,
+                        K, bias, C, out_dtype, ldc, ws, ws_bytes, stream);
+}
+
 // The MX gate/up GEMM + gated GELU; H8 (with H8t) set: H quantized in the epilogue.
-static int geglu_mx_entry(const char* who, const uint8_t* X, int64_t ldx, const uint8_t* X_scales,
-                          int64_t ldx_sc, const uint8_t* W, int64_t ldw, const uint8_t* W_scales,
-                          int64_t ldw_sc, int64_t M, int64_t I, int64_t K, void* H, int64_t ldh,
-                          uint8_t* H8, uint8_t* H8_scales, int64_t ldh8_sc, uint8_t* H8t,
-                          uint8_t* H8t_scales, int64_t ldh8t_sc, void* GU, void* stream) {
+static int geglu_mx_args(const char* who, int64_t M, int64_t I, int64_t K, const void* H,
+                         int64_t ldh, const uint8_t* H8, const uint8_t* H8t, const void* GU) {
   BF8_CHECK(M >= 1 && I >= 1 && K >= 32, "%s: bad shape", who);
   BF8_CHECK(I % 128 == 0, "%s: I must be a multiple of 128 (got %lld)", who, (long long)I);
   BF8_CHECK(K % 32 == 0, "%s: K must be a multiple of 32", who);
@@ -876,34 +924,51 @@ static int geglu_mx_entry(const char* who, const uint8_t* X, int64_t ldx, const 
   BF8_CHECK(!H || (ldh >= I && ldh % 4 == 0), "%s: bad ldh", who);
   BF8_CHECK(((uintptr_t)H & 15) == 0 && ((uintptr_t)GU & 15) == 0,
             "%s: H, GU must be 16-byte aligned", who);
-  if (H8) {
-    BF8_CHECK(H8_scales && ldh8_sc >= I / 32 && ((uintptr_t)H8 & 7) == 0,
-              "%s: H8 needs 8-byte alignment and scales with row stride >= I / 32", who);
-    BF8_CHECK(M * I < (1LL << 31), "%s: H8 larger than 2 GiB", who);
-  }
+  BF8_CHECK(!H8 || M * I < (1LL << 31), "%s: H8 larger than 2 GiB", who);
+  BF8_CHECK(((uintptr_t)H8 & 7) == 0, "%s: H8 needs 8-byte alignment", who);
   BF8_CHECK(!H8t || H8, "%s: H8t needs H8", who);
-  if (H8t) {
-    BF8_CHECK(M % 32 == 0, "%s: H8t blocks along M need M %% 32 == 0 (got %lld)", who,
-              (long long)M);
-    BF8_CHECK(H8t_scales && ldh8t_sc >= bf8_mx_scale_ld(M) && ((uintptr_t)H8t & 15) == 0,
-              "%s: H8t needs 16-byte alignment and scales with row stride >= %lld", who,
-              (long long)bf8_mx_scale_ld(M));
-  }
-  int rc = check_mx_operand(who, "X", X, ldx, X_scales, ldx_sc, M, K);
-  if (rc) return rc;
-  rc = check_mx_operand(who, "W", W, ldw, W_scales, ldw_sc, 2 * I, K);
-  if (rc) return rc;
+  BF8_CHECK(!H8t || (M % 32 == 0 && ((uintptr_t)H8t & 15) == 0),
+            "%s: H8t blocks along M need M %% 32 == 0 (got %lld) and 16-byte alignment", who,
+            (long long)M);
+  return BF8_OK;
+}
+
+static int geglu_mx_launch(const uint8_t* X, int64_t ldx, MxScales x_sc, const uint8_t* W,
+                           int64_t ldw, MxScales w_sc, int64_t M, int64_t I, int64_t K, void* H,
+                           int64_t ldh, uint8_t* H8, MxScales h8_sc, uint8_t* H8t,
+                           MxScales h8t_sc, void* GU, void* stream) {
   GemmParams p{};
   p.A = X; p.B = W; p.lda = ldx; p.ldb = ldw;
   p.M = (int)M; p.N = (int)(2 * I); p.K = (int)K; p.I = (int)I;
-  p.a_sc = X_scales; p.b_sc = W_scales; p.a_sc_ld = ldx_sc; p.b_sc_ld = ldw_sc;
+  p.a_sc = x_sc; p.b_sc = w_sc;
   p.n_seg = 1;
   p.C = H; p.ldc = ldh; p.GU = (uint16_t*)GU; p.partials = nullptr;
-  p.h8 = H8; p.h8_sc = H8_scales; p.h8_sc_ld = ldh8_sc;
-  p.h8t = H8t; p.h8t_sc = H8t_scales; p.h8t_sc_ld = ldh8t_sc;
+  p.h8 = H8; p.h8_sc = h8_sc;
+  p.h8t = H8t; p.h8t_sc = h8t_sc;
   Plan pl = choose_plan(M, 2 * I, K, true, 0, true);
   return launch_plan(pl, p, EPI_GEGLU, BF8_OUT_BF16, BF8_E4M3, BF8_E4M3, nullptr,
                      as_stream(stream), true);
+}
+
+static int geglu_mx_entry(const char* who, const uint8_t* X, int64_t ldx, const uint8_t* X_scales,
+                          int64_t ldx_sc, const uint8_t* W, int64_t ldw, const uint8_t* W_scales,
+                          int64_t ldw_sc, int64_t M, int64_t I, int64_t K, void* H, int64_t ldh,
+                          uint8_t* H8, uint8_t* H8_scales, int64_t ldh8_sc, uint8_t* H8t,
+                          uint8_t* H8t_scales, int64_t ldh8t_sc, void* GU, void* stream) {
+  int rc = geglu_mx_args(who, M, I, K, H, ldh, H8, H8t, GU);
+  if (rc) return rc;
+  BF8_CHECK(!H8 || (H8_scales && ldh8_sc >= I / 32),
+            "%s: H8 needs scales with row stride >= I / 32", who);
+  BF8_CHECK(!H8t || (H8t_scales && ldh8t_sc >= bf8_mx_scale_ld(M)),
+            "%s: H8t needs scales with row stride >= %lld", who, (long long)bf8_mx_scale_ld(M));
+  rc = check_mx_operand(who, "X", X, ldx, X_scales, ldx_sc, M, K);
+  if (rc) return rc;
+  rc = check_mx_operand(who, "W", W, ldw, W_scales, ldw_sc, 2 * I, K);
+  if (rc) return rc;
+  return geglu_mx_launch(X, ldx, row_scales(X_scales, ldx_sc), W, ldw,
+                         row_scales(W_scales, ldw_sc), M, I, K, H, ldh, H8,
+                         row_scales(H8_scales, ldh8_sc), H8t, row_scales(H8t_scales, ldh8t_sc),
+                         GU, stream);
 }
 
 int bf8_gemm_geglu_mx(const uint8_t* X, int64_t ldx, const uint8_t* X_scales, int64_t ldx_sc,
@@ -924,6 +989,26 @@ int bf8_gemm_geglu_mx_quant(const uint8_t* X, int64_t ldx, const uint8_t* X_scal
   return geglu_mx_entry("bf8_gemm_geglu_mx_quant", X, ldx, X_scales, ldx_sc, W, ldw, W_scales,
                         ldw_sc, M, I, K, H, ldh, H8, H8_scales, ldh8_sc, H8t, H8t_scales,
                         ldh8t_sc, GU, stream);
+}
+
+int bf8_gemm_geglu_mx_planes(const uint8_t* X, int64_t ldx, const uint32_t* X_planes,
+                             const uint8_t* W, int64_t ldw, const uint32_t* W_planes, int64_t M,
+                             int64_t I, int64_t K, void* H, int64_t ldh, uint8_t* H8,
+                             uint32_t* H8_planes, uint8_t* H8t, uint32_t* H8t_planes, void* GU,
+                             void* stream) {
+  const char* who = "bf8_gemm_geglu_mx_planes";
+  int rc = geglu_mx_args(who, M, I, K, H, ldh, H8, H8t, GU);
+  if (rc) return rc;
+  BF8_CHECK((!H8 || (H8_planes && ((uintptr_t)H8_planes & 3) == 0)) &&
+                (!H8t || (H8t_planes && ((uintptr_t)H8t_planes & 3) == 0)),
+            "%s: H8 and H8t need 4-byte aligned scale planes", who);
+  rc = check_mx_planes(who, "X", X, ldx, X_planes, M, K);
+  if (rc) return rc;
+  rc = check_mx_planes(who, "W", W, ldw, W_planes, 2 * I, K);
+  if (rc) return rc;
+  return geglu_mx_launch(X, ldx, plane_scales(X_planes, M), W, ldw, plane_scales(W_planes, 2 * I),
+                         M, I, K, H, ldh, H8, plane_scales(H8_planes, M), H8t,
+                         plane_scales(H8t_planes, I), GU, stream);
 }
 
 }  // extern "C"

@@ -13,6 +13,11 @@ enum GemmEpi { EPI_LINEAR = 0, EPI_GEGLU = 1 };
 // lda and ldb are passed in bytes); the FP8 formats are BF8_E4M3 (0) and BF8_E5M2 (1).
 constexpr int kFmtBf16 = 2;
 
+struct MxScales {
+  uint8_t* p;
+  int64_t rs, gs;  // bytes per operand row and per group of 128 K-values
+};
+
 struct GemmParams {
   const uint8_t* A;  // [M, K] row-major, row stride lda bytes
   const uint8_t* B;  // [N, K] row-major (nn.Linear weight layout), row stride ldb bytes
@@ -25,9 +30,10 @@ struct GemmParams {
   const float* a_sinv;    // a_vec: one per row of A (M), else a single value
   const float* b_sinv;    // b_vec: one per row of B (N), else n_seg values b_stride apart
   int a_vec, b_vec;       // LINEAR only
-  const uint8_t* a_sc;    // MX: E8M0 block scales [M, a_sc_ld] (byte k/32 of row m)
-  const uint8_t* b_sc;    // MX: [N, b_sc_ld]
-  int64_t a_sc_ld, b_sc_ld;
+  // MX: E8M0 block scales. Byte k/32 of operand row m lies at m * rs + (k/128) * gs + (k/32) % 4:
+  // rows of bytes (rs = the row stride, gs = 4) or one plane of dwords per 128-byte K step
+  // (rs = 4, gs = 4 * rows), whose 64 rows' dwords a wave loads as two lines instead of 64.
+  MxScales a_sc, b_sc;
   int b_stride;
   int n_seg;
   int seg_end[4];
@@ -38,14 +44,13 @@ struct GemmParams {
   uint32_t* partials;     // GEGLU: one amax key of |H| per tile
   // GEGLU with H quantized in the epilogue (C, the bf16 H, may then be NULL). h8: e4m3
   // [M, I]; h8t (optional, needs M % 32 == 0): e4m3 H^T [I, M]. MX: E8M0 block scales
-  // h8_sc [M, h8_sc_ld] (blocks along I) and h8t_sc [I, h8t_sc_ld] (blocks along M);
+  // h8_sc of H (blocks along I) and h8t_sc of H^T (blocks along M), laid out as a_sc;
   // otherwise one scale, read from the device word h8_scale.
   const float* h8_scale;
   uint8_t* h8;
-  uint8_t* h8_sc;
+  MxScales h8_sc;
   uint8_t* h8t;
-  uint8_t* h8t_sc;
-  int64_t h8_sc_ld, h8t_sc_ld;
+  MxScales h8t_sc;
   int64_t split_stride;   // splits > 1: C is fp32 [splits][M][ldc], raw sums, this many
                           // elements apart (a reduce kernel applies scales and bias)
   // Tail-split schedule (tail_pieces > 0, linear epilogues, splits == 1): workgroups

@@ -48,13 +48,28 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 constexpr int kBK = 128;       // K bytes per LDS stage
 constexpr int kNumXcd = 8;
+enum { EXTRA_NONE = 0, EXTRA_TABLE };  // what a K step does besides
 constexpr uint32_t kOob = 0x80000000u;  // buffer offset that always reads as zero
 
-// LDS bytes a variant needs besides its NS pipeline stages: the gated-GELU epilogue keeps
-// the fp32 gelu table (kGeluA32) there, at LDS offset 0 ahead of the stages, so that its
-// byte offsets (below 64 KB) address it directly from packed 16-bit arithmetic.
-template <int EPI>
-constexpr int extra_lds() { return EPI == EPI_GEGLU ? kGeluA32Bytes : 0; }
+// The gated-GELU epilogue reads the fp32 gelu table (kGeluA32, 26 KB) at LDS offset 0, so that
+// its byte offsets (below 64 KB) address it directly from packed 16-bit arithmetic. Tiles with
+// two stages load it into stage slot 0 while the last K step runs: the slots alternate so
+// that the last step always sits in slot 1, and slot 0 is free from the mid-step barrier of the
+// step before (no LDS beyond the stages, and the tile's first loads do not queue behind it).
+// Deeper rings, rings with extra B slots and stages below 26 KB keep it ahead of the stages
+// for the whole tile.
+constexpr bool late_table(int epi, int ns, int xb, int kg, int stage_bytes) {
+  return epi == EPI_GEGLU && ns == 2 && xb == 0 && kg == 1 && stage_bytes >= kGeluA32Bytes;
+}
+// LDS bytes a variant needs besides its NS pipeline stages.
+constexpr int extra_lds(int epi, bool late) { return epi == EPI_GEGLU && !late ? kGeluA32Bytes : 0; }
+
+// MX block scales in LDS: one dword (4 blocks of 32) per tile row in every stage. From scale
+// rows a wave's load touches 64 lines; from scale planes (MxScales) two. That was what held
+// the MX GEMMs below the FP8 ones: 8192^3 on the eight-wave tile 495.1 us from rows, 418.8 from
+// planes (FP8 416.5; the four-wave tile 523.5 from rows), (4096, 2560, 10240) 121.2 -> 94.5 us on
+// the 256x160 tile.
+constexpr int kMxStageBytes = 2048;
 
 // Buffer resource (4 SGPRs): base, stride 0, `bytes` valid bytes (offsets at or beyond
 // read as zero), raw-buffer flags of gfx9/gfx950.
@@ -288,7 +303,8 @@ __device__ __forceinline__ void mx_h_epilogue(const GemmParams& p, const uint8_t
       const float mult = mx_multiplier(e);
       *reinterpret_cast<uint2*>(p.h8 + (int64_t)gm * p.I + n) =
           FAST ? quant8_bf16_finite<BF8_E4M3, false>(d, mult) : quant8_bf16<BF8_E4M3>(d, mult);
-      if ((c & 3) == 0) p.h8_sc[(int64_t)gm * p.h8_sc_ld + (n >> 5)] = (uint8_t)e;
+      if ((c & 3) == 0)
+        p.h8_sc.p[(int64_t)gm * p.h8_sc.rs + (n >> 7) * p.h8_sc.gs + ((n >> 5) & 3)] = (uint8_t)e;
     }
   }
   if (p.h8t == nullptr) return;
@@ -333,15 +349,15 @@ __device__ __forceinline__ void mx_h_epilogue(const GemmParams& p, const uint8_t
     d0[1] = make_uint4(q0[4], q0[5], q0[6], q0[7]);
     d1[0] = make_uint4(q1[0], q1[1], q1[2], q1[3]);
     d1[1] = make_uint4(q1[4], q1[5], q1[6], q1[7]);
-    uint8_t* r0 = p.h8t_sc + (int64_t)n * p.h8t_sc_ld;
-    uint8_t* r1 = r0 + p.h8t_sc_ld;
-    r0[gm >> 5] = (uint8_t)e0;
-    r1[gm >> 5] = (uint8_t)e1;
+    uint8_t* r0 = p.h8t_sc.p + (int64_t)n * p.h8t_sc.rs + (gm >> 7) * p.h8t_sc.gs;
+    uint8_t* r1 = r0 + p.h8t_sc.rs;
+    r0[(gm >> 5) & 3] = (uint8_t)e0;
+    r1[(gm >> 5) & 3] = (uint8_t)e1;
     if ((gm >> 5) == nblk - 1) {
-      // the column's last block also pads its scale row to whole dwords
+      // the column's last block also pads its last dword of scales
       for (int pb = nblk; pb < sc_pad_end; ++pb) {
-        r0[pb] = (uint8_t)kMxPadScale;
-        r1[pb] = (uint8_t)kMxPadScale;
+        r0[pb & 3] = (uint8_t)kMxPadScale;
+        r1[pb & 3] = (uint8_t)kMxPadScale;
       }
     }
   }
@@ -447,11 +463,12 @@ gemm_kernel(GemmParams p) {
   constexpr int kA = BM * kBK;               // A tile bytes per stage
   // MX: each stage also holds the E8M0 block scales of its K step: one dword (4 blocks of
   // 32) per tile row, A rows at kData + 4 r, B rows at kData + 1024 + 4 r (r < 256).
+  constexpr bool MX8 = MX && NW == 8;
   constexpr int kData = (BM + BN) * kBK;
-  constexpr int kStage = kData + (MX ? 2048 : 0);  // [A tile | B tile | scales]
+  constexpr int kStage = kData + (MX ? kMxStageBytes : 0);  // [A tile | B tile | scales]
   constexpr int DA = BM / (8 * NW), DB = BN / (8 * NW);  // 1 KB DMA blocks per wave per stage
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole 1 KB blocks per wave");
-  constexpr int ND = DA + DB + (MX ? 2 : 0);  // loads per wave per stage
+  constexpr int ND = DA + DB + (MX ? (MX8 ? 1 : 2) : 0);  // loads per wave per stage
   constexpr int NM = FM * FN;                // MFMAs per sub-step
   constexpr int NH = 2 * (FM + FN);          // 16-byte fragment halves per sub-step
   static_assert(EPI != EPI_GEGLU || FN % 2 == 0 || (T::WN == 1 && BN % 16 == 0 && BN % 64 != 0),
@@ -459,17 +476,17 @@ gemm_kernel(GemmParams p) {
                 "and up halves are whole runs of 8 columns");
   static_assert(!(EPI == EPI_GEGLU && MX && FN % 2 != 0), "MX GEGLU: 32-column H blocks per tile");
   static_assert(!MX || (BM <= 256 && BN <= 256), "MX scale rows: one dword per lane");
-  static_assert(!MX || NW == 4, "MX scale dwords: four waves of 64 rows");
+  static_assert(!MX8 || (BM == 256 && BN == 256), "MX, eight waves: one scale row per lane");
   static_assert(KM == 0 || (NW == 8 && BM == 256 && BN == 256 && EPI == EPI_LINEAR && !MX),
                 "K-major operands: eight-wave 256 x 256 linear tiles");
   constexpr bool AKM = (KM & 1) != 0, BKM = (KM & 2) != 0;
   static_assert(XB == 0 || (NS == 2 && KG == 1 && !MX), "extra B slots: two stages, one K group");
-  constexpr int kStageOff = extra_lds<EPI>();  // GEGLU: the gelu table, then the stages
+  constexpr bool kLateTab = late_table(EPI, NS, XB, KG, kStage);
+  constexpr int kStageOff = extra_lds(EPI, kLateTab);  // GEGLU: a resident gelu table first
   constexpr int kB = BN * kBK;  // B tile bytes per stage
-  static_assert((KG * NS * kStage + XB * kB + extra_lds<EPI>()) * T::OCC <= 160 * 1024,
-                "LDS budget");
-  __shared__ __attribute__((aligned(1024)))
-  uint8_t smem[KG * NS * kStage + XB * kB + extra_lds<EPI>()];
+  constexpr int kLds = kStageOff + KG * NS * kStage + XB * kB;
+  static_assert(kLds * T::OCC <= 160 * 1024, "LDS budget");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kLds];
 
   // Dequant scales: read at the start, so their latency hides behind the first loads.
   const float sa = MX ? 1.0f : *p.a_sinv;
@@ -515,51 +532,74 @@ gemm_kernel(GemmParams p) {
   // l and wid & 1 (= blk & 1, NW even), so one K mask serves every block of the lane.
   const int lrow = lane >> 3;
   const int lchunk = (lane & 7) ^ (((wid & 1) << 2) | (lrow >> 1));
-  uint32_t a_off[DA], b_off[DB];
   // K-major: lane l of 1 KB block blk covers K row blk*4 + l/16 (of the step) and 16-byte
-  // position l%16 of that row's 256 bytes, holding logical chunk (l%16) ^ kmaj_swz(row)
+  // position l%16 of that row's 256 bytes, holding logical chunk (l%16) ^ kmaj_swz(row); row
+  // mod 8 does not depend on j either.
   const int kmrow = lane >> 4;
-  auto kmaj_chunk = [&](int j) { return (lane & 15) ^ kmaj_swz((j * NW + wid) * 4 + kmrow); };
-#pragma unroll
-  for (int j = 0; j < DA; ++j) {
-    if constexpr (AKM) {
-      const int am = m0 + kmaj_chunk(j) * 16;  // M % 16 == 0: whole chunks in or out
-      a_off[j] = am < p.M ? (uint32_t)((int64_t)((j * NW + wid) * 4 + kmrow) * p.lda + am)
-                          : kOob;
-    } else {
-      const int am = m0 + (j * NW + wid) * 8 + lrow;
-      a_off[j] = am < p.M ? (uint32_t)((int64_t)am * p.lda + lchunk * 16) : kOob;
-    }
+  const int kmchunk = (lane & 15) ^ kmaj_swz(wid * 4 + kmrow);
+  static_assert(!(AKM || BKM) || NW % 2 == 0, "K-major chunk swizzle is the same for every block");
+  // Block j of the lane lies a constant number of rows past block 0, so one offset register
+  // and scalar strides address them all (not one register a block). Row offsets past the
+  // tensor must read as zero and never wrap: operands are below 2 GiB, so a block-0 offset or a
+  // stride of 2^31 - 1 or more is past their end whatever is added (offsets are capped at
+  // kOob = 2^31, strides at 2^31 - 1, and the sums stay below 2^32).
+  auto stride_of = [&](int64_t rows, int64_t ld) {
+    const int64_t v = rows * ld;
+    return (uint32_t)(v < 0x7FFFFFFF ? v : 0x7FFFFFFF);
+  };
+  uint32_t a_off, b_off;
+  if constexpr (AKM) {
+    const int am = m0 + kmchunk * 16;  // M % 16 == 0: whole chunks in or out
+    a_off = am < p.M ? (uint32_t)((int64_t)(wid * 4 + kmrow) * p.lda + am) : kOob;
+  } else {
+    const int am = m0 + wid * 8 + lrow;
+    a_off = am < p.M ? (uint32_t)((int64_t)am * p.lda + lchunk * 16) : kOob;
   }
+  uint32_t a_str[DA];
+#pragma unroll
+  for (int j = 0; j < DA; ++j) a_str[j] = stride_of((int64_t)j * NW * (AKM ? 4 : 8), p.lda);
+  // B likewise; gated GELU: the first half of the tile's rows are gate rows, the second the up
+  // rows I further on (whole blocks on either side, every row in range since I % 128 == 0),
+  // except for the odd-FN tile, whose halves are not whole blocks: one register a block there.
+  constexpr bool kBSplit = EPI == EPI_GEGLU && (BN / 2) % (8 * NW) != 0;
+  uint32_t b_blk[kBSplit ? DB : 1];
+  if constexpr (BKM) {
+    const int bc = n0 + kmchunk * 16;  // N % 16 == 0: whole chunks in or out
+    b_off = bc < p.N ? (uint32_t)((int64_t)(wid * 4 + kmrow) * p.ldb + bc) : kOob;
+  } else {
+    const int bn = n0 + wid * 8 + lrow;
+    b_off = bn < (EPI == EPI_GEGLU ? p.I : p.N) ? (uint32_t)((int64_t)bn * p.ldb + lchunk * 16)
+                                                : kOob;
+  }
+  uint32_t b_str[DB];
 #pragma unroll
   for (int j = 0; j < DB; ++j) {
-    const int r = (j * NW + wid) * 8 + lrow;
-    int bn;
-    bool bvalid;
-    if (EPI == EPI_GEGLU) {
-      const int rr = r < BN / 2 ? r : r - BN / 2;
-      bn = (r < BN / 2 ? 0 : p.I) + n0 + rr;
-      bvalid = n0 + rr < p.I;
+    if constexpr (EPI == EPI_GEGLU && !kBSplit) {
+      constexpr int half = BN / 2 / (8 * NW);  // blocks per half
+      b_str[j] = stride_of((int64_t)(j % half) * 8 * NW + (j < half ? 0 : p.I), p.ldb);
     } else {
-      bn = n0 + r;
-      bvalid = bn < p.N;
+      b_str[j] = stride_of((int64_t)j * NW * (BKM ? 4 : 8), p.ldb);
     }
-    b_off[j] = bvalid ? (uint32_t)((int64_t)bn * p.ldb + lchunk * 16) : kOob;
-    if constexpr (BKM) {
-      const int bc = n0 + kmaj_chunk(j) * 16;  // N % 16 == 0: whole chunks in or out
-      b_off[j] = bc < p.N ? (uint32_t)((int64_t)((j * NW + wid) * 4 + kmrow) * p.ldb + bc)
-                          : kOob;
+    if constexpr (kBSplit) {
+      const int r = (j * NW + wid) * 8 + lrow;
+      const int rr = r < BN / 2 ? r : r - BN / 2;
+      const int bn = (r < BN / 2 ? 0 : p.I) + n0 + rr;
+      b_blk[j] = n0 + rr < p.I ? (uint32_t)((int64_t)bn * p.ldb + lchunk * 16) : kOob;
     }
   }
-  // MX: lane l of wave w loads the scale dword of tile row w * 64 + l (A and B), from
-  // the [rows, ld] E8M0 arrays; rows outside the tile or the tensor read as zero.
+  // MX: lane l of wave w loads the scale dword of tile row w * 64 + l (A and B) or, with eight
+  // waves, waves 0-3 those of A and waves 4-7 those of B; rows outside the tile or the tensor
+  // read as zero.
   i32x4 srd_sa = {0, 0, 0, 0}, srd_sb = {0, 0, 0, 0};
-  uint32_t sa_off = kOob, sb_off = kOob;
+  uint32_t sa_off = kOob, sb_off = kOob, sa_gs = 0, sb_gs = 0;
   if constexpr (MX) {
-    srd_sa = make_srd(p.a_sc, (uint32_t)((int64_t)p.M * p.a_sc_ld));
-    srd_sb = make_srd(p.b_sc, (uint32_t)((int64_t)p.N * p.b_sc_ld));
-    const int r = wid * 64 + lane;
-    if (r < BM && m0 + r < p.M) sa_off = (uint32_t)((int64_t)(m0 + r) * p.a_sc_ld);
+    auto sc_srd = [&](const MxScales& m, int rows) {
+      const int64_t by_row = rows * m.rs, by_group = ksteps * m.gs;  // whichever is the outer
+      return make_srd(m.p, (uint32_t)(by_row > by_group ? by_row : by_group));
+    };
+    const int r = (MX8 ? wid & 3 : wid) * 64 + lane;
+    uint32_t oa = kOob, ob = kOob;
+    if (r < BM && m0 + r < p.M) oa = (uint32_t)((int64_t)(m0 + r) * p.a_sc.rs);
     if (r < BN) {
       int bn;
       bool bvalid;
@@ -571,7 +611,16 @@ gemm_kernel(GemmParams p) {
         bn = n0 + r;
         bvalid = bn < p.N;
       }
-      if (bvalid) sb_off = (uint32_t)((int64_t)bn * p.b_sc_ld);
+      if (bvalid) ob = (uint32_t)((int64_t)bn * p.b_sc.rs);
+    }
+    const bool second = MX8 && __builtin_amdgcn_readfirstlane(wid) >= 4;
+    srd_sa = second ? sc_srd(p.b_sc, p.N) : sc_srd(p.a_sc, p.M);
+    sa_off = second ? ob : oa;
+    sa_gs = (uint32_t)(second ? p.b_sc.gs : p.a_sc.gs);
+    if constexpr (!MX8) {
+      srd_sb = sc_srd(p.b_sc, p.N);
+      sb_off = ob;
+      sb_gs = (uint32_t)p.b_sc.gs;
     }
   }
   // A partial last K step (K % 128 != 0) must read its chunks at or beyond K as zero.
@@ -585,22 +634,22 @@ gemm_kernel(GemmParams p) {
                       uint8_t* bdst) {
     const uint32_t base = lds_addr(stage);
     if (x < DA) {
-      if constexpr (AKM)
-        dma16(ra, base + (x * NW + wid) * 1024, kill_sc ? kOob : a_off[x], k0 * (uint32_t)p.lda);
-      else
-        dma16(ra, base + (x * NW + wid) * 1024, kill ? kOob : a_off[x], k0);
+      const uint32_t off = ((AKM ? kill_sc : kill) ? kOob : a_off) + a_str[x];
+      dma16(ra, base + (x * NW + wid) * 1024, off, AKM ? k0 * (uint32_t)p.lda : k0);
     } else if (x < DA + DB) {
-      if constexpr (BKM)
-        dma16(rb, lds_addr(bdst) + ((x - DA) * NW + wid) * 1024,
-              kill_sc ? kOob : b_off[x - DA], k0 * (uint32_t)p.ldb);
+      const int j = x - DA;
+      const bool dead = BKM ? kill_sc : kill;
+      uint32_t off;
+      if constexpr (kBSplit)
+        off = dead ? kOob : b_blk[j];
       else
-        dma16(rb, lds_addr(bdst) + ((x - DA) * NW + wid) * 1024, kill ? kOob : b_off[x - DA],
-              k0);
+        off = (dead ? kOob : b_off) + b_str[j];
+      dma16(rb, lds_addr(bdst) + (j * NW + wid) * 1024, off, BKM ? k0 * (uint32_t)p.ldb : k0);
     }
     else if (x == DA + DB)
-      dma4(srd_sa, base + kData + wid * 256, kill_sc ? kOob : sa_off, k0 >> 5);
+      dma4(srd_sa, base + kData + wid * 256, kill_sc ? kOob : sa_off, (k0 / kBK) * sa_gs);
     else
-      dma4(srd_sb, base + kData + 1024 + wid * 256, kill_sc ? kOob : sb_off, k0 >> 5);
+      dma4(srd_sb, base + kData + 1024 + wid * 256, kill_sc ? kOob : sb_off, (k0 / kBK) * sb_gs);
   };
   // Stages past this split's last step are filled with zeros (never read); the partial
   // last K step of the tensor masks lanes beyond K. (ls: the group's local step.)
@@ -609,7 +658,12 @@ gemm_kernel(GemmParams p) {
   auto stage_kill = [&](int ls) {
     return kstep(ls) >= nsteps || (gstep(ls) == ksteps - 1 && lane_ktail_dead);
   };
-  auto stage_ptr = [&](int ls) { return smem + kStageOff + (kg * NS + ls % NS) * kStage; };
+  auto stage_ptr = [&](int ls) {
+    if constexpr (kLateTab)  // the last step in slot 1
+      return smem + ((ls + niters) & 1) * kStage;
+    else
+      return smem + kStageOff + (kg * NS + ls % NS) * kStage;
+  };
   // the B tile of local step ls: the B part of a stage slot, or (XB) a B-only slot
   auto b_ptr = [&](int ls) {
     if constexpr (XB == 0) {
@@ -657,17 +711,22 @@ gemm_kernel(GemmParams p) {
   // MX scales of the current stage (per fragment: the row's four block scales, shifted
   // so that byte 2 kk holds block 2 kk + (lane >> 5)) and of the next one.
   uint32_t scA[MX ? FM : 1], scB[MX ? FN : 1], scA_n[MX ? FM : 1], scB_n[MX ? FN : 1];
+  // the scale dword of A fragment j / B fragment i of a stage, unshifted
+  auto read_sa = [&](const uint8_t* stage, int j) __attribute__((always_inline)) {
+    return *reinterpret_cast<const uint32_t*>(stage + kData +
+                                              (wave_m0 + j * 32 + (lane & 31)) * 4);
+  };
+  auto read_sb = [&](const uint8_t* stage, int i) __attribute__((always_inline)) {
+    return *reinterpret_cast<const uint32_t*>(stage + kData + 1024 + (brow[i] + (lane & 31)) * 4);
+  };
   auto read_scales = [&](const uint8_t* stage, uint32_t* sa_, uint32_t* sb_)
       __attribute__((always_inline)) {
     if constexpr (MX) {
-      const uint8_t* sc = stage + kData;
       const int sh = (lane >> 5) * 8;
 #pragma unroll
-      for (int j = 0; j < FM; ++j)
-        sa_[j] = *reinterpret_cast<const uint32_t*>(sc + (wave_m0 + j * 32 + (lane & 31)) * 4) >> sh;
+      for (int j = 0; j < FM; ++j) sa_[j] = read_sa(stage, j) >> (MX8 ? 0 : sh);
 #pragma unroll
-      for (int i = 0; i < FN; ++i)
-        sb_[i] = *reinterpret_cast<const uint32_t*>(sc + 1024 + (brow[i] + (lane & 31)) * 4) >> sh;
+      for (int i = 0; i < FN; ++i) sb_[i] = read_sb(stage, i) >> (MX8 ? 0 : sh);
     }
   };
   auto mma_one = [&](const Frags<NH>& f, int x, auto kk_tag) __attribute__((always_inline)) {
@@ -675,6 +734,12 @@ gemm_kernel(GemmParams p) {
     const int i = x / FM, j = x % FM;
     const int hb = i == 0 ? 0 : 2 * (FM + i);
     const int ha = 2 * (1 + j);
+    if constexpr (MX8 && kk == 0) {
+      // the step's scale dwords, read raw in the previous half-step: byte 2 kk becomes the
+      // lane half's own block
+      if (i == 0) scA[j] >>= (lane >> 5) * 8;
+      if (j == 0) scB[i] >>= (lane >> 5) * 8;
+    }
     if constexpr (MX)
       acc[i][j] = mfma_mx<FB, FA, 2 * kk>(join(f.h[hb], f.h[hb + 1]), join(f.h[ha], f.h[ha + 1]),
                                          acc[i][j], scB[i], scA[j]);
@@ -693,16 +758,20 @@ gemm_kernel(GemmParams p) {
   // mid-step wait drains every load instead (the next stage is then the last one issued,
   // or none: the trailing fragment reads of the final step go to a stale slot and are
   // never used). Prologue stages past the end are zero-filled.
-  if constexpr (EPI == EPI_GEGLU) {
-    // the fp32 gelu table (26 KB) into LDS ahead of the stage loads, so the prologue's wait
-    // for stage 0 also covers it; wave w copies KB w, w + NW, .., below 26
-    static_assert(kGeluA32Bytes == 26 * 1024, "gelu table copy assumes 26 KB");
-    const i32x4 rt = make_srd(kGeluA32, (uint32_t)kGeluA32Bytes);
-    const uint32_t tab = lds_addr(smem);
+  // the fp32 gelu table (26 KB) to LDS offset 0; wave w copies KB w, w + NW, .., below 26
+  auto load_table = [&]() {
+    if constexpr (EPI == EPI_GEGLU) {
+      static_assert(kGeluA32Bytes == 26 * 1024, "gelu table copy assumes 26 KB");
+      const i32x4 rt = make_srd(kGeluA32, (uint32_t)kGeluA32Bytes);
+      const uint32_t tab = lds_addr(smem);
 #pragma unroll
-    for (int c = 0; c < (26 + NW - 1) / NW; ++c)
-      if (wid + NW * c < 26) dma16(rt, tab + (wid + NW * c) * 1024, lane * 16, (wid + NW * c) * 1024);
-  }
+      for (int c = 0; c < (26 + NW - 1) / NW; ++c)
+        if (wid + NW * c < 26)
+          dma16(rt, tab + (wid + NW * c) * 1024, lane * 16, (wid + NW * c) * 1024);
+    }
+  };
+  // a resident table goes ahead of the stage loads, so the prologue's wait for stage 0 covers it
+  if constexpr (EPI == EPI_GEGLU && !kLateTab) load_table();
 #pragma unroll
   for (int ls = 0; ls < NS; ++ls) {
 #pragma unroll
@@ -731,8 +800,12 @@ gemm_kernel(GemmParams p) {
     __builtin_amdgcn_sched_barrier(0);
   }
   read_scales(stage_ptr(0), scA, scB);
-  auto step = [&](auto with_dma, int ls) __attribute__((always_inline)) {
+  // with_dma: the step issues the loads of step ls + NS. extra: what else its second half does
+  // (EXTRA_*). Compile-time, since a branch inside a step lets the compiler sink the first
+  // half's MFMAs past the mid-step barrier.
+  auto step = [&](auto with_dma, auto extra_tag, int ls) __attribute__((always_inline)) {
     constexpr bool kDma = decltype(with_dma)::value;
+    constexpr int extra = decltype(extra_tag)::value;
     uint8_t* cur = stage_ptr(ls);
     uint8_t* nxt = stage_ptr(ls + 1);
     uint8_t* curb = b_ptr(ls);
@@ -764,10 +837,16 @@ gemm_kernel(GemmParams p) {
     const uint32_t knb = (uint32_t)gstep(ls + NSB) * kBK;  // = kn without XB
     const bool killnb = stage_kill(ls + NSB);
     const bool killnb_end = kstep(ls + NSB) >= nsteps;
-    read_scales(nxt, scA_n, scB_n);
+    // step niters - 2 leaves slot 0 to the gelu table; the last step's mid-step wait covers it
+    if constexpr (extra == EXTRA_TABLE) load_table();
+    if constexpr (!MX8) read_scales(nxt, scA_n, scB_n);
 #pragma unroll
     for (int x = 0; x < NM; ++x) {
       mma_one(f1, x, std::integral_constant<int, 1>{});
+      if constexpr (MX8) {  // each scale register takes the next step's dword after its last use
+        if (x % FM == FM - 1) scB[x / FM] = read_sb(nxt, x / FM);
+        if (x / FM == FN - 1) scA[x % FM] = read_sa(nxt, x % FM);
+      }
 #pragma unroll
       for (int h = x * NH / NM; h < (x + 1) * NH / NM; ++h) read_one(f0, nxt, nxtb, 0, h);
       if constexpr (kDma) {
@@ -781,7 +860,7 @@ gemm_kernel(GemmParams p) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (MX) {
+    if constexpr (MX && !MX8) {
 #pragma unroll
       for (int j = 0; j < FM; ++j) scA[j] = scA_n[j];
 #pragma unroll
@@ -789,8 +868,17 @@ gemm_kernel(GemmParams p) {
     }
   };
   int ls = 0;
-  for (; ls < niters - NS; ++ls) step(std::true_type{}, ls);
-  for (; ls < niters; ++ls) step(std::false_type{}, ls);
+  const std::integral_constant<int, EXTRA_NONE> none{};
+  for (; ls < niters - NS; ++ls) step(std::true_type{}, none, ls);
+  if constexpr (kLateTab) {
+    if (niters >= 2)
+      step(std::false_type{}, std::integral_constant<int, EXTRA_TABLE>{}, ls++);
+    else
+      load_table();  // no earlier step to load it behind: slot 0 holds no step
+    step(std::false_type{}, none, ls);
+  } else {
+    for (; ls < niters; ++ls) step(std::false_type{}, none, ls);
+  }
   // Let every wave finish with the stages before the epilogue reuses the space.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -984,8 +1072,9 @@ gemm_kernel(GemmParams p) {
     using Runs = GegluRuns<FN, BN>;
     constexpr int RUNS = Runs::kRuns;
     constexpr int CH = RUNS;  // 16-byte chunks per staged H row (8 bf16 per run)
-    static_assert(NW * ROWS * CH * 16 <= NS * kStage, "per-wave staging fits the ring");
-    uint8_t* wbuf = smem + kStageOff + wid * (ROWS * CH * 16);
+    static_assert((kLateTab ? kGeluA32Bytes : 0) + NW * ROWS * CH * 16 <= NS * kStage,
+                  "per-wave staging fits the ring");
+    uint8_t* wbuf = smem + kGeluA32Bytes + wid * (ROWS * CH * 16);  // past the gelu table
     const int wave_h0 = n0 + wn * RUNS * 8;
     uint32_t hkeys = 0;  // packed max of the |H| bf16 keys staged by this lane
     uint32_t hmax = 0;   // the same as one fp32-bit amax key
@@ -1166,9 +1255,10 @@ int launch_typed(const GemmParams& p, int fa, int fb, hipStream_t s) {
 // two steps ahead).
 template <class T, int EPI, bool MX>
 struct FitTile {
+  static constexpr int kStageBytes = (T::BM + T::BN) * kBK + (MX ? kMxStageBytes : 0);
   static constexpr int bytes(int ns, int xb = 0) {
-    return (ns * ((T::BM + T::BN) * kBK + (MX ? 2048 : 0)) + xb * T::BN * kBK +
-            extra_lds<EPI>()) * T::OCC;
+    return (ns * kStageBytes + xb * T::BN * kBK +
+            extra_lds(EPI, late_table(EPI, ns, xb, T::KG, kStageBytes))) * T::OCC;
   }
   // 256 bytes stay free for the epilogue's block reductions
   static constexpr int kLimit = 160 * 1024 - 256;
@@ -1208,7 +1298,7 @@ int launch_gemm_tile(const GemmParams& p, int epi, int out_dtype, int fmt_a, int
   if (epi == EPI_GEGLU) {
     if constexpr (T::FN % 2 == 0) {
       if (mx) {
-        if constexpr (T::NW == 4) {
+        if constexpr (T::NW == 4 || (T::BM == 256 && T::BN == 256)) {
           using TG = typename FitTile<T, EPI_GEGLU, true>::type;
           hipLaunchKernelGGL((gemm_kernel<TG, 0, 0, EPI_GEGLU, BF8_OUT_BF16, true>), grid, block,
                              0, stream, p);
@@ -1248,8 +1338,8 @@ int launch_gemm_tile(const GemmParams& p, int epi, int out_dtype, int fmt_a, int
     }
   }
   if (mx) {
-    if constexpr (T::NW == 4) {
-      // MX block scales (e4m3 operands): each stage also holds 2 KB of scale dwords
+    if constexpr (T::NW == 4 || (T::BM == 256 && T::BN == 256)) {
+      // MX block scales (e4m3 operands) beside the stages
       using TM = typename FitTile<T, EPI_LINEAR, true>::type;
       if (out_dtype == BF8_OUT_BF16)
         hipLaunchKernelGGL((gemm_kernel<TM, 0, 0, EPI_LINEAR, BF8_OUT_BF16, true>), grid, block,

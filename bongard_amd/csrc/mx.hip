@@ -22,96 +22,8 @@ namespace bf8 {
 namespace {
 
 constexpr int kMxNT = 256;
-constexpr int kMxMaxRowBlocks = 8192;
 constexpr int kMT = 128;               // tile of the two-copy kernel (rows x cols)
 constexpr int kMaxMxTileBlocks = 2048;
-// Rowwise: a 16-lane group handles 128 consecutive elements of a row (4 blocks, 4 lanes
-// each, 8 elements per lane) and writes the dword of their 4 scale bytes. Grid-stride over
-// (row, 128-element group) pairs; groups past the row's last block write padding scales.
-// (Block blk of the nblk blocks that quantize x.)
-template <int FMT>
-__device__ __forceinline__ void mx_row_body(const uint16_t* __restrict__ x, int64_t rows,
-                                            int64_t cols, uint8_t* __restrict__ out,
-                                            uint8_t* __restrict__ sc, int64_t ld_sc,
-                                            int64_t blk, int64_t nblk) {
-  const int lane = threadIdx.x & 63;
-  const int sub = lane & 15;                 // lane within the 16-lane group
-  const int64_t groups_per_row = ld_sc / 4;  // dwords of scales per row
-  const int64_t ngroups = rows * groups_per_row;
-  const int64_t gstride = nblk * (kMxNT / 16);
-  for (int64_t g = blk * (kMxNT / 16) + (threadIdx.x >> 4); g < ngroups; g += gstride) {
-    const int64_t r = g / groups_per_row, cg = g % groups_per_row;
-    const int64_t c = cg * 128 + sub * 8;
-    const bool valid = c < cols;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (valid) v = *reinterpret_cast<const uint4*>(x + r * cols + c);
-    uint32_t m = absmax_key8(v);
-    m = max(m, (uint32_t)__shfl_xor((int)m, 1, 64));
-    m = max(m, (uint32_t)__shfl_xor((int)m, 2, 64));
-    const bool block_valid = valid;  // cols % 32 == 0: a block is valid iff its lanes are
-    const uint32_t e = block_valid ? mx_exponent<FMT>(m) : kMxPadScale;
-    if (valid) {
-      const float mult = mx_multiplier(e);
-      *reinterpret_cast<uint2*>(out + r * cols + c) = quant8_bf16<FMT>(v, mult);
-    }
-    // gather the 4 block exponents of the group (lanes 0, 4, 8, 12 of the group)
-    const int base = lane & ~15;
-    const uint32_t e0 = (uint32_t)__shfl((int)e, base + 0, 64);
-    const uint32_t e1 = (uint32_t)__shfl((int)e, base + 4, 64);
-    const uint32_t e2 = (uint32_t)__shfl((int)e, base + 8, 64);
-    const uint32_t e3 = (uint32_t)__shfl((int)e, base + 12, 64);
-    if (sub == 0)
-      *reinterpret_cast<uint32_t*>(sc + r * ld_sc + cg * 4) = e0 | (e1 << 8) | (e2 << 16) | (e3 << 24);
-  }
-}
-
-template <int FMT>
-__global__ __launch_bounds__(kMxNT) void mx_row_kernel(const uint16_t* __restrict__ x,
-                                                       int64_t rows, int64_t cols,
-                                                       uint8_t* __restrict__ out,
-                                                       uint8_t* __restrict__ sc, int64_t ld_sc) {
-  mx_row_body<FMT>(x, rows, cols, out, sc, ld_sc, blockIdx.x, gridDim.x);
-}
-
-// Rowwise MX quantization of up to kMxMany tensors in one launch: tensor t owns blocks
-// [first, first + blocks) and runs exactly the grid-stride loop mx_row_kernel runs for it
-// alone, so its bytes and scales are unchanged; the shared launch fills the chip when one
-// tensor would not and saves a launch per extra tensor.
-constexpr int kMxMany = 8;
-
-struct MxManySeg {
-  const uint16_t* x;
-  int64_t rows, cols;
-  uint8_t* out;
-  uint8_t* sc;
-  int64_t ld_sc;
-  int64_t first, blocks;
-  int fmt;
-};
-
-struct MxManyArgs {
-  MxManySeg seg[kMxMany];
-  int count;
-};
-
-__global__ __launch_bounds__(kMxNT) void mx_row_many_kernel(MxManyArgs a) {
-  int t = 0;
-  for (int k = 1; k < a.count; ++k)
-    if ((int64_t)blockIdx.x >= a.seg[k].first) t = k;
-  const MxManySeg& g = a.seg[t];
-  const int64_t blk = (int64_t)blockIdx.x - g.first;
-  if (g.fmt == BF8_E4M3)
-    mx_row_body<BF8_E4M3>(g.x, g.rows, g.cols, g.out, g.sc, g.ld_sc, blk, g.blocks);
-  else
-    mx_row_body<BF8_E5M2>(g.x, g.rows, g.cols, g.out, g.sc, g.ld_sc, blk, g.blocks);
-}
-
-int64_t mx_row_blocks(int64_t rows, int64_t ld_sc) {
-  const int64_t groups = rows * (ld_sc / 4);
-  return std::max<int64_t>(1, std::min<int64_t>((groups + kMxNT / 16 - 1) / (kMxNT / 16),
-                                                kMxMaxRowBlocks));
-}
-
 // Exponents (mx_exponent) of two packed |x| maxima given as finite bf16 keys: fp8_max is
 // 1.75 x 2^S, so amax / fp8_max rounds up to a power of two with exponent E - S where the
 // mantissa is at most 1.75 (96 / 128 above 1) and E - S + 1 past it, i.e. ((key + 31) >> 7) - S,
@@ -154,26 +66,32 @@ __device__ __forceinline__ uint2 mx_quant8_vs(uint4 v, const float* s) {
   return make_uint2(q[0], q[1]);
 }
 
-// Both copies of x in one pass (or the columnwise one alone). A block takes 128 x 128 tiles,
-// each wave 32 rows of all 128 columns: lane l holds columns 8 (l & 15) .. +7 of the rows
-// 4 k + l / 16, k < 8, so a row block of 32 is four neighbouring lanes (two DPP exchanges) and a
-// column block of 32 rows is the wave's eight pieces and the four lanes of a column group (two
-// lane exchanges of packed 16-bit maxima). The columnwise bytes meet in LDS; each wave then
-// turns 32 columns of all 128 rows. Every store instruction of either output writes whole
-// 128-byte lines, and every scale store a whole dword of four blocks.
+// Either or both copies of x in one pass. A block takes 128 x 128 tiles, each wave 32 rows of
+// all 128 columns: lane l holds columns 8 (l & 15) .. +7 of the rows 4 k + l / 16, k < 8, so a
+// row block of 32 is four neighbouring lanes (two DPP exchanges) and a column block of 32 rows is
+// the wave's eight pieces and the four lanes of a column group (two lane exchanges of packed
+// 16-bit maxima). The columnwise bytes meet in LDS; each wave then turns 32 columns of all 128
+// rows. Every store instruction of either output writes whole 128-byte lines, and a scale dword
+// holds the four blocks of 128 K-values: rows of bytes (sc) and / or planes, one dword per row
+// and group of 128 (the layout the GEMM loads in whole lines).
 // HBM-bound: 2 B read, 1 B (+ 1/32) written per element and copy; x is read once for the two
 // copies, where a rowwise and a columnwise pass read it twice. Both copies, inputs rotated past
 // the MALL: [4096, 20480] 133.1 us in two passes, 78.4 us in one (4.3 TB/s); [20480, 2560]
 // 72.9 -> 45.4 us (4.7 TB/s); one pass over 64 x 64 tiles per wave, whose stores are half
-// lines, 99.7 and 56.3 us.
+// lines, 99.7 and 56.3 us. With planes in place of the scale rows' scattered dwords 75.2 and
+// 43.0 us; the rowwise copy alone 45.9 and 29.8 us (5.5 TB/s).
 struct MxTile {
+  const uint16_t* x;
   int64_t rows, cols;
   uint8_t* out;
   uint8_t* sc;
+  uint32_t* planes;
   int64_t ld_sc;
   uint8_t* out_t;
   uint8_t* sc_t;
+  uint32_t* planes_t;
   int64_t ld_sc_t;
+  int fmt;
 };
 
 constexpr int kMPitch = kMT / 4 + 1;  // dwords per staged row (odd)
@@ -182,7 +100,7 @@ template <int FMT, bool FINITE>
 __device__ __forceinline__ void mx_tile_body(const MxTile& p, int64_t r0, int64_t c0,
                                              const uint4 (&v)[8], const uint32_t (&rk)[8],
                                              const uint32_t (&cm)[4], uint32_t* stage,
-                                             uint8_t* ecol, int wid, int lane) {
+                                             uint32_t* erow, uint8_t* ecol, int wid, int lane) {
   const int cl = lane & 15, lr = lane >> 4;
   const int64_t c = c0 + 8 * cl;
   const int64_t wr0 = r0 + 32 * wid;
@@ -204,9 +122,15 @@ __device__ __forceinline__ void mx_tile_body(const MxTile& p, int64_t r0, int64_
       // lanes 0, 4, 8, 12 of the 16 hold the four blocks: gather into lane 0
       e |= (uint32_t)__shfl_down((int)e, 4, 64) << 8;
       e |= (uint32_t)__shfl_down((int)e, 8, 64) << 16;
-      if (cl == 0 && r < p.rows)
-        *reinterpret_cast<uint32_t*>(p.sc + r * p.ld_sc + (c0 >> 5)) = e;
+      if (cl == 0) {
+        erow[32 * wid + 4 * k + lr] = e;
+        if (p.sc && r < p.rows)
+          *reinterpret_cast<uint32_t*>(p.sc + r * p.ld_sc + (c0 >> 5)) = e;
+      }
     }
+    // the wave's own 32 dwords as one line of the plane (a wave's LDS accesses are in order)
+    if (p.planes && lane < 32 && wr0 + lane < p.rows)
+      p.planes[(c0 >> 7) * p.rows + wr0 + lane] = erow[32 * wid + lane];
   }
   if (!p.out_t) return;
   float s[8];
@@ -237,16 +161,16 @@ __device__ __forceinline__ void mx_tile_body(const MxTile& p, int64_t r0, int64_
   }
 }
 
+// The tiles blk, blk + nblk, .. of p (every thread of the block calls it alike).
 template <int FMT>
-__global__ __launch_bounds__(kMxNT) void mx_tile_kernel(const uint16_t* __restrict__ x, MxTile p) {
-  __shared__ uint32_t stage[kMT * kMPitch];
-  __shared__ __attribute__((aligned(4))) uint8_t ecol[kMT * 4];  // [column][row block]
+__device__ __forceinline__ void mx_tiles(const MxTile& p, int64_t blk, int64_t nblk,
+                                         uint32_t* stage, uint32_t* erow, uint32_t* ecol) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int64_t tiles_c = (p.cols + kMT - 1) / kMT, tiles_r = (p.rows + kMT - 1) / kMT;
   const int64_t ntiles = tiles_c * tiles_r;
   const int cl = lane & 15, lr = lane >> 4;
-  const bool sc_dwords = ((uintptr_t)p.sc_t & 3) == 0;
-  for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+  const bool sct_dwords = ((uintptr_t)p.sc_t & 3) == 0;
+  for (int64_t t = blk; t < ntiles; t += nblk) {
     const int64_t r0 = (t / tiles_c) * kMT, c0 = (t % tiles_c) * kMT;
     const int64_t c = c0 + 8 * cl;
     uint4 v[8];
@@ -255,7 +179,7 @@ __global__ __launch_bounds__(kMxNT) void mx_tile_kernel(const uint16_t* __restri
       const int64_t r = r0 + 32 * wid + 4 * k + lr;
       v[k] = make_uint4(0u, 0u, 0u, 0u);
       if (r < p.rows && c < p.cols)
-        v[k] = *reinterpret_cast<const uint4*>(x + r * p.cols + c);
+        v[k] = *reinterpret_cast<const uint4*>(p.x + r * p.cols + c);
     }
     uint32_t rk[8], cm[4] = {};
     uint32_t top = 0;
@@ -271,44 +195,91 @@ __global__ __launch_bounds__(kMxNT) void mx_tile_kernel(const uint16_t* __restri
       rk[k] = max(m & 0xFFFFu, m >> 16);
       top = max(top, rk[k]);
     }
+    if (p.out_t) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 16, 64));
-      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 32, 64));
-    }
-    if (__builtin_expect(__any(top >= 0x7F80u), 0))
-      mx_tile_body<FMT, false>(p, r0, c0, v, rk, cm, stage, ecol, wid, lane);
-    else
-      mx_tile_body<FMT, true>(p, r0, c0, v, rk, cm, stage, ecol, wid, lane);
-    __syncthreads();
-    // lane: 16 rows (lane & 7) x 4 columns (lane >> 3) of the wave's 32 columns
-    const int rg = (lane & 7) * 16, cg = 8 * wid + (lane >> 3);
-    uint32_t d[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) d[i] = stage[(rg + i) * kMPitch + cg];
-    uint4 tq[4];
-    transpose_4x16(d, tq);
-    const int64_t tc = r0 + rg;  // column of out_t (a row of x)
-    if (tc < p.rows) {
-#pragma unroll
-      for (int cc = 0; cc < 4; ++cc) {
-        const int64_t tr = c0 + 4 * cg + cc;  // row of out_t (a column of x)
-        if (tr < p.cols) *reinterpret_cast<uint4*>(p.out_t + tr * p.rows + tc) = tq[cc];
+      for (int i = 0; i < 4; ++i) {
+        cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 16, 64));
+        cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 32, 64));
       }
     }
-    if (threadIdx.x < kMT && c0 + threadIdx.x < p.cols) {
-      // four blocks of one column; the last tile row's absent blocks pad the scale row
-      const uint32_t e4 = *reinterpret_cast<const uint32_t*>(ecol + 4 * threadIdx.x);
-      uint8_t* dst = p.sc_t + (c0 + threadIdx.x) * p.ld_sc_t + (r0 >> 5);
-      if (sc_dwords) {
-        *reinterpret_cast<uint32_t*>(dst) = e4;
-      } else {
+    uint8_t* ecolb = reinterpret_cast<uint8_t*>(ecol);
+    if (__builtin_expect(__any(top >= 0x7F80u), 0))
+      mx_tile_body<FMT, false>(p, r0, c0, v, rk, cm, stage, erow, ecolb, wid, lane);
+    else
+      mx_tile_body<FMT, true>(p, r0, c0, v, rk, cm, stage, erow, ecolb, wid, lane);
+    if (!p.out_t) continue;
+    __syncthreads();
+    {
+      // lane: 16 rows (lane & 7) x 4 columns (lane >> 3) of the wave's 32 columns
+      const int rg = (lane & 7) * 16, cg = 8 * wid + (lane >> 3);
+      uint32_t d[16];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) dst[b] = (uint8_t)(e4 >> (8 * b));
+      for (int i = 0; i < 16; ++i) d[i] = stage[(rg + i) * kMPitch + cg];
+      uint4 tq[4];
+      transpose_4x16(d, tq);
+      const int64_t tc = r0 + rg;  // column of out_t (a row of x)
+      if (tc < p.rows) {
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {
+          const int64_t tr = c0 + 4 * cg + cc;  // row of out_t (a column of x)
+          if (tr < p.cols) *reinterpret_cast<uint4*>(p.out_t + tr * p.rows + tc) = tq[cc];
+        }
+      }
+      if (threadIdx.x < kMT && c0 + threadIdx.x < p.cols) {
+        // four blocks of one column; the last tile row's absent blocks pad the last dword
+        const uint32_t e4 = ecol[threadIdx.x];
+        if (p.planes_t) p.planes_t[(r0 >> 7) * p.cols + c0 + threadIdx.x] = e4;
+        if (p.sc_t) {
+          uint8_t* dst = p.sc_t + (c0 + threadIdx.x) * p.ld_sc_t + (r0 >> 5);
+          if (sct_dwords) {
+            *reinterpret_cast<uint32_t*>(dst) = e4;
+          } else {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) dst[b] = (uint8_t)(e4 >> (8 * b));
+          }
+        }
       }
     }
     __syncthreads();
   }
+}
+
+// Up to kMxMany tensors in one launch: tensor t owns blocks [first, next tensor's first), so
+// that a forward's small tensors fill the chip together and save launches.
+constexpr int kMxMany = 8;
+
+struct MxManyArgs {
+  MxTile t[kMxMany];
+  int64_t first[kMxMany + 1];
+  int count;
+};
+
+__global__ __launch_bounds__(kMxNT) void mx_tile_kernel(MxManyArgs a) {
+  __shared__ uint32_t stage[kMT * kMPitch];
+  __shared__ uint32_t erow[kMT], ecol[kMT];  // scale dwords of the tile's rows and columns
+  int i = 0;
+  for (int k = 1; k < a.count; ++k)
+    if ((int64_t)blockIdx.x >= a.first[k]) i = k;
+  const int64_t blk = (int64_t)blockIdx.x - a.first[i], nblk = a.first[i + 1] - a.first[i];
+  if (a.t[i].fmt == BF8_E4M3)
+    mx_tiles<BF8_E4M3>(a.t[i], blk, nblk, stage, erow, ecol);
+  else
+    mx_tiles<BF8_E5M2>(a.t[i], blk, nblk, stage, erow, ecol);
+}
+
+// Adds a tensor to a launch.
+void mx_add(MxManyArgs& a, const MxTile& t) {
+  const int64_t tiles = ((t.rows + kMT - 1) / kMT) * ((t.cols + kMT - 1) / kMT);
+  a.t[a.count] = t;
+  a.first[a.count + 1] = a.first[a.count] + std::min<int64_t>(tiles, kMaxMxTileBlocks);
+  ++a.count;
+}
+
+int mx_launch(const MxManyArgs& a, void* stream) {
+  if (a.count == 0) return BF8_OK;
+  hipLaunchKernelGGL(mx_tile_kernel, dim3((unsigned)a.first[a.count]), dim3(kMxNT), 0,
+                     as_stream(stream), a);
+  return launch_status("mx_tile_kernel");
 }
 
 }  // namespace
@@ -318,95 +289,71 @@ using namespace bf8;
 
 extern "C" {
 
+int bf8_quantize_mx_planes_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
+                                uint8_t* out_scales, uint32_t* out_planes, uint8_t* out_t,
+                                uint8_t* out_t_scales, uint32_t* out_t_planes, void* stream) {
+  const char* who = "bf8_quantize_mx_bf16";
+  BF8_CHECK(fmt == BF8_E4M3 || fmt == BF8_E5M2, "%s: bad fmt %d", who, fmt);
+  BF8_CHECK(rows >= 0 && cols >= 0, "%s: negative shape", who);
+  BF8_CHECK((out == nullptr) == (!out_scales && !out_planes) &&
+                (out_t == nullptr) == (!out_t_scales && !out_t_planes) && (out || out_t),
+            "%s: give out with out_scales and/or out_t with out_t_scales", who);
+  BF8_CHECK(!out || cols % 32 == 0, "%s: rowwise blocks need cols %% 32 == 0 (got %lld)", who,
+            (long long)cols);
+  BF8_CHECK(!out_t || (rows % 32 == 0 && cols % 16 == 0),
+            "%s: columnwise blocks need rows %% 32 == 0 and cols %% 16 == 0 (got %lld x %lld)", who,
+            (long long)rows, (long long)cols);
+  if (rows == 0 || cols == 0) return BF8_OK;
+  BF8_CHECK(x != nullptr, "%s: x is NULL", who);
+  BF8_CHECK(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 7) == 0 && ((uintptr_t)out_t & 15) == 0 &&
+                (((uintptr_t)out_scales | (uintptr_t)out_planes | (uintptr_t)out_t_planes) & 3) == 0,
+            "%s: x, out_t 16-byte, out 8-byte, out_scales and planes 4-byte aligned", who);
+  MxManyArgs a{};
+  mx_add(a, MxTile{(const uint16_t*)x, rows, cols, out, out_scales, out_planes,
+                   out ? bf8_mx_scale_ld(cols) : 0, out_t, out_t_scales, out_t_planes,
+                   bf8_mx_scale_ld(rows), fmt});
+  return mx_launch(a, stream);
+}
+
 int bf8_quantize_mx_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
                          uint8_t* out_scales, uint8_t* out_t, uint8_t* out_t_scales,
                          void* stream) {
-  BF8_CHECK(fmt == BF8_E4M3 || fmt == BF8_E5M2, "bf8_quantize_mx_bf16: bad fmt %d", fmt);
-  BF8_CHECK(rows >= 0 && cols >= 0, "bf8_quantize_mx_bf16: negative shape");
-  BF8_CHECK((out == nullptr) == (out_scales == nullptr) &&
-                (out_t == nullptr) == (out_t_scales == nullptr) && (out || out_t),
-            "bf8_quantize_mx_bf16: give out with out_scales and/or out_t with out_t_scales");
-  BF8_CHECK(!out || cols % 32 == 0,
-            "bf8_quantize_mx_bf16: rowwise blocks need cols %% 32 == 0 (got %lld)", (long long)cols);
-  BF8_CHECK(!out_t || (rows % 32 == 0 && cols % 16 == 0),
-            "bf8_quantize_mx_bf16: columnwise blocks need rows %% 32 == 0 and cols %% 16 == 0 "
-            "(got %lld x %lld)", (long long)rows, (long long)cols);
-  if (rows == 0 || cols == 0) return BF8_OK;
-  BF8_CHECK(x != nullptr, "bf8_quantize_mx_bf16: x is NULL");
-  BF8_CHECK(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 7) == 0 && ((uintptr_t)out_t & 15) == 0 &&
-                ((uintptr_t)out_scales & 3) == 0,
-            "bf8_quantize_mx_bf16: x, out_t 16-byte, out 8-byte, out_scales 4-byte aligned");
-  hipStream_t s = as_stream(stream);
-  const uint16_t* xs = (const uint16_t*)x;
-  if (!out_t) {
-    const int64_t ld = bf8_mx_scale_ld(cols);
-    const unsigned grid = (unsigned)mx_row_blocks(rows, ld);
-    if (fmt == BF8_E4M3)
-      hipLaunchKernelGGL(mx_row_kernel<BF8_E4M3>, dim3(grid), dim3(kMxNT), 0, s, xs, rows, cols,
-                         out, out_scales, ld);
-    else
-      hipLaunchKernelGGL(mx_row_kernel<BF8_E5M2>, dim3(grid), dim3(kMxNT), 0, s, xs, rows, cols,
-                         out, out_scales, ld);
-    return launch_status("mx_row_kernel");
+  return bf8_quantize_mx_planes_bf16(x, rows, cols, fmt, out, out_scales, nullptr, out_t,
+                                     out_t_scales, nullptr, stream);
+}
+
+int bf8_quantize_mx_many_planes_bf16(int count, const void* const* x, const int64_t* rows,
+                                     const int64_t* cols, const int* fmt, uint8_t* const* out,
+                                     uint8_t* const* out_scales, uint32_t* const* out_planes,
+                                     void* stream) {
+  const char* who = "bf8_quantize_mx_many_bf16";
+  BF8_CHECK(count >= 1 && count <= kMxMany, "%s: count %d outside [1, %d]", who, count, kMxMany);
+  BF8_CHECK(x && rows && cols && fmt && out && out_scales, "%s: NULL array", who);
+  MxManyArgs a{};
+  for (int t = 0; t < count; ++t) {
+    BF8_CHECK(fmt[t] == BF8_E4M3 || fmt[t] == BF8_E5M2, "%s: tensor %d: bad fmt %d", who, t, fmt[t]);
+    BF8_CHECK(rows[t] >= 0 && cols[t] >= 0, "%s: tensor %d: negative shape", who, t);
+    BF8_CHECK(cols[t] % 32 == 0,
+              "%s: tensor %d: rowwise blocks need cols %% 32 == 0 (got %lld)", who, t,
+              (long long)cols[t]);
+    if (rows[t] == 0 || cols[t] == 0) continue;
+    uint32_t* planes = out_planes ? out_planes[t] : nullptr;
+    BF8_CHECK(x[t] && out[t] && (out_scales[t] || planes),
+              "%s: tensor %d: x, out or out_scales is NULL", who, t);
+    BF8_CHECK(((uintptr_t)x[t] & 15) == 0 && ((uintptr_t)out[t] & 7) == 0 &&
+                  (((uintptr_t)out_scales[t] | (uintptr_t)planes) & 3) == 0,
+              "%s: tensor %d: x 16-byte, out 8-byte, out_scales 4-byte aligned", who, t);
+    mx_add(a, MxTile{(const uint16_t*)x[t], rows[t], cols[t], out[t], out_scales[t], planes,
+                     bf8_mx_scale_ld(cols[t]), nullptr, nullptr, nullptr, 0, fmt[t]});
   }
-  MxTile p{};
-  p.rows = rows;
-  p.cols = cols;
-  p.out = out;
-  p.sc = out_scales;
-  p.ld_sc = out ? bf8_mx_scale_ld(cols) : 0;
-  p.out_t = out_t;
-  p.sc_t = out_t_scales;
-  p.ld_sc_t = bf8_mx_scale_ld(rows);
-  const int64_t tiles = ((rows + kMT - 1) / kMT) * ((cols + kMT - 1) / kMT);
-  const unsigned grid = (unsigned)std::min<int64_t>(tiles, kMaxMxTileBlocks);
-  if (fmt == BF8_E4M3)
-    hipLaunchKernelGGL(mx_tile_kernel<BF8_E4M3>, dim3(grid), dim3(kMxNT), 0, s, xs, p);
-  else
-    hipLaunchKernelGGL(mx_tile_kernel<BF8_E5M2>, dim3(grid), dim3(kMxNT), 0, s, xs, p);
-  return launch_status("mx_tile_kernel");
+  return mx_launch(a, stream);
 }
 
 int bf8_quantize_mx_many_bf16(int count, const void* const* x, const int64_t* rows,
                               const int64_t* cols, const int* fmt, uint8_t* const* out,
                               uint8_t* const* out_scales, void* stream) {
-  BF8_CHECK(count >= 1 && count <= kMxMany,
-            "bf8_quantize_mx_many_bf16: count %d outside [1, %d]", count, kMxMany);
-  BF8_CHECK(x && rows && cols && fmt && out && out_scales,
-            "bf8_quantize_mx_many_bf16: NULL array");
-  MxManyArgs a{};
-  int64_t total = 0;
-  for (int t = 0; t < count; ++t) {
-    BF8_CHECK(fmt[t] == BF8_E4M3 || fmt[t] == BF8_E5M2,
-              "bf8_quantize_mx_many_bf16: tensor %d: bad fmt %d", t, fmt[t]);
-    BF8_CHECK(rows[t] >= 0 && cols[t] >= 0, "bf8_quantize_mx_many_bf16: tensor %d: negative shape",
-              t);
-    BF8_CHECK(cols[t] % 32 == 0,
-              "bf8_quantize_mx_many_bf16: tensor %d: rowwise blocks need cols %% 32 == 0 (got %lld)",
-              t, (long long)cols[t]);
-    if (rows[t] == 0 || cols[t] == 0) continue;
-    BF8_CHECK(x[t] && out[t] && out_scales[t],
-              "bf8_quantize_mx_many_bf16: tensor %d: x, out or out_scales is NULL", t);
-    BF8_CHECK(((uintptr_t)x[t] & 15) == 0 && ((uintptr_t)out[t] & 7) == 0 &&
-                  ((uintptr_t)out_scales[t] & 3) == 0,
-              "bf8_quantize_mx_many_bf16: tensor %d: x 16-byte, out 8-byte, out_scales 4-byte "
-              "aligned", t);
-    MxManySeg& g = a.seg[a.count++];
-    g.x = (const uint16_t*)x[t];
-    g.rows = rows[t];
-    g.cols = cols[t];
-    g.out = out[t];
-    g.sc = out_scales[t];
-    g.ld_sc = bf8_mx_scale_ld(cols[t]);
-    g.first = total;
-    g.blocks = mx_row_blocks(rows[t], g.ld_sc);
-    g.fmt = fmt[t];
-    total += g.blocks;
-  }
-  if (a.count == 0) return BF8_OK;
-  hipLaunchKernelGGL(mx_row_many_kernel, dim3((unsigned)total), dim3(kMxNT), 0,
-                     as_stream(stream), a);
-  return launch_status("mx_row_many_kernel");
+  return bf8_quantize_mx_many_planes_bf16(count, x, rows, cols, fmt, out, out_scales, nullptr,
+                                          stream);
 }
 
 }  // extern "C"

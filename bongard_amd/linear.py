@@ -372,7 +372,8 @@ class GegluGateUpNvfp4Function(_Fp8Function):
 def quantize_weight_mx(weight, *, transpose=True):
     """MXFP8 copy of a weight [N, K]: blocks along K (forward), and with ``transpose`` the
     [K, N] copy with blocks along N (the input-gradient GEMM's operand)."""
-    return ops.quantize_mx(weight.detach(), E4M3, rowwise=True, colwise=transpose)
+    return ops.quantize_mx(weight.detach(), E4M3, rowwise=True, colwise=transpose,
+                           scale_rows=False)
 
 
 class Fp8LinearMxFunction(_Fp8Function):
@@ -390,26 +391,27 @@ class Fp8LinearMxFunction(_Fp8Function):
     def forward(ctx, x, weight, wq):
         need_dx, need_dw = _forward_needs(ctx, 2)
         if wq is None and not (need_dx or need_dw):
-            xq, wq = ops.quantize_mx_many([x, weight.detach()])   # inference: one launch
+            xq, wq = ops.quantize_mx_many([x, weight.detach()], scale_rows=False)  # one launch
         else:
-            xq = ops.quantize_mx(x, E4M3, rowwise=True, colwise=need_dw)
+            xq = ops.quantize_mx(x, E4M3, rowwise=True, colwise=need_dw, scale_rows=False)
         if wq is None:
             wq = quantize_weight_mx(weight, transpose=need_dx)
-        y = ops.gemm_mx(xq.data, xq.scales, wq.data, wq.scales)
-        ctx.save_for_backward(xq.data_t, xq.scales_t, wq.data_t if need_dx else None,
-                              wq.scales_t if need_dx else None)
+        y = ops.gemm_mx(xq.data, None, wq.data, None, a_planes=xq.planes, b_planes=wq.planes)
+        ctx.save_for_backward(xq.data_t, xq.planes_t, wq.data_t if need_dx else None,
+                              wq.planes_t if need_dx else None)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x8t, xst, w8t, wst = ctx.saved_tensors
+        x8t, xpt, w8t, wpt = ctx.saved_tensors
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        dyq = ops.quantize_mx(dy.contiguous(), E4M3, rowwise=need_dx, colwise=need_dw)
+        dyq = ops.quantize_mx(dy.contiguous(), E4M3, rowwise=need_dx, colwise=need_dw,
+                              scale_rows=False)
         dx = dw = None
         if need_dx:
-            dx = ops.gemm_mx(dyq.data, dyq.scales, w8t, wst)
+            dx = ops.gemm_mx(dyq.data, None, w8t, None, a_planes=dyq.planes, b_planes=wpt)
         if need_dw:
-            dw = ops.gemm_mx(dyq.data_t, dyq.scales_t, x8t, xst)
+            dw = ops.gemm_mx(dyq.data_t, None, x8t, None, a_planes=dyq.planes_t, b_planes=xpt)
         return dx, dw, None
 
 
@@ -429,45 +431,48 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
         if not train and (gu_q is None or down_q is None):
             # inference: x and the uncached weights in one rowwise launch
             ws = [w for w, q in ((w_gu, gu_q), (w_down, down_q)) if q is None]
-            qs = ops.quantize_mx_many([x] + [w.detach() for w in ws])
+            qs = ops.quantize_mx_many([x] + [w.detach() for w in ws], scale_rows=False)
             xq = qs[0]
             if gu_q is None:
                 gu_q = qs[1]
             if down_q is None:
                 down_q = qs[-1]
         else:
-            xq = ops.quantize_mx(x, E4M3, rowwise=True, colwise=need_dgu)
+            xq = ops.quantize_mx(x, E4M3, rowwise=True, colwise=need_dgu, scale_rows=False)
         if gu_q is None:
             gu_q = quantize_weight_mx(w_gu, transpose=need_dx)
         # H is quantized (rowwise, plus the columnwise copy for the down wgrad) in the
         # GEMM's epilogue; the bf16 H itself is never written
-        hq, GU, _ = ops.gemm_geglu_mx_quant(xq.data, xq.scales, gu_q.data, gu_q.scales, I,
-                                            colwise=need_dd, keep_gu=train)
+        hq, GU = ops.gemm_geglu_mx_planes(xq.data, xq.planes, gu_q.data, gu_q.planes, I,
+                                          colwise=need_dd, keep_gu=train)
         if down_q is None:
             down_q = quantize_weight_mx(w_down, transpose=need_dx or need_dgu)
-        y = ops.gemm_mx(hq.data, hq.scales, down_q.data, down_q.scales)
+        y = ops.gemm_mx(hq.data, None, down_q.data, None, a_planes=hq.planes,
+                        b_planes=down_q.planes)
         ctx.intermediate = I
-        ctx.save_for_backward(GU, xq.data_t, xq.scales_t, hq.data_t, hq.scales_t, gu_q.data_t,
-                              gu_q.scales_t, down_q.data_t, down_q.scales_t)
+        ctx.save_for_backward(GU, xq.data_t, xq.planes_t, hq.data_t, hq.planes_t, gu_q.data_t,
+                              gu_q.planes_t, down_q.data_t, down_q.planes_t)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        GU, x8t, xst, h8t, hst, gu8t, gust, d8t, dst = ctx.saved_tensors
+        GU, x8t, xpt, h8t, hpt, gu8t, gupt, d8t, dpt = ctx.saved_tensors
         need_dx, need_dgu, need_dd = ctx.needs_input_grad[:3]
         dyq = ops.quantize_mx(dy.contiguous(), E4M3, rowwise=need_dx or need_dgu,
-                              colwise=need_dd)
+                              colwise=need_dd, scale_rows=False)
         dx = dgu = dd = None
         if need_dd:
-            dd = ops.gemm_mx(dyq.data_t, dyq.scales_t, h8t, hst)
+            dd = ops.gemm_mx(dyq.data_t, None, h8t, None, a_planes=dyq.planes_t, b_planes=hpt)
         if need_dx or need_dgu:
-            dH = ops.gemm_mx(dyq.data, dyq.scales, d8t, dst)
+            dH = ops.gemm_mx(dyq.data, None, d8t, None, a_planes=dyq.planes, b_planes=dpt)
             dGU, _ = ops.geglu_bwd(dH, GU)
-            dq = ops.quantize_mx(dGU, E4M3, rowwise=need_dx, colwise=need_dgu)
+            dq = ops.quantize_mx(dGU, E4M3, rowwise=need_dx, colwise=need_dgu,
+                                 scale_rows=False)
             if need_dx:
-                dx = ops.gemm_mx(dq.data, dq.scales, gu8t, gust)
+                dx = ops.gemm_mx(dq.data, None, gu8t, None, a_planes=dq.planes, b_planes=gupt)
             if need_dgu:
-                dgu = ops.gemm_mx(dq.data_t, dq.scales_t, x8t, xst)
+                dgu = ops.gemm_mx(dq.data_t, None, x8t, None, a_planes=dq.planes_t,
+                                  b_planes=xpt)
         return dx, dgu, dd, None, None, None
 
 

@@ -497,7 +497,9 @@ class MxFp8Tensor:
     """An MXFP8 tensor of x [rows, cols] (32-element blocks, one E8M0 byte each):
     ``data`` [rows, cols] with ``scales`` [rows, mx_scale_ld(cols)] (blocks along rows)
     and/or ``data_t`` [cols, rows] with ``scales_t`` [cols, mx_scale_ld(rows)] (blocks along
-    columns of x, stored transposed)."""
+    columns of x, stored transposed). ``planes`` int32 [ceil(cols / 128), rows] and
+    ``planes_t`` [ceil(rows / 128), cols] hold the same scales as one plane of dwords per 128
+    K-values, which the GEMMs load in whole lines (``gemm_mx(..., a_planes=, b_planes=)``)."""
 
     data: Optional[torch.Tensor]
     scales: Optional[torch.Tensor]
@@ -506,34 +508,55 @@ class MxFp8Tensor:
     fmt: int
     rows: int
     cols: int
+    planes: Optional[torch.Tensor] = None
+    planes_t: Optional[torch.Tensor] = None
 
 
 def mx_scale_ld(K):
-    return int(_lib.lib().bf8_mx_scale_ld(int(K)))
+    return (int(K) + 127) // 128 * 4
 
 
-def quantize_mx(x, fmt=E4M3, *, rowwise=True, colwise=False):
-    """MXFP8 quantization of a bf16 tensor (TE MXFP8BlockScaling arithmetic)."""
+def _new_planes(K, rows, device):
+    """Scale planes of an operand [rows, K]."""
+    return torch.empty(((K + 127) // 128, rows), dtype=torch.int32, device=device)
+
+
+def _mx_planes(who, rows, K, **planes):
+    for name, t in planes.items():
+        if t.dtype != torch.int32 or tuple(t.shape) != ((K + 127) // 128, rows[name]) \
+                or not t.is_contiguous():
+            raise ValueError(f"{who}: {name} must be contiguous int32 "
+                             f"[{(K + 127) // 128}, {rows[name]}] (got {t.dtype} {tuple(t.shape)})")
+
+
+def quantize_mx(x, fmt=E4M3, *, rowwise=True, colwise=False, scale_rows=True):
+    """MXFP8 quantization of a bf16 tensor (TE MXFP8BlockScaling arithmetic). ``scale_rows``
+    False: the scales as planes only (``scales`` and ``scales_t`` None), for a tensor that
+    only feeds the GEMMs."""
     _require_gpu(x)
     x = _bf16_2d(x)
     rows, cols = x.shape
     dev = x.device
     if not (rowwise or colwise):
         raise ValueError("quantize_mx: nothing requested")
-    out = sc = out_t = sc_t = None
+    out = sc = pl = out_t = sc_t = pl_t = None
     if rowwise:
         out = torch.empty((rows, cols), dtype=TORCH_FP8[fmt], device=dev)
-        sc = torch.empty((rows, mx_scale_ld(cols)), dtype=torch.uint8, device=dev)
+        if scale_rows:
+            sc = torch.empty((rows, mx_scale_ld(cols)), dtype=torch.uint8, device=dev)
+        pl = _new_planes(cols, rows, dev)
     if colwise:
         out_t = torch.empty((cols, rows), dtype=TORCH_FP8[fmt], device=dev)
-        sc_t = torch.empty((cols, mx_scale_ld(rows)), dtype=torch.uint8, device=dev)
-    _lib.check(_lib.lib().bf8_quantize_mx_bf16(_ptr(x), rows, cols, fmt, _ptr(out), _ptr(sc),
-                                               _ptr(out_t), _ptr(sc_t), _stream(dev)),
-               "bf8_quantize_mx_bf16")
-    return MxFp8Tensor(out, sc, out_t, sc_t, fmt, rows, cols)
+        if scale_rows:
+            sc_t = torch.empty((cols, mx_scale_ld(rows)), dtype=torch.uint8, device=dev)
+        pl_t = _new_planes(rows, cols, dev)
+    _lib.check(_lib.lib().bf8_quantize_mx_planes_bf16(
+        _ptr(x), rows, cols, fmt, _ptr(out), _ptr(sc), _ptr(pl), _ptr(out_t), _ptr(sc_t),
+        _ptr(pl_t), _stream(dev)), "bf8_quantize_mx_planes_bf16")
+    return MxFp8Tensor(out, sc, out_t, sc_t, fmt, rows, cols, pl, pl_t)
 
 
-def quantize_mx_many(xs, fmts=None):
+def quantize_mx_many(xs, fmts=None, *, scale_rows=True):
     """Rowwise :func:`quantize_mx` of up to 8 bf16 tensors in one launch; each result
     equals that tensor's own ``quantize_mx(x, fmt)`` (bytes and scales). ``fmts``: one
     format for all or one per tensor (default e4m3)."""
@@ -551,23 +574,37 @@ def quantize_mx_many(xs, fmts=None):
         raise ValueError("quantize_mx_many: one format per tensor")
     outs = [torch.empty(x.shape, dtype=TORCH_FP8[f], device=dev) for x, f in zip(xs, fmts)]
     scs = [torch.empty((x.shape[0], mx_scale_ld(x.shape[1])), dtype=torch.uint8, device=dev)
-           for x in xs]
-    _lib.check(_lib.lib().bf8_quantize_mx_many_bf16(
+           if scale_rows else None for x in xs]
+    pls = [_new_planes(x.shape[1], x.shape[0], dev) for x in xs]
+    _lib.check(_lib.lib().bf8_quantize_mx_many_planes_bf16(
         count, (ctypes.c_void_p * count)(*[x.data_ptr() for x in xs]),
         (ctypes.c_int64 * count)(*[x.shape[0] for x in xs]),
         (ctypes.c_int64 * count)(*[x.shape[1] for x in xs]), (ctypes.c_int * count)(*fmts),
         (ctypes.c_void_p * count)(*[o.data_ptr() for o in outs]),
-        (ctypes.c_void_p * count)(*[c.data_ptr() for c in scs]), _stream(dev)),
-        "bf8_quantize_mx_many_bf16")
-    return [MxFp8Tensor(o, c, None, None, f, x.shape[0], x.shape[1])
-            for x, o, c, f in zip(xs, outs, scs, fmts)]
+        (ctypes.c_void_p * count)(*[_ptr(c) for c in scs]),
+        (ctypes.c_void_p * count)(*[c.data_ptr() for c in pls]), _stream(dev)),
+        "bf8_quantize_mx_many_planes_bf16")
+    return [MxFp8Tensor(o, c, None, None, f, x.shape[0], x.shape[1], pl)
+            for x, o, c, f, pl in zip(xs, outs, scs, fmts, pls)]
 
 
-def gemm_mx(a, a_scales, b, b_scales, *, out_dtype=torch.bfloat16, bias=None, out=None):
+@functools.lru_cache(maxsize=4096)
+def _gemm_mx_ws_cached(M, N, K, override):
+    return int(_lib.lib().bf8_gemm_mx_workspace(M, N, K))
+
+
+def gemm_mx(a, a_scales, b, b_scales, *, out_dtype=torch.bfloat16, bias=None, out=None,
+            a_planes=None, b_planes=None):
     """``C = a @ b.T`` on MXFP8 (e4m3) operands a [M, K], b [N, K] with their E8M0 block
-    scales [M, >= mx_scale_ld(K)], [N, ...]."""
-    _require_gpu(a, b, a_scales, b_scales)
-    _byte_matrix("gemm_mx", a=a, b=b, a_scales=a_scales, b_scales=b_scales)
+    scales [M, >= mx_scale_ld(K)], [N, ...], or with both operands' scale planes (the scale
+    rows are then not read and may be None; the same result, faster)."""
+    by_planes = a_planes is not None and b_planes is not None
+    if by_planes:
+        _require_gpu(a, b, a_planes, b_planes)
+        _byte_matrix("gemm_mx", a=a, b=b)
+    else:
+        _require_gpu(a, b, a_scales, b_scales)
+        _byte_matrix("gemm_mx", a=a, b=b, a_scales=a_scales, b_scales=b_scales)
     M, K = a.shape
     N, Kb = b.shape
     if K != Kb:
@@ -582,9 +619,17 @@ def gemm_mx(a, a_scales, b, b_scales, *, out_dtype=torch.bfloat16, bias=None, ou
             raise TypeError("gemm_mx: bias must be bfloat16")
         bias = bias.contiguous()
     L = _lib.lib()
-    ws_bytes = int(L.bf8_gemm_mx_workspace(M, N, K))
+    ws_bytes = _gemm_mx_ws_cached(M, N, K, _tile_override())
     ws = gemm_workspace(ws_bytes, a.device) if ws_bytes else None
     ws_bytes = ws.numel() if ws is not None else 0
+    if by_planes:
+        _mx_planes("gemm_mx", {"a_planes": M, "b_planes": N}, K, a_planes=a_planes,
+                   b_planes=b_planes)
+        _lib.check(L.bf8_gemm_mx_planes(
+            _ptr(a), a.stride(0), _ptr(a_planes), _ptr(b), b.stride(0), _ptr(b_planes), M, N, K,
+            _ptr(bias), _ptr(out), OUT_BF16 if out_dtype == torch.bfloat16 else OUT_F32,
+            out.stride(0), _ptr(ws), ws_bytes, _stream(a.device)), "bf8_gemm_mx_planes")
+        return out
     _lib.check(L.bf8_gemm_mx(_ptr(a), a.stride(0), _ptr(a_scales), a_scales.stride(0), _ptr(b),
                              b.stride(0), _ptr(b_scales), b_scales.stride(0), M, N, K, _ptr(bias),
                              _ptr(out), OUT_BF16 if out_dtype == torch.bfloat16 else OUT_F32,
@@ -639,6 +684,33 @@ def gemm_geglu_mx_quant(x8, x_scales, w8, w_scales, intermediate, *, colwise=Fal
         h8_sc.stride(0), _ptr(h8t), _ptr(h8t_sc), h8t_sc.stride(0) if colwise else 0, _ptr(GU),
         _stream(dev)), "bf8_gemm_geglu_mx_quant")
     return MxFp8Tensor(h8, h8_sc, h8t, h8t_sc, E4M3, M, I), GU, H
+
+
+def gemm_geglu_mx_planes(x8, x_planes, w8, w_planes, intermediate, *, colwise=False,
+                         keep_gu=False):
+    """:func:`gemm_geglu_mx_quant` on scale planes, H's scales written as planes: ``(hq, GU
+    or None)``, ``hq`` an :class:`MxFp8Tensor` with ``planes`` / ``planes_t`` and no scale
+    rows; the same bytes and scale values."""
+    who = "gemm_geglu_mx_planes"
+    _require_gpu(x8, x_planes, w8, w_planes)
+    _byte_matrix(who, x8=x8, w8=w8)
+    M, K = x8.shape
+    I = int(intermediate)
+    if w8.shape != (2 * I, K):
+        raise ValueError(f"{who}: W must be [{2 * I}, {K}]")
+    _mx_planes(who, {"x_planes": M, "w_planes": 2 * I}, K, x_planes=x_planes, w_planes=w_planes)
+    dev = x8.device
+    fp8 = TORCH_FP8[E4M3]
+    h8 = torch.empty((M, I), dtype=fp8, device=dev)
+    hp = _new_planes(I, M, dev)
+    h8t = torch.empty((I, M), dtype=fp8, device=dev) if colwise else None
+    hpt = _new_planes(M, I, dev) if colwise else None
+    GU = torch.empty((M, 2 * I), dtype=torch.bfloat16, device=dev) if keep_gu else None
+    _lib.check(_lib.lib().bf8_gemm_geglu_mx_planes(
+        _ptr(x8), x8.stride(0), _ptr(x_planes), _ptr(w8), w8.stride(0), _ptr(w_planes), M, I, K,
+        None, I, _ptr(h8), _ptr(hp), _ptr(h8t), _ptr(hpt), _ptr(GU), _stream(dev)),
+        "bf8_gemm_geglu_mx_planes")
+    return MxFp8Tensor(h8, None, h8t, None, E4M3, M, I, hp, hpt), GU
 
 
 def geglu_partials_count(M, intermediate):

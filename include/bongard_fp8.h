@@ -356,6 +356,19 @@ int bf8_quantize_mx_many_bf16(int count, const void* const* x, const int64_t* ro
                               const int64_t* cols, const int* fmt, uint8_t* const* out,
                               uint8_t* const* out_scales, void* stream);
 
+/* The same quantizers that (also) write the scales as planes: out_planes is uint32
+ * [(cols + 127) / 128][rows], plane g holding the dword of blocks 4 g .. 4 g + 3 of every row
+ * (bytes past the last block 127), out_t_planes likewise [(rows + 127) / 128][cols]; 4-byte
+ * aligned. Rows and planes of an output: at least one of the two. In planes a GEMM tile's
+ * scales of one K step are consecutive dwords, in rows they are a line apart each. */
+int bf8_quantize_mx_planes_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
+                                uint8_t* out_scales, uint32_t* out_planes, uint8_t* out_t,
+                                uint8_t* out_t_scales, uint32_t* out_t_planes, void* stream);
+int bf8_quantize_mx_many_planes_bf16(int count, const void* const* x, const int64_t* rows,
+                                     const int64_t* cols, const int* fmt, uint8_t* const* out,
+                                     uint8_t* const* out_scales, uint32_t* const* out_planes,
+                                     void* stream);
+
 /* ---------------------------------------------------------------------------------
  * NVFP4 (TE NVFP4BlockScaling under the 'nvfp4' recipe: bongard/te_linear.py:17,38,
  * bongard/fused_mlp.py:9,32). Round to nearest even everywhere, 1-D blocks of 16 along
@@ -491,6 +504,20 @@ size_t bf8_rmsnorm_bwd_workspace(int64_t rows, int64_t cols);
 int bf8_rmsnorm_bwd_bf16(const void* x, const void* dy, int64_t rows, int64_t cols,
                          const void* gamma, float eps, int zero_centered, void* dx,
                          void* dgamma, void* ws, size_t ws_bytes, void* stream);
+
+/* bf8_gemm_mx and bf8_gemm_geglu_mx_quant (H8 NULL: bf8_gemm_geglu_mx) on scale planes
+ * (bf8_quantize_mx_planes_bf16): A_planes [(K + 127) / 128][M], B_planes [..][N], X_planes
+ * [..][M], W_planes [..][2 I]; H8_planes [I / 128][M] and H8t_planes [(M + 127) / 128][I] are
+ * written. Same results, bit for bit. */
+int bf8_gemm_mx_planes(const uint8_t* A, int64_t lda, const uint32_t* A_planes, const uint8_t* B,
+                       int64_t ldb, const uint32_t* B_planes, int64_t M, int64_t N, int64_t K,
+                       const void* bias, void* C, int out_dtype, int64_t ldc, void* ws,
+                       size_t ws_bytes, void* stream);
+int bf8_gemm_geglu_mx_planes(const uint8_t* X, int64_t ldx, const uint32_t* X_planes,
+                             const uint8_t* W, int64_t ldw, const uint32_t* W_planes, int64_t M,
+                             int64_t I, int64_t K, void* H, int64_t ldh, uint8_t* H8,
+                             uint32_t* H8_planes, uint8_t* H8t, uint32_t* H8t_planes, void* GU,
+                             void* stream);
 
 #ifdef __cplusplus
 }

@@ -83,6 +83,50 @@ def test_quantize_mx_errors(gpu):
         ops.quantize_mx(torch.zeros(48, 64, dtype=torch.bfloat16, device=gpu), colwise=True)
 
 
+def _planes_of(rows_scales):
+    """The scale planes [ld / 4, rows] of scale rows [rows, ld]."""
+    r, ld = rows_scales.shape
+    return rows_scales.contiguous().view(torch.int32).reshape(r, ld // 4).t().contiguous()
+
+
+@pytest.mark.parametrize("rows,cols", [(32, 32), (160, 96), (288, 416), (512, 2560)])
+def test_mx_scale_planes(gpu, rows, cols):
+    """The quantizers' scale planes hold the scale rows' dwords (either copy, one tensor or
+    several), and a GEMM on planes gives the bits of the GEMM on rows."""
+    x = _x(rows, cols, rows - cols).to(gpu)
+    w = _x(64, cols, cols, spread=False).to(gpu)
+    q, qw = ops.quantize_mx(x, colwise=True), ops.quantize_mx(w)
+    many = ops.quantize_mx_many([x, w])
+    assert torch.equal(q.planes, _planes_of(q.scales))
+    assert torch.equal(q.planes_t, _planes_of(q.scales_t))
+    for a, b in zip(many, (q, qw)):
+        assert torch.equal(a.planes, b.planes) and torch.equal(a.scales, b.scales)
+    y = ops.gemm_mx(q.data, q.scales, qw.data, qw.scales)
+    yp = ops.gemm_mx(q.data, None, qw.data, None, a_planes=q.planes, b_planes=qw.planes)
+    assert torch.equal(y, yp)
+    with pytest.raises(ValueError, match="a_planes"):
+        ops.gemm_mx(q.data, None, qw.data, None, a_planes=qw.planes, b_planes=q.planes)
+
+
+@pytest.mark.parametrize("M,I,K", [(32, 128, 96), (288, 384, 512), (512, 1280, 2560)])
+def test_gemm_geglu_mx_planes(gpu, M, I, K):
+    """The gated-GELU GEMM on planes: H's bytes, its planes (both copies) and GU equal those of
+    the GEMM on scale rows."""
+    x = _x(M, K, M, spread=False).to(gpu)
+    w = (_x(2 * I, K, I, spread=False).float() * 0.02).to(torch.bfloat16).to(gpu)
+    qx, qw = ops.quantize_mx(x), ops.quantize_mx(w)
+    hq, gu, _ = ops.gemm_geglu_mx_quant(qx.data, qx.scales, qw.data, qw.scales, I, colwise=True,
+                                        keep_gu=True)
+    hp, gup = ops.gemm_geglu_mx_planes(qx.data, qx.planes, qw.data, qw.planes, I, colwise=True,
+                                       keep_gu=True)
+    u8 = torch.uint8
+    assert torch.equal(hq.data.view(u8), hp.data.view(u8)) and torch.equal(gu, gup)
+    assert torch.equal(hq.data_t.view(u8), hp.data_t.view(u8))
+    ld = ops.mx_scale_ld(I)
+    assert torch.equal(_planes_of(hq.scales[:, :ld]), hp.planes)
+    assert torch.equal(_planes_of(hq.scales_t), hp.planes_t)
+
+
 def _mx_gemm_case(gpu, M, N, K, seed, bias=False):
     g = torch.Generator().manual_seed(seed)
     a = (torch.randn(M, K, generator=g) * torch.logspace(-2, 2, K)[None, :]).to(torch.bfloat16)
