@@ -43,30 +43,38 @@ enum TileId {
 
 struct TileInfo {
   int bm, bn, occ;
-  double rate;        // modelled dense FP8 rate of one CU running this tile, TFLOP/s
-  double geglu_rate;  // the same with the gated-GELU epilogue; 0: no such variant (the
-                      // gated GELU pairs gate and up sub-tiles, so FN must be even)
+  double step_us;     // linear plans: one 128-byte K step of a round with every slot busy
+  double fixed_us;    // ... and what a round takes besides (pipeline fill, epilogue, relaunch)
+  double geglu_rate;  // modelled FP8 rate of one CU with the gated-GELU epilogue, TFLOP/s; 0: no
+                      // such variant (the gated GELU pairs gate and up sub-tiles: even FN)
   const char* name;
   bool mx;            // has an MX (block-scaled) variant (tiles whose stages would overflow
                       // the LDS with the scale dwords run it with one stage fewer)
 };
 
-// Rates are per-CU throughputs measured on MI355X (time per K step of one workgroup, with
-// every CU busy, over the tile's FLOP per step).
+// step_us and fixed_us: least squares over 600 measured (shape, tile, split) times of FP8
+// linear GEMMs (M 64 .. 16384, five (N, K) of the text layer, every tile and 2-4 splits),
+// together with the constants of plan_cost. Picking by them loses at most 7% on one of those
+// shapes and under 4% on the others; per-tile rates with two steps of overhead a round picked up
+// to 22% slower plans (M = 2048, N = 2560, K = 10240 on 192x256 82.0 us, 256x160 in two K pieces
+// 67.0; M = 4096, N = 10240, K = 2560 on 256x160 117.5 us, eight-wave 256x256 101.5; M = 4096,
+// N = 2048, K = 2560 on 128x128 28.5 us, 160x256 25.8). geglu_rate: time per K step of one
+// workgroup, with every CU busy, over the tile's FLOP per step. Tiles never picked by cost
+// (1e3): run by an override or in place of a twin.
 constexpr TileInfo kTiles[NUM_TILES] = {
-    {256, 256, 1, 9.6, 8.8, "256x256", true},
-    {256, 160, 1, 9.2, 8.0, "256x160", true},
-    {160, 256, 1, 9.0, 7.6, "160x256", true},
-    {128, 128, 1, 8.0, 6.2, "128x128", true},
-    {192, 256, 1, 9.0, 8.0, "192x256", true},
-    {128, 64, 2, 6.5, 0.0, "128x64", true},
-    {64, 128, 2, 6.5, 4.0, "64x128", true},
-    {256, 128, 1, 0.1, 0.1, "256x128", true},
-    {128, 64, 1, 0.1, 0.0, "128x64k2", false},
-    {64, 128, 1, 0.1, 0.0, "64x128k2", false},
-    {128, 128, 1, 0.1, 0.0, "128x128k2", false},
-    {256, 256, 1, 10.0, 9.2, "256x256w8", true},
-    {256, 256, 1, 10.0, 0.0, "256x256w8x", false},
+    {256, 256, 1, 1e3, 1e3, 8.8, "256x256", true},
+    {256, 160, 1, 1.006, 8.19, 8.0, "256x160", true},
+    {160, 256, 1, 0.936, 8.35, 7.6, "160x256", true},
+    {128, 128, 1, 0.501, 4.44, 6.2, "128x128", true},
+    {192, 256, 1, 1.058, 10.18, 8.0, "192x256", true},
+    {128, 64, 2, 0.605, 3.24, 0.0, "128x64", true},
+    {64, 128, 2, 0.620, 3.78, 4.0, "64x128", true},
+    {256, 128, 1, 1e3, 1e3, 0.1, "256x128", true},
+    {128, 64, 1, 1e3, 1e3, 0.0, "128x64k2", false},
+    {64, 128, 1, 1e3, 1e3, 0.0, "64x128k2", false},
+    {128, 128, 1, 1e3, 1e3, 0.0, "128x128k2", false},
+    {256, 256, 1, 1.097, 14.07, 9.2, "256x256w8", true},
+    {256, 256, 1, 1.097, 14.07, 0.0, "256x256w8x", false},
 };
 // Whether `tile` has a gated-GELU variant for I = N / 2: tiles of 128 or 64 H columns take
 // any I (a multiple of 128); the 256x160 tile (80 gate + 80 up columns, one wave column)
@@ -113,15 +121,9 @@ Plan make_plan(int tile, int64_t M, int64_t N, int64_t ksteps, int splits) {
 // into pieces = min(256 / t, 8) K ranges, one workgroup each, so the last round has every
 // CU busy for a fraction of a tile instead of t CUs for a whole one. Valid for tiles that
 // run one workgroup per CU with one K group. Returns false when it does not apply.
-// Per-CU FP8 rate of a long run of K steps (no epilogue) for the tiles that take tail
-// splits: the 256x256 tile, ~1.5 us per 128-byte step on MI355X with every CU busy (8192^3
-// and c5's dX shape). Measured gain at c5 (interleaved A/B): dX (M=8192, N=2560,
-// K=20480) 343.5 -> 341.0 us, dW_gu (M=20480, N=2560, K=8192) 338.8 -> 332.6 us against
-// two rounds of 256x160 tiles; a shape with a smaller tail gains more.
-constexpr double kTailStepRate256 = 11.2;
-// the eight-wave 256x256 tile on the same long-K shapes (8192^3: 394.8 -> 385.4 us)
-constexpr double kTailStepRate256w8 = 11.5;
-
+// Measured gain at c5 (interleaved A/B, four-wave tile): dX (M=8192, N=2560, K=20480) 343.5 ->
+// 341.0 us, dW_gu (M=20480, N=2560, K=8192) 338.8 -> 332.6 us against two rounds of 256x160
+// tiles; a shape with a smaller tail gains more.
 // Linear GEMMs with at least this many K steps run the eight-wave tile with its third B
 // slot (Tile256x256w8x): in a training step their operands come from HBM, not the MALL,
 // and B loaded two steps ahead hides that (operands rotated through more than the MALL
@@ -157,41 +159,52 @@ bool make_tail_plan(int tile, int64_t M, int64_t N, int64_t ksteps, Plan& p) {
 constexpr double kStepFloorNs = 520.0;
 constexpr double kStepFloorNsOcc2 = 450.0;
 
-// Modelled time (ns): rounds of co-resident workgroups, each running its K steps plus
-// about two steps of pipeline fill and epilogue, plus the split-K partials' HBM round
-// trip and the reduction's launch. A step costs the MFMA work of the workgroups sharing
-// a CU in the busiest round, or the latency floor.
-double plan_cost(const Plan& p, int64_t M, int64_t N, bool geglu, int64_t ksteps = 0) {
+// The split or tail partials' fp32 round trip through HBM and their reduction.
+constexpr double kPartialUsPerMB = 0.308, kReduceUs = 6.2;
+
+// Modelled time (us) of a linear plan: rounds of co-resident workgroups. A last round that only
+// a fraction f of the slots run, after whole rounds, takes a + (1 - a) f of a whole one, a lone
+// partial round b + (1 - b) f: the busy CUs share the memory system and the power budget with
+// fewer others. One workgroup per CU: a 0.75, b 0.80 (a round is as slow as its slowest tile);
+// two (occ 2): a 0.24, b 0.56 (half a round leaves every workgroup a CU of its own).
+double linear_cost(const Plan& p, int64_t ksteps) {
   const TileInfo& ti = kTiles[p.tile];
+  const double ws_us = kPartialUsPerMB * (double)p.ws_bytes / 1e6 + kReduceUs;
   if (p.tail_pieces > 0) {
-    // whole rounds of whole tiles, one round of pieces, the pieces' partials written and
-    // read back, the reduction's launch
-    const double rate =
-        p.tile == TILE_256x256 ? kTailStepRate256 : kTailStepRate256w8;  // w8 and w8x alike
-    const double step_ns = 2.0 * ti.bm * ti.bn * kStepBytes / (rate * 1e3);
+    // whole rounds of whole tiles, then one round of pieces
     const double rounds = (double)p.full_tiles / kNumCus;
-    return rounds * (ksteps + 2) * step_ns + (p.kps + 2) * step_ns + 2.0 * p.ws_bytes / 5e3 + 5000.0;
+    return rounds * (ksteps * ti.step_us + ti.fixed_us) + p.kps * ti.step_us + ti.fixed_us + ws_us;
   }
-  const int64_t ctas = (int64_t)p.tiles_m * p.tiles_n * p.splits;
-  const int64_t rounds = cdiv(ctas, (int64_t)kNumCus * ti.occ);
-  const int64_t per_cu = std::min<int64_t>(ti.occ, cdiv(ctas, (int64_t)kNumCus));
-  const double rate = geglu ? ti.geglu_rate : ti.rate;
-  const double work_ns = per_cu * 2.0 * ti.bm * ti.bn * kStepBytes / (rate * 1e3);
-  const double step_ns = std::max(work_ns, ti.occ > 1 ? kStepFloorNsOcc2 : kStepFloorNs);
-  // A last round that only part of the CUs run, after whole rounds, steps faster than a
-  // whole one (the busy CUs share the memory system and the power budget with fewer
-  // others): costed as 0.35 + 0.65 f of a round for a fraction f of the workgroup slots.
-  // Measured on c5's dW_down (M = 2560, N = 10240, K = 8192): one round and 56% of a
-  // second of eight-wave 256x256 tiles 164 us, two rounds and 50% of a third of 256x160
-  // tiles 188 us. A lone partial round (small M) is latency-bound and keeps its full cost.
   const int64_t slots = (int64_t)kNumCus * ti.occ;
+  const int64_t ctas = (int64_t)p.tiles_m * p.tiles_n * p.splits;
+  const int64_t whole = ctas / slots;
+  const double frac = (double)(ctas - whole * slots) / slots;
+  const double base = whole > 0 ? (ti.occ > 1 ? 0.24 : 0.75) : (ti.occ > 1 ? 0.56 : 0.80);
+  const double rounds = whole + (frac > 0 ? base + (1 - base) * frac : 0.0);
+  return rounds * (p.kps * ti.step_us + ti.fixed_us) + (p.splits > 1 ? ws_us : 0.0);
+}
+
+// Modelled time (us) of a gated-GELU plan: rounds of co-resident workgroups, each running its K
+// steps plus about two steps of pipeline fill and epilogue. A step costs the MFMA work of the
+// workgroups sharing a CU in the busiest round, or the latency floor. A partial last round
+// after whole ones counts 0.35 + 0.65 f (fewer CUs share the memory system and the power).
+double geglu_cost(const Plan& p) {
+  const TileInfo& ti = kTiles[p.tile];
+  const int64_t slots = (int64_t)kNumCus * ti.occ;
+  const int64_t ctas = (int64_t)p.tiles_m * p.tiles_n;
+  const int64_t rounds = cdiv(ctas, slots);
+  const int64_t per_cu = std::min<int64_t>(ti.occ, cdiv(ctas, (int64_t)kNumCus));
+  const double work_ns = per_cu * 2.0 * ti.bm * ti.bn * kStepBytes / (ti.geglu_rate * 1e3);
+  const double step_ns = std::max(work_ns, ti.occ > 1 ? kStepFloorNsOcc2 : kStepFloorNs);
   const int64_t whole = ctas / slots;
   const double frac = (double)(ctas - whole * slots) / slots;
   const double eff_rounds =
       whole >= 1 && frac > 0 ? whole + 0.35 + 0.65 * frac : (double)rounds;
-  double t = eff_rounds * (p.kps + 2) * step_ns;
-  if (p.splits > 1) t += 2.0 * p.splits * M * N * 4 / 5e3 + 5000.0;
-  return t;
+  return eff_rounds * (p.kps + 2) * step_ns / 1e3;
+}
+
+double plan_cost(const Plan& p, bool geglu, int64_t ksteps) {
+  return geglu ? geglu_cost(p) : linear_cost(p, ksteps);
 }
 
 // Tuning override, read on every call: BONGARD_FP8_GEMM_TILE=<bm>x<bn>[:<splits>|:t]
@@ -248,8 +261,8 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
       const Plan p = make_plan(tile, M, N, geglu ? kGegluNominalSteps : ksteps, s);
       if (p.splits != s || (s > 1 && p.kps < kMinStepsPerSplit) || p.ws_bytes > ws_avail)
         continue;
-      const double c = plan_cost(p, M, N, geglu);
-      if (!have || c < best_cost * 0.97) {  // prefer earlier (larger, unsplit) plans on ties
+      const double c = plan_cost(p, geglu, ksteps);
+      if (!have || c < best_cost * 0.99) {  // prefer earlier (larger, unsplit) plans on ties
         best = p;
         best_cost = c;
         have = true;
@@ -257,8 +270,8 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
     }
     Plan tp;
     if (!geglu && make_tail_plan(tile, M, N, ksteps, tp) && tp.ws_bytes <= ws_avail) {
-      const double c = plan_cost(tp, M, N, false, ksteps);
-      if (!have || c < best_cost * 0.97) {
+      const double c = plan_cost(tp, false, ksteps);
+      if (!have || c < best_cost * 0.99) {
         best = tp;
         best_cost = c;
         have = true;
@@ -292,8 +305,8 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
 // entry point transposes B^T [K, N] into its workspace and runs the row-major plan. (The
 // wgrad form, A and B K-major, measured level or faster on the same shapes, so it always
 // runs K-major.)
-constexpr double kTransposeBytesPerNs = 2.5e3;  // a small transpose: ~2.5 TB/s read + write
-constexpr double kTransposeLaunchNs = 4000.0;
+constexpr double kTransposeBytesPerUs = 2.5e6;  // a small transpose: ~2.5 TB/s read + write
+constexpr double kTransposeLaunchUs = 2.0;
 constexpr double kKmajorFallbackGain = 0.8;  // transpose only when that is 20% cheaper
 
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -319,12 +332,12 @@ KmajorChoice choose_kmajor(int64_t M, int64_t N, int64_t K, bool a_kmajor, size_
     if (q.tile == TILE_128x64k2) q.tile = TILE_128x64;
     if (q.tile == TILE_64x128k2) q.tile = TILE_64x128;
     if (q.tile == TILE_256x256w8x) q.tile = TILE_256x256w8;
-    return plan_cost(q, M, N, false, ksteps);
+    return linear_cost(q, ksteps);
   };
   const double ck = costed(c.plan);
-  const double cr = costed(pr) + 2.0 * (double)N * K / kTransposeBytesPerNs + kTransposeLaunchNs;
+  const double cr = costed(pr) + 2.0 * (double)N * K / kTransposeBytesPerUs + kTransposeLaunchUs;
   if (const char* d = std::getenv("BONGARD_FP8_GEMM_DEBUG"); d && d[0] == '1')
-    std::fprintf(stderr, "bf8 kmajor M=%lld N=%lld K=%lld: K-major %.0f ns, transposed B %.0f ns\n",
+    std::fprintf(stderr, "bf8 kmajor M=%lld N=%lld K=%lld: K-major %.1f us, transposed B %.1f us\n",
                  (long long)M, (long long)N, (long long)K, ck, cr);
   if (cr < kKmajorFallbackGain * ck) {
     c.plan = pr;
