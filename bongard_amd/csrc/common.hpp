@@ -80,6 +80,11 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
+// bf16 sums of two packed pairs, each rounded once.
+__device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b) {
+  return pack_bf16x2(bf16_lo(a) + bf16_lo(b), bf16_hi(a) + bf16_hi(b));
+}
+
 // A packed bf16 pair with each NaN replaced by 0x7FC0 (torch's canonical bf16 NaN), so
 // that pack_bf16x2 then gives f32_to_bf16_bits bit for bit. A half h is NaN iff
 // (h & 0x7FFF) + 0x7F carries into bit 15; the low half's sum cannot reach bit 16.

@@ -419,6 +419,7 @@ struct ReduceOut {
   void* C;
   int64_t ldc;
   int a_vec, b_vec, unit;
+  int add;  // add the bf16 result to C (GemmParams::add)
 };
 
 template <int OUT>
@@ -459,12 +460,20 @@ __device__ __forceinline__ void reduce_store(const ReduceOut& o, float (&v)[8], 
   }
   if (OUT == BF8_OUT_BF16) {
     uint16_t* dst = reinterpret_cast<uint16_t*>(o.C) + m * o.ldc + n;
-    uint32_t w[4];
+    uint32_t w[4], c[4] = {0u, 0u, 0u, 0u};
+    if (o.add) {
+      const uint2 c0 = reinterpret_cast<const uint2*>(dst)[0], c1 = reinterpret_cast<const uint2*>(dst)[1];
+      c[0] = c0.x; c[1] = c0.y; c[2] = c1.x; c[3] = c1.y;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       w[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(
                  (float __attribute__((ext_vector_type(2)))){v[2 * e], v[2 * e + 1]},
                  __bf16 __attribute__((ext_vector_type(2)))));
+    if (o.add) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = add_bf16x2(c[e], w[e]);
+    }
     if ((o.ldc & 7) == 0) {
       *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
     } else {
@@ -553,6 +562,7 @@ int launch_plan(const Plan& pl, GemmParams p, int epi, int out_dtype, int fa, in
   o.a_sinv = p.a_sinv; o.b_sinv = p.b_sinv; o.b_stride = p.b_stride; o.n_seg = p.n_seg;
   for (int i = 0; i < 4; ++i) o.seg_end.e[i] = p.seg_end[i];
   o.bias = p.bias; o.C = p.C; o.ldc = p.ldc; o.a_vec = p.a_vec; o.b_vec = p.b_vec;
+  o.add = p.add;
   o.unit = mx ? 1 : 0;
   if (pl.tail_pieces > 0) {
     // whole tiles write C; the tail tiles' pieces write raw partials, reduced after
@@ -673,11 +683,11 @@ size_t bf8_gemm_kmajor_workspace(int64_t M, int64_t N, int64_t K) {
   return std::max(both, b_only.b_bytes + b_only.plan.ws_bytes);
 }
 
-int bf8_gemm_kmajor(const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor, const uint8_t* B,
-                    int fmt_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
-                    const float* a_scale_inv, const float* b_scale_inv, void* C, int out_dtype,
-                    int64_t ldc, void* ws, size_t ws_bytes, void* stream) {
-  const char* who = "bf8_gemm_kmajor";
+static int kmajor_entry(const char* who, const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor,
+                        const uint8_t* B, int fmt_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                        const float* a_scale_inv, const float* b_scale_inv, void* C,
+                        int out_dtype, int64_t ldc, int add, void* ws, size_t ws_bytes,
+                        void* stream) {
   BF8_CHECK(fmt_a == BF8_E5M2 && fmt_b == BF8_E4M3,
             "%s: formats %d x %d (supported: e5m2 x e4m3)", who, fmt_a, fmt_b);
   BF8_CHECK(a_kmajor == 0 || a_kmajor == 1, "%s: a_kmajor must be 0 or 1", who);
@@ -708,6 +718,7 @@ int bf8_gemm_kmajor(const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor, cons
   for (int s = 0; s < 4; ++s) p.seg_end[s] = (int)N;
   p.C = C; p.ldc = ldc;
   p.kmajor = a_kmajor ? 3 : 2;
+  p.add = add;
   hipStream_t s = as_stream(stream);
   const KmajorChoice ch = choose_kmajor(M, N, K, a_kmajor != 0, ws ? ws_bytes : 0);
   if (!ch.transpose_b) return launch_plan(ch.plan, p, EPI_LINEAR, out_dtype, fmt_a, fmt_b, ws, s);
@@ -723,6 +734,23 @@ int bf8_gemm_kmajor(const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor, cons
   p.kmajor = 0;
   return launch_plan(ch.plan, p, EPI_LINEAR, out_dtype, fmt_a, fmt_b,
                      ch.plan.ws_bytes ? bt + ch.b_bytes : nullptr, s);
+}
+
+int bf8_gemm_kmajor(const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor, const uint8_t* B,
+                    int fmt_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                    const float* a_scale_inv, const float* b_scale_inv, void* C, int out_dtype,
+                    int64_t ldc, void* ws, size_t ws_bytes, void* stream) {
+  return kmajor_entry("bf8_gemm_kmajor", A, fmt_a, lda, a_kmajor, B, fmt_b, ldb, M, N, K,
+                      a_scale_inv, b_scale_inv, C, out_dtype, ldc, 0, ws, ws_bytes, stream);
+}
+
+int bf8_gemm_kmajor_add(const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor, const uint8_t* B,
+                        int fmt_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                        const float* a_scale_inv, const float* b_scale_inv, void* C,
+                        int out_dtype, int64_t ldc, void* ws, size_t ws_bytes, void* stream) {
+  BF8_CHECK(out_dtype == BF8_OUT_BF16, "bf8_gemm_kmajor_add: the sum is formed in bf16");
+  return kmajor_entry("bf8_gemm_kmajor_add", A, fmt_a, lda, a_kmajor, B, fmt_b, ldb, M, N, K,
+                      a_scale_inv, b_scale_inv, C, out_dtype, ldc, 1, ws, ws_bytes, stream);
 }
 
 int bf8_gemm_bf16(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M, int64_t N,

@@ -63,6 +63,7 @@ struct GemmParams {
   // Operand layout (linear epilogues of the eight-wave 256 x 256 tiles): 0 = A [M, K] and
   // B [N, K]; 2 = B given as B^T [K, N] (row stride ldb >= N); 3 = A as A^T [K, M] as well.
   int kmajor;
+  int add;  // linear, bf16 out: C = bf16(C + bf16(result)) (element by element, in place)
 };
 
 constexpr int kGroupM = 8;  // tile rows walked together (the tile order of a launch)

@@ -1008,11 +1008,19 @@ gemm_kernel(GemmParams p) {
     for (int it = 0; it < ROWS * CH / 64; ++it) {
       const int idx = it * 64 + lane;
       const int row = idx / CH, c = idx % CH;
-      const uint4 d = stage_get<CH>(wbuf, row, c);
+      uint4 d = stage_get<CH>(wbuf, row, c);
       const int gm = m0 + wave_m0 + row;
       const int gn = wave_n0 + c * 8;
-      if (gm < p.M && gn < p.N)
-        store_bf16x8(reinterpret_cast<uint16_t*>(p.C) + (int64_t)gm * p.ldc + gn, d, p.ldc);
+      if (gm < p.M && gn < p.N) {
+        uint16_t* dst = reinterpret_cast<uint16_t*>(p.C) + (int64_t)gm * p.ldc + gn;
+        if (p.add) {
+          const uint2 c0 = reinterpret_cast<const uint2*>(dst)[0];
+          const uint2 c1 = reinterpret_cast<const uint2*>(dst)[1];
+          d = make_uint4(add_bf16x2(c0.x, d.x), add_bf16x2(c0.y, d.y), add_bf16x2(c1.x, d.z),
+                         add_bf16x2(c1.y, d.w));
+        }
+        store_bf16x8(dst, d, p.ldc);
+      }
     }
   } else if constexpr (EPI == EPI_LINEAR) {
     // fp32 out; with a K split, raw partial sums into this split's slice of C

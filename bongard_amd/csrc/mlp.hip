@@ -354,7 +354,8 @@ int bf8_geglu_bwd_delayed(const void* dH, const void* GU, int64_t M, int64_t I, 
   BF8_CHECK(fmt == BF8_E4M3 || fmt == BF8_E5M2, "bf8_geglu_bwd_delayed: bad fmt %d", fmt);
   BF8_CHECK(M >= 0 && I >= kTT && I % kTT == 0,
             "bf8_geglu_bwd_delayed: need I %% 64 == 0 (I=%lld)", (long long)I);
-  BF8_CHECK(M % 16 == 0, "bf8_geglu_bwd_delayed: need M %% 16 == 0 (M=%lld)", (long long)M);
+  BF8_CHECK(!out_t || M % 16 == 0,
+            "bf8_geglu_bwd_delayed: a transposed copy needs M %% 16 == 0 (M=%lld)", (long long)M);
   BF8_CHECK(dH && GU && state && partials_out && (out || out_t),
             "bf8_geglu_bwd_delayed: NULL pointer");
   BF8_CHECK(len >= 1 && len <= 1024 && pos >= 0 && pos < len,

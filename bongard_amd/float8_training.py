@@ -78,9 +78,11 @@ class Float8Linear(torch.nn.Linear):
         flat = inputs.reshape(-1, shape[-1])
         if flat.dtype != torch.bfloat16:
             flat = flat.to(torch.bfloat16)
-        length = flat.shape[0]
-        # pad_inner_dim: the wgrad GEMM reduces over tokens, so keep them a multiple of 16
-        aligned = (length + 15) // 16 * 16
+        length = aligned = flat.shape[0]
+        if self.config.recipe == "rowwise":
+            # pad_inner_dim: its wgrad GEMM reduces over the tokens of transposed copies, whose
+            # rows are 16-byte vectors (the other recipes' kernels take any token count)
+            aligned = (length + 15) // 16 * 16
         if aligned != length:
             flat = F.pad(flat, (0, 0, 0, aligned - length))
         weight = self.weight if self.weight.dtype == torch.bfloat16 else self.weight.to(torch.bfloat16)

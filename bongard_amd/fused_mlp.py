@@ -27,8 +27,8 @@ import torch
 from . import linear as _linear
 from . import ops as _ops
 from . import scaling as _scaling
-from .te_linear import (RECIPES, _is_mx, _is_nvfp4, _make_recipe, _new_scaling, _pad_rows, _ScalingExtraState,
-                        present)
+from .te_linear import (RECIPES, _is_blocked, _is_mx, _is_nvfp4, _make_recipe, _new_scaling,
+                        _pad_rows, _ScalingExtraState, present)
 
 __all__ = ["RECIPES", "FusedMLP", "enable_fused_mlp", "hf_state_dict"]
 
@@ -54,7 +54,8 @@ class _FusedRMSNorm(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight = ctx.saved_tensors
-        dx, dw = _ops.rmsnorm_backward(x, dy.contiguous(), weight, ctx.eps, zero_centered=True,
+        dx, dw = _ops.rmsnorm_backward(x, _linear.dense_rows(dy), weight, ctx.eps,
+                                       zero_centered=True,
                                        need_dx=ctx.needs_input_grad[0],
                                        need_dw=ctx.needs_input_grad[1])
         return dx, dw, None, None
@@ -128,9 +129,13 @@ class FusedMLP(_ScalingExtraState, torch.nn.Module):
         first = versions != self._cached_weight_versions or self._fp8_weights is None
         self._cached_weight_versions = versions
         self.counts['weight_quantizations' if first else 'cached_weights'] += 1
-        flat, length, aligned = _pad_rows(flat)
+        length = flat.shape[0]
+        # the token count of the 32-row granularity the reference pads to; only the
+        # block-scaled recipes' kernels need the padded rows themselves
         self.counts['real_tokens'] += length
-        self.counts['kernel_tokens'] += aligned
+        self.counts['kernel_tokens'] += (length + 31) // 32 * 32
+        if _is_blocked(self.recipe):
+            flat, _, _ = _pad_rows(flat)
         fc1, fc2 = self.scaling if self.scaling is not None else (None, None)
         mx = _is_mx(self.recipe)
         if _is_nvfp4(self.recipe):
@@ -151,7 +156,7 @@ class FusedMLP(_ScalingExtraState, torch.nn.Module):
                                              split_scales=False),
                     _linear.quantize_weight(self.fc2_weight))
         gu_q, down_q = self._fp8_weights
-        flat = flat.to(torch.bfloat16).contiguous()
+        flat = _linear.dense_rows(flat.to(torch.bfloat16))
         if mx:
             # block scales need no tensor-wide amax: the norm's partials go unused
             if _ops.rmsnorm_supported(flat.shape[1]):
@@ -180,8 +185,7 @@ class FusedMLP(_ScalingExtraState, torch.nn.Module):
         out = _linear.Fp8GegluMlpFunction.apply(normed, self.fc1_weight, self.fc2_weight, gu_q,
                                                 down_q, self.intermediate_size, False,
                                                 self.scaling, x_amax)
-        return out[:length].reshape_as(x)
-
+        return out.reshape_as(x)
 
     def _nvfp4_forward(self, x, flat, length, first):
         """'nvfp4': the fused norm, fc1 as an NVFP4 GEMM (operands dequantized exactly to

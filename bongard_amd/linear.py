@@ -93,6 +93,15 @@ def _quantize_input(x, scaler, x_amax, transpose):
     return scaler.quantize(x, rowwise=True, transpose=transpose, producer_count=int(x_amax))
 
 
+def dense_rows(t):
+    """``t`` as the kernels read it: contiguous and 16-byte aligned. Row counts that are not
+    multiples of 16 reach the per-tensor-scaled kernels as they are (every GEMM takes them,
+    the weight-gradient GEMM's reduction included); a copy is made only of a tensor whose
+    storage the kernels cannot read."""
+    t = t.contiguous()
+    return t if t.shape[0] % 16 == 0 or t.data_ptr() % 16 == 0 else t.clone()
+
+
 def linear_kmajor(in_features, out_features):
     """Whether a tensorwise FP8 linear can train: its backward reads the forward's fp8 X and
     W as they are (K-major dgrad / wgrad operands, bf8_gemm_kmajor), which needs both row
@@ -115,6 +124,7 @@ def linear_forward(x, weight, bias, wq, scaling, need_dx, need_dw):
     launch, in training as in inference."""
     if need_dx or need_dw:
         _check_trainable("fp8 linear", x.shape[-1], weight.shape[0])
+    x = dense_rows(x)
     if scaling is None and wq is None:
         xq, wq = ops.quantize_many([x, weight.detach()])
     else:
@@ -129,7 +139,7 @@ def linear_backward(dy, saved, scaling, need_dx, need_dw):
     """Tensorwise FP8 linear backward: dY in e5m2 (its own scale), dX = dY8 . W8 and
     dW = dY8^T . X8 with W8 and X8 (and dY8 for dW) read as K-major operands."""
     x8, x_meta, w8, w_meta = saved
-    dyq = _quantize(dy.contiguous(), E5M2, scaling and scaling.grad_output)
+    dyq = _quantize(dense_rows(dy), E5M2, scaling and scaling.grad_output)
     dx = ops.gemm_kmajor(dyq.data, E5M2, dyq.meta, w8, E4M3, w_meta) if need_dx else None
     dw = (ops.gemm_kmajor(dyq.data, E5M2, dyq.meta, x8, E4M3, x_meta, a_kmajor=True)
           if need_dw else None)
@@ -170,6 +180,7 @@ def linear_axiswise_forward(x, weight, bias, recipe, need_dx, need_dw):
     if recipe not in AXISWISE_RECIPES:
         raise ValueError(f"axiswise recipe must be one of {AXISWISE_RECIPES}")
     hp_wgrad = recipe == "rowwise_with_gw_hp"
+    x = dense_rows(x)
     xq = ops.quantize_axiswise(x, E4M3, rowwise=True, colwise=need_dw and not hp_wgrad)
     wq = ops.quantize_axiswise(weight.detach(), E4M3, rowwise=True,
                                colwise=need_dx and not hp_wgrad)
@@ -180,7 +191,7 @@ def linear_axiswise_forward(x, weight, bias, recipe, need_dx, need_dw):
 
 
 def linear_axiswise_backward(dy, saved, recipe, need_dx, need_dw):
-    dy = dy.contiguous()
+    dy = dense_rows(dy)
     dx = dw = None
     if recipe == "rowwise":
         x8t, x_cs, w8t, w_cs = saved
@@ -196,7 +207,7 @@ def linear_axiswise_backward(dy, saved, recipe, need_dx, need_dw):
             wt = ops.quantize(weight, E4M3, rowwise=False, transpose=True, pow2=True)
             dx = ops.gemm_axiswise(dyq.data, E4M3, dyq.row_sinv, wt.data_t, E4M3, wt.meta[2:3])
         if need_dw:
-            dw = torch.mm(dy.t().contiguous(), x)
+            dw = torch.mm(dy.t(), x)
     return dx, dw
 
 
@@ -490,6 +501,7 @@ def mlp_forward(x, w_gu, w_down, gu_q, down_q, intermediate, split_scales, scali
         _check_trainable("fp8 gated MLP", x.shape[-1], I, w_down.shape[0])
     if scaling is not None and split_scales:
         raise NotImplementedError("delayed scaling needs the fused [gate; up] weight")
+    x = dense_rows(x)
     gs, ds = scaling if scaling is not None else (None, None)
     if (scaling is None and x_amax is None and not split_scales
             and (gu_q is None or down_q is None)):
@@ -550,7 +562,7 @@ def mlp_backward(dy, saved, intermediate, split_scales, scaling, needs):
     I = int(intermediate)
     need_dx, need_dgu, need_dd = needs
     gs, ds = scaling if scaling is not None else (None, None)
-    dyq = _quantize(dy.contiguous(), E5M2, ds and ds.grad_output)
+    dyq = _quantize(dense_rows(dy), E5M2, ds and ds.grad_output)
 
     def gemm_b(a, a_meta, b, b_meta, *, a_kmajor=False):
         # e5m2 gradient A (or A^T) against the saved e4m3 B, given as B^T [K, N]

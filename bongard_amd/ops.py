@@ -367,11 +367,13 @@ def _gemm_kmajor_ws_cached(M, N, K, override):
 
 
 def gemm_kmajor(a, a_fmt, a_meta, b_t, b_fmt, b_meta, *, a_kmajor=False,
-                out_dtype=torch.bfloat16, out=None):
+                out_dtype=torch.bfloat16, out=None, accumulate=False):
     """:func:`gemm` with B given as ``b_t`` = B^T [K, N] (and, when ``a_kmajor``, A as ``a``
     = A^T [K, M]): the backward's dgrad and wgrad GEMMs on the fp8 tensors as their
     producers wrote them, no transposed copies (bf8_gemm_kmajor; e5m2 x e4m3). Same
-    products and fp32 sums as :func:`gemm` on the transposed operands."""
+    products and fp32 sums as :func:`gemm` on the transposed operands. ``accumulate``: the
+    bf16 result is added to ``out`` (one rounding of the sum of the two bf16 values, as
+    ``out + result`` rounds it)."""
     _require_gpu(a, b_t, a_meta, b_meta)
     _byte_matrix("gemm_kmajor", a=a, b_t=b_t)
     if a_kmajor:
@@ -383,13 +385,17 @@ def gemm_kmajor(a, a_fmt, a_meta, b_t, b_fmt, b_meta, *, a_kmajor=False,
         raise ValueError(f"gemm_kmajor: inner dims differ ({K} vs {Kb})")
     if out_dtype not in (torch.bfloat16, torch.float32):
         raise TypeError("gemm_kmajor: out_dtype must be bfloat16 or float32")
+    if accumulate and (out is None or out_dtype != torch.bfloat16):
+        raise ValueError("gemm_kmajor: accumulate needs a bfloat16 out")
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=a.device)
     _out_matrix("gemm_kmajor", out, (M, N), out_dtype)
     ws_bytes = _gemm_kmajor_ws_cached(M, N, K, _tile_override())
     ws = gemm_workspace(ws_bytes, a.device) if ws_bytes else None
     ws_bytes = ws.numel() if ws is not None else 0
-    _lib.check(_lib.lib().bf8_gemm_kmajor(
+    L = _lib.lib()
+    entry = L.bf8_gemm_kmajor_add if accumulate else L.bf8_gemm_kmajor
+    _lib.check(entry(
         _ptr(a), a_fmt, a.stride(0), int(bool(a_kmajor)), _ptr(b_t), b_fmt, b_t.stride(0), M, N,
         K, _sinv_ptr(a_meta), _sinv_ptr(b_meta), _ptr(out),
         OUT_BF16 if out_dtype == torch.bfloat16 else OUT_F32, out.stride(0), _ptr(ws), ws_bytes,

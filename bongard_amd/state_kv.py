@@ -16,15 +16,15 @@ import torch
 
 from . import ops
 from .ops import E4M3, E5M2
-from .linear import _Fp8Function, _check_trainable, _forward_needs
-from .te_linear import Float8CurrentScaling, TELinear, _pad_rows
+from .linear import _Fp8Function, _check_trainable, _forward_needs, dense_rows
+from .te_linear import Float8CurrentScaling, TELinear
 
 __all__ = ["project_state_kv"]
 
 
 class _SharedInputFp8Function(_Fp8Function):
     """y_i = x @ W_i^T for several per-tensor-scaled FP8 projections of one input x
-    [M, K] (M % 32 == 0): one e4m3 quantization of x, one GEMM per cached weight; backward
+    [M, K]: one e4m3 quantization of x, one GEMM per cached weight; backward
     per projection as Fp8LinearFunction (X8, W8_i and dY8 read as K-major operands), the
     input gradients summed in bf16 in projection order."""
 
@@ -36,6 +36,7 @@ class _SharedInputFp8Function(_Fp8Function):
         if need_dx or need_dw:
             _check_trainable("shared-input projections", x.shape[-1],
                              *[wq.data.shape[0] for wq in wqs])
+        x = dense_rows(x)
         xq = ops.quantize(x, E4M3)
         outs = [ops.gemm(xq.data, E4M3, xq.meta, wq.data, E4M3, wq.meta) for wq in wqs]
         ctx.n = len(wqs)
@@ -52,16 +53,23 @@ class _SharedInputFp8Function(_Fp8Function):
         x8, x_meta = saved[0], saved[1]
         dx = None
         dws = []
-        for i, dy in enumerate(dys):
+        # every dY in one amax and one cast launch
+        given = [i for i, dy in enumerate(dys) if dy is not None]
+        qs = {}
+        for j in range(0, len(given), 8):
+            part = given[j:j + 8]
+            qs.update(zip(part, ops.quantize_many([dense_rows(dys[i]) for i in part], E5M2)))
+        for i in range(len(dys)):
             w8, w_meta = saved[2 + 2 * i], saved[3 + 2 * i]
             need_dw = ctx.needs_input_grad[2 + i]
-            if dy is None:
+            if i not in qs:
                 dws.append(None)
                 continue
-            dyq = ops.quantize(dy.contiguous(), E5M2)
+            dyq = qs[i]
             if ctx.need_dx:
-                part = ops.gemm_kmajor(dyq.data, E5M2, dyq.meta, w8, E4M3, w_meta)
-                dx = part if dx is None else dx + part
+                # a later projection's bf16 product is added to dx in its GEMM's epilogue
+                dx = ops.gemm_kmajor(dyq.data, E5M2, dyq.meta, w8, E4M3, w_meta, out=dx,
+                                     accumulate=dx is not None)
             dws.append(ops.gemm_kmajor(dyq.data, E5M2, dyq.meta, x8, E4M3, x_meta, a_kmajor=True)
                        if need_dw else None)
         return (dx, None, *dws)
@@ -78,17 +86,11 @@ def shared_input_projections(x, projections):
     torch.compile, like the projections themselves: the reference compiles
     project_state_kv (bongard/model.py:279), which then runs this part eagerly."""
     flat = x.reshape(-1, x.shape[-1])
-    flat, length, aligned = _pad_rows(flat)
     if flat.dtype != torch.bfloat16:
         flat = flat.to(torch.bfloat16)
     wqs = [p.fp8_weight(p._note_microbatch()) for p in projections]
     outs = _SharedInputFp8Function.apply(flat, wqs, *[p.weight for p in projections])
-    res = []
-    for out in outs:
-        if aligned != length:
-            out = out[:length]
-        res.append(out.reshape(*x.shape[:-1], out.shape[-1]))
-    return res
+    return [out.reshape(*x.shape[:-1], out.shape[-1]) for out in outs]
 
 
 def project_state_kv(attention, state):

@@ -100,6 +100,11 @@ def _is_nvfp4(recipe):
     return isinstance(recipe, NVFP4BlockScaling)
 
 
+def _is_blocked(recipe):
+    """Whether a recipe quantizes blocks along the rows (the columnwise copies)."""
+    return _is_mx(recipe) or _is_nvfp4(recipe)
+
+
 def _new_scaling(recipe):
     """The delayed-scaling state a module needs for ``recipe`` (None: stateless)."""
     if isinstance(recipe, DelayedScaling):
@@ -240,8 +245,9 @@ class TELinear(_ScalingExtraState, torch.nn.Module):
             return F.linear(x, self.weight)
         flat = x.reshape(-1, x.shape[-1])
         first_microbatch = self._note_microbatch()
-        # Pad to a multiple of 32 rows (zeros leave the amax unchanged), slice after.
-        flat, length, aligned = _pad_rows(flat)
+        # The block-scaled recipes quantize blocks of rows: pad to a multiple of 32 rows (zeros
+        # leave the amax unchanged), slice after. Per-tensor scaling takes any row count.
+        flat, length, aligned = _pad_rows(flat, 32 if _is_blocked(self.recipe) else 1)
         if flat.dtype != torch.bfloat16:
             flat = flat.to(torch.bfloat16)
         if _is_mx(self.recipe):
@@ -310,7 +316,7 @@ class TEMLP(torch.nn.Module):
             return self.down(h.reshape(*shape[:-1], shape[-1] // 2), x_partials=h_partials)
         I = self.intermediate_size
         flat = x.reshape(-1, x.shape[-1])
-        flat, length, aligned = _pad_rows(flat)
+        flat, length, aligned = _pad_rows(flat, 32 if _is_blocked(self.down.recipe) else 1)
         if flat.dtype != torch.bfloat16:
             flat = flat.to(torch.bfloat16)
         down_first = self.down._note_microbatch()

@@ -164,6 +164,15 @@ int bf8_gemm_kmajor(const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor, cons
                     const float* a_scale_inv, const float* b_scale_inv, void* C, int out_dtype,
                     int64_t ldc, void* ws, size_t ws_bytes, void* stream);
 
+/* bf8_gemm_kmajor whose bf16 result is added to C: C = bf16(C + bf16(result)), one rounding of
+ * the sum of two bf16 values (out_dtype BF8_OUT_BF16). The input gradient of several
+ * projections of one input, which autograd forms as such a sum (project_state_kv,
+ * bongard/model.py:342-347). */
+int bf8_gemm_kmajor_add(const uint8_t* A, int fmt_a, int64_t lda, int a_kmajor, const uint8_t* B,
+                    int fmt_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                    const float* a_scale_inv, const float* b_scale_inv, void* C, int out_dtype,
+                    int64_t ldc, void* ws, size_t ws_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------
  * Gate/up GEMM with the gated-GELU(tanh) epilogue.
  * Replaces TEMLP.forward's gate_up GEMM + F.gelu(gate, approximate='tanh') * up

@@ -582,3 +582,25 @@ def test_gemm_kmajor_small_output_runs_on_transposed_b(gpu, M, N, K):
         torch.cuda.synchronize()
         iv = torch.int16 if dt == torch.bfloat16 else torch.int32
         assert torch.equal(got.view(iv), want.view(iv)), f"{M}x{N}x{K} {dt}"
+
+
+@pytest.mark.parametrize("M,N,K,plan", [
+    (33, 48, 80, ""), (512, 2560, 1024, ""),             # the row-major plan on a transposed B
+    (300, 272, 512, "256x256w8"), (260, 256, 2048, "256x256w8:3"), (4160, 3856, 2048, "256x256w8:t"),
+])
+def test_gemm_kmajor_accumulate(gpu, monkeypatch, M, N, K, plan):
+    """accumulate adds the bf16 result to ``out`` in the epilogue (whole, split and tail-split
+    plans): bit for bit ``out + gemm_kmajor(...)``."""
+    g = torch.Generator().manual_seed(M + N + K)
+    aq = ops.quantize((torch.randn(M, K, generator=g) * 1e-3).to(torch.bfloat16).to(gpu), ops.E5M2)
+    bq = ops.quantize((torch.randn(K, N, generator=g) * 0.02).to(torch.bfloat16).to(gpu), ops.E4M3)
+    base = (torch.randn(M, N, generator=g) * 1e-4).to(torch.bfloat16).to(gpu)
+    if plan:
+        monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", plan)
+    part = ops.gemm_kmajor(aq.data, ops.E5M2, aq.meta, bq.data, ops.E4M3, bq.meta)
+    got = ops.gemm_kmajor(aq.data, ops.E5M2, aq.meta, bq.data, ops.E4M3, bq.meta,
+                          out=base.clone(), accumulate=True)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), (base + part).view(torch.int16))
+    with pytest.raises(ValueError, match="accumulate"):
+        ops.gemm_kmajor(aq.data, ops.E5M2, aq.meta, bq.data, ops.E4M3, bq.meta, accumulate=True)

@@ -518,3 +518,57 @@ def test_inference_forward_shares_quantize_launches(gpu, monkeypatch):
     assert len(calls) == 5
     assert torch.equal(y_train.detach(), y_inf)
 
+
+
+@pytest.mark.parametrize("rows", [1, 15, 77, 301])
+@pytest.mark.parametrize("kind", ["te_fp8", "te_delayed", "tensorwise", "gw_hp"])
+def test_ragged_rows_equal_padded_rows(gpu, rows, kind):
+    """Row counts that are not multiples of 16 or 32 run without padded copies: the gradients
+    and outputs are those of the zero-padded rows (fp32 sums of the same products; the K split
+    may differ), also for an input view off 16-byte alignment and an expanded gradient."""
+    from bongard_amd import linear, scaling
+    K, N, pad = 512, 384, (rows + 31) // 32 * 32
+    g = torch.Generator().manual_seed(rows)
+    buf = torch.randn(rows * K + 3, generator=g).to(torch.bfloat16).to(gpu)
+    x = buf[3:].view(rows, K)                       # 6 bytes past the allocation's alignment
+    w = (torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    dy = torch.full((1, N), 1e-3, dtype=torch.bfloat16, device=gpu).expand(rows, N)
+
+    def run(x, dy):
+        xg, wg = x.detach().requires_grad_(True), w.detach().clone().requires_grad_(True)
+        if kind == "gw_hp":
+            y = linear.Fp8LinearAxiswiseFunction.apply(xg, wg, None, "rowwise_with_gw_hp")
+        else:
+            sc = scaling.LinearScaling(16) if kind == "te_delayed" else None
+            y = linear.Fp8LinearFunction.apply(xg, wg, None, None, sc)
+        return (y, *torch.autograd.grad(y, [xg, wg], dy))
+
+    F = torch.nn.functional
+    y, dx, dw = run(x, dy)
+    py, pdx, pdw = run(F.pad(x, (0, 0, 0, pad - rows)), F.pad(dy, (0, 0, 0, pad - rows)))
+    torch.cuda.synchronize()
+    for what, a, b in (("y", y, py[:rows]), ("dx", dx, pdx[:rows]), ("dw", dw, pdw)):
+        _close(a, b, f"ragged {kind} {rows} {what}", tol=1e-3)
+
+
+@pytest.mark.parametrize("recipe", ["fp8", "fp8_delayed"])
+@pytest.mark.parametrize("rows", [5, 301])
+def test_temlp_ragged_rows_equal_padded_rows(gpu, recipe, rows):
+    """The gated MLP on ragged rows against the same rows padded to 32 by the caller, two steps
+    (delayed: the second uses the first's amaxes)."""
+    F = torch.nn.functional
+    pad = (rows + 31) // 32 * 32 - rows
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, 256, generator=g).to(torch.bfloat16).to(gpu)
+    dy = (torch.randn(rows, 256, generator=g) * 1e-3).to(torch.bfloat16).to(gpu)
+    a, b = (te_linear.TEMLP(_mlp(256, 512, 3, gpu), recipe).train() for _ in range(2))
+    for _ in range(2):
+        out = []
+        for m, xi, di in ((a, x, dy), (b, F.pad(x, (0, 0, 0, pad)), F.pad(dy, (0, 0, 0, pad)))):
+            xg = xi.detach().requires_grad_(True)
+            y = m(xg)
+            out.append((y, *torch.autograd.grad(y, [xg, m.gate_up.weight, m.down.weight], di)))
+    torch.cuda.synchronize()
+    for i, (u, v) in enumerate(zip(*out)):
+        _close_requant(u, v[:rows] if i < 2 else v, f"ragged temlp {recipe} {rows} {i}",
+                       max_tol=0.2, rms_tol=0.005)
