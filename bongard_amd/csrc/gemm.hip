@@ -54,13 +54,17 @@ struct TileInfo {
 
 // step_us and fixed_us: least squares over 600 measured (shape, tile, split) times of FP8
 // linear GEMMs (M 64 .. 16384, five (N, K) of the text layer, every tile and 2-4 splits),
-// together with the constants of plan_cost. Picking by them loses at most 7% on one of those
-// shapes and under 4% on the others; per-tile rates with two steps of overhead a round picked up
+// together with the constants of linear_cost. Picking by them loses 0.9% on average against the
+// best measured plan, 15% at most (M = 64: 2 us); per-tile rates with two steps of overhead a round picked up
 // to 22% slower plans (M = 2048, N = 2560, K = 10240 on 192x256 82.0 us, 256x160 in two K pieces
 // 67.0; M = 4096, N = 10240, K = 2560 on 256x160 117.5 us, eight-wave 256x256 101.5; M = 4096,
-// N = 2048, K = 2560 on 128x128 28.5 us, 160x256 25.8). geglu_rate: time per K step of one
-// workgroup, with every CU busy, over the tile's FLOP per step. Tiles never picked by cost
-// (1e3): run by an override or in place of a twin.
+// N = 2048, K = 2560 on 128x128 28.5 us, 160x256 25.8). The eight-wave tile's pair
+// is the one whose picks are best over these and 18 shapes of long K (48-160 steps), where it
+// runs 15-20% over its fit on the shorter ones as no other tile does: that fit
+// (1.097, 14.07) put M = 8192, N = 2560, K = 10240 on
+// its tail split (196 us; 256x160 186) and M = 2048, K = 20480 on three pieces (126; 256x160 in
+// two 109). geglu_rate: time per K step of one workgroup, with every CU busy, over the tile's
+// FLOP per step. Tiles never picked by cost (1e3): run by an override or in place of a twin.
 constexpr TileInfo kTiles[NUM_TILES] = {
     {256, 256, 1, 1e3, 1e3, 8.8, "256x256", true},
     {256, 160, 1, 1.006, 8.19, 8.0, "256x160", true},
@@ -73,8 +77,8 @@ constexpr TileInfo kTiles[NUM_TILES] = {
     {128, 64, 1, 1e3, 1e3, 0.0, "128x64k2", false},
     {64, 128, 1, 1e3, 1e3, 0.0, "64x128k2", false},
     {128, 128, 1, 1e3, 1e3, 0.0, "128x128k2", false},
-    {256, 256, 1, 1.097, 14.07, 9.2, "256x256w8", true},
-    {256, 256, 1, 1.097, 14.07, 0.0, "256x256w8x", false},
+    {256, 256, 1, 1.30, 12.0, 9.2, "256x256w8", true},
+    {256, 256, 1, 1.30, 12.0, 0.0, "256x256w8x", false},
 };
 // Whether `tile` has a gated-GELU variant for I = N / 2: tiles of 128 or 64 H columns take
 // any I (a multiple of 128); the 256x160 tile (80 gate + 80 up columns, one wave column)
