@@ -17,8 +17,7 @@
 //   axis_row_kernel      one pass over x: per-row amax -> scale -> cast (row output), and
 //                        per-block column amax partials (bf16 keys) for the column scales;
 //   axis_col_scale_kernel the column partials -> per-column scale and scale_inv;
-//   axis_col_cast_kernel  second pass over x: per-column cast through a wave-level LDS
-//                        transpose.
+//   axis_col_cast_kernel  second pass over x: per-column cast, turned in LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -33,7 +32,9 @@ constexpr int kAxMaxCols = 16384;       // widest row the row kernel holds in re
 constexpr int kAxBlocksPartials = 512;  // row-kernel blocks when it writes column partials
 constexpr int kAxBlocksPlain = 2048;    // ... when it does not
 constexpr int kColNT = 256;
-constexpr int kCT = 64;                 // column-cast tile (rows x cols)
+constexpr int kScaleNT = 1024;          // threads of the column-scale kernel
+constexpr int kCT = 128;                // column-cast tile (rows x cols)
+constexpr int kCPitch = kCT / 4 + 1;    // dwords per staged row (odd)
 constexpr int kMaxColCastBlocks = 2048;
 
 // |x| keys of two packed bf16: clearing the sign makes the unsigned order of each half the
@@ -42,12 +43,17 @@ __device__ __forceinline__ uint4 abs_keys(uint4 v) {
   return make_uint4(v.x & 0x7FFF7FFFu, v.y & 0x7FFF7FFFu, v.z & 0x7FFF7FFFu, v.w & 0x7FFF7FFFu);
 }
 
-// Quantize 8 bf16 values with one scale each.
-template <int FMT>
+// Quantize 8 bf16 values with one scale each. FINITE: no value and no scale is inf or NaN.
+template <int FMT, bool FINITE>
 __device__ __forceinline__ uint2 quant8_bf16_vs(uint4 v, const float* sc) {
   const float x0 = bf16_lo(v.x), x1 = bf16_hi(v.x), x2 = bf16_lo(v.y), x3 = bf16_hi(v.y);
   const float x4 = bf16_lo(v.z), x5 = bf16_hi(v.z), x6 = bf16_lo(v.w), x7 = bf16_hi(v.w);
   uint2 r;
+  if constexpr (FINITE) {
+    r.x = quant4_finite<FMT, true>(x0 * sc[0], x1 * sc[1], x2 * sc[2], x3 * sc[3]);
+    r.y = quant4_finite<FMT, true>(x4 * sc[4], x5 * sc[5], x6 * sc[6], x7 * sc[7]);
+    return r;
+  }
   r.x = quant4<FMT>(x0 * sc[0], x1 * sc[1], x2 * sc[2], x3 * sc[3], x0, x1, x2, x3, sc[0]);
   r.y = quant4<FMT>(x4 * sc[4], x5 * sc[5], x6 * sc[6], x7 * sc[7], x4, x5, x6, x7, sc[4]);
   // quant4 takes one scale for the sign of a NaN product; patch lanes whose own scale is
@@ -88,6 +94,10 @@ __device__ __forceinline__ uint32_t group_max(uint32_t m) {
 // Rows [blockIdx.x * strip, + strip) of x, one row per TPR-thread group at a time (strip is
 // a multiple of the kAxNT / TPR groups, so every group runs the same number of steps).
 // Thread tl of a group holds the row's 16-byte vectors tl, tl + TPR, ... (V of them).
+// The next row's vectors are loaded before the current row's maximum is known, and V is the
+// row's exact number of vectors per thread. Memory-bound: rows alone (2 B read, 1 B written per
+// element) [4096, 10240] 25.1 us with V rounded up to 8 and no load ahead, 22.5 so (5.6 TB/s);
+// [2560, 10240] 17.2 and 15.7.
 // out / row_sinv: per-row quantization (NULL: skipped). colpart: per-block max |x| keys
 // of each column (bf16 keys, [gridDim.x][cols]), or NULL.
 template <int FMT, int TPR, int V>
@@ -102,16 +112,23 @@ __global__ __launch_bounds__(kAxNT) void axis_row_kernel(
 #pragma unroll
   for (int j = 0; j < V; ++j) ck[j] = make_uint4(0u, 0u, 0u, 0u);
   const int r0 = blockIdx.x * strip;
-  for (int rr = g; rr < strip; rr += G) {
-    const int r = r0 + rr;
-    const bool valid = r < rows;
+  uint4 next[V];
+  auto load = [&](int r) {
     const uint4* xr = reinterpret_cast<const uint4*>(x + (int64_t)r * cols);
-    uint4 xv[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const int v = tl + TPR * j;
-      xv[j] = (valid && v < nvec) ? xr[v] : make_uint4(0u, 0u, 0u, 0u);
+      next[j] = (r < rows && v < nvec) ? xr[v] : make_uint4(0u, 0u, 0u, 0u);
     }
+  };
+  load(r0 + g);
+  for (int rr = g; rr < strip; rr += G) {
+    const int r = r0 + rr;
+    const bool valid = r < rows;
+    uint4 xv[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) xv[j] = next[j];
+    if (rr + G < strip) load(r + G);  // in flight during this row's reduction and cast
     uint32_t m = 0;
 #pragma unroll
     for (int j = 0; j < V; ++j) m = max(m, absmax_key8(xv[j]));
@@ -130,10 +147,18 @@ __global__ __launch_bounds__(kAxNT) void axis_row_kernel(
       if (row_sinv && tl == 0) row_sinv[r] = sinv;
       if (out) {
         uint2* orow = reinterpret_cast<uint2*>(out + (int64_t)r * cols);
+        if (__builtin_expect(m < 0x7F800000u, 1)) {
 #pragma unroll
-        for (int j = 0; j < V; ++j) {
-          const int v = tl + TPR * j;
-          if (v < nvec) orow[v] = quant8_bf16<FMT>(xv[j], scale);
+          for (int j = 0; j < V; ++j) {
+            const int v = tl + TPR * j;
+            if (v < nvec) orow[v] = quant8_bf16_finite<FMT, true>(xv[j], scale);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < V; ++j) {
+            const int v = tl + TPR * j;
+            if (v < nvec) orow[v] = quant8_bf16<FMT>(xv[j], scale);
+          }
         }
       }
     }
@@ -175,112 +200,122 @@ __global__ __launch_bounds__(kAxNT) void axis_row_kernel(
 }
 
 // Column scales from the row kernel's partials [nblk][cols]: a block covers 64 columns
-// (8 threads x 8 columns) and splits the nblk partial rows over 32 thread rows.
+// (8 threads x 8 columns) and splits the nblk partial rows over 128 thread rows, so that each
+// thread's few loads are in flight together; one thread per column computes its scale.
+// Latency-bound: at 512 partial rows of 2560 columns 256 threads, whose last 8 computed 8
+// scales each (fp64 divisions) one after the other, took 6.0 us, this 4.9.
 template <int FMT>
-__global__ __launch_bounds__(kColNT) void axis_col_scale_kernel(
+__global__ __launch_bounds__(kScaleNT) void axis_col_scale_kernel(
     const uint16_t* __restrict__ colpart, int nblk, int cols, int pow2,
     float* __restrict__ col_scale, float* __restrict__ col_sinv) {
-  __shared__ uint4 red[32][8];
+  constexpr int kTR = kScaleNT / 8, kW = kScaleNT / 64;
+  __shared__ uint4 red[kW][8];
   const int cg = threadIdx.x & 7, rg = threadIdx.x >> 3;
   const int nvec = cols >> 3;
   const int v = blockIdx.x * 8 + cg;
-  uint4 k = make_uint4(0u, 0u, 0u, 0u);
+  uint32_t k[4] = {0u, 0u, 0u, 0u};
   if (v < nvec) {
-    // four independent loads in flight per thread (the partial rows are a latency-bound
-    // gather of ~nblk / 32 loads each)
     const uint4* src = reinterpret_cast<const uint4*>(colpart);
-    uint4 k4[4] = {k, k, k, k};
-    int b = rg;
-    for (; b + 96 < nblk; b += 128) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint4 o = src[(int64_t)(b + 32 * u) * nvec + v];
-        k4[u] = make_uint4(pk_max_u16(k4[u].x, o.x), pk_max_u16(k4[u].y, o.y),
-                           pk_max_u16(k4[u].z, o.z), pk_max_u16(k4[u].w, o.w));
-      }
-    }
-    for (; b < nblk; b += 32) {
-      const uint4 o = src[(int64_t)b * nvec + v];
-      k4[0] = make_uint4(pk_max_u16(k4[0].x, o.x), pk_max_u16(k4[0].y, o.y),
-                         pk_max_u16(k4[0].z, o.z), pk_max_u16(k4[0].w, o.w));
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      k = make_uint4(pk_max_u16(k.x, k4[u].x), pk_max_u16(k.y, k4[u].y), pk_max_u16(k.z, k4[u].z),
-                     pk_max_u16(k.w, k4[u].w));
-  }
-  red[rg][cg] = k;
-  __syncthreads();
-  if (rg != 0 || v >= nvec) return;
 #pragma unroll 4
-  for (int i = 1; i < 32; ++i) {
-    const uint4 o = red[i][cg];
-    k = make_uint4(pk_max_u16(k.x, o.x), pk_max_u16(k.y, o.y), pk_max_u16(k.z, o.z),
-                   pk_max_u16(k.w, o.w));
+    for (int b = rg; b < nblk; b += kTR) {
+      const uint4 o = src[(int64_t)b * nvec + v];
+      k[0] = pk_max_u16(k[0], o.x);
+      k[1] = pk_max_u16(k[1], o.y);
+      k[2] = pk_max_u16(k[2], o.z);
+      k[3] = pk_max_u16(k[3], o.w);
+    }
   }
-  const uint32_t w[4] = {k.x, k.y, k.z, k.w};
+  // the 8 thread rows of a wave, then the waves
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const uint32_t key = ((w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu) << 16;
-    float scale, sinv;
-    scale_from_amax_key(key, Fp8Max<FMT>::value, pow2 != 0, scale, sinv);
-    col_scale[v * 8 + e] = scale;
-    col_sinv[v * 8 + e] = sinv;
+  for (int off = 8; off < 64; off <<= 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) k[i] = pk_max_u16(k[i], (uint32_t)__shfl_xor((int)k[i], off, 64));
   }
+  if ((threadIdx.x & 63) < 8) red[threadIdx.x >> 6][cg] = make_uint4(k[0], k[1], k[2], k[3]);
+  __syncthreads();
+  const int c = blockIdx.x * 64 + threadIdx.x;
+  if (threadIdx.x >= 64 || c >= cols) return;
+  uint32_t m = 0;
+#pragma unroll
+  for (int w = 0; w < kW; ++w)
+    m = max(m, (uint32_t)reinterpret_cast<const uint16_t*>(red[w])[threadIdx.x]);
+  float scale, sinv;
+  scale_from_amax_key(m << 16, Fp8Max<FMT>::value, pow2 != 0, scale, sinv);
+  col_scale[c] = scale;
+  col_sinv[c] = sinv;
 }
 
-// q_t [cols, rows] = per-column cast of x: one 64 x 64 tile per wave (grid-stride), loaded
-// as eight 8-row x 128-byte pieces, cast with the lane's 8 column scales, staged in the
-// wave's own LDS region and stored transposed (wave_transpose64_staged), as the tensorwise
-// cast-transpose does with one scale per column.
+// q_t [cols, rows] = per-column cast of x. A block takes 128 x 128 tiles, each wave 32 rows of
+// all 128 columns: lane l holds columns 8 (l & 15) .. +7 of the rows 4 k + l / 16, k < 8, and
+// casts them with its 8 column scales; the bytes meet in LDS and each wave turns 32 columns of
+// all 128 rows, so that every store instruction writes whole 128-byte lines.
+// Memory-bound: 2 B read (x again, from the MALL where it fits), 1 B written per element. On
+// 64 x 64 tiles per wave, whose stores were half lines: [10240, 2560] 20.9 us, now 15.6
+// (5.0 TB/s); [4096, 10240] 25.9 and 23.7 us (5.3 TB/s).
 template <int FMT>
 __global__ __launch_bounds__(kColNT) void axis_col_cast_kernel(
     const uint16_t* __restrict__ x, int64_t rows, int64_t cols,
     const float* __restrict__ col_scale, uint8_t* __restrict__ out_t) {
-  constexpr int kWaves = kColNT / 64;
-  __shared__ uint32_t stage[kWaves][kWaveTileDwords];
+  __shared__ uint32_t stage[kCT * kCPitch];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int64_t tiles_c = (cols + kCT - 1) / kCT;
   const int64_t ntiles = tiles_c * ((rows + kCT - 1) / kCT);
   const bool t16 = (rows & 15) == 0;
-  const int ch = lane & 7;
-  uint32_t* lds = stage[wid];
-  for (int64_t tile_id = (int64_t)blockIdx.x * kWaves + wid; tile_id < ntiles;
-       tile_id += (int64_t)gridDim.x * kWaves) {
-    const int64_t r0 = (tile_id / tiles_c) * kCT, c0 = (tile_id % tiles_c) * kCT;
-    const int64_t c = c0 + 8 * ch;
-    const bool cv = c < cols;
+  const int cl = lane & 15, lr = lane >> 4;
+  for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int64_t r0 = (t / tiles_c) * kCT, c0 = (t % tiles_c) * kCT;
+    const int64_t c = c0 + 8 * cl;
     uint4 v[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const int64_t r = r0 + 8 * k + (lane >> 3);
+      const int64_t r = r0 + 32 * wid + 4 * k + lr;
       v[k] = make_uint4(0u, 0u, 0u, 0u);
-      if (r < rows && cv) v[k] = *reinterpret_cast<const uint4*>(x + r * cols + c);
+      if (r < rows && c < cols) v[k] = *reinterpret_cast<const uint4*>(x + r * cols + c);
     }
     float sc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (cv) {
+    if (c < cols) {
       const float4 s0 = reinterpret_cast<const float4*>(col_scale + c)[0];
       const float4 s1 = reinterpret_cast<const float4*>(col_scale + c)[1];
       sc[0] = s0.x; sc[1] = s0.y; sc[2] = s0.z; sc[3] = s0.w;
       sc[4] = s1.x; sc[5] = s1.y; sc[6] = s1.z; sc[7] = s1.w;
     }
+    // a column of finite values has a finite scale above 0; an inf gives 0, a NaN gives NaN
+    bool special = false;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int lr = 8 * k + (lane >> 3);
-      const uint2 q = quant8_bf16_vs<FMT>(v[k], sc);
-      lds[lr * kWaveTilePitch + 2 * ch] = q.x;
-      lds[lr * kWaveTilePitch + 2 * ch + 1] = q.y;
+    for (int e = 0; e < 8; ++e) special |= c < cols && !(sc[e] > 0.f);
+    if (__builtin_expect(__any(special), 0)) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint2 q = quant8_bf16_vs<FMT, false>(v[k], sc);
+        uint32_t* d = stage + (32 * wid + 4 * k + lr) * kCPitch + 2 * cl;
+        d[0] = q.x;
+        d[1] = q.y;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint2 q = quant8_bf16_vs<FMT, true>(v[k], sc);
+        uint32_t* d = stage + (32 * wid + 4 * k + lr) * kCPitch + 2 * cl;
+        d[0] = q.x;
+        d[1] = q.y;
+      }
     }
+    __syncthreads();
+    // lane: 16 rows (lane & 7) x 4 columns (lane >> 3) of the wave's 32 columns
+    const int rg = (lane & 7) * 16, cg = 8 * wid + (lane >> 3);
+    uint32_t d[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) d[i] = stage[(rg + i) * kCPitch + cg];
     uint4 tq[4];
-    wave_transpose64_staged(lds, lane, tq);
-    const int64_t tc = r0 + (lane >> 4) * 16;  // column of out_t (a row of x)
+    transpose_4x16(d, tq);
+    const int64_t tc = r0 + rg;  // column of out_t (a row of x)
     if (tc < rows) {
 #pragma unroll
       for (int cc = 0; cc < 4; ++cc) {
-        const int64_t tr = c0 + 4 * (lane & 15) + cc;  // row of out_t (a column of x)
+        const int64_t tr = c0 + 4 * cg + cc;  // row of out_t (a column of x)
         if (tr >= cols) continue;
         uint8_t* dst = out_t + tr * rows + tc;
-        if (t16 && tc + 16 <= rows) {
+        if (t16) {
           *reinterpret_cast<uint4*>(dst) = tq[cc];
         } else {
           const uint32_t w[4] = {tq[cc].x, tq[cc].y, tq[cc].z, tq[cc].w};
@@ -289,6 +324,7 @@ __global__ __launch_bounds__(kColNT) void axis_col_cast_kernel(
         }
       }
     }
+    __syncthreads();
   }
 }
 
@@ -302,7 +338,7 @@ AxisPlan axis_plan(int64_t rows, int64_t cols, bool colwise) {
   const int64_t nvec = cols / 8;
   p.tpr = cols <= 4096 ? 64 : 256;
   const int64_t per = (nvec + p.tpr - 1) / p.tpr;
-  p.v = per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : 8;
+  p.v = (int)per;  // <= 8: cols <= kAxMaxCols
   p.groups = kAxNT / p.tpr;
   const int64_t cap = colwise ? kAxBlocksPartials : kAxBlocksPlain;
   int64_t strip = (rows + cap - 1) / cap;
@@ -325,7 +361,11 @@ void launch_row(const AxisPlan& p, const uint16_t* x, int rows, int cols, int po
   switch (p.v) {
     case 1: BF8_AXIS_ROW(1); break;
     case 2: BF8_AXIS_ROW(2); break;
+    case 3: BF8_AXIS_ROW(3); break;
     case 4: BF8_AXIS_ROW(4); break;
+    case 5: BF8_AXIS_ROW(5); break;
+    case 6: BF8_AXIS_ROW(6); break;
+    case 7: BF8_AXIS_ROW(7); break;
     default: BF8_AXIS_ROW(8); break;
   }
 #undef BF8_AXIS_ROW
@@ -345,12 +385,11 @@ int run_axiswise(const uint16_t* x, int rows, int cols, int pow2, uint8_t* out, 
   if (rc != BF8_OK || !colwise) return rc;
   float* col_scale = reinterpret_cast<float*>(ws + p.part_bytes);
   hipLaunchKernelGGL(axis_col_scale_kernel<FMT>, dim3((unsigned)((cols / 8 + 7) / 8)),
-                     dim3(kColNT), 0, s, colpart, p.blocks, cols, pow2, col_scale, col_sinv);
+                     dim3(kScaleNT), 0, s, colpart, p.blocks, cols, pow2, col_scale, col_sinv);
   rc = launch_status("axis_col_scale_kernel");
   if (rc != BF8_OK) return rc;
   const int64_t tiles = ((int64_t)(rows + kCT - 1) / kCT) * ((cols + kCT - 1) / kCT);
-  const unsigned grid = (unsigned)std::min<int64_t>((tiles + kColNT / 64 - 1) / (kColNT / 64),
-                                                    kMaxColCastBlocks);
+  const unsigned grid = (unsigned)std::min<int64_t>(tiles, kMaxColCastBlocks);
   hipLaunchKernelGGL(axis_col_cast_kernel<FMT>, dim3(grid), dim3(kColNT), 0, s, x,
                      (int64_t)rows, (int64_t)cols, col_scale, out_t);
   return launch_status("axis_col_cast_kernel");

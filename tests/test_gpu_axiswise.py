@@ -51,6 +51,31 @@ def test_quantize_axiswise_bit_exact(gpu, rows, cols, fmt):
         assert torch.equal(q.col_sinv.cpu(), cs[0].reciprocal())
 
 
+@pytest.mark.parametrize("rows,cols", [(128, 128), (127, 1536), (129, 144), (272, 3072),
+                                       (385, 3584), (1040, 272)])
+def test_quantize_axiswise_tile_edges(gpu, rows, cols):
+    """Whole and partial 128 x 128 column-cast tiles, rows of 1 to 7 vectors per thread, and
+    tiles with and without a column whose scale is 0 (inf) or NaN, against the oracle bit for
+    bit (a NaN column's bytes modulo the sign, as in the test below)."""
+    x = _x(rows, cols, rows + cols)
+    x[rows - 1, cols - 3] = float("inf")
+    x[rows // 2, cols - 7] = float("nan")
+    x[rows // 3, cols - 11] = float("-inf")
+    q = ops.quantize_axiswise(x.to(gpu), ops.E4M3, rowwise=True, colwise=True)
+    torch.cuda.synchronize()
+    rq, rs = orc.quantize_axiswise(x, ops.E4M3, -1)
+    cq, cs = orc.quantize_axiswise(x, ops.E4M3, 0)
+    assert torch.equal(q.data.view(torch.uint8).cpu(), rq)
+    rfin = ~rs[:, 0].isnan()
+    assert torch.equal(q.row_sinv.cpu()[rfin], rs[:, 0].reciprocal()[rfin])
+    got, want = q.data_t.view(torch.uint8).cpu(), cq.t().contiguous()
+    nan_col = cs[0].isnan()[:, None]
+    assert torch.equal(torch.where(nan_col, got & 0x7F, got),
+                       torch.where(nan_col, want & 0x7F, want))
+    finite = ~cs[0].isnan()
+    assert torch.equal(q.col_sinv.cpu()[finite], cs[0].reciprocal()[finite])
+
+
 def test_quantize_axiswise_one_side_and_specials(gpu):
     x = _x(96, 256, 5)
     x[10, 4] = float("nan")
