@@ -167,7 +167,8 @@ class FusedMLP(_ScalingExtraState, torch.nn.Module):
                 normed = _rms_norm(flat, self.layer_norm_weight, self.eps)
             out = _linear.Fp8GegluMlpMxFunction.apply(normed, self.fc1_weight, self.fc2_weight,
                                                       gu_q, down_q, self.intermediate_size)
-            return out[:length].reshape_as(x)
+            # sliced only if padded: a slice's backward fills and copies the whole gradient
+            return (out if length == flat.shape[0] else out[:length]).reshape_as(x)
         count = _ops.rmsnorm_partials_count(flat.shape[0])
         if not _ops.rmsnorm_supported(flat.shape[1]):
             # rows wider than the fused kernel holds in registers: norm in torch ops on the
@@ -208,7 +209,7 @@ class FusedMLP(_ScalingExtraState, torch.nn.Module):
         h, h_partials = _linear.GegluGateUpNvfp4Function.apply(normed, self.fc1_weight, gu_q,
                                                                 self.intermediate_size, parts)
         out = _linear.Fp8LinearNvfp4Function.apply(h, self.fc2_weight, down_q, h_partials)
-        return out[:length].reshape_as(x)
+        return (out if length == flat.shape[0] else out[:length]).reshape_as(x)
 
 
 def enable_fused_mlp(model, recipe):

@@ -317,11 +317,14 @@ class GegluFunction(torch.autograd.Function):
         H, parts = ops.geglu(GU)
         ctx.save_for_backward(GU)
         ctx.mark_non_differentiable(parts)
+        ctx.set_materialize_grads(False)  # no zeros for the partials' absent gradient
         return H, parts
 
     @staticmethod
     def backward(ctx, dH, _d_partials):
         (GU,) = ctx.saved_tensors
+        if dH is None:
+            dH = GU.new_zeros(GU.shape[0], GU.shape[1] // 2)
         dGU, _ = ops.geglu_bwd(dH.contiguous(), GU)
         return dGU
 
@@ -360,12 +363,15 @@ class GegluGateUpNvfp4Function(_Fp8Function):
                               wq.scales_t if need_dx else None, wq.meta)
         ctx.wq = wq if need_dx and wq.cache_dequant else None
         ctx.mark_non_differentiable(h_partials)
+        ctx.set_materialize_grads(False)  # no zeros for the partials' absent gradient
         return H, h_partials
 
     @staticmethod
     def backward(ctx, dH, _d_partials):
         GU, x4t, xst, x_meta, w4t, wst, w_meta = ctx.saved_tensors
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        if dH is None:
+            dH = GU.new_zeros(GU.shape[0], GU.shape[1] // 2)
         dGU, dparts = ops.geglu_bwd(dH.contiguous(), GU)
         dq = ops.quantize_nvfp4(dGU, rowwise=need_dx, colwise=need_dw, partials=dparts,
                                 dequant_rows=True, dequant_cols=True)
