@@ -16,6 +16,9 @@
 // stores are plain 16-byte vector accesses, several in flight per lane (the non-temporal
 // hint measured up to 30% slower on gfx950 for these streams).
 //
+// A tensor of at most kSmallQuantMax elements takes both passes in one launch, every block
+// reading the whole tensor for its amax (quantize_small_kernel).
+//
 // Delayed scaling (amax history, TE DelayedScaling semantics) needs no pre-pass: the
 // cast kernel derives the scale from the history (after folding in the previous step's
 // amax partials) and writes this step's amax partials while it casts, so a delayed
@@ -57,6 +60,11 @@ constexpr int64_t kMaxCastBlocks = 2048;  // 8 blocks per CU
 // Consumers reduce up to this many partials in every block; a longer list (the gated-GELU
 // GEMM writes one per tile: 5200 at M = 16.6k) is first reduced by a one-block kernel.
 constexpr int64_t kMaxInlinePartials = 2048;
+// Largest tensor (elements) that bf8_quantize_bf16 quantizes in one launch (rowwise copy only):
+// up to here the launch saved is worth more than the extra reading. Host-bound calls in a row
+// 12.1 us with two launches, 9.6 with one (16K .. 256K elements alike); the device time alone,
+// replayed from a graph, 4.95 and 4.15 us at 16K, 5.6 and 5.8 at 100K, 5.7 and 8.4 at 200K.
+constexpr int64_t kSmallQuantMax = 192 * 1024;
 // Slots of the library-owned scratch of bf8_quantize_bf16_noalloc: the most amax partials
 // any tensor's quantization writes.
 constexpr int64_t kNoAllocSlots = kMaxAmaxBlocks;
@@ -222,6 +230,50 @@ __global__ __launch_bounds__(kNT) void cast_kernel(const uint16_t* __restrict__ 
                                                    ScaleSrc src, uint8_t* __restrict__ out,
                                                    uint32_t* __restrict__ amax_out) {
   cast_body<FMT>(x, n, src, out, amax_out, blockIdx.x, gridDim.x);
+}
+
+// Amax and cast of a small tensor in one launch: every block reads all of x for the amax (from
+// its XCD's L2 after the first), then casts its own kSmallNT groups of 16, which each thread
+// loads before. A call this small is bound by its launches and their host time, not by the
+// nblk-fold read (64 x 2560: 12.1 us for the two launches, 9.6 for this one; longer or
+// overlapped batches of loads measured slower).
+constexpr int kSmallNT = 1024;
+template <int FMT>
+__global__ __launch_bounds__(kSmallNT) void quantize_small_kernel(
+    const uint16_t* __restrict__ x, int64_t n, int pow2, uint8_t* __restrict__ out,
+    float* __restrict__ meta) {
+  const uint4* xv = reinterpret_cast<const uint4*>(x);
+  const int64_t nvec = n >> 3, n16 = n >> 4;
+  const int64_t i = (int64_t)blockIdx.x * kSmallNT + threadIdx.x;
+  uint4 c0 = make_uint4(0u, 0u, 0u, 0u), c1 = c0;
+  if (i < n16) { c0 = xv[2 * i]; c1 = xv[2 * i + 1]; }
+  uint32_t m = 0;
+  for (int64_t j = threadIdx.x; j < nvec; j += (int64_t)kVecPerThread * kSmallNT) {
+    uint4 v[kVecPerThread];
+#pragma unroll
+    for (int k = 0; k < kVecPerThread; ++k)
+      v[k] = j + k * kSmallNT < nvec ? xv[j + k * kSmallNT] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int k = 0; k < kVecPerThread; ++k) m = max(m, absmax_key8(v[k]));
+  }
+  const int64_t tail = (nvec << 3) + threadIdx.x;
+  if (tail < n) m = max(m, (uint32_t)(x[tail] & 0x7FFFu) << 16);
+  m = block_max_u32<kSmallNT>(m);
+  float scale, sinv;
+  scale_from_amax_key(m, Fp8Max<FMT>::value, pow2 != 0, scale, sinv);
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    write_meta_from_amax(m, Fp8Max<FMT>::value, meta, pow2 != 0);
+  if (i < n16) {
+    const uint2 q0 = quant8_bf16<FMT>(c0, scale), q1 = quant8_bf16<FMT>(c1, scale);
+    reinterpret_cast<uint4*>(out)[i] = make_uint4(q0.x, q0.y, q1.x, q1.y);
+  }
+  if (blockIdx.x == 0) {
+    const int64_t j = (n16 << 4) + threadIdx.x;
+    if (j < n) {
+      const float xf = __uint_as_float((uint32_t)x[j] << 16);
+      out[j] = (uint8_t)(quant4<FMT>(xf * scale, 0.f, 0.f, 0.f, xf, 0.f, 0.f, 0.f, scale) & 0xFFu);
+    }
+  }
 }
 
 // Cast with a transposed copy, over kTR x 64 tiles of x, one tile per wave (grid-stride,
@@ -716,6 +768,18 @@ int bf8_quantize_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_
   BF8_CHECK(!out_t || cols % 16 == 0,
             "bf8_quantize_bf16: transposed cast needs cols %% 16 == 0 (got %lld)", (long long)cols);
   const int64_t n = rows * cols;
+  if (out && !out_t && n > 0 && n <= kSmallQuantMax) {
+    BF8_CHECK(x != nullptr && partials != nullptr, "bf8_quantize_bf16: x or partials is NULL");
+    const unsigned blocks = (unsigned)(n / 16 / kSmallNT + 1);
+    const int pow2 = (fmt & BF8_SCALE_POW2) ? 1 : 0;
+    if ((fmt & ~BF8_SCALE_POW2) == BF8_E4M3)
+      hipLaunchKernelGGL(quantize_small_kernel<BF8_E4M3>, dim3(blocks), dim3(kSmallNT), 0,
+                         as_stream(stream), (const uint16_t*)x, n, pow2, out, meta);
+    else
+      hipLaunchKernelGGL(quantize_small_kernel<BF8_E5M2>, dim3(blocks), dim3(kSmallNT), 0,
+                         as_stream(stream), (const uint16_t*)x, n, pow2, out, meta);
+    return launch_status("quantize_small_kernel");
+  }
   int rc = bf8_amax_bf16(x, n, partials, stream);
   if (rc) return rc;
   return bf8_cast_partials_bf16(x, rows, cols, partials, amax_blocks(n), fmt, meta, out, out_t,

@@ -161,6 +161,27 @@ def test_quantize_many_equals_quantize(gpu):
         assert torch.equal(q.meta, r.meta)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 5), (1, 16), (7, 33), (64, 256), (65, 2560),
+                                       (1, 16385), (192, 1024), (193, 1024)])
+@pytest.mark.parametrize("special", [None, "inf", "nan", "zero"])
+def test_quantize_one_launch_equals_two(gpu, rows, cols, special):
+    """A small tensor's one-launch quantization (up to 192 x 1024 elements, and the first size
+    past it) against the amax and cast passes of quantize_many: the same bytes and meta."""
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols)).bfloat16()
+    if special == "zero":
+        x.zero_()
+    elif special:
+        x.view(-1)[-1] = float(special)   # the last element: the tail of n % 16
+    x = x.to(gpu)
+    for fmt in (ops.E4M3, ops.E5M2):
+        for pow2 in (False, True):
+            one = ops.quantize(x, fmt, pow2=pow2)
+            two = ops.quantize_many([x], fmt, pow2=pow2)[0]
+            torch.cuda.synchronize()
+            assert torch.equal(one.data.view(torch.uint8), two.data.view(torch.uint8))
+            assert torch.equal(one.meta.view(torch.int32), two.meta.view(torch.int32))
+
+
 def test_quantize_many_rejects_bad_lists(gpu):
     x = torch.randn(64, 64, device=gpu).to(torch.bfloat16)
     with pytest.raises(ValueError):
