@@ -9,7 +9,7 @@ from ctypes import c_float, c_int, c_int64, c_size_t, c_uint32, c_void_p, POINTE
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().with_name("libbongard_fp8.so")
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 # name -> (restype, argtypes); mirrors include/bongard_fp8.h one to one.
 SIGNATURES = {
@@ -84,6 +84,8 @@ SIGNATURES = {
     "bf8_quantize_nvfp4_dequant2_bf16": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int64,
                                                  c_void_p, c_void_p, c_void_p, c_void_p,
                                                  c_void_p, c_void_p]),
+    "bf8_geglu_bwd_mx_planes": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p,
+                                        c_void_p, c_void_p, c_void_p, c_void_p]),
     "bf8_quantize_mx_planes_bf16": (c_int, [c_void_p, c_int64, c_int64, c_int, c_void_p,
         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "bf8_quantize_mx_many_planes_bf16": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p,

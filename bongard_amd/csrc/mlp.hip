@@ -33,49 +33,6 @@ int64_t bwd_blocks(int64_t M, int64_t I) {
 }
 
 
-// The chain for 8 elements (4 packed bf16 pairs of dh, g, u): d_g, d_u as packed bf16
-// pairs (NaNs 0xFFFF) and the running amax key of |d_g|, |d_u|. ta / tf: the LDS copies
-// of the gelu tables; all 16 table reads are issued before any is used, gates outside the
-// tables take a wave-uniform slow path.
-__device__ __forceinline__ void geglu_bwd8(const uint32_t (&dhw)[4], const uint32_t (&gw)[4],
-                                           const uint32_t (&uw)[4], const uint16_t* ta,
-                                           const uint32_t* tf, uint32_t (&dg)[4],
-                                           uint32_t (&du)[4], uint32_t& m) {
-  uint32_t outside = 0, ia[4], jf[4], va[8], vf[8];
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    ia[w] = gelu_index2(gw[w], outside);
-    jf[w] = gelu_factor_index2(gw[w], outside);
-  }
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    va[2 * w] = ta[ia[w] & 0xFFFFu];
-    va[2 * w + 1] = ta[ia[w] >> 16];
-    vf[2 * w] = tf[jf[w] & 0xFFFFu];
-    vf[2 * w + 1] = tf[jf[w] >> 16];
-  }
-  if (__builtin_expect(__any(outside != 0), 0)) {
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      va[2 * w] = gelu_finish(gw[w], va[2 * w]);
-      va[2 * w + 1] = gelu_finish(gw[w] >> 16, va[2 * w + 1]);
-      vf[2 * w] = gelu_factor_finish(gw[w], vf[2 * w]);
-      vf[2 * w + 1] = gelu_factor_finish(gw[w] >> 16, vf[2 * w + 1]);
-    }
-  }
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const float d0 = bf16_lo(dhw[w]), d1 = bf16_hi(dhw[w]);
-    const uint32_t a = va[2 * w] | (va[2 * w + 1] << 16);                          // bf16(gelu(g))
-    const uint32_t da = pack_bf16x2(d0 * bf16_lo(uw[w]), d1 * bf16_hi(uw[w]));    // bf16(dh * u)
-    du[w] = nan_ffff_bf16x2(pack_bf16x2(d0 * bf16_lo(a), d1 * bf16_hi(a)));
-    dg[w] = nan_ffff_bf16x2(pack_bf16x2(bf16_lo(da) * __uint_as_float(vf[2 * w]),
-                                        bf16_hi(da) * __uint_as_float(vf[2 * w + 1])));
-    const uint32_t kg = dg[w] & 0x7FFF7FFFu, ku = du[w] & 0x7FFF7FFFu;
-    m = max(m, max(max(kg << 16, kg & 0xFFFF0000u), max(ku << 16, ku & 0xFFFF0000u)));
-  }
-}
-
 // H for 8 elements (4 packed pairs of g, u), with the table reads issued together.
 __device__ __forceinline__ uint4 geglu_fwd8(uint4 g, uint4 u, const uint16_t* ta) {
   const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};

@@ -17,6 +17,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "gelu.hpp"
 
 namespace bf8 {
 namespace {
@@ -161,6 +162,75 @@ __device__ __forceinline__ void mx_tile_body(const MxTile& p, int64_t r0, int64_
   }
 }
 
+// The loaded tile at (r0, c0), by four waves (wid 0 .. 3) that share stage, erow and ecol; every
+// wave of the block calls it alike. A tile with r0 >= p.rows writes nothing.
+template <int FMT>
+__device__ __forceinline__ void mx_tile_finish(const MxTile& p, int64_t r0, int64_t c0,
+                                               const uint4 (&v)[8], uint32_t* stage,
+                                               uint32_t* erow, uint32_t* ecol, int wid, int lane) {
+  uint32_t rk[8], cm[4] = {};
+  uint32_t top = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint32_t a[4] = {v[k].x & 0x7FFF7FFFu, v[k].y & 0x7FFF7FFFu, v[k].z & 0x7FFF7FFFu,
+                           v[k].w & 0x7FFF7FFFu};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cm[i] = pk_max_u16(cm[i], a[i]);
+    uint32_t m = pk_max_u16(pk_max_u16(a[0], a[1]), pk_max_u16(a[2], a[3]));
+    m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true));
+    m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, true));
+    rk[k] = max(m & 0xFFFFu, m >> 16);
+    top = max(top, rk[k]);
+  }
+  if (p.out_t) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 16, 64));
+      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 32, 64));
+    }
+  }
+  uint8_t* ecolb = reinterpret_cast<uint8_t*>(ecol);
+  if (__builtin_expect(__any(top >= 0x7F80u), 0))
+    mx_tile_body<FMT, false>(p, r0, c0, v, rk, cm, stage, erow, ecolb, wid, lane);
+  else
+    mx_tile_body<FMT, true>(p, r0, c0, v, rk, cm, stage, erow, ecolb, wid, lane);
+  if (!p.out_t) return;
+  __syncthreads();
+  {
+    // lane: 16 rows (lane & 7) x 4 columns (lane >> 3) of the wave's 32 columns
+    const int rg = (lane & 7) * 16, cg = 8 * wid + (lane >> 3);
+    uint32_t d[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) d[i] = stage[(rg + i) * kMPitch + cg];
+    uint4 tq[4];
+    transpose_4x16(d, tq);
+    const int64_t tc = r0 + rg;  // column of out_t (a row of x)
+    if (tc < p.rows) {
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) {
+        const int64_t tr = c0 + 4 * cg + cc;  // row of out_t (a column of x)
+        if (tr < p.cols) *reinterpret_cast<uint4*>(p.out_t + tr * p.rows + tc) = tq[cc];
+      }
+    }
+    const int tid = 64 * wid + lane;
+    if (tid < kMT && c0 + tid < p.cols && r0 < p.rows) {
+      // four blocks of one column; the last tile row's absent blocks pad the last dword
+      const uint32_t e4 = ecol[tid];
+      if (p.planes_t) p.planes_t[(r0 >> 7) * p.cols + c0 + tid] = e4;
+      if (p.sc_t) {
+        uint8_t* dst = p.sc_t + (c0 + tid) * p.ld_sc_t + (r0 >> 5);
+        if (((uintptr_t)p.sc_t & 3) == 0) {
+          *reinterpret_cast<uint32_t*>(dst) = e4;
+        } else {
+#pragma unroll
+          for (int b = 0; b < 4; ++b) dst[b] = (uint8_t)(e4 >> (8 * b));
+        }
+      }
+    }
+  }
+  __syncthreads();
+}
+
 // The tiles blk, blk + nblk, .. of p (every thread of the block calls it alike).
 template <int FMT>
 __device__ __forceinline__ void mx_tiles(const MxTile& p, int64_t blk, int64_t nblk,
@@ -169,7 +239,6 @@ __device__ __forceinline__ void mx_tiles(const MxTile& p, int64_t blk, int64_t n
   const int64_t tiles_c = (p.cols + kMT - 1) / kMT, tiles_r = (p.rows + kMT - 1) / kMT;
   const int64_t ntiles = tiles_c * tiles_r;
   const int cl = lane & 15, lr = lane >> 4;
-  const bool sct_dwords = ((uintptr_t)p.sc_t & 3) == 0;
   for (int64_t t = blk; t < ntiles; t += nblk) {
     const int64_t r0 = (t / tiles_c) * kMT, c0 = (t % tiles_c) * kMT;
     const int64_t c = c0 + 8 * cl;
@@ -181,66 +250,109 @@ __device__ __forceinline__ void mx_tiles(const MxTile& p, int64_t blk, int64_t n
       if (r < p.rows && c < p.cols)
         v[k] = *reinterpret_cast<const uint4*>(p.x + r * p.cols + c);
     }
-    uint32_t rk[8], cm[4] = {};
-    uint32_t top = 0;
+    mx_tile_finish<FMT>(p, r0, c0, v, stage, erow, ecol, wid, lane);
+  }
+}
+
+// d_g (G) or d_u of 8 elements: the chain of geglu_bwd8, one half of it.
+template <bool G>
+__device__ __forceinline__ uint4 geglu_bwd8_half(uint4 dh, uint4 g, uint4 u, const uint16_t* ta,
+                                                 const uint32_t* tf) {
+  const uint32_t dw[4] = {dh.x, dh.y, dh.z, dh.w}, gw[4] = {g.x, g.y, g.z, g.w};
+  const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
+  uint32_t outside = 0, ix[4], t[8], o[4];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const uint32_t a[4] = {v[k].x & 0x7FFF7FFFu, v[k].y & 0x7FFF7FFFu, v[k].z & 0x7FFF7FFFu,
-                             v[k].w & 0x7FFF7FFFu};
+  for (int w = 0; w < 4; ++w)
+    ix[w] = G ? gelu_factor_index2(gw[w], outside) : gelu_index2(gw[w], outside);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) cm[i] = pk_max_u16(cm[i], a[i]);
-      uint32_t m = pk_max_u16(pk_max_u16(a[0], a[1]), pk_max_u16(a[2], a[3]));
-      m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true));
-      m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, true));
-      rk[k] = max(m & 0xFFFFu, m >> 16);
-      top = max(top, rk[k]);
+  for (int w = 0; w < 4; ++w) {
+    t[2 * w] = G ? tf[ix[w] & 0xFFFFu] : ta[ix[w] & 0xFFFFu];
+    t[2 * w + 1] = G ? tf[ix[w] >> 16] : ta[ix[w] >> 16];
+  }
+  if (__builtin_expect(__any(outside != 0), 0)) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      t[2 * w] = G ? gelu_factor_finish(gw[w], t[2 * w]) : gelu_finish(gw[w], t[2 * w]);
+      t[2 * w + 1] = G ? gelu_factor_finish(gw[w] >> 16, t[2 * w + 1])
+                       : gelu_finish(gw[w] >> 16, t[2 * w + 1]);
     }
-    if (p.out_t) {
+  }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 16, 64));
-        cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], 32, 64));
+  for (int w = 0; w < 4; ++w) {
+    const float d0 = bf16_lo(dw[w]), d1 = bf16_hi(dw[w]);
+    if constexpr (G) {
+      const uint32_t da = pack_bf16x2(d0 * bf16_lo(uw[w]), d1 * bf16_hi(uw[w]));
+      o[w] = pack_bf16x2(bf16_lo(da) * __uint_as_float(t[2 * w]),
+                         bf16_hi(da) * __uint_as_float(t[2 * w + 1]));
+    } else {
+      const uint32_t a = t[2 * w] | (t[2 * w + 1] << 16);
+      o[w] = pack_bf16x2(d0 * bf16_lo(a), d1 * bf16_hi(a));
+    }
+    o[w] = nan_ffff_bf16x2(o[w]);
+  }
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// d_g or d_u of the lane's eight rows 4 k of a tile, in two batches of loads.
+template <bool G>
+__device__ __forceinline__ void geglu_bwd_rows(const uint16_t* dp, const uint16_t* gp, int64_t I,
+                                               int64_t rows_left, const uint16_t* ta,
+                                               const uint32_t* tf, uint4 (&v)[8]) {
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    uint4 d[4], g[4], u[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = 4 * (4 * q + k);
+      d[k] = g[k] = u[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (row < rows_left) {
+        d[k] = *reinterpret_cast<const uint4*>(dp + row * I);
+        g[k] = *reinterpret_cast<const uint4*>(gp + row * 2 * I);
+        if (G) u[k] = *reinterpret_cast<const uint4*>(gp + row * 2 * I + I);
       }
     }
-    uint8_t* ecolb = reinterpret_cast<uint8_t*>(ecol);
-    if (__builtin_expect(__any(top >= 0x7F80u), 0))
-      mx_tile_body<FMT, false>(p, r0, c0, v, rk, cm, stage, erow, ecolb, wid, lane);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[4 * q + k] = geglu_bwd8_half<G>(d[k], g[k], u[k], ta, tf);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// The gated-GELU backward fused with the quantization of its output: dGU [M, 2I] of dH [M, I]
+// and GU [M, 2I] goes from registers to its MX copies (p: rows M, cols 2I; I % 128 == 0), the
+// bf16 dGU itself is never written. The first four waves of a block take the d_g tile of a
+// 128 x 128 tile of I, the others its d_u tile: neither holds both (one wave holding d_g and d_u
+// spilled 140 registers), and dH and g come from the CU's own cache the second time. The gelu
+// tables (39 KB of LDS) and two stages let two blocks, 16 waves, run on a CU.
+// HBM-bound: 6 B read, 4 B (+ 1/8) written per element of H, where the two passes read 10 B and
+// wrote 8. [4096, 10240]: 73 + 72 us in two passes, 126 in one (3.4 TB/s: at 16 waves a CU the
+// table lookups and the turning are not all hidden; loading the next tile during them spilled).
+constexpr int kBwdNT = 512;
+constexpr int kMaxBwdBlocks = 512;
+template <int FMT>
+__global__ __launch_bounds__(kBwdNT, 4) void geglu_bwd_mx_kernel(
+    const uint16_t* __restrict__ dH, const uint16_t* __restrict__ GU, int64_t I, MxTile p) {
+  __shared__ __attribute__((aligned(16))) uint16_t ta[kGeluABytes / 2];
+  __shared__ __attribute__((aligned(16))) uint32_t tf[kGeluFBytes / 4];
+  __shared__ uint32_t stage[2][kMT * kMPitch];
+  __shared__ uint32_t erow[2][kMT], ecol[2][kMT];
+  load_gelu_tables<kBwdNT>(ta, tf);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wid = (threadIdx.x >> 6) & 3;
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int64_t tiles_c = I / kMT, tiles_r = (p.rows + kMT - 1) / kMT;
+  const int64_t ntiles = tiles_c * tiles_r;
+  const int cl = lane & 15, lr = lane >> 4;
+  for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int64_t r0 = (t / tiles_c) * kMT, c0 = (t % tiles_c) * kMT;
+    const int64_t rw = r0 + 32 * wid + lr;
+    const uint16_t* dp = dH + rw * I + c0 + 8 * cl;
+    const uint16_t* gp = GU + rw * 2 * I + c0 + 8 * cl;
+    uint4 v[8];
+    if (half == 0)
+      geglu_bwd_rows<true>(dp, gp, I, p.rows - rw, ta, tf, v);
     else
-      mx_tile_body<FMT, true>(p, r0, c0, v, rk, cm, stage, erow, ecolb, wid, lane);
-    if (!p.out_t) continue;
-    __syncthreads();
-    {
-      // lane: 16 rows (lane & 7) x 4 columns (lane >> 3) of the wave's 32 columns
-      const int rg = (lane & 7) * 16, cg = 8 * wid + (lane >> 3);
-      uint32_t d[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) d[i] = stage[(rg + i) * kMPitch + cg];
-      uint4 tq[4];
-      transpose_4x16(d, tq);
-      const int64_t tc = r0 + rg;  // column of out_t (a row of x)
-      if (tc < p.rows) {
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
-          const int64_t tr = c0 + 4 * cg + cc;  // row of out_t (a column of x)
-          if (tr < p.cols) *reinterpret_cast<uint4*>(p.out_t + tr * p.rows + tc) = tq[cc];
-        }
-      }
-      if (threadIdx.x < kMT && c0 + threadIdx.x < p.cols) {
-        // four blocks of one column; the last tile row's absent blocks pad the last dword
-        const uint32_t e4 = ecol[threadIdx.x];
-        if (p.planes_t) p.planes_t[(r0 >> 7) * p.cols + c0 + threadIdx.x] = e4;
-        if (p.sc_t) {
-          uint8_t* dst = p.sc_t + (c0 + threadIdx.x) * p.ld_sc_t + (r0 >> 5);
-          if (sct_dwords) {
-            *reinterpret_cast<uint32_t*>(dst) = e4;
-          } else {
-#pragma unroll
-            for (int b = 0; b < 4; ++b) dst[b] = (uint8_t)(e4 >> (8 * b));
-          }
-        }
-      }
-    }
-    __syncthreads();
+      geglu_bwd_rows<false>(dp, gp, I, p.rows - rw, ta, tf, v);
+    mx_tile_finish<FMT>(p, r0, half * I + c0, v, stage[half], erow[half], ecol[half], wid, lane);
   }
 }
 
@@ -313,6 +425,37 @@ int bf8_quantize_mx_planes_bf16(const void* x, int64_t rows, int64_t cols, int f
                    out ? bf8_mx_scale_ld(cols) : 0, out_t, out_t_scales, out_t_planes,
                    bf8_mx_scale_ld(rows), fmt});
   return mx_launch(a, stream);
+}
+
+int bf8_geglu_bwd_mx_planes(const void* dH, const void* GU, int64_t M, int64_t I, int fmt,
+                            uint8_t* out, uint32_t* out_planes, uint8_t* out_t,
+                            uint32_t* out_t_planes, void* stream) {
+  const char* who = "bf8_geglu_bwd_mx_planes";
+  BF8_CHECK(fmt == BF8_E4M3 || fmt == BF8_E5M2, "%s: bad fmt %d", who, fmt);
+  BF8_CHECK(M >= 0 && I >= 0 && I % kMT == 0, "%s: need I %% 128 == 0 (M=%lld, I=%lld)", who,
+            (long long)M, (long long)I);
+  BF8_CHECK((out == nullptr) == (out_planes == nullptr) &&
+                (out_t == nullptr) == (out_t_planes == nullptr) && (out || out_t),
+            "%s: give out with out_planes and/or out_t with out_t_planes", who);
+  BF8_CHECK(!out_t || M % 32 == 0, "%s: columnwise blocks need M %% 32 == 0 (got %lld)", who,
+            (long long)M);
+  if (M == 0 || I == 0) return BF8_OK;
+  BF8_CHECK(dH && GU, "%s: NULL pointer", who);
+  BF8_CHECK((((uintptr_t)dH | (uintptr_t)GU | (uintptr_t)out_t) & 15) == 0 &&
+                ((uintptr_t)out & 7) == 0 &&
+                (((uintptr_t)out_planes | (uintptr_t)out_t_planes) & 3) == 0,
+            "%s: dH, GU, out_t 16-byte, out 8-byte, planes 4-byte aligned", who);
+  const MxTile p{nullptr, M, 2 * I, out, nullptr, out_planes, 0, out_t, nullptr, out_t_planes, 0,
+                 fmt};
+  const int64_t tiles = ((M + kMT - 1) / kMT) * (I / kMT);
+  const dim3 grid((unsigned)std::min<int64_t>(tiles, kMaxBwdBlocks));
+  if (fmt == BF8_E4M3)
+    hipLaunchKernelGGL(geglu_bwd_mx_kernel<BF8_E4M3>, grid, dim3(kBwdNT), 0, as_stream(stream),
+                       (const uint16_t*)dH, (const uint16_t*)GU, I, p);
+  else
+    hipLaunchKernelGGL(geglu_bwd_mx_kernel<BF8_E5M2>, grid, dim3(kBwdNT), 0, as_stream(stream),
+                       (const uint16_t*)dH, (const uint16_t*)GU, I, p);
+  return launch_status("geglu_bwd_mx_kernel");
 }
 
 int bf8_quantize_mx_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,

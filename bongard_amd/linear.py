@@ -474,6 +474,7 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
     @staticmethod
     def backward(ctx, dy):
         GU, x8t, xpt, h8t, hpt, gu8t, gupt, d8t, dpt = ctx.saved_tensors
+        I = ctx.intermediate
         need_dx, need_dgu, need_dd = ctx.needs_input_grad[:3]
         dyq = ops.quantize_mx(dy.contiguous(), E4M3, rowwise=need_dx or need_dgu,
                               colwise=need_dd, scale_rows=False)
@@ -482,9 +483,13 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
             dd = ops.gemm_mx(dyq.data_t, None, h8t, None, a_planes=dyq.planes_t, b_planes=hpt)
         if need_dx or need_dgu:
             dH = ops.gemm_mx(dyq.data, None, d8t, None, a_planes=dyq.planes, b_planes=dpt)
-            dGU, _ = ops.geglu_bwd(dH, GU)
-            dq = ops.quantize_mx(dGU, E4M3, rowwise=need_dx, colwise=need_dgu,
-                                 scale_rows=False)
+            if I % 128 == 0:
+                # d_g and d_u go from registers to their MX copies (whole 128 x 128 tiles of I)
+                dq = ops.geglu_bwd_mx(dH, GU, rowwise=need_dx, colwise=need_dgu)
+            else:
+                dGU, _ = ops.geglu_bwd(dH, GU)
+                dq = ops.quantize_mx(dGU, E4M3, rowwise=need_dx, colwise=need_dgu,
+                                     scale_rows=False)
             if need_dx:
                 dx = ops.gemm_mx(dq.data, None, gu8t, None, a_planes=dq.planes, b_planes=gupt)
             if need_dgu:

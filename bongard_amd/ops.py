@@ -562,6 +562,29 @@ def quantize_mx(x, fmt=E4M3, *, rowwise=True, colwise=False, scale_rows=True):
     return MxFp8Tensor(out, sc, out_t, sc_t, fmt, rows, cols, pl, pl_t)
 
 
+def geglu_bwd_mx(dH, GU, fmt=E4M3, *, rowwise=True, colwise=False):
+    """:func:`geglu_bwd` and the :func:`quantize_mx` of its dGU [M, 2I] in one pass (planes
+    only, the same bytes and scales; the bf16 dGU is not written). I must be a multiple of 128."""
+    _require_gpu(dH, GU)
+    dH = dH.contiguous()
+    M, I = dH.shape
+    GU = _gu_operand("geglu_bwd_mx", GU, M, I)
+    dev = dH.device
+    if not (rowwise or colwise):
+        raise ValueError("geglu_bwd_mx: nothing requested")
+    out = pl = out_t = pl_t = None
+    if rowwise:
+        out = torch.empty((M, 2 * I), dtype=TORCH_FP8[fmt], device=dev)
+        pl = _new_planes(2 * I, M, dev)
+    if colwise:
+        out_t = torch.empty((2 * I, M), dtype=TORCH_FP8[fmt], device=dev)
+        pl_t = _new_planes(M, 2 * I, dev)
+    _lib.check(_lib.lib().bf8_geglu_bwd_mx_planes(
+        _ptr(dH), _ptr(GU), M, I, fmt, _ptr(out), _ptr(pl), _ptr(out_t), _ptr(pl_t),
+        _stream(dev)), "bf8_geglu_bwd_mx_planes")
+    return MxFp8Tensor(out, None, out_t, None, fmt, M, 2 * I, pl, pl_t)
+
+
 def quantize_mx_many(xs, fmts=None, *, scale_rows=True):
     """Rowwise :func:`quantize_mx` of up to 8 bf16 tensors in one launch; each result
     equals that tensor's own ``quantize_mx(x, fmt)`` (bytes and scales). ``fmts``: one

@@ -379,6 +379,16 @@ int bf8_quantize_mx_many_planes_bf16(int count, const void* const* x, const int6
                                      uint8_t* const* out_scales, uint32_t* const* out_planes,
                                      void* stream);
 
+/* bf8_geglu_bwd and the MX quantization of its dGU [M, 2I] in one pass: the same bytes and scale
+ * planes as bf8_quantize_mx_planes_bf16 of bf8_geglu_bwd's output, which is not written. out
+ * [M, 2I] with out_planes and / or out_t [2I, M] with out_t_planes; I % 128 == 0, M % 32 == 0
+ * with out_t.
+ * Replaces the gated-GELU backward and the quantization of its result in TE's LayerNormMLP and
+ * Linear backward under 'mxfp8' (bongard/te_linear.py:98-103, bongard/fused_mlp.py:25-33). */
+int bf8_geglu_bwd_mx_planes(const void* dH, const void* GU, int64_t M, int64_t I, int fmt,
+                            uint8_t* out, uint32_t* out_planes, uint8_t* out_t,
+                            uint32_t* out_t_planes, void* stream);
+
 /* ---------------------------------------------------------------------------------
  * NVFP4 (TE NVFP4BlockScaling under the 'nvfp4' recipe: bongard/te_linear.py:17,38,
  * bongard/fused_mlp.py:9,32). Round to nearest even everywhere, 1-D blocks of 16 along

@@ -254,6 +254,27 @@ def test_gemm_geglu_mx_quant_errors(gpu):
         ops.gemm_geglu_mx_quant(qx.data, qx.scales, qw.data, qw.scales, 256, colwise=True)
 
 
+@pytest.mark.parametrize("M,I", [(32, 128), (96, 384), (128, 256), (160, 128), (1056, 640)])
+@pytest.mark.parametrize("rowwise,colwise", [(True, True), (True, False), (False, True)])
+def test_geglu_bwd_mx_equals_two_passes(gpu, M, I, rowwise, colwise):
+    """The fused gated-GELU backward and MX quantizer (one tile of I per half block, odd tile
+    counts, partial tile rows, an inf and a NaN gradient) against geglu_bwd and quantize_mx: the
+    same bytes and scale planes."""
+    g = torch.Generator().manual_seed(M + I)
+    dH = torch.randn(M, I, generator=g)
+    dH[M - 1, I - 1], dH[M // 2, 5] = float("inf"), float("nan")
+    GU = 3 * torch.randn(M, 2 * I, generator=g)
+    dH, GU = dH.bfloat16().to(gpu), GU.bfloat16().to(gpu)
+    one = ops.geglu_bwd_mx(dH, GU, rowwise=rowwise, colwise=colwise)
+    two = ops.quantize_mx(ops.geglu_bwd(dH, GU)[0], rowwise=rowwise, colwise=colwise,
+                          scale_rows=False)
+    torch.cuda.synchronize()
+    for a, b in ((one.data, two.data), (one.planes, two.planes), (one.data_t, two.data_t),
+                 (one.planes_t, two.planes_t)):
+        assert (a is None) == (b is None)
+        assert a is None or torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
 # ---- the TE modules under 'mxfp8' ------------------------------------------------------
 import types  # noqa: E402
 
