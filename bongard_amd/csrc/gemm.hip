@@ -38,6 +38,8 @@ enum TileId {
   TILE_128x128k2,
   TILE_256x256w8,
   TILE_256x256w8x,
+  TILE_192x128o2,
+  TILE_128x128o2,
   NUM_TILES
 };
 
@@ -54,16 +56,16 @@ struct TileInfo {
 
 // step_us and fixed_us: least squares over 600 measured (shape, tile, split) times of FP8
 // linear GEMMs (M 64 .. 16384, five (N, K) of the text layer, every tile and 2-4 splits),
-// together with the constants of linear_cost. Picking by them loses 0.9% on average against the
-// best measured plan, 15% at most (M = 64: 2 us); per-tile rates with two steps of overhead a round picked up
-// to 22% slower plans (M = 2048, N = 2560, K = 10240 on 192x256 82.0 us, 256x160 in two K pieces
-// 67.0; M = 4096, N = 10240, K = 2560 on 256x160 117.5 us, eight-wave 256x256 101.5; M = 4096,
-// N = 2048, K = 2560 on 128x128 28.5 us, 160x256 25.8). The eight-wave tile's pair
-// is the one whose picks are best over these and 18 shapes of long K (48-160 steps), where it
-// runs 15-20% over its fit on the shorter ones as no other tile does: that fit
-// (1.097, 14.07) put M = 8192, N = 2560, K = 10240 on
-// its tail split (196 us; 256x160 186) and M = 2048, K = 20480 on three pieces (126; 256x160 in
-// two 109). geglu_rate: time per K step of one workgroup, with every CU busy, over the tile's
+// together with the constants of linear_cost; per-tile rates with two steps of overhead a round
+// picked up to 22% slower plans (M = 2048, N = 2560, K = 10240 on 192x256 82.0 us, 256x160 in two
+// K pieces 67.0; M = 4096, N = 10240, K = 2560 on 256x160 117.5 us, eight-wave 256x256 101.5;
+// M = 4096, N = 2048, K = 2560 on 128x128 28.5 us, 160x256 25.8). The eight-wave tile's pair is
+// the one whose picks are best over these and 18 shapes of long K (48-160 steps), where it runs
+// 15-20% over its fit on the shorter ones as no other tile does: that fit (1.097, 14.07) put
+// M = 8192, N = 2560, K = 10240 on its tail split (196 us; 256x160 186) and M = 2048, K = 20480
+// on three pieces (126; 256x160 in two 109). The two-stage tiles' pairs were chosen the same way
+// over all 106 shapes, FP8 and bf16: picking by the table loses 0.8% on average against the best
+// measured plan, 8% at most, without these tiles 2.8% and 25%. geglu_rate: time per K step of one workgroup, with every CU busy, over the tile's
 // FLOP per step. Tiles never picked by cost (1e3): run by an override or in place of a twin.
 constexpr TileInfo kTiles[NUM_TILES] = {
     {256, 256, 1, 1e3, 1e3, 8.8, "256x256", true},
@@ -79,6 +81,8 @@ constexpr TileInfo kTiles[NUM_TILES] = {
     {128, 128, 1, 1e3, 1e3, 0.0, "128x128k2", false},
     {256, 256, 1, 1.30, 12.0, 9.2, "256x256w8", true},
     {256, 256, 1, 1.30, 12.0, 0.0, "256x256w8x", false},
+    {192, 128, 2, 1.15, 8.0, 0.0, "192x128o2", false},
+    {128, 128, 2, 0.87, 6.2, 0.0, "128x128o2", true},
 };
 // Whether `tile` has a gated-GELU variant for I = N / 2: tiles of 128 or 64 H columns take
 // any I (a multiple of 128); the 256x160 tile (80 gate + 80 up columns, one wave column)
@@ -170,7 +174,8 @@ constexpr double kPartialUsPerMB = 0.308, kReduceUs = 6.2;
 // a fraction f of the slots run, after whole rounds, takes a + (1 - a) f of a whole one, a lone
 // partial round b + (1 - b) f: the busy CUs share the memory system and the power budget with
 // fewer others. One workgroup per CU: a 0.75, b 0.80 (a round is as slow as its slowest tile);
-// two (occ 2): a 0.24, b 0.56 (half a round leaves every workgroup a CU of its own).
+// two (occ 2): a 0.24 (tiles of 128 x 128 and more 0.40), b 0.56 (half a round leaves every
+// workgroup a CU of its own).
 double linear_cost(const Plan& p, int64_t ksteps) {
   const TileInfo& ti = kTiles[p.tile];
   const double ws_us = kPartialUsPerMB * (double)p.ws_bytes / 1e6 + kReduceUs;
@@ -183,7 +188,8 @@ double linear_cost(const Plan& p, int64_t ksteps) {
   const int64_t ctas = (int64_t)p.tiles_m * p.tiles_n * p.splits;
   const int64_t whole = ctas / slots;
   const double frac = (double)(ctas - whole * slots) / slots;
-  const double base = whole > 0 ? (ti.occ > 1 ? 0.24 : 0.75) : (ti.occ > 1 ? 0.56 : 0.80);
+  const double a = ti.occ == 1 ? 0.75 : ti.bm * ti.bn >= 128 * 128 ? 0.40 : 0.24;
+  const double base = whole > 0 ? a : ti.occ == 1 ? 0.80 : 0.56;
   const double rounds = whole + (frac > 0 ? base + (1 - base) * frac : 0.0);
   return rounds * (p.kps * ti.step_us + ti.fixed_us) + (p.splits > 1 ? ws_us : 0.0);
 }
@@ -261,11 +267,16 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
     if (tile == TILE_256x256) continue;
     // the extra-B-slot twin of the eight-wave tile is substituted below, by K
     if (tile == TILE_256x256w8x) continue;
-    for (int s = 1; s <= (geglu ? 1 : kMaxSplits); ++s) {
+    // the two-stage tiles run unsplit: in K pieces the modelled time is up to 13% short (M = 1024,
+    // N = 2560, K = 20480 in three pieces: 78 us, 256x160 65)
+    const bool two_stage = tile == TILE_192x128o2 || tile == TILE_128x128o2;
+    for (int s = 1; s <= (geglu || two_stage ? 1 : kMaxSplits); ++s) {
       const Plan p = make_plan(tile, M, N, geglu ? kGegluNominalSteps : ksteps, s);
       if (p.splits != s || (s > 1 && p.kps < kMinStepsPerSplit) || p.ws_bytes > ws_avail)
         continue;
-      const double c = plan_cost(p, geglu, ksteps);
+      // (MX: the scales' traffic weighs more on the smaller tile, M = 2048, N = 2560, K = 10240
+      // modelled 63 us, measured 67-69, 256x160 in two pieces 65)
+      const double c = plan_cost(p, geglu, ksteps) * (mx && two_stage ? 1.08 : 1.0);
       if (!have || c < best_cost * 0.99) {  // prefer earlier (larger, unsplit) plans on ties
         best = p;
         best_cost = c;
@@ -402,6 +413,8 @@ int launch_tile(const Plan& pl, const GemmParams& p, int epi, int out_dtype, int
     case TILE_64x128k2: return launch_gemm_tile<Tile64x128k2>(p, epi, out_dtype, fa, fb, s, mx);
     case TILE_128x128k2: return launch_gemm_tile<Tile128x128k2>(p, epi, out_dtype, fa, fb, s, mx);
     case TILE_256x256w8: return launch_gemm_tile<Tile256x256w8>(p, epi, out_dtype, fa, fb, s, mx);
+    case TILE_192x128o2: return launch_gemm_tile<Tile192x128o2>(p, epi, out_dtype, fa, fb, s, mx);
+    case TILE_128x128o2: return launch_gemm_tile<Tile128x128o2>(p, epi, out_dtype, fa, fb, s, mx);
     case TILE_256x256w8x: return launch_gemm_tile<Tile256x256w8x>(p, epi, out_dtype, fa, fb, s, mx);
     default: return launch_gemm_tile<Tile128x128>(p, epi, out_dtype, fa, fb, s, mx);
   }

@@ -115,6 +115,15 @@ using Tile256x256w8 = GemmTile<2, 4, 4, 2, 2, 1>;
 // the same with a third B slot in the 32 KB its stages leave free (B loads two steps
 // ahead): for long-K linear GEMMs whose operands come from HBM rather than the MALL
 using Tile256x256w8x = GemmTile<2, 4, 4, 2, 2, 1, 1, 1>;
+// Two workgroups per CU of two stages each: one's fill and epilogue run beside the other's K
+// loop, where a lone workgroup leaves the CU 8-14 us a round without MFMA work. For the middle
+// of the range, where a tile has few K steps or the larger tiles leave CUs idle (M = 2001,
+// N = 2560, K = 4096: 160x256 32.1 us, 128x128o2 27.8; 3008 x 2560 x 1024: 14.5 and 12.3;
+// bf16 20480 x 2560 x 1024: 118.4 on the eight-wave 256x256, 192x128o2 110.9); their operands
+// cross the LDS more often, so long K on a full chip stays with the larger tiles (8192 x 2560 x
+// 2048 50.8 and 48.0, 4096 x 2560 x 10240 on 256x160 88.8 and 101.3).
+using Tile192x128o2 = GemmTile<2, 2, 3, 2, 2, 2>;
+using Tile128x128o2 = GemmTile<2, 2, 2, 2, 2, 2>;
 // two K groups (skinny GEMMs): 8 waves, alternate K steps
 using Tile128x64k2 = GemmTile<2, 2, 2, 1, 3, 1, 2>;
 using Tile64x128k2 = GemmTile<2, 2, 1, 2, 3, 1, 2>;

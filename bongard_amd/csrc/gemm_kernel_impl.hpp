@@ -1293,6 +1293,28 @@ int launch_gemm_tile(const GemmParams& p, int epi, int out_dtype, int fmt_a, int
     if (out_dtype == BF8_OUT_BF16)
       return launch_typed<T, EPI_LINEAR, BF8_OUT_BF16>(p, fmt_a, fmt_b, stream);
     return launch_typed<T, EPI_LINEAR, BF8_OUT_F32>(p, fmt_a, fmt_b, stream);
+  } else if constexpr (T::OCC == 2 && T::NS == 2) {
+    // two stages of two workgroups: no room for the gelu table; MX scales fit 128 x 128 only
+    if (epi == EPI_GEGLU) {
+      set_error("gemm: tile %dx%d of two stages has linear epilogues only", T::BM, T::BN);
+      return BF8_EINVAL;
+    }
+    if (mx) {
+      if constexpr (T::BM == 128 && T::BN == 128) {
+        if (out_dtype == BF8_OUT_BF16)
+          hipLaunchKernelGGL((gemm_kernel<T, 0, 0, EPI_LINEAR, BF8_OUT_BF16, true>), grid, block,
+                             0, stream, p);
+        else
+          hipLaunchKernelGGL((gemm_kernel<T, 0, 0, EPI_LINEAR, BF8_OUT_F32, true>), grid, block,
+                             0, stream, p);
+        return launch_status("gemm_kernel(mx)");
+      }
+      set_error("gemm: tile %dx%d of two stages has no MX variant", T::BM, T::BN);
+      return BF8_EINVAL;
+    }
+    if (out_dtype == BF8_OUT_BF16)
+      return launch_typed<T, EPI_LINEAR, BF8_OUT_BF16>(p, fmt_a, fmt_b, stream);
+    return launch_typed<T, EPI_LINEAR, BF8_OUT_F32>(p, fmt_a, fmt_b, stream);
   } else if constexpr (T::KG != 1) {
     if (epi == EPI_GEGLU || mx) {
       set_error("gemm: tile %dx%d with two K groups has linear non-MX epilogues only", T::BM,

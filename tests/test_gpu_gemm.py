@@ -299,6 +299,34 @@ def test_split_k_deterministic(gpu, monkeypatch, tile):
     _assert_fp32_close(outs[0], orc.scaled_mm(ra, sa, 0, rb, sb, 0), what=f"split4 {tile}")
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (300, 328, 1056), (192, 128, 128), (385, 264, 256),
+                                   (40, 520, 384)])
+@pytest.mark.parametrize("tile", ["192x128o2", "128x128o2"])
+def test_two_workgroup_tiles(gpu, monkeypatch, tile, M, N, K):
+    """The two-stage tiles of which two share a CU, unsplit and in K pieces: 1 to 9 K steps, M, N
+    and K tails, against the oracle; bf16 and (128 x 128) MX operands against the four-stage 128 x
+    128 tile, which adds the same products in the same order."""
+    for plan in (tile, f"{tile}:3"):
+        monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", plan)
+        _gemm_case(gpu, M, N, K, seed=M + K, bias=True)
+        _gemm_case(gpu, M, N, K, fa=ops.E5M2, seed=18, a_std=1e-3)
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randn(M, K, generator=g).bfloat16().to(gpu)
+    b = torch.randn(N, K, generator=g).bfloat16().to(gpu)
+    qa, qb = ops.quantize_mx(a), ops.quantize_mx(b)
+    na, nb = (ops.quantize_nvfp4(t, rowwise=True) for t in (a, b))
+    got = []
+    for plan in (tile, "128x128"):
+        monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", plan)
+        got.append([ops.gemm_nvfp4(na.data, na.scales, na.meta, nb.data, nb.scales, nb.meta)])
+        if tile == "128x128o2":
+            for dt in (torch.bfloat16, torch.float32):
+                got[-1].append(ops.gemm_mx(qa.data, qa.scales, qb.data, qb.scales, out_dtype=dt))
+    torch.cuda.synchronize()
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("tile", ["256x256", "160x256", "128x128", "192x256", "256x128",
                                   "64x128", "256x160", "256x256w8"])
 def test_geglu_tiles(gpu, monkeypatch, tile):
