@@ -142,8 +142,8 @@ class FusedMLP(_ScalingExtraState, torch.nn.Module):
             return self._nvfp4_forward(x, flat, length, first)
         if first:
             if mx:
-                self._fp8_weights = (_linear.quantize_weight_mx(self.fc1_weight),
-                                     _linear.quantize_weight_mx(self.fc2_weight))
+                self._fp8_weights = (_linear.quantize_weight_mx(self.fc1_weight, scale_rows=False),
+                                     _linear.quantize_weight_mx(self.fc2_weight, scale_rows=False))
             elif fc1 is not None:
                 # delayed scaling: both weights in one launch
                 wq, dq = _scaling.quantize_many([

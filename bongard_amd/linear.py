@@ -386,11 +386,13 @@ class GegluGateUpNvfp4Function(_Fp8Function):
         return dx, dw, None, None, None
 
 
-def quantize_weight_mx(weight, *, transpose=True):
+def quantize_weight_mx(weight, *, transpose=True, scale_rows=True):
     """MXFP8 copy of a weight [N, K]: blocks along K (forward), and with ``transpose`` the
-    [K, N] copy with blocks along N (the input-gradient GEMM's operand)."""
+    [K, N] copy with blocks along N (the input-gradient GEMM's operand). ``scale_rows`` as in
+    ``ops.quantize_mx``: a caller of ``fp8_weight`` may read the scale rows, the layers'
+    GEMMs read the planes alone."""
     return ops.quantize_mx(weight.detach(), E4M3, rowwise=True, colwise=transpose,
-                           scale_rows=False)
+                           scale_rows=scale_rows)
 
 
 class Fp8LinearMxFunction(_Fp8Function):
@@ -412,7 +414,7 @@ class Fp8LinearMxFunction(_Fp8Function):
         else:
             xq = ops.quantize_mx(x, E4M3, rowwise=True, colwise=need_dw, scale_rows=False)
         if wq is None:
-            wq = quantize_weight_mx(weight, transpose=need_dx)
+            wq = quantize_weight_mx(weight, transpose=need_dx, scale_rows=False)
         y = ops.gemm_mx(xq.data, None, wq.data, None, a_planes=xq.planes, b_planes=wq.planes)
         ctx.save_for_backward(xq.data_t, xq.planes_t, wq.data_t if need_dx else None,
                               wq.planes_t if need_dx else None)
@@ -457,16 +459,15 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
         else:
             xq = ops.quantize_mx(x, E4M3, rowwise=True, colwise=need_dgu, scale_rows=False)
         if gu_q is None:
-            gu_q = quantize_weight_mx(w_gu, transpose=need_dx)
+            gu_q = quantize_weight_mx(w_gu, transpose=need_dx, scale_rows=False)
         # H is quantized (rowwise, plus the columnwise copy for the down wgrad) in the
         # GEMM's epilogue; the bf16 H itself is never written
         hq, GU = ops.gemm_geglu_mx_planes(xq.data, xq.planes, gu_q.data, gu_q.planes, I,
                                           colwise=need_dd, keep_gu=train)
         if down_q is None:
-            down_q = quantize_weight_mx(w_down, transpose=need_dx or need_dgu)
+            down_q = quantize_weight_mx(w_down, transpose=need_dx or need_dgu, scale_rows=False)
         y = ops.gemm_mx(hq.data, None, down_q.data, None, a_planes=hq.planes,
                         b_planes=down_q.planes)
-        ctx.intermediate = I
         ctx.save_for_backward(GU, xq.data_t, xq.planes_t, hq.data_t, hq.planes_t, gu_q.data_t,
                               gu_q.planes_t, down_q.data_t, down_q.planes_t)
         return y
@@ -474,7 +475,6 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
     @staticmethod
     def backward(ctx, dy):
         GU, x8t, xpt, h8t, hpt, gu8t, gupt, d8t, dpt = ctx.saved_tensors
-        I = ctx.intermediate
         need_dx, need_dgu, need_dd = ctx.needs_input_grad[:3]
         dyq = ops.quantize_mx(dy.contiguous(), E4M3, rowwise=need_dx or need_dgu,
                               colwise=need_dd, scale_rows=False)
@@ -483,13 +483,9 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
             dd = ops.gemm_mx(dyq.data_t, None, h8t, None, a_planes=dyq.planes_t, b_planes=hpt)
         if need_dx or need_dgu:
             dH = ops.gemm_mx(dyq.data, None, d8t, None, a_planes=dyq.planes, b_planes=dpt)
-            if I % 128 == 0:
-                # d_g and d_u go from registers to their MX copies (whole 128 x 128 tiles of I)
-                dq = ops.geglu_bwd_mx(dH, GU, rowwise=need_dx, colwise=need_dgu)
-            else:
-                dGU, _ = ops.geglu_bwd(dH, GU)
-                dq = ops.quantize_mx(dGU, E4M3, rowwise=need_dx, colwise=need_dgu,
-                                     scale_rows=False)
+            # d_g and d_u go from registers to their MX copies (whole 128 x 128 tiles of I: the
+            # forward's gated-GELU GEMM takes only multiples of 128)
+            dq = ops.geglu_bwd_mx(dH, GU, rowwise=need_dx, colwise=need_dgu)
             if need_dx:
                 dx = ops.gemm_mx(dq.data, None, gu8t, None, a_planes=dq.planes, b_planes=gupt)
             if need_dgu:

@@ -395,7 +395,7 @@ class TEMLP(torch.nn.Module):
             first_u = self.up_proj._note_microbatch()
             if first_g or first_u or self._split_cache is None:
                 self._split_cache = _linear.quantize_weight_mx(
-                    torch.cat([self.gate_proj.weight, self.up_proj.weight], 0))
+                    torch.cat([self.gate_proj.weight, self.up_proj.weight], 0), scale_rows=False)
             gu_q = self._split_cache
             w_gu = _SplitGateUp.apply(self.gate_proj.weight, self.up_proj.weight)
         out = _linear.Fp8GegluMlpMxFunction.apply(flat, w_gu, self.down.weight, gu_q, down_q, I)

@@ -457,3 +457,21 @@ def test_quantize_mx_many_equals_quantize_mx(gpu, monkeypatch):
         y_inf = linear.Fp8LinearMxFunction.apply(x, w_o, None)
     assert len(calls) == 2
     assert torch.equal(y_train.detach(), y_inf)
+
+
+def test_module_weight_keeps_scale_rows(gpu):
+    """The cached MXFP8 weight a module hands out still holds its scales as rows, for a caller's
+    own ``gemm_mx`` on them."""
+    g = torch.Generator().manual_seed(5)
+    lin = torch.nn.Linear(160, 96, bias=False, dtype=torch.bfloat16)
+    with torch.no_grad():
+        lin.weight.copy_(torch.randn(96, 160, generator=g) * 0.02)
+    layer = te_linear.TELinear([lin], "mxfp8").to(gpu)
+    q = layer.fp8_weight(True)
+    r = ops.quantize_mx(layer.weight.detach(), rowwise=True, colwise=True)
+    for name in ("data", "scales", "data_t", "scales_t", "planes", "planes_t"):
+        assert torch.equal(getattr(q, name).view(torch.uint8), getattr(r, name).view(torch.uint8))
+    x = ops.quantize_mx(torch.randn(33, 160, generator=g).to(torch.bfloat16).to(gpu))
+    assert torch.equal(ops.gemm_mx(x.data, x.scales, q.data, q.scales),
+                       ops.gemm_mx(x.data, None, q.data, None, a_planes=x.planes,
+                                   b_planes=q.planes))
