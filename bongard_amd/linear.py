@@ -95,11 +95,11 @@ def _quantize_input(x, scaler, x_amax, transpose):
 
 def dense_rows(t):
     """``t`` as the kernels read it: contiguous and 16-byte aligned. Row counts that are not
-    multiples of 16 reach the per-tensor-scaled kernels as they are (every GEMM takes them,
-    the weight-gradient GEMM's reduction included); a copy is made only of a tensor whose
-    storage the kernels cannot read."""
+    multiples of 32 reach the per-tensor-scaled kernels as they are (every GEMM takes them,
+    the weight-gradient GEMM's reduction included), where callers once passed a padded and so
+    aligned copy; a copy is made only of a tensor whose storage the kernels cannot read."""
     t = t.contiguous()
-    return t if t.shape[0] % 16 == 0 or t.data_ptr() % 16 == 0 else t.clone()
+    return t if t.shape[0] % 32 == 0 or t.data_ptr() % 16 == 0 else t.clone()
 
 
 def linear_kmajor(in_features, out_features):
