@@ -25,6 +25,7 @@ namespace {
 constexpr int kMxNT = 256;
 constexpr int kMT = 128;               // tile of the two-copy kernel (rows x cols)
 constexpr int kMaxMxTileBlocks = 2048;
+constexpr int kMaxMxRowBlocks = 8192;
 // Exponents (mx_exponent) of two packed |x| maxima given as finite bf16 keys: fp8_max is
 // 1.75 x 2^S, so amax / fp8_max rounds up to a power of two with exponent E - S where the
 // mantissa is at most 1.75 (96 / 128 above 1) and E - S + 1 past it, i.e. ((key + 31) >> 7) - S,
@@ -67,7 +68,7 @@ __device__ __forceinline__ uint2 mx_quant8_vs(uint4 v, const float* s) {
   return make_uint2(q[0], q[1]);
 }
 
-// Either or both copies of x in one pass. A block takes 128 x 128 tiles, each wave 32 rows of
+// Both copies of x in one pass, or the columnwise one. A block takes 128 x 128 tiles, each wave 32 rows of
 // all 128 columns: lane l holds columns 8 (l & 15) .. +7 of the rows 4 k + l / 16, k < 8, so a
 // row block of 32 is four neighbouring lanes (two DPP exchanges) and a column block of 32 rows is
 // the wave's eight pieces and the four lanes of a column group (two lane exchanges of packed
@@ -80,7 +81,7 @@ __device__ __forceinline__ uint2 mx_quant8_vs(uint4 v, const float* s) {
 // the MALL: [4096, 20480] 133.1 us in two passes, 78.4 us in one (4.3 TB/s); [20480, 2560]
 // 72.9 -> 45.4 us (4.7 TB/s); one pass over 64 x 64 tiles per wave, whose stores are half
 // lines, 99.7 and 56.3 us. With planes in place of the scale rows' scattered dwords 75.2 and
-// 43.0 us; the rowwise copy alone 45.9 and 29.8 us (5.5 TB/s).
+// 43.0 us. The rowwise copy alone is mx_rows_kernel's.
 struct MxTile {
   const uint16_t* x;
   int64_t rows, cols;
@@ -379,16 +380,113 @@ __global__ __launch_bounds__(kMxNT) void mx_tile_kernel(MxManyArgs a) {
     mx_tiles<BF8_E5M2>(a.t[i], blk, nblk, stage, erow, ecol);
 }
 
-// Adds a tensor to a launch.
+constexpr int kLR = 4;  // rows per lane of the rowwise kernel
+// Rowwise quantization of a wave's 16 rows x 128 columns: lane l holds columns 8 (l & 15) .. +7
+// of the rows 4 (l / 16) + k, k < 4 (rk: the maximum of its block of 32, a bf16 key).
+template <int FMT, bool FINITE>
+__device__ __forceinline__ void mx_rows_body(const MxTile& p, int64_t r0, int64_t c0,
+                                             const uint4 (&v)[kLR], const uint32_t (&rk)[kLR],
+                                             int lane) {
+  const int cl = lane & 15;
+  const int64_t c = c0 + 8 * cl, rl = r0 + kLR * (lane >> 4);
+  uint32_t mine = 0;  // the scale dword of row rl + cl, in the lanes cl < kLR
+#pragma unroll
+  for (int k = 0; k < kLR; ++k) {
+    uint32_t e;
+    if constexpr (FINITE)
+      e = mx_exponent_finite_pk<FMT>(rk[k]) & 0xFFFFu;
+    else
+      e = mx_exponent<FMT>(rk[k] << 16);
+    if (rl + k < p.rows && c < p.cols) {
+      const float mult = mx_multiplier(e);
+      *reinterpret_cast<uint2*>(p.out + (rl + k) * p.cols + c) =
+          FINITE ? quant8_bf16_finite<FMT, false>(v[k], mult) : quant8_bf16<FMT>(v[k], mult);
+    }
+    if (c >= p.cols) e = kMxPadScale;  // blocks past the row pad its last dword of scales
+    e <<= 8 * (cl >> 2);
+    e |= (uint32_t)__shfl_xor((int)e, 4, 64);
+    e |= (uint32_t)__shfl_xor((int)e, 8, 64);
+    if (cl == k) mine = e;
+  }
+  const int64_t r = rl + cl;
+  if (cl < kLR && r < p.rows) {
+    if (p.planes) p.planes[(c0 >> 7) * p.rows + r] = mine;
+    if (p.sc) *reinterpret_cast<uint32_t*>(p.sc + r * p.ld_sc + (c0 >> 5)) = mine;
+  }
+}
+
+template <int FMT>
+__device__ __forceinline__ void mx_rows(const MxTile& p, int64_t blk, int64_t nblk) {
+  const int lane = threadIdx.x & 63;
+  // wave-uniform 32-bit tile arithmetic (a tile is 2048 elements)
+  const uint32_t groups = (uint32_t)((p.cols + kMT - 1) / kMT);
+  const uint32_t ntiles = groups * (uint32_t)((p.rows + kLR * 4 - 1) / (kLR * 4));
+  const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  for (uint32_t t = (uint32_t)blk * (kMxNT / 64) + wid; t < ntiles;
+       t += (uint32_t)nblk * (kMxNT / 64)) {
+    const int64_t r0 = (int64_t)(t / groups) * (kLR * 4), c0 = (int64_t)(t % groups) * kMT;
+    const int64_t c = c0 + 8 * (lane & 15), rl = r0 + kLR * (lane >> 4);
+    uint4 v[kLR];
+#pragma unroll
+    for (int k = 0; k < kLR; ++k) {
+      v[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (rl + k < p.rows && c < p.cols)
+        v[k] = *reinterpret_cast<const uint4*>(p.x + (rl + k) * p.cols + c);
+    }
+    uint32_t rk[kLR], top = 0;
+#pragma unroll
+    for (int k = 0; k < kLR; ++k) {
+      uint32_t m = pk_max_u16(pk_max_u16(v[k].x & 0x7FFF7FFFu, v[k].y & 0x7FFF7FFFu),
+                              pk_max_u16(v[k].z & 0x7FFF7FFFu, v[k].w & 0x7FFF7FFFu));
+      m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true));
+      m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, true));
+      rk[k] = max(m & 0xFFFFu, m >> 16);
+      top = max(top, rk[k]);
+    }
+    if (__builtin_expect(__any(top >= 0x7F80u), 0))
+      mx_rows_body<FMT, false>(p, r0, c0, v, rk, lane);
+    else
+      mx_rows_body<FMT, true>(p, r0, c0, v, rk, lane);
+  }
+}
+
+// The rowwise copies alone, of up to kMxMany tensors. Memory-bound like the tile kernel, whose
+// registers and LDS for the columnwise copy hold it to 4 waves per SIMD; this one runs 8 (60
+// VGPRs, no LDS). Planes only, inputs repeated / rotated past the MALL, tile kernel -> this one:
+// [4096, 10240] 24.4 / 26.5 -> 20.8 / 22.3 us (5.7 TB/s), [20480, 2560] 27.9 / 29.7 -> 24.9 / 26.5,
+// [8192, 2560] 15.0 / 16.7 -> 11.5 / 13.1; with scale rows as well 27.9 / 29.4 -> 22.0 / 23.4.
+// Eight rows per lane (94 VGPRs) 22.8 / 24.7 us at [4096, 10240], two 20.1 / 23.0.
+__global__ __launch_bounds__(kMxNT) void mx_rows_kernel(MxManyArgs a) {
+  int i = 0;
+  for (int k = 1; k < a.count; ++k)
+    if ((int64_t)blockIdx.x >= a.first[k]) i = k;
+  const int64_t blk = (int64_t)blockIdx.x - a.first[i], nblk = a.first[i + 1] - a.first[i];
+  if (a.t[i].fmt == BF8_E4M3)
+    mx_rows<BF8_E4M3>(a.t[i], blk, nblk);
+  else
+    mx_rows<BF8_E5M2>(a.t[i], blk, nblk);
+}
+
+// Adds a tensor to a launch (one with a columnwise copy is launched alone).
 void mx_add(MxManyArgs& a, const MxTile& t) {
-  const int64_t tiles = ((t.rows + kMT - 1) / kMT) * ((t.cols + kMT - 1) / kMT);
+  const int64_t tiles_c = (t.cols + kMT - 1) / kMT;
+  // rowwise: a block's four waves take a tile of 4 kLR rows x 128 columns each
+  const int64_t blocks =
+      t.out_t ? std::min<int64_t>((t.rows + kMT - 1) / kMT * tiles_c, kMaxMxTileBlocks)
+              : std::min<int64_t>(((t.rows + 4 * kLR - 1) / (4 * kLR) * tiles_c + 3) / 4,
+                                  kMaxMxRowBlocks);
   a.t[a.count] = t;
-  a.first[a.count + 1] = a.first[a.count] + std::min<int64_t>(tiles, kMaxMxTileBlocks);
+  a.first[a.count + 1] = a.first[a.count] + blocks;
   ++a.count;
 }
 
 int mx_launch(const MxManyArgs& a, void* stream) {
   if (a.count == 0) return BF8_OK;
+  if (!a.t[0].out_t) {
+    hipLaunchKernelGGL(mx_rows_kernel, dim3((unsigned)a.first[a.count]), dim3(kMxNT), 0,
+                       as_stream(stream), a);
+    return launch_status("mx_rows_kernel");
+  }
   hipLaunchKernelGGL(mx_tile_kernel, dim3((unsigned)a.first[a.count]), dim3(kMxNT), 0,
                      as_stream(stream), a);
   return launch_status("mx_tile_kernel");

@@ -83,6 +83,29 @@ def test_quantize_mx_errors(gpu):
         ops.quantize_mx(torch.zeros(48, 64, dtype=torch.bfloat16, device=gpu), colwise=True)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 32), (33, 128), (95, 160), (128, 416), (300, 1056)])
+def test_quantize_mx_rows_alone(gpu, rows, cols):
+    """The rowwise copy alone: rows and columns that leave partial 32 x 128 wave tiles, with and
+    without inf, NaN and the largest and smallest magnitudes; bytes and both layouts of the scales,
+    one tensor or several, against the oracle."""
+    x = _x(rows, cols, rows + cols, spread=False)
+    y = x.float()
+    y[0, :16], y[rows - 1, 16:32] = 3.38e38, 1e-39
+    y[rows // 2, cols - 1], y[rows - 1, 3] = float("nan"), -float("inf")
+    xs = [x, y.to(torch.bfloat16)]
+    for fmt in (ops.E4M3, ops.E5M2):
+        many = ops.quantize_mx_many([t.to(gpu) for t in xs], fmt)
+        for t, m in zip(xs, many):
+            rq, re = orc.quantize_mx(t, fmt, -1)
+            for q in (ops.quantize_mx(t.to(gpu), fmt), m):
+                assert torch.equal(q.data.view(torch.uint8).cpu(), rq)
+                assert torch.equal(q.scales.cpu(), orc.mx_scale_rows(re))
+                assert torch.equal(q.planes, _planes_of(q.scales))
+            alone = ops.quantize_mx(t.to(gpu), fmt, scale_rows=False)
+            assert torch.equal(alone.data.view(torch.uint8), m.data.view(torch.uint8))
+            assert torch.equal(alone.planes, m.planes)
+
+
 def _planes_of(rows_scales):
     """The scale planes [ld / 4, rows] of scale rows [rows, ld]."""
     r, ld = rows_scales.shape
