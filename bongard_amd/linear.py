@@ -94,12 +94,11 @@ def _quantize_input(x, scaler, x_amax, transpose):
 
 
 def dense_rows(t):
-    """``t`` as the kernels read it: contiguous and 16-byte aligned. Row counts that are not
-    multiples of 32 reach the per-tensor-scaled kernels as they are (every GEMM takes them,
-    the weight-gradient GEMM's reduction included), where callers once passed a padded and so
-    aligned copy; a copy is made only of a tensor whose storage the kernels cannot read."""
+    """``t`` as the kernels read it: contiguous and 16-byte aligned. Rows and gradients reach the
+    kernels as a caller's program hands them over (no padding or slice of this package copies
+    them first), so a tensor whose storage starts off that alignment is copied here."""
     t = t.contiguous()
-    return t if t.shape[0] % 32 == 0 or t.data_ptr() % 16 == 0 else t.clone()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def linear_kmajor(in_features, out_features):
@@ -290,7 +289,7 @@ class Fp8LinearNvfp4Function(_Fp8Function):
     def backward(ctx, dy):
         x4t, xst, x_meta, w4t, wst, w_meta = ctx.saved_tensors
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        dyq = ops.quantize_nvfp4(dy.contiguous(), rowwise=need_dx, colwise=need_dw,
+        dyq = ops.quantize_nvfp4(dense_rows(dy), rowwise=need_dx, colwise=need_dw,
                                  dequant_rows=True, dequant_cols=True)
         dx = dw = None
         if need_dx:
@@ -424,7 +423,7 @@ class Fp8LinearMxFunction(_Fp8Function):
     def backward(ctx, dy):
         x8t, xpt, w8t, wpt = ctx.saved_tensors
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        dyq = ops.quantize_mx(dy.contiguous(), E4M3, rowwise=need_dx, colwise=need_dw,
+        dyq = ops.quantize_mx(dense_rows(dy), E4M3, rowwise=need_dx, colwise=need_dw,
                               scale_rows=False)
         dx = dw = None
         if need_dx:
@@ -476,7 +475,7 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
     def backward(ctx, dy):
         GU, x8t, xpt, h8t, hpt, gu8t, gupt, d8t, dpt = ctx.saved_tensors
         need_dx, need_dgu, need_dd = ctx.needs_input_grad[:3]
-        dyq = ops.quantize_mx(dy.contiguous(), E4M3, rowwise=need_dx or need_dgu,
+        dyq = ops.quantize_mx(dense_rows(dy), E4M3, rowwise=need_dx or need_dgu,
                               colwise=need_dd, scale_rows=False)
         dx = dgu = dd = None
         if need_dd:

@@ -572,3 +572,36 @@ def test_temlp_ragged_rows_equal_padded_rows(gpu, recipe, rows):
     for i, (u, v) in enumerate(zip(*out)):
         _close_requant(u, v[:rows] if i < 2 else v, f"ragged temlp {recipe} {rows} {i}",
                        max_tol=0.2, rms_tol=0.005)
+
+
+@pytest.mark.parametrize("rows", [64, 77])
+@pytest.mark.parametrize("recipe", ["fp8", "fp8_delayed", "mxfp8", "nvfp4"])
+def test_gradient_off_alignment(gpu, recipe, rows):
+    """A gradient whose storage starts 2 bytes past 16-byte alignment (a view into a larger
+    buffer, as the backward of a concatenation makes them) gives FusedMLP and TELinear the
+    gradients of an aligned one, bit for bit, at whole and ragged multiples of 32 rows."""
+    g = torch.Generator().manual_seed(rows)
+    hidden, inter = 256, 512
+    x = torch.randn(rows, hidden, generator=g).to(torch.bfloat16).to(gpu)
+    buf = torch.zeros(rows * hidden + 1, dtype=torch.bfloat16, device=gpu)
+    buf[1:] = (torch.randn(rows * hidden, generator=g) * 1e-3).to(torch.bfloat16).to(gpu)
+    off = buf[1:].view(rows, hidden)
+    assert off.data_ptr() % 16 == 2
+
+    def fused():
+        norm = T5Gemma2RMSNorm(hidden, eps=1e-6).to(torch.bfloat16).to(gpu)
+        return fused_mlp.FusedMLP(_mlp(hidden, inter, 3, gpu), norm, recipe).train()
+
+    def linear():
+        torch.manual_seed(3)
+        return te_linear.TELinear([nn.Linear(hidden, hidden, bias=False)], recipe).to(gpu).train()
+
+    for make in (fused, linear):
+        grads = []
+        for dy in (off.clone(), off):
+            m = make()
+            xg = x.detach().requires_grad_(True)
+            grads.append(torch.autograd.grad(m(xg), [xg, *m.parameters()], dy))
+        torch.cuda.synchronize()
+        for a, b in zip(*grads):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
