@@ -241,7 +241,7 @@ constexpr int kSmallNT = 1024;
 template <int FMT>
 __global__ __launch_bounds__(kSmallNT) void quantize_small_kernel(
     const uint16_t* __restrict__ x, int64_t n, int pow2, uint8_t* __restrict__ out,
-    float* __restrict__ meta) {
+    float* __restrict__ meta, uint32_t* __restrict__ partials, int np) {
   const uint4* xv = reinterpret_cast<const uint4*>(x);
   const int64_t nvec = n >> 3, n16 = n >> 4;
   const int64_t i = (int64_t)blockIdx.x * kSmallNT + threadIdx.x;
@@ -261,8 +261,11 @@ __global__ __launch_bounds__(kSmallNT) void quantize_small_kernel(
   m = block_max_u32<kSmallNT>(m);
   float scale, sinv;
   scale_from_amax_key(m, Fp8Max<FMT>::value, pow2 != 0, scale, sinv);
-  if (blockIdx.x == 0 && threadIdx.x == 0)
-    write_meta_from_amax(m, Fp8Max<FMT>::value, meta, pow2 != 0);
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) write_meta_from_amax(m, Fp8Max<FMT>::value, meta, pow2 != 0);
+    // the amax pass's slots hold the tensor's amax too, for a caller that reads them
+    if (threadIdx.x < np) partials[threadIdx.x] = threadIdx.x == 0 ? m : 0u;
+  }
   if (i < n16) {
     const uint2 q0 = quant8_bf16<FMT>(c0, scale), q1 = quant8_bf16<FMT>(c1, scale);
     reinterpret_cast<uint4*>(out)[i] = make_uint4(q0.x, q0.y, q1.x, q1.y);
@@ -756,8 +759,10 @@ int bf8_cast_delayed_bf16(const void* x, int64_t rows, int64_t cols, float* stat
                      "bf8_cast_delayed_bf16");
 }
 
-int bf8_quantize_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
-                      uint8_t* out_t, float* meta, uint32_t* partials, void* stream) {
+// keep_partials: the caller may read the partials afterwards (they are not mere scratch).
+static int quantize_entry(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
+                          uint8_t* out_t, float* meta, uint32_t* partials, bool keep_partials,
+                          void* stream) {
   BF8_CHECK(rows >= 0 && cols >= 0, "bf8_quantize_bf16: negative shape");
   BF8_CHECK((fmt & ~BF8_SCALE_POW2) == BF8_E4M3 || (fmt & ~BF8_SCALE_POW2) == BF8_E5M2,
             "bf8_quantize_bf16: bad fmt %d", fmt);
@@ -772,18 +777,24 @@ int bf8_quantize_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_
     BF8_CHECK(x != nullptr && partials != nullptr, "bf8_quantize_bf16: x or partials is NULL");
     const unsigned blocks = (unsigned)(n / 16 / kSmallNT + 1);
     const int pow2 = (fmt & BF8_SCALE_POW2) ? 1 : 0;
+    const int np = keep_partials ? (int)amax_blocks(n) : 0;
     if ((fmt & ~BF8_SCALE_POW2) == BF8_E4M3)
       hipLaunchKernelGGL(quantize_small_kernel<BF8_E4M3>, dim3(blocks), dim3(kSmallNT), 0,
-                         as_stream(stream), (const uint16_t*)x, n, pow2, out, meta);
+                         as_stream(stream), (const uint16_t*)x, n, pow2, out, meta, partials, np);
     else
       hipLaunchKernelGGL(quantize_small_kernel<BF8_E5M2>, dim3(blocks), dim3(kSmallNT), 0,
-                         as_stream(stream), (const uint16_t*)x, n, pow2, out, meta);
+                         as_stream(stream), (const uint16_t*)x, n, pow2, out, meta, partials, np);
     return launch_status("quantize_small_kernel");
   }
   int rc = bf8_amax_bf16(x, n, partials, stream);
   if (rc) return rc;
   return bf8_cast_partials_bf16(x, rows, cols, partials, amax_blocks(n), fmt, meta, out, out_t,
                                 stream);
+}
+
+int bf8_quantize_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
+                      uint8_t* out_t, float* meta, uint32_t* partials, void* stream) {
+  return quantize_entry(x, rows, cols, fmt, out, out_t, meta, partials, true, stream);
 }
 
 int bf8_quantize_bf16_noalloc(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
@@ -797,7 +808,7 @@ int bf8_quantize_bf16_noalloc(const void* x, int64_t rows, int64_t cols, int fmt
   const int rc = noalloc_scratch(as_stream(stream), &partials);
   if (rc != BF8_OK) return rc;
   // the amax pass writes every slot [0, need) that the cast then reads: nothing to clear
-  return bf8_quantize_bf16(x, rows, cols, fmt, out, out_t, meta, partials, stream);
+  return quantize_entry(x, rows, cols, fmt, out, out_t, meta, partials, false, stream);
 }
 
 int64_t bf8_quantize_many_partials(int count, const int64_t* n) {

@@ -90,9 +90,10 @@ int bf8_cast_partials_bf16(const void* x, int64_t rows, int64_t cols, const uint
                            int64_t n_partials, int fmt, float* meta, uint8_t* out,
                            uint8_t* out_t, void* stream);
 
-/* amax -> scale -> cast (two kernels: bf8_amax_bf16, bf8_cast_partials_bf16; one, that leaves
- * partials as they were, for a small tensor's rowwise copy); meta gets {amax, scale, scale_inv,
- * 0}. partials: uint32 scratch [bf8_amax_partials(rows * cols)]. */
+/* amax -> scale -> cast (two kernels: bf8_amax_bf16, bf8_cast_partials_bf16; one for a small
+ * tensor's rowwise copy); meta gets {amax, scale, scale_inv, 0}. partials: uint32
+ * [bf8_amax_partials(rows * cols)], left holding keys whose largest is the tensor's amax (as
+ * after bf8_amax_bf16, though a small tensor's may be spread over the slots differently). */
 int bf8_quantize_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
                       uint8_t* out_t, float* meta, uint32_t* partials, void* stream);
 

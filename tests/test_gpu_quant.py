@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from bongard_amd import ops, workloads
+from bongard_amd import _lib, ops, workloads
 from oracle import fp8_oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -180,6 +180,28 @@ def test_quantize_one_launch_equals_two(gpu, rows, cols, special):
             torch.cuda.synchronize()
             assert torch.equal(one.data.view(torch.uint8), two.data.view(torch.uint8))
             assert torch.equal(one.meta.view(torch.int32), two.meta.view(torch.int32))
+
+
+@pytest.mark.parametrize("n", [1, 16, 16385, 64 * 1024, 64 * 1024 + 16, 192 * 1024, 192 * 1024 + 8])
+def test_quantize_leaves_the_amax_partials(gpu, n):
+    """bf8_quantize_bf16 leaves the tensor's amax in the partials it was given, in one launch or
+    two: a second cast of x from them equals its own quantization, and no slot past
+    bf8_amax_partials is written."""
+    L = _lib.lib()
+    x = torch.randn(1, n, generator=torch.Generator().manual_seed(n)).bfloat16().to(gpu)
+    np_ = L.bf8_amax_partials(n)
+    parts = torch.full((np_ + 4,), 0x7F123456, dtype=torch.int32, device=gpu)
+    out, meta = torch.empty(n, dtype=torch.uint8, device=gpu), ops.new_meta(gpu)
+    _lib.check(L.bf8_quantize_bf16(x.data_ptr(), 1, n, ops.E4M3, out.data_ptr(), None,
+                                   meta.data_ptr(), parts.data_ptr(),
+                                   torch.cuda.current_stream().cuda_stream), "bf8_quantize_bf16")
+    torch.cuda.synchronize()
+    assert (parts[np_:] == 0x7F123456).all()
+    assert parts[:np_].max().item() == meta[0].view(torch.int32).item()
+    second = ops.cast_partials(x, parts[:np_], ops.E5M2)
+    want = ops.quantize_many([x], ops.E5M2)[0]
+    assert torch.equal(second.data.view(torch.uint8), want.data.view(torch.uint8))
+    assert torch.equal(second.meta, want.meta)
 
 
 def test_quantize_many_rejects_bad_lists(gpu):
