@@ -61,10 +61,14 @@ constexpr int64_t kMaxCastBlocks = 2048;  // 8 blocks per CU
 // GEMM writes one per tile: 5200 at M = 16.6k) is first reduced by a one-block kernel.
 constexpr int64_t kMaxInlinePartials = 2048;
 // Largest tensor (elements) that bf8_quantize_bf16 quantizes in one launch (rowwise copy only):
-// up to here the launch saved is worth more than the extra reading. Host-bound calls in a row
-// 12.1 us with two launches, 9.6 with one (16K .. 256K elements alike); the device time alone,
-// replayed from a graph, 4.95 and 4.15 us at 16K, 5.6 and 5.8 at 100K, 5.7 and 8.4 at 200K.
-constexpr int64_t kSmallQuantMax = 192 * 1024;
+// what one block reads for its amax in one batch of loads (128 KB of x). Every block reads all of
+// x at what one CU loads (70-85 GB/s by these figures), so past that the reading costs more than
+// the launch saved. Device time in a replayed graph, one launch / two, x repeated and, in brackets, x not
+// seen before: 33K elements 4.1 / 4.7 us (4.4 / 5.3), 67K 4.7 / 5.1 (5.7 / 6.2), 82K 5.6 / 5.2
+// (6.6 / 6.3), 164K 6.9 / 5.3 (8.4 / 6.4). Back-to-back eager calls, bound by the host: 7 / 9.3 us
+// at every one of these sizes.
+constexpr int kSmallNT = 1024;
+constexpr int64_t kSmallQuantMax = (int64_t)kSmallNT * kVecPerThread * 8;
 // Slots of the library-owned scratch of bf8_quantize_bf16_noalloc: the most amax partials
 // any tensor's quantization writes.
 constexpr int64_t kNoAllocSlots = kMaxAmaxBlocks;
@@ -233,11 +237,9 @@ __global__ __launch_bounds__(kNT) void cast_kernel(const uint16_t* __restrict__ 
 }
 
 // Amax and cast of a small tensor in one launch: every block reads all of x for the amax (from
-// its XCD's L2 after the first), then casts its own kSmallNT groups of 16, which each thread
-// loads before. A call this small is bound by its launches and their host time, not by the
-// nblk-fold read (64 x 2560: 12.1 us for the two launches, 9.6 for this one; longer or
-// overlapped batches of loads measured slower).
-constexpr int kSmallNT = 1024;
+// its XCD's L2 after the first) in one batch of loads, then casts its own kSmallNT groups of 16,
+// which each thread loads before. A call this small is bound by its launches and their host time,
+// not by the nblk-fold read (figures at kSmallQuantMax).
 template <int FMT>
 __global__ __launch_bounds__(kSmallNT) void quantize_small_kernel(
     const uint16_t* __restrict__ x, int64_t n, int pow2, uint8_t* __restrict__ out,
@@ -248,14 +250,14 @@ __global__ __launch_bounds__(kSmallNT) void quantize_small_kernel(
   uint4 c0 = make_uint4(0u, 0u, 0u, 0u), c1 = c0;
   if (i < n16) { c0 = xv[2 * i]; c1 = xv[2 * i + 1]; }
   uint32_t m = 0;
-  for (int64_t j = threadIdx.x; j < nvec; j += (int64_t)kVecPerThread * kSmallNT) {
-    uint4 v[kVecPerThread];
+  uint4 v[kVecPerThread];
 #pragma unroll
-    for (int k = 0; k < kVecPerThread; ++k)
-      v[k] = j + k * kSmallNT < nvec ? xv[j + k * kSmallNT] : make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-    for (int k = 0; k < kVecPerThread; ++k) m = max(m, absmax_key8(v[k]));
+  for (int k = 0; k < kVecPerThread; ++k) {
+    const int64_t j = threadIdx.x + k * kSmallNT;
+    v[k] = j < nvec ? xv[j] : make_uint4(0u, 0u, 0u, 0u);
   }
+#pragma unroll
+  for (int k = 0; k < kVecPerThread; ++k) m = max(m, absmax_key8(v[k]));
   const int64_t tail = (nvec << 3) + threadIdx.x;
   if (tail < n) m = max(m, (uint32_t)(x[tail] & 0x7FFFu) << 16);
   m = block_max_u32<kSmallNT>(m);

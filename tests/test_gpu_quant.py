@@ -162,11 +162,12 @@ def test_quantize_many_equals_quantize(gpu):
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 5), (1, 16), (7, 33), (64, 256), (65, 2560),
-                                       (1, 16385), (192, 1024), (193, 1024)])
+                                       (1, 16385), (64, 1024), (4096, 16), (1, 64 * 1024 + 1),
+                                       (192, 1024), (193, 1024)])
 @pytest.mark.parametrize("special", [None, "inf", "nan", "zero"])
 def test_quantize_one_launch_equals_two(gpu, rows, cols, special):
-    """A small tensor's one-launch quantization (up to 192 x 1024 elements, and the first size
-    past it) against the amax and cast passes of quantize_many: the same bytes and meta."""
+    """A small tensor's one-launch quantization (up to 64 x 1024 elements) and the first sizes past
+    it against the amax and cast passes of quantize_many: the same bytes and meta."""
     x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols)).bfloat16()
     if special == "zero":
         x.zero_()
@@ -186,7 +187,8 @@ def test_quantize_one_launch_equals_two(gpu, rows, cols, special):
 def test_quantize_leaves_the_amax_partials(gpu, n):
     """bf8_quantize_bf16 leaves the tensor's amax in the partials it was given, in one launch or
     two: a second cast of x from them equals its own quantization, and no slot past
-    bf8_amax_partials is written."""
+    bf8_amax_partials is written. Past 64 x 1024 elements, where the one launch would be the
+    slower, the slots are those of the amax pass."""
     L = _lib.lib()
     x = torch.randn(1, n, generator=torch.Generator().manual_seed(n)).bfloat16().to(gpu)
     np_ = L.bf8_amax_partials(n)
@@ -198,6 +200,8 @@ def test_quantize_leaves_the_amax_partials(gpu, n):
     torch.cuda.synchronize()
     assert (parts[np_:] == 0x7F123456).all()
     assert parts[:np_].max().item() == meta[0].view(torch.int32).item()
+    if n > 64 * 1024:
+        assert torch.equal(parts[:np_], ops.amax(x))
     second = ops.cast_partials(x, parts[:np_], ops.E5M2)
     want = ops.quantize_many([x], ops.E5M2)[0]
     assert torch.equal(second.data.view(torch.uint8), want.data.view(torch.uint8))
