@@ -414,9 +414,10 @@ class Fp8LinearMxFunction(_Fp8Function):
             xq = ops.quantize_mx(x, E4M3, rowwise=True, colwise=need_dw, scale_rows=False)
         if wq is None:
             wq = quantize_weight_mx(weight, transpose=need_dx, scale_rows=False)
-        y = ops.gemm_mx(xq.data, None, wq.data, None, a_planes=xq.planes, b_planes=wq.planes)
+        y = ops.gemm_mx(xq.data, None, wq.data, None, a_planes=xq.planes,
+                        b_planes=wq.scale_planes())
         ctx.save_for_backward(xq.data_t, xq.planes_t, wq.data_t if need_dx else None,
-                              wq.planes_t if need_dx else None)
+                              wq.scale_planes(transpose=True) if need_dx else None)
         return y
 
     @staticmethod
@@ -461,14 +462,16 @@ class Fp8GegluMlpMxFunction(_Fp8Function):
             gu_q = quantize_weight_mx(w_gu, transpose=need_dx, scale_rows=False)
         # H is quantized (rowwise, plus the columnwise copy for the down wgrad) in the
         # GEMM's epilogue; the bf16 H itself is never written
-        hq, GU = ops.gemm_geglu_mx_planes(xq.data, xq.planes, gu_q.data, gu_q.planes, I,
+        hq, GU = ops.gemm_geglu_mx_planes(xq.data, xq.planes, gu_q.data, gu_q.scale_planes(), I,
                                           colwise=need_dd, keep_gu=train)
         if down_q is None:
             down_q = quantize_weight_mx(w_down, transpose=need_dx or need_dgu, scale_rows=False)
         y = ops.gemm_mx(hq.data, None, down_q.data, None, a_planes=hq.planes,
-                        b_planes=down_q.planes)
+                        b_planes=down_q.scale_planes())
         ctx.save_for_backward(GU, xq.data_t, xq.planes_t, hq.data_t, hq.planes_t, gu_q.data_t,
-                              gu_q.planes_t, down_q.data_t, down_q.planes_t)
+                              gu_q.scale_planes(transpose=True) if need_dx else None,
+                              down_q.data_t, down_q.scale_planes(transpose=True)
+                              if need_dx or need_dgu else None)
         return y
 
     @staticmethod

@@ -517,6 +517,17 @@ class MxFp8Tensor:
     planes: Optional[torch.Tensor] = None
     planes_t: Optional[torch.Tensor] = None
 
+    def scale_planes(self, transpose=False):
+        """``planes`` (``planes_t``), made from the scale rows for a tensor that has only
+        those, as one put together from bf8_quantize_mx_bf16's outputs does; None without a
+        copy of that direction."""
+        planes, scales = ((self.planes_t, self.scales_t) if transpose
+                          else (self.planes, self.scales))
+        if planes is not None or scales is None:
+            return planes
+        ld = mx_scale_ld(self.rows if transpose else self.cols)
+        return scales[:, :ld].contiguous().view(torch.int32).t().contiguous()
+
 
 def mx_scale_ld(K):
     return (int(K) + 127) // 128 * 4

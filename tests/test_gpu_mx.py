@@ -498,3 +498,45 @@ def test_module_weight_keeps_scale_rows(gpu):
     assert torch.equal(ops.gemm_mx(x.data, x.scales, q.data, q.scales),
                        ops.gemm_mx(x.data, None, q.data, None, a_planes=x.planes,
                                    b_planes=q.planes))
+
+
+@pytest.mark.parametrize("hidden,inter", [(256, 384), (160, 128)])
+def test_weights_of_scale_rows_alone(gpu, hidden, inter):
+    """MXFP8 weights put together from scale rows, without planes (as from the C quantizer's
+    outputs; here with rows wider than the scales), run the linear and the gated MLP with the
+    outputs and gradients of a weight that holds both, bit for bit."""
+    from bongard_amd import linear
+    g = torch.Generator().manual_seed(hidden)
+    M = 96
+    x = torch.randn(M, hidden, generator=g).to(torch.bfloat16).to(gpu)
+    w_gu = (torch.randn(2 * inter, hidden, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    w_d = (torch.randn(hidden, inter, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    dy = (torch.randn(M, hidden, generator=g) * 1e-3).to(torch.bfloat16).to(gpu)
+
+    def rows_alone(q):
+        def wide(s):
+            w = torch.full((s.shape[0], s.shape[1] + 8), 0xFF, dtype=torch.uint8, device=gpu)
+            w[:, :s.shape[1]] = s
+            return w[:, :s.shape[1]]
+        return ops.MxFp8Tensor(q.data, wide(q.scales), q.data_t, wide(q.scales_t), q.fmt, q.rows,
+                               q.cols)
+
+    def both(q):
+        return q
+
+    out = []
+    for form in (both, rows_alone):
+        gu_q, d_q = form(linear.quantize_weight_mx(w_gu)), form(linear.quantize_weight_mx(w_d))
+        xg, gu, wd = (t.detach().clone().requires_grad_(True) for t in (x, w_gu, w_d))
+        y = linear.Fp8GegluMlpMxFunction.apply(xg, gu, wd, gu_q, d_q, inter)
+        res = [y, *torch.autograd.grad(y, [xg, gu, wd], dy)]
+        h = torch.randn(M, inter, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+        hg = h.to(gpu).requires_grad_(True)
+        z = linear.Fp8LinearMxFunction.apply(hg, wd, d_q)
+        res += [z, *torch.autograd.grad(z, [hg, wd], dy)]
+        with torch.no_grad():
+            res.append(linear.Fp8LinearMxFunction.apply(hg, wd, d_q))
+        out.append(res)
+    torch.cuda.synchronize()
+    for a, b in zip(*out):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
