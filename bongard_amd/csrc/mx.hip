@@ -499,15 +499,15 @@ using namespace bf8;
 
 extern "C" {
 
-int bf8_quantize_mx_planes_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
-                                uint8_t* out_scales, uint32_t* out_planes, uint8_t* out_t,
-                                uint8_t* out_t_scales, uint32_t* out_t_planes, void* stream) {
-  const char* who = "bf8_quantize_mx_bf16";
+static int quantize_mx_entry(const char* who, const void* x, int64_t rows, int64_t cols, int fmt,
+                             uint8_t* out, uint8_t* out_scales, uint32_t* out_planes,
+                             uint8_t* out_t, uint8_t* out_t_scales, uint32_t* out_t_planes,
+                             void* stream) {
   BF8_CHECK(fmt == BF8_E4M3 || fmt == BF8_E5M2, "%s: bad fmt %d", who, fmt);
   BF8_CHECK(rows >= 0 && cols >= 0, "%s: negative shape", who);
   BF8_CHECK((out == nullptr) == (!out_scales && !out_planes) &&
                 (out_t == nullptr) == (!out_t_scales && !out_t_planes) && (out || out_t),
-            "%s: give out with out_scales and/or out_t with out_t_scales", who);
+            "%s: give out and / or out_t, each with its scale rows or planes", who);
   BF8_CHECK(!out || cols % 32 == 0, "%s: rowwise blocks need cols %% 32 == 0 (got %lld)", who,
             (long long)cols);
   BF8_CHECK(!out_t || (rows % 32 == 0 && cols % 16 == 0),
@@ -517,12 +517,19 @@ int bf8_quantize_mx_planes_bf16(const void* x, int64_t rows, int64_t cols, int f
   BF8_CHECK(x != nullptr, "%s: x is NULL", who);
   BF8_CHECK(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 7) == 0 && ((uintptr_t)out_t & 15) == 0 &&
                 (((uintptr_t)out_scales | (uintptr_t)out_planes | (uintptr_t)out_t_planes) & 3) == 0,
-            "%s: x, out_t 16-byte, out 8-byte, out_scales and planes 4-byte aligned", who);
+            "%s: x, out_t 16-byte, out 8-byte, out_scales and scale planes 4-byte aligned", who);
   MxManyArgs a{};
   mx_add(a, MxTile{(const uint16_t*)x, rows, cols, out, out_scales, out_planes,
                    out ? bf8_mx_scale_ld(cols) : 0, out_t, out_t_scales, out_t_planes,
                    bf8_mx_scale_ld(rows), fmt});
   return mx_launch(a, stream);
+}
+
+int bf8_quantize_mx_planes_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
+                                uint8_t* out_scales, uint32_t* out_planes, uint8_t* out_t,
+                                uint8_t* out_t_scales, uint32_t* out_t_planes, void* stream) {
+  return quantize_mx_entry("bf8_quantize_mx_planes_bf16", x, rows, cols, fmt, out, out_scales,
+                           out_planes, out_t, out_t_scales, out_t_planes, stream);
 }
 
 int bf8_geglu_bwd_mx_planes(const void* dH, const void* GU, int64_t M, int64_t I, int fmt,
@@ -559,15 +566,14 @@ int bf8_geglu_bwd_mx_planes(const void* dH, const void* GU, int64_t M, int64_t I
 int bf8_quantize_mx_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
                          uint8_t* out_scales, uint8_t* out_t, uint8_t* out_t_scales,
                          void* stream) {
-  return bf8_quantize_mx_planes_bf16(x, rows, cols, fmt, out, out_scales, nullptr, out_t,
-                                     out_t_scales, nullptr, stream);
+  return quantize_mx_entry("bf8_quantize_mx_bf16", x, rows, cols, fmt, out, out_scales, nullptr,
+                           out_t, out_t_scales, nullptr, stream);
 }
 
-int bf8_quantize_mx_many_planes_bf16(int count, const void* const* x, const int64_t* rows,
-                                     const int64_t* cols, const int* fmt, uint8_t* const* out,
-                                     uint8_t* const* out_scales, uint32_t* const* out_planes,
-                                     void* stream) {
-  const char* who = "bf8_quantize_mx_many_bf16";
+static int quantize_mx_many_entry(const char* who, int count, const void* const* x,
+                                  const int64_t* rows, const int64_t* cols, const int* fmt,
+                                  uint8_t* const* out, uint8_t* const* out_scales,
+                                  uint32_t* const* out_planes, void* stream) {
   BF8_CHECK(count >= 1 && count <= kMxMany, "%s: count %d outside [1, %d]", who, count, kMxMany);
   BF8_CHECK(x && rows && cols && fmt && out && out_scales, "%s: NULL array", who);
   MxManyArgs a{};
@@ -580,21 +586,29 @@ int bf8_quantize_mx_many_planes_bf16(int count, const void* const* x, const int6
     if (rows[t] == 0 || cols[t] == 0) continue;
     uint32_t* planes = out_planes ? out_planes[t] : nullptr;
     BF8_CHECK(x[t] && out[t] && (out_scales[t] || planes),
-              "%s: tensor %d: x, out or out_scales is NULL", who, t);
+              "%s: tensor %d: x, out or the scales (rows and planes alike) is NULL", who, t);
     BF8_CHECK(((uintptr_t)x[t] & 15) == 0 && ((uintptr_t)out[t] & 7) == 0 &&
                   (((uintptr_t)out_scales[t] | (uintptr_t)planes) & 3) == 0,
-              "%s: tensor %d: x 16-byte, out 8-byte, out_scales 4-byte aligned", who, t);
+              "%s: tensor %d: x 16-byte, out 8-byte, out_scales and scale planes 4-byte aligned", who, t);
     mx_add(a, MxTile{(const uint16_t*)x[t], rows[t], cols[t], out[t], out_scales[t], planes,
                      bf8_mx_scale_ld(cols[t]), nullptr, nullptr, nullptr, 0, fmt[t]});
   }
   return mx_launch(a, stream);
 }
 
+int bf8_quantize_mx_many_planes_bf16(int count, const void* const* x, const int64_t* rows,
+                                     const int64_t* cols, const int* fmt, uint8_t* const* out,
+                                     uint8_t* const* out_scales, uint32_t* const* out_planes,
+                                     void* stream) {
+  return quantize_mx_many_entry("bf8_quantize_mx_many_planes_bf16", count, x, rows, cols, fmt, out,
+                                out_scales, out_planes, stream);
+}
+
 int bf8_quantize_mx_many_bf16(int count, const void* const* x, const int64_t* rows,
                               const int64_t* cols, const int* fmt, uint8_t* const* out,
                               uint8_t* const* out_scales, void* stream) {
-  return bf8_quantize_mx_many_planes_bf16(count, x, rows, cols, fmt, out, out_scales, nullptr,
-                                          stream);
+  return quantize_mx_many_entry("bf8_quantize_mx_many_bf16", count, x, rows, cols, fmt, out,
+                                out_scales, nullptr, stream);
 }
 
 }  // extern "C"

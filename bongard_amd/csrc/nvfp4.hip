@@ -488,22 +488,9 @@ int bf8_quantize_nvfp4_bf16(const void* x, int64_t rows, int64_t cols, uint8_t* 
                      partials, bf8_amax_partials(n), meta, as_stream(stream));
 }
 
-int bf8_quantize_nvfp4_dequant_bf16(const void* x, int64_t rows, int64_t cols,
-                                    uint32_t* partials, int64_t n_partials, void* deq,
-                                    uint8_t* out_t, uint8_t* out_t_scales, float* meta,
-                                    void* stream) {
-  BF8_CHECK(deq != nullptr && cols % 16 == 0,
-            "bf8_quantize_nvfp4_dequant_bf16: needs deq and cols %% 16 == 0 (got %lld)",
-            (long long)cols);
-  return bf8_quantize_nvfp4_dequant2_bf16(x, rows, cols, partials, n_partials, deq, nullptr, out_t,
-                                          out_t_scales, meta, stream);
-}
-
-int bf8_quantize_nvfp4_dequant2_bf16(const void* x, int64_t rows, int64_t cols,
-                                     uint32_t* partials, int64_t n_partials, void* deq,
-                                     void* deq_t, uint8_t* out_t, uint8_t* out_t_scales,
-                                     float* meta, void* stream) {
-  const char* who = "bf8_quantize_nvfp4_dequant_bf16";
+static int nvfp4_dequant_entry(const char* who, const void* x, int64_t rows, int64_t cols,
+                               uint32_t* partials, int64_t n_partials, void* deq, void* deq_t,
+                               uint8_t* out_t, uint8_t* out_t_scales, float* meta, void* stream) {
   BF8_CHECK(rows >= 0 && cols >= 0, "%s: negative shape", who);
   BF8_CHECK(deq != nullptr || deq_t != nullptr, "%s: deq and deq_t are both NULL", who);
   BF8_CHECK(!deq || cols % 16 == 0, "%s: needs cols %% 16 == 0 (got %lld)", who, (long long)cols);
@@ -532,6 +519,25 @@ int bf8_quantize_nvfp4_dequant2_bf16(const void* x, int64_t rows, int64_t cols,
                      NvTile{rows, cols, nullptr, nullptr, (uint16_t*)deq, out_t, out_t_scales,
                             (uint16_t*)deq_t},
                      partials, n_partials, meta, as_stream(stream));
+}
+
+int bf8_quantize_nvfp4_dequant_bf16(const void* x, int64_t rows, int64_t cols,
+                                    uint32_t* partials, int64_t n_partials, void* deq,
+                                    uint8_t* out_t, uint8_t* out_t_scales, float* meta,
+                                    void* stream) {
+  const char* who = "bf8_quantize_nvfp4_dequant_bf16";
+  BF8_CHECK(deq != nullptr && cols % 16 == 0, "%s: needs deq and cols %% 16 == 0 (got %lld)", who,
+            (long long)cols);
+  return nvfp4_dequant_entry(who, x, rows, cols, partials, n_partials, deq, nullptr, out_t,
+                             out_t_scales, meta, stream);
+}
+
+int bf8_quantize_nvfp4_dequant2_bf16(const void* x, int64_t rows, int64_t cols,
+                                     uint32_t* partials, int64_t n_partials, void* deq,
+                                     void* deq_t, uint8_t* out_t, uint8_t* out_t_scales,
+                                     float* meta, void* stream) {
+  return nvfp4_dequant_entry("bf8_quantize_nvfp4_dequant2_bf16", x, rows, cols, partials,
+                             n_partials, deq, deq_t, out_t, out_t_scales, meta, stream);
 }
 
 int bf8_dequant_nvfp4(const uint8_t* q, const uint8_t* scales, int64_t rows, int64_t cols,

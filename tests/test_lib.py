@@ -211,3 +211,32 @@ def test_nvfp4_and_bf16_geglu_entries_reject_bad_arguments():
     rc = L.bf8_gemm_geglu_bf16(ptr, 32, ptr, 32, 32, 100, 32, ptr, ptr, ptr, 128, null, ptr,
                                null)
     assert rc == 1 and b"multiple of 128" in L.bf8_last_error()
+
+
+def test_errors_name_the_entry_called():
+    """Entry points that share their checks report the name that was called, and what is missing
+    in that entry's own terms."""
+    L = _lib.lib()
+    null, ptr = ctypes.c_void_p(0), ctypes.c_void_p(256)
+    one = ctypes.c_void_p * 1
+    rows, fm = (ctypes.c_int64 * 1)(32), (ctypes.c_int * 1)(0)
+    calls = {
+        "bf8_quantize_mx_bf16": (ptr, 32, 32, 0, ptr, null, null, null, null),
+        "bf8_quantize_mx_planes_bf16": (ptr, 32, 32, 0, ptr, null, null, null, null, null, null),
+        "bf8_quantize_mx_many_bf16": (1, one(256), rows, rows, fm, one(256), one(0), null),
+        "bf8_quantize_mx_many_planes_bf16": (1, one(256), rows, rows, fm, one(256), one(0), one(0),
+                                             null),
+        "bf8_quantize_nvfp4_dequant_bf16": (ptr, 32, 32, ptr, -1, ptr, null, null, ptr, null),
+        "bf8_quantize_nvfp4_dequant2_bf16": (ptr, 32, 32, ptr, -1, ptr, null, null, null, ptr,
+                                             null),
+        "bf8_gemm_kmajor": (null, 1, 16, 2, null, 0, 16, 16, 16, 16, null, null, null, 0, 16, null,
+                            0, null),
+        "bf8_gemm_kmajor_add": (null, 1, 16, 2, null, 0, 16, 16, 16, 16, null, null, null, 0, 16,
+                                null, 0, null),
+    }
+    for name, args in calls.items():
+        assert getattr(L, name)(*args) == 1, name
+        message = L.bf8_last_error().decode()
+        assert message.startswith(name + ":"), message
+        if "planes" in name:
+            assert "planes" in message, message
