@@ -43,46 +43,69 @@ enum TileId {
   NUM_TILES
 };
 
+// A round of a linear plan's co-resident workgroups (us). K steps of 128 bytes: s0 .. s1 as the
+// CUs with one workgroup go from none to all, s2 .. s3 as those with a second one do (occ 2).
+// Besides (pipeline fill, epilogue): f1 .. f1 + g1, and f2 .. f2 + g2.
+struct RoundCost {
+  double s0, s1, f1, g1;
+  double s2, s3, f2, g2;
+};
+
 struct TileInfo {
   int bm, bn, occ;
-  double step_us;     // linear plans: one 128-byte K step of a round with every slot busy
-  double fixed_us;    // ... and what a round takes besides (pipeline fill, epilogue, relaunch)
-  double geglu_rate;  // modelled FP8 rate of one CU with the gated-GELU epilogue, TFLOP/s; 0: no
-                      // such variant (the gated GELU pairs gate and up sub-tiles: even FN)
+  bool planned;       // choose_plan considers it; else run by an override or in place of a twin
+  double geglu_rate;  // modelled FP8 rate of one CU with the gated-GELU epilogue, TFLOP/s (time
+                      // per K step of one workgroup, with every CU busy, over its FLOP); 0: no
+                      // such variant (the gated GELU pairs gate and up sub-tiles: even FN). Of a
+                      // tile that is not planned only its being above 0 counts
   const char* name;
   bool mx;            // has an MX (block-scaled) variant (tiles whose stages would overflow
                       // the LDS with the scale dwords run it with one stage fewer)
+  RoundCost rows, mx_rows;  // FP8 and bf16 operands; MXFP8 on scale planes
 };
 
-// step_us and fixed_us: least squares over 600 measured (shape, tile, split) times of FP8
-// linear GEMMs (M 64 .. 16384, five (N, K) of the text layer, every tile and 2-4 splits),
-// together with the constants of linear_cost; per-tile rates with two steps of overhead a round
-// picked up to 22% slower plans (M = 2048, N = 2560, K = 10240 on 192x256 82.0 us, 256x160 in two
-// K pieces 67.0; M = 4096, N = 10240, K = 2560 on 256x160 117.5 us, eight-wave 256x256 101.5;
-// M = 4096, N = 2048, K = 2560 on 128x128 28.5 us, 160x256 25.8). The eight-wave tile's pair is
-// the one whose picks are best over these and 18 shapes of long K (48-160 steps), where it runs
-// 15-20% over its fit on the shorter ones as no other tile does: that fit (1.097, 14.07) put
-// M = 8192, N = 2560, K = 10240 on its tail split (196 us; 256x160 186) and M = 2048, K = 20480
-// on three pieces (126; 256x160 in two 109). The two-stage tiles' pairs were chosen the same way
-// over all 106 shapes, FP8 and bf16: picking by the table loses 0.8% on average against the best
-// measured plan, 8% at most, without these tiles 2.8% and 25%. geglu_rate: time per K step of one workgroup, with every CU busy, over the tile's
-// FLOP per step. Tiles never picked by cost (1e3): run by an override or in place of a twin.
+// The round costs are least squares over the measured times (operands repeated and operands
+// rotated past the L2s, their geometric mean) of every plan of 560 random shapes each in FP8,
+// bf16 and MXFP8: M 8 .. 20480 against the text layer's (N, K) and against N 16 .. 12288, K 32 ..
+// 20480. Plans within 1.6 of a shape's best count, 16,900 (6,800 MXFP8) in all; the residual is
+// 5%. On 300 more shapes of each kind the picks lose 1.0% on average against the best measured
+// plan, 4% in one of ten, 9% in one of a hundred; the worst, 25%, is a tall product of few columns
+// (4147 x 208 x 7136), whose re-read rows the model does not see. With one step time per tile,
+// fitted at M >= 64 and at five (N, K), they lost 5-6% on average and 28-40% at worst: it
+// took a second workgroup on a few CUs for a fraction of one (1137 x 2048 x 2560: 288 tiles of
+// 128x64 16.3 us, 144 of 128x128 14.4), a small reduction for as long as a large one (MXFP8 47 x
+// 2560 x 2560: unsplit 11.3 us, in five pieces 8.9) and MXFP8 and bf16 for FP8.
 constexpr TileInfo kTiles[NUM_TILES] = {
-    {256, 256, 1, 1e3, 1e3, 8.8, "256x256", true},
-    {256, 160, 1, 1.006, 8.19, 8.0, "256x160", true},
-    {160, 256, 1, 0.936, 8.35, 7.6, "160x256", true},
-    {128, 128, 1, 0.501, 4.44, 6.2, "128x128", true},
-    {192, 256, 1, 1.058, 10.18, 8.0, "192x256", true},
-    {128, 64, 2, 0.605, 3.24, 0.0, "128x64", true},
-    {64, 128, 2, 0.620, 3.78, 4.0, "64x128", true},
-    {256, 128, 1, 1e3, 1e3, 0.1, "256x128", true},
-    {128, 64, 1, 1e3, 1e3, 0.0, "128x64k2", false},
-    {64, 128, 1, 1e3, 1e3, 0.0, "64x128k2", false},
-    {128, 128, 1, 1e3, 1e3, 0.0, "128x128k2", false},
-    {256, 256, 1, 1.30, 12.0, 9.2, "256x256w8", true},
-    {256, 256, 1, 1.30, 12.0, 0.0, "256x256w8x", false},
-    {192, 128, 2, 1.15, 8.0, 0.0, "192x128o2", false},
-    {128, 128, 2, 0.87, 6.2, 0.0, "128x128o2", true},
+    {256, 256, 1, false, 1.0, "256x256", true,
+     {}, {}},
+    {256, 160, 1, true, 8.0, "256x160", true,
+     {0.755, 1.056, 9.053, 0.243}, {1.17, 1.177, 7.123, 2.13}},
+    {160, 256, 1, true, 7.6, "160x256", true,
+     {0.815, 1.047, 6.392, 1.89}, {1.047, 1.159, 5.242, 2.151}},
+    {128, 128, 1, true, 6.2, "128x128", true,
+     {0.464, 0.514, 5.189, 1.859}, {0.54, 0.586, 4.856, 1.52}},
+    {192, 256, 1, true, 8.0, "192x256", true,
+     {1.026, 1.223, 7.913, 1.334}, {1.21, 1.248, 6.947, 1.412}},
+    {128, 64, 2, true, 0.0, "128x64", true,
+     {0.37, 0.449, 3.889, 0.677, 0.586, 0.649, 4.806, 0.479}, {0.424, 0.495, 3.762, 0.556, 0.687, 0.706, 4.602, 0.416}},
+    {64, 128, 2, true, 4.0, "64x128", true,
+     {0.36, 0.48, 4.197, 0.484, 0.627, 0.608, 5.139, 1.324}, {0.405, 0.521, 4.142, 0.804, 0.677, 0.678, 5.353, 0.256}},
+    {256, 128, 1, false, 1.0, "256x128", true,
+     {}, {}},
+    {128, 64, 1, true, 0.0, "128x64k2", false,
+     {0.25, 0.364, 4.996, 0.346}, {}},
+    {64, 128, 1, true, 0.0, "64x128k2", false,
+     {0.24, 0.398, 5.724, 0.158}, {}},
+    {128, 128, 1, false, 0.0, "128x128k2", false,
+     {}, {}},
+    {256, 256, 1, true, 9.2, "256x256w8", true,
+     {0.955, 1.538, 6.272, 0.952}, {1.179, 1.541, 5.548, 2.4}},
+    {256, 256, 1, false, 0.0, "256x256w8x", false,
+     {}, {}},
+    {192, 128, 2, true, 0.0, "192x128o2", false,
+     {0.624, 0.92, 5.416, 0.009, 1.049, 1.313, 5.816, 1.16}, {}},
+    {128, 128, 2, true, 0.0, "128x128o2", true,
+     {0.496, 0.811, 4.862, 0.018, 0.827, 0.977, 4.205, 1.793}, {0.553, 0.892, 4.534, 0.001, 0.984, 1.044, 3.718, 1.881}},
 };
 // Whether `tile` has a gated-GELU variant for I = N / 2: tiles of 128 or 64 H columns take
 // any I (a multiple of 128); the 256x160 tile (80 gate + 80 up columns, one wave column)
@@ -124,14 +147,6 @@ Plan make_plan(int tile, int64_t M, int64_t N, int64_t ksteps, int splits) {
   return p;
 }
 
-// Tail split: with T tiles filling R rounds and a partial last round of t = T mod 256
-// tiles (t <= 128), the whole rounds run whole tiles and each of the t tail tiles is split
-// into pieces = min(256 / t, 8) K ranges, one workgroup each, so the last round has every
-// CU busy for a fraction of a tile instead of t CUs for a whole one. Valid for tiles that
-// run one workgroup per CU with one K group. Returns false when it does not apply.
-// Measured gain at c5 (interleaved A/B, four-wave tile): dX (M=8192, N=2560, K=20480) 343.5 ->
-// 341.0 us, dW_gu (M=20480, N=2560, K=8192) 338.8 -> 332.6 us against two rounds of 256x160
-// tiles; a shape with a smaller tail gains more.
 // Linear GEMMs with at least this many K steps run the eight-wave tile with its third B
 // slot (Tile256x256w8x): in a training step their operands come from HBM, not the MALL,
 // and B loaded two steps ahead hides that (operands rotated through more than the MALL
@@ -140,6 +155,14 @@ Plan make_plan(int tile, int64_t M, int64_t N, int64_t ksteps, int splits) {
 // costs 1.5-2%, warm or cold.
 constexpr int64_t kExtraBSlotMinSteps = 48;
 
+// Tail split: with T tiles filling R rounds and a partial last round of t = T mod 256
+// tiles (t <= 128), the whole rounds run whole tiles and each of the t tail tiles is split
+// into pieces = min(256 / t, 8) K ranges, one workgroup each, so the last round has every
+// CU busy for a fraction of a tile instead of t CUs for a whole one. Valid for tiles that
+// run one workgroup per CU with one K group. Returns false when it does not apply.
+// Measured gain at c5 (interleaved A/B, four-wave tile): dX (M=8192, N=2560, K=20480) 343.5 ->
+// 341.0 us, dW_gu (M=20480, N=2560, K=8192) 338.8 -> 332.6 us against two rounds of 256x160
+// tiles; a shape with a smaller tail gains more.
 bool make_tail_plan(int tile, int64_t M, int64_t N, int64_t ksteps, Plan& p) {
   const TileInfo& ti = kTiles[tile];
   if (tile != TILE_256x256 && tile != TILE_256x256w8 && tile != TILE_256x256w8x) return false;
@@ -160,39 +183,58 @@ bool make_tail_plan(int tile, int64_t M, int64_t N, int64_t ksteps, Plan& p) {
   return true;
 }
 
+// A split or tail plan's fp32 partials: their round trip and the reduction's launch, which counts
+// more after a product of two K-major operands (K pieces of it measured up to 7 us over the
+// model: 2048 x 640 x 1929 in two 28.7 us, unsplit 21.9; with 5.0 its picks lose 0.4% on average
+// over 800 shapes and 24% at worst, with 2.83 0.6% and 36%).
+constexpr double kPartialUsPerMB = 0.386, kReduceUs = 2.83, kReduceBothKmajorUs = 5.0;
+// Rounds after the first pay this share less of f (their fill and epilogue run beside the round
+// before), by occ; a tile mostly outside the output steps up to kEmptySaves faster (it loads less);
+// a round's bf16 output takes kOutUsPerMB, of which kOutHidden of the round's K steps hide (it
+// matters at few K steps: 9161 x 4176 x 192 on 256x256w8 42.1 us, on 192x128o2 37.4).
+constexpr double kLaterSaves[2] = {0.44, 0.761};
+constexpr double kEmptySaves = 0.145, kOutUsPerMB = 0.143, kOutHidden = 0.175;
+
+// Modelled time (us) of a linear plan of C [M, N]. kmajor: as GemmParams::kmajor.
+double linear_cost(const Plan& p, int64_t M, int64_t N, int64_t ksteps, bool mx, int kmajor) {
+  // the extra-B-slot twin is costed as the tile it replaces
+  const TileInfo& ti = kTiles[p.tile == TILE_256x256w8x ? (int)TILE_256x256w8 : p.tile];
+  const RoundCost& rc = mx ? ti.mx_rows : ti.rows;
+  const double loaded =
+      (double)(std::min<int64_t>(M, ti.bm) + std::min<int64_t>(N, ti.bn)) / (ti.bm + ti.bn);
+  const double fill = 1 - kEmptySaves * (1 - loaded);
+  const double out_mb = 2e-6 * M * N / ((double)p.tiles_m * p.tiles_n);  // of a workgroup
+  auto round = [&](int64_t ctas, int64_t steps, bool first, bool writes_out) {
+    const double x = (double)std::min<int64_t>(ctas, kNumCus) / kNumCus;
+    const double y = (double)(ctas - kNumCus) / kNumCus;
+    const bool two = ctas > kNumCus;  // occ 2
+    const double loop = steps * fill * (two ? rc.s2 + (rc.s3 - rc.s2) * y : rc.s0 + (rc.s1 - rc.s0) * x);
+    const double fixed = two ? rc.f2 + rc.g2 * y : rc.f1 + rc.g1 * x;
+    const double out = writes_out ? kOutUsPerMB * out_mb * ctas - kOutHidden * loop : 0.0;
+    return loop + fixed * (first ? 1.0 : 1.0 - kLaterSaves[ti.occ - 1]) + std::max(out, 0.0);
+  };
+  const int64_t slots = (int64_t)kNumCus * ti.occ;
+  const bool tail = p.tail_pieces > 0, split = p.splits > 1;
+  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+  const int64_t ctas = tail ? p.full_tiles : tiles * p.splits;
+  const int64_t steps = tail ? ksteps : p.kps;
+  const int64_t whole = ctas / slots, rest = ctas % slots;
+  double t = 0;
+  if (whole > 0)
+    t = round(slots, steps, true, !split) + (whole - 1) * round(slots, steps, false, !split);
+  if (rest > 0) t += round(rest, steps, whole == 0, !split);
+  if (tail) t += round((tiles - p.full_tiles) * p.tail_pieces, p.kps, false, false);
+  if (tail || split)
+    t += (kmajor == 3 ? kReduceBothKmajorUs : kReduceUs) + kPartialUsPerMB * (double)p.ws_bytes / 1e6;
+  return t;
+}
+
 // A K step never takes less than this, however little MFMA work it holds: with few
 // workgroups per CU the loads of the stages in flight no longer cover their latency
 // (measured at M = 512: ~520 ns per step for one workgroup per CU, ~450 ns when the tile
 // is small enough for two to share the CU).
 constexpr double kStepFloorNs = 520.0;
 constexpr double kStepFloorNsOcc2 = 450.0;
-
-// The split or tail partials' fp32 round trip through HBM and their reduction.
-constexpr double kPartialUsPerMB = 0.308, kReduceUs = 6.2;
-
-// Modelled time (us) of a linear plan: rounds of co-resident workgroups. A last round that only
-// a fraction f of the slots run, after whole rounds, takes a + (1 - a) f of a whole one, a lone
-// partial round b + (1 - b) f: the busy CUs share the memory system and the power budget with
-// fewer others. One workgroup per CU: a 0.75, b 0.80 (a round is as slow as its slowest tile);
-// two (occ 2): a 0.24 (tiles of 128 x 128 and more 0.40), b 0.56 (half a round leaves every
-// workgroup a CU of its own).
-double linear_cost(const Plan& p, int64_t ksteps) {
-  const TileInfo& ti = kTiles[p.tile];
-  const double ws_us = kPartialUsPerMB * (double)p.ws_bytes / 1e6 + kReduceUs;
-  if (p.tail_pieces > 0) {
-    // whole rounds of whole tiles, then one round of pieces
-    const double rounds = (double)p.full_tiles / kNumCus;
-    return rounds * (ksteps * ti.step_us + ti.fixed_us) + p.kps * ti.step_us + ti.fixed_us + ws_us;
-  }
-  const int64_t slots = (int64_t)kNumCus * ti.occ;
-  const int64_t ctas = (int64_t)p.tiles_m * p.tiles_n * p.splits;
-  const int64_t whole = ctas / slots;
-  const double frac = (double)(ctas - whole * slots) / slots;
-  const double a = ti.occ == 1 ? 0.75 : ti.bm * ti.bn >= 128 * 128 ? 0.40 : 0.24;
-  const double base = whole > 0 ? a : ti.occ == 1 ? 0.80 : 0.56;
-  const double rounds = whole + (frac > 0 ? base + (1 - base) * frac : 0.0);
-  return rounds * (p.kps * ti.step_us + ti.fixed_us) + (p.splits > 1 ? ws_us : 0.0);
-}
 
 // Modelled time (us) of a gated-GELU plan: rounds of co-resident workgroups, each running its K
 // steps plus about two steps of pipeline fill and epilogue. A step costs the MFMA work of the
@@ -211,10 +253,6 @@ double geglu_cost(const Plan& p) {
   const double eff_rounds =
       whole >= 1 && frac > 0 ? whole + 0.35 + 0.65 * frac : (double)rounds;
   return eff_rounds * (p.kps + 2) * step_ns / 1e3;
-}
-
-double plan_cost(const Plan& p, bool geglu, int64_t ksteps) {
-  return geglu ? geglu_cost(p) : linear_cost(p, ksteps);
 }
 
 // Tuning override, read on every call: BONGARD_FP8_GEMM_TILE=<bm>x<bn>[:<splits>|:t]
@@ -240,7 +278,7 @@ bool env_override(int& tile, int& splits) {
 // Chooses the tile and K split for C[M, N] = A[M, K] . B[N, K]^T. GEGLU plans never split
 // and depend on (M, N) only, so the per-tile amax partial count is known without K.
 Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, bool mx = false,
-                 bool kmajor = false) {
+                 int kmajor = 0) {
   const int64_t ksteps = std::max<int64_t>(cdiv(K, kStepBytes), 1);
   int otile, osplits;
   if (env_override(otile, osplits) && (!geglu || geglu_tile_ok(otile, N, mx)) &&
@@ -259,24 +297,23 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
   double best_cost = 0;
   bool have = false;
   for (int tile = 0; tile < NUM_TILES; ++tile) {
-    if ((geglu && !geglu_tile_ok(tile, N, mx)) || (mx && !kTiles[tile].mx)) continue;
+    if (!kTiles[tile].planned || (geglu && !geglu_tile_ok(tile, N, mx)) || (mx && !kTiles[tile].mx))
+      continue;
     // K-major operands: the eight-wave 256x256 tiles only
     if (kmajor && tile != TILE_256x256w8) continue;
-    // the eight-wave 256x256 tile replaces the four-wave one wherever it has a variant
-    // (measured faster on every large shape, same bits)
-    if (tile == TILE_256x256) continue;
-    // the extra-B-slot twin of the eight-wave tile is substituted below, by K
-    if (tile == TILE_256x256w8x) continue;
-    // the two-stage tiles run unsplit: in K pieces the modelled time is up to 13% short (M = 1024,
-    // N = 2560, K = 20480 in three pieces: 78 us, 256x160 65)
+    // The two-stage tiles run unsplit: in K pieces the modelled time is up to 13% short (M = 1024,
+    // N = 2560, K = 20480 in three pieces: 78 us, 256x160 65). So do the small tiles' two-K-group
+    // twins, where one workgroup per CU is left: two pipelines take alternate K steps (M = 512,
+    // N = 4096, K = 2560: 10.5 vs 11.5 us; with more tiles than CUs the one-group tile already
+    // shares each CU between two workgroups).
     const bool two_stage = tile == TILE_192x128o2 || tile == TILE_128x128o2;
-    for (int s = 1; s <= (geglu || two_stage ? 1 : kMaxSplits); ++s) {
+    const bool two_groups = tile == TILE_128x64k2 || tile == TILE_64x128k2;
+    for (int s = 1; s <= (geglu || two_stage || two_groups ? 1 : kMaxSplits); ++s) {
       const Plan p = make_plan(tile, M, N, geglu ? kGegluNominalSteps : ksteps, s);
       if (p.splits != s || (s > 1 && p.kps < kMinStepsPerSplit) || p.ws_bytes > ws_avail)
         continue;
-      // (MX: the scales' traffic weighs more on the smaller tile, M = 2048, N = 2560, K = 10240
-      // modelled 63 us, measured 67-69, 256x160 in two pieces 65)
-      const double c = plan_cost(p, geglu, ksteps) * (mx && two_stage ? 1.08 : 1.0);
+      if (two_groups && (int64_t)p.tiles_m * p.tiles_n > kNumCus) continue;
+      const double c = geglu ? geglu_cost(p) : linear_cost(p, M, N, ksteps, mx, kmajor);
       if (!have || c < best_cost * 0.99) {  // prefer earlier (larger, unsplit) plans on ties
         best = p;
         best_cost = c;
@@ -285,7 +322,7 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
     }
     Plan tp;
     if (!geglu && make_tail_plan(tile, M, N, ksteps, tp) && tp.ws_bytes <= ws_avail) {
-      const double c = plan_cost(tp, false, ksteps);
+      const double c = linear_cost(tp, M, N, ksteps, mx, kmajor);
       if (!have || c < best_cost * 0.99) {
         best = tp;
         best_cost = c;
@@ -296,15 +333,6 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
   if (geglu) best.kps = (int)ksteps;
   if (!geglu && !mx && best.tile == TILE_256x256w8 && ksteps >= kExtraBSlotMinSteps)
     best.tile = TILE_256x256w8x;  // same geometry, so the plan (tiles, pieces) stands
-  // A small tile that leaves one workgroup per CU (no K split) runs as its two-K-group
-  // twin: two pipelines per CU take alternate K steps (measured ~10% faster at M = 512,
-  // e.g. N = 4096, K = 2560: 10.5 vs 11.5 us; with more tiles than CUs the one-group tile
-  // already shares each CU between two workgroups).
-  if (!geglu && !mx && best.splits == 1 &&
-      (int64_t)best.tiles_m * best.tiles_n <= kNumCus &&
-      (best.tile == TILE_128x64 || best.tile == TILE_64x128)) {
-    best.tile = best.tile == TILE_128x64 ? TILE_128x64k2 : TILE_64x128k2;
-  }
   if (const char* d = std::getenv("BONGARD_FP8_GEMM_DEBUG"); d && d[0] == '1')
     std::fprintf(stderr, "bf8 plan %s%s M=%lld N=%lld K=%lld: tile %s splits %d (%d x %d tiles, tail pieces %d)\n",
                  geglu ? "geglu" : "gemm", mx ? " mx" : "", (long long)M, (long long)N, (long long)K,
@@ -316,13 +344,14 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, bool geglu, size_t ws_avail, b
 // The K-major GEMM runs on the eight-wave 256x256 tiles only, which leave most CUs idle when
 // the output is small (M = 512, N = 2560, K = 2048: 20 tiles; measured 30 us against 12 us
 // for the row-major plan on a transposed copy of B). For a call with only B K-major whose
-// plan the cost model prices well above the row-major plan plus a byte transpose of B, the
+// plan the cost model prices above the row-major plan plus a byte transpose of B, the
 // entry point transposes B^T [K, N] into its workspace and runs the row-major plan. (The
 // wgrad form, A and B K-major, measured level or faster on the same shapes, so it always
-// runs K-major.)
-constexpr double kTransposeBytesPerUs = 2.5e6;  // a small transpose: ~2.5 TB/s read + write
-constexpr double kTransposeLaunchUs = 2.0;
-constexpr double kKmajorFallbackGain = 0.8;  // transpose only when that is 20% cheaper
+// runs K-major.) The transpose: what 373 such calls took over their row-major plan, 3.0 us in
+// the median at 0.25 MB of B, 3.7 at 1 MB, 5.3 at 4 MB, 8.8 at 15 MB. Picks so, over 800
+// shapes, lose 0.9% on average; with the K-major plan kept unless 20% dearer 8%.
+constexpr double kTransposeBytesPerUs = 4.5e6;  // read + write
+constexpr double kTransposeLaunchUs = 3.0;
 
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
@@ -334,27 +363,20 @@ struct KmajorChoice {
 
 KmajorChoice choose_kmajor(int64_t M, int64_t N, int64_t K, bool a_kmajor, size_t ws_avail) {
   KmajorChoice c;
-  c.plan = choose_plan(M, N, K, false, ws_avail, false, true);
+  c.plan = choose_plan(M, N, K, false, ws_avail, false, a_kmajor ? 3 : 2);
   int otile, osplits;
   if (a_kmajor || env_override(otile, osplits)) return c;  // a forced plan stays as asked
   const size_t bb = align256((size_t)N * K);
   if (ws_avail < bb) return c;
   const int64_t ksteps = std::max<int64_t>(cdiv(K, kStepBytes), 1);
   const Plan pr = choose_plan(M, N, K, false, ws_avail - bb);
-  // costed as the planner costed them: the two-K-group and extra-B-slot tiles replace
-  // their plain twins after the choice, on the twins' costs
-  auto costed = [&](Plan q) {
-    if (q.tile == TILE_128x64k2) q.tile = TILE_128x64;
-    if (q.tile == TILE_64x128k2) q.tile = TILE_64x128;
-    if (q.tile == TILE_256x256w8x) q.tile = TILE_256x256w8;
-    return linear_cost(q, ksteps);
-  };
-  const double ck = costed(c.plan);
-  const double cr = costed(pr) + 2.0 * (double)N * K / kTransposeBytesPerUs + kTransposeLaunchUs;
+  const double ck = linear_cost(c.plan, M, N, ksteps, false, 2);
+  const double cr = linear_cost(pr, M, N, ksteps, false, 0) +
+                    2.0 * (double)N * K / kTransposeBytesPerUs + kTransposeLaunchUs;
   if (const char* d = std::getenv("BONGARD_FP8_GEMM_DEBUG"); d && d[0] == '1')
     std::fprintf(stderr, "bf8 kmajor M=%lld N=%lld K=%lld: K-major %.1f us, transposed B %.1f us\n",
                  (long long)M, (long long)N, (long long)K, ck, cr);
-  if (cr < kKmajorFallbackGain * ck) {
+  if (cr < ck) {
     c.plan = pr;
     c.transpose_b = true;
     c.b_bytes = bb;

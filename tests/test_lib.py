@@ -93,6 +93,33 @@ def test_tail_split_plans(monkeypatch):
     assert L.bf8_gemm_workspace(4096, 4096, 4096) == 0                # 256 tiles: no tail
 
 
+@pytest.mark.parametrize("entry,M,N,K,tiles,splits", [
+    # few rows: K pieces (measured 11.3 us unsplit, 8.9 in five; 10.7 and 8.8; 9.7 and 7.4)
+    ("mx", 47, 2560, 2560, {"128x64"}, range(3, 8)),
+    ("bf16", 244, 272, 1440, {"128x64"}, range(3, 8)),
+    ("mx", 17, 640, 2048, {"128x64"}, range(3, 6)),
+    # 288 tiles of 128x64 give 32 CUs two workgroups: 16.3 us, one a CU on 128x128 14.4
+    ("gemm", 1137, 2048, 2560, {"128x128"}, [1]),
+    ("mx", 1137, 2048, 2560, {"128x128"}, [1]),
+    ("gemm", 3613, 704, 2016, {"128x128"}, [1]),
+    ("bf16", 3613, 704, 2016, {"128x128"}, [1]),
+    # few columns: 128x64 55.1 us, 128x128 41.4
+    ("gemm", 11080, 176, 8608, {"128x128"}, [1]),
+    # bf16 on 192x256 334 us, 256x256w8 310
+    ("bf16", 6914, 10240, 2560, {"256x256w8"}, [1]),
+])
+def test_planner_picks(monkeypatch, capfd, entry, M, N, K, tiles, splits):
+    """The planner's choice on shapes whose plans measure 9-34% apart."""
+    L = _lib.lib()
+    monkeypatch.delenv("BONGARD_FP8_GEMM_TILE", raising=False)
+    monkeypatch.setenv("BONGARD_FP8_GEMM_DEBUG", "1")
+    {"gemm": lambda: L.bf8_gemm_workspace(M, N, K), "mx": lambda: L.bf8_gemm_mx_workspace(M, N, K),
+     "bf16": lambda: L.bf8_gemm_bf16_workspace(M, N, K),
+     "geglu": lambda: L.bf8_geglu_partials(M, N)}[entry]()
+    tile, pieces = re.search(r"tile (\S+) splits (\d+)", capfd.readouterr().err).groups()
+    assert tile in tiles and int(pieces) in splits
+
+
 def test_quantize_many_rejects_bad_arguments():
     """The multi-tensor quantization checks its lists on the host (no launch)."""
     L = _lib.lib()
