@@ -107,6 +107,8 @@ def test_tail_split_plans(monkeypatch):
     ("gemm", 11080, 176, 8608, {"128x128"}, [1]),
     # bf16 on 192x256 334 us, 256x256w8 310
     ("bf16", 6914, 10240, 2560, {"256x256w8"}, [1]),
+    # gated GELU of I = N columns on 256x256w8 223.5 us, 192x256 200.9
+    ("geglu", 4457, 2560, 10240, {"192x256"}, [1]),
 ])
 def test_planner_picks(monkeypatch, capfd, entry, M, N, K, tiles, splits):
     """The planner's choice on shapes whose plans measure 9-34% apart."""
