@@ -60,15 +60,18 @@ constexpr int64_t kMaxCastBlocks = 2048;  // 8 blocks per CU
 // Consumers reduce up to this many partials in every block; a longer list (the gated-GELU
 // GEMM writes one per tile: 5200 at M = 16.6k) is first reduced by a one-block kernel.
 constexpr int64_t kMaxInlinePartials = 2048;
-// Largest tensor (elements) that bf8_quantize_bf16 quantizes in one launch (rowwise copy only):
-// what one block reads for its amax in one batch of loads (128 KB of x). Every block reads all of
-// x at what one CU loads (70-85 GB/s by these figures), so past that the reading costs more than
-// the launch saved. Device time in a replayed graph, one launch / two, x repeated and, in brackets, x not
-// seen before: 33K elements 4.1 / 4.7 us (4.4 / 5.3), 67K 4.7 / 5.1 (5.7 / 6.2), 82K 5.6 / 5.2
-// (6.6 / 6.3), 164K 6.9 / 5.3 (8.4 / 6.4). Back-to-back eager calls, bound by the host: 7 / 9.3 us
-// at every one of these sizes.
+// Largest tensor (elements) that bf8_quantize_bf16 quantizes in one launch (rowwise copy only).
+// Every block reads all of x for its amax at what one CU loads (70-85 GB/s by these figures), in
+// batches of 128 KB: past the first batch the reading costs more device time than the launch
+// saved. In a captured graph, where launches cost no host time, that is the limit; an eager program
+// whose tensors are this small waits for the host, and there the launch is the dearer up to
+// kSmallQuantMax. Device time in a replayed graph, one launch / two, x repeated and, in brackets,
+// x not seen before: 33K elements 4.1 / 4.7 us (4.4 / 5.3), 67K 4.7 / 5.1 (5.7 / 6.2), 82K 5.6 / 5.2
+// (6.6 / 6.3), 164K 6.9 / 5.3 (8.4 / 6.4). Eager, a linear of 64 x 2560 (164K) back to back, its
+// weight cached: 33.9 / 40.7 us; behind a full queue such a call pays the device's 2 us instead.
 constexpr int kSmallNT = 1024;
-constexpr int64_t kSmallQuantMax = (int64_t)kSmallNT * kVecPerThread * 8;
+constexpr int64_t kSmallQuantCaptured = (int64_t)kSmallNT * kVecPerThread * 8;
+constexpr int64_t kSmallQuantMax = 192 * 1024;
 // Slots of the library-owned scratch of bf8_quantize_bf16_noalloc: the most amax partials
 // any tensor's quantization writes.
 constexpr int64_t kNoAllocSlots = kMaxAmaxBlocks;
@@ -237,9 +240,10 @@ __global__ __launch_bounds__(kNT) void cast_kernel(const uint16_t* __restrict__ 
 }
 
 // Amax and cast of a small tensor in one launch: every block reads all of x for the amax (from
-// its XCD's L2 after the first) in one batch of loads, then casts its own kSmallNT groups of 16,
-// which each thread loads before. A call this small is bound by its launches and their host time,
-// not by the nblk-fold read (figures at kSmallQuantMax).
+// its XCD's L2 after the first), then casts its own kSmallNT groups of 16, which each thread
+// loads before. A call this small is bound by its launches and their host time, not by the
+// nblk-fold read (figures at kSmallQuantMax; longer or overlapped batches of loads measured
+// slower).
 template <int FMT>
 __global__ __launch_bounds__(kSmallNT) void quantize_small_kernel(
     const uint16_t* __restrict__ x, int64_t n, int pow2, uint8_t* __restrict__ out,
@@ -250,14 +254,14 @@ __global__ __launch_bounds__(kSmallNT) void quantize_small_kernel(
   uint4 c0 = make_uint4(0u, 0u, 0u, 0u), c1 = c0;
   if (i < n16) { c0 = xv[2 * i]; c1 = xv[2 * i + 1]; }
   uint32_t m = 0;
-  uint4 v[kVecPerThread];
+  for (int64_t j = threadIdx.x; j < nvec; j += (int64_t)kVecPerThread * kSmallNT) {
+    uint4 v[kVecPerThread];
 #pragma unroll
-  for (int k = 0; k < kVecPerThread; ++k) {
-    const int64_t j = threadIdx.x + k * kSmallNT;
-    v[k] = j < nvec ? xv[j] : make_uint4(0u, 0u, 0u, 0u);
+    for (int k = 0; k < kVecPerThread; ++k)
+      v[k] = j + k * kSmallNT < nvec ? xv[j + k * kSmallNT] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int k = 0; k < kVecPerThread; ++k) m = max(m, absmax_key8(v[k]));
   }
-#pragma unroll
-  for (int k = 0; k < kVecPerThread; ++k) m = max(m, absmax_key8(v[k]));
   const int64_t tail = (nvec << 3) + threadIdx.x;
   if (tail < n) m = max(m, (uint32_t)(x[tail] & 0x7FFFu) << 16);
   m = block_max_u32<kSmallNT>(m);
@@ -761,6 +765,11 @@ int bf8_cast_delayed_bf16(const void* x, int64_t rows, int64_t cols, float* stat
                      "bf8_cast_delayed_bf16");
 }
 
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // keep_partials: the caller may read the partials afterwards (they are not mere scratch).
 static int quantize_entry(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
                           uint8_t* out_t, float* meta, uint32_t* partials, bool keep_partials,
@@ -775,7 +784,8 @@ static int quantize_entry(const void* x, int64_t rows, int64_t cols, int fmt, ui
   BF8_CHECK(!out_t || cols % 16 == 0,
             "bf8_quantize_bf16: transposed cast needs cols %% 16 == 0 (got %lld)", (long long)cols);
   const int64_t n = rows * cols;
-  if (out && !out_t && n > 0 && n <= kSmallQuantMax) {
+  if (out && !out_t && n > 0 && n <= kSmallQuantMax &&
+      (n <= kSmallQuantCaptured || !capturing(as_stream(stream)))) {
     BF8_CHECK(x != nullptr && partials != nullptr, "bf8_quantize_bf16: x or partials is NULL");
     const unsigned blocks = (unsigned)(n / 16 / kSmallNT + 1);
     const int pow2 = (fmt & BF8_SCALE_POW2) ? 1 : 0;

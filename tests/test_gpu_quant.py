@@ -166,7 +166,7 @@ def test_quantize_many_equals_quantize(gpu):
                                        (192, 1024), (193, 1024)])
 @pytest.mark.parametrize("special", [None, "inf", "nan", "zero"])
 def test_quantize_one_launch_equals_two(gpu, rows, cols, special):
-    """A small tensor's one-launch quantization (up to 64 x 1024 elements) and the first sizes past
+    """A small tensor's one-launch quantization (up to 192 x 1024 elements) and the first size past
     it against the amax and cast passes of quantize_many: the same bytes and meta."""
     x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols)).bfloat16()
     if special == "zero":
@@ -187,8 +187,7 @@ def test_quantize_one_launch_equals_two(gpu, rows, cols, special):
 def test_quantize_leaves_the_amax_partials(gpu, n):
     """bf8_quantize_bf16 leaves the tensor's amax in the partials it was given, in one launch or
     two: a second cast of x from them equals its own quantization, and no slot past
-    bf8_amax_partials is written. Past 64 x 1024 elements, where the one launch would be the
-    slower, the slots are those of the amax pass."""
+    bf8_amax_partials is written."""
     L = _lib.lib()
     x = torch.randn(1, n, generator=torch.Generator().manual_seed(n)).bfloat16().to(gpu)
     np_ = L.bf8_amax_partials(n)
@@ -200,12 +199,43 @@ def test_quantize_leaves_the_amax_partials(gpu, n):
     torch.cuda.synchronize()
     assert (parts[np_:] == 0x7F123456).all()
     assert parts[:np_].max().item() == meta[0].view(torch.int32).item()
-    if n > 64 * 1024:
-        assert torch.equal(parts[:np_], ops.amax(x))
     second = ops.cast_partials(x, parts[:np_], ops.E5M2)
     want = ops.quantize_many([x], ops.E5M2)[0]
     assert torch.equal(second.data.view(torch.uint8), want.data.view(torch.uint8))
     assert torch.equal(second.meta, want.meta)
+
+
+@pytest.mark.parametrize("n", [64 * 1024, 64 * 1024 + 16, 164 * 1024, 192 * 1024])
+def test_quantize_captured_in_a_graph(gpu, n):
+    """Captured in a graph, tensors past 64 x 1024 elements take the two launches, whose device
+    time is the shorter (their partials are then the amax pass's, slot for slot); every replay, on
+    new values and between eager calls of the one-launch path, gives the eager bytes and meta."""
+    L = _lib.lib()
+    x = torch.zeros(1, n, dtype=torch.bfloat16, device=gpu)
+    parts = torch.zeros(L.bf8_amax_partials(n), dtype=torch.int32, device=gpu)
+    out, meta = torch.empty(n, dtype=torch.uint8, device=gpu), ops.new_meta(gpu)
+
+    def call():
+        _lib.check(L.bf8_quantize_bf16(x.data_ptr(), 1, n, ops.E4M3, out.data_ptr(), None,
+                                       meta.data_ptr(), parts.data_ptr(),
+                                       torch.cuda.current_stream().cuda_stream), "quantize")
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call()
+    for seed in range(3):
+        x.copy_(torch.randn(1, n, generator=torch.Generator().manual_seed(seed)).bfloat16() * 3 ** seed)
+        want = ops.quantize(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want.data.view(torch.uint8).view(-1))
+        assert torch.equal(meta, want.meta)
+        assert torch.equal(parts, ops.amax(x)) == (n > 64 * 1024)
 
 
 def test_quantize_many_rejects_bad_lists(gpu):
