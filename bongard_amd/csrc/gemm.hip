@@ -185,9 +185,14 @@ bool make_tail_plan(int tile, int64_t M, int64_t N, int64_t ksteps, Plan& p) {
 
 // A split or tail plan's fp32 partials: their round trip and the reduction's launch, which counts
 // more after a product of two K-major operands (K pieces of it measured up to 7 us over the
-// model: 2048 x 640 x 1929 in two 28.7 us, unsplit 21.9; with 5.0 its picks lose 0.4% on average
-// over 800 shapes and 24% at worst, with 2.83 0.6% and 36%).
-constexpr double kPartialUsPerMB = 0.386, kReduceUs = 2.83, kReduceBothKmajorUs = 5.0;
+// model: 2048 x 640 x 1929 in two 28.7 us, unsplit 21.9; with 5.0 in all its picks lose 0.4% on
+// average over 800 shapes and 24% at worst, with 2.83 0.6% and 36%).
+constexpr double kPartialUsPerMB = 0.386, kReduceUs = 2.83, kReduceBothKmajorUs = 4.3;
+// What a plan's second launch (a reduction, a transpose) has to save besides: the host time of a
+// caller that waits for it. 64 x 2048 x 2560 is level on the device, 128x64 in four pieces against
+// 128x64k2 unsplit (9.0 / 9.7 us, operands not seen before 10.1 / 10.1), but an eager linear of it is
+// 5 us longer in two launches. Costs the picks 0.2% of device time on average.
+constexpr double kSecondLaunchUs = 0.7;
 // Rounds after the first pay this share less of f (their fill and epilogue run beside the round
 // before), by occ; a tile mostly outside the output steps up to kEmptySaves faster (it loads less);
 // a round's bf16 output takes kOutUsPerMB, of which kOutHidden of the round's K steps hide (it
@@ -225,7 +230,8 @@ double linear_cost(const Plan& p, int64_t M, int64_t N, int64_t ksteps, bool mx,
   if (rest > 0) t += round(rest, steps, whole == 0, !split);
   if (tail) t += round((tiles - p.full_tiles) * p.tail_pieces, p.kps, false, false);
   if (tail || split)
-    t += (kmajor == 3 ? kReduceBothKmajorUs : kReduceUs) + kPartialUsPerMB * (double)p.ws_bytes / 1e6;
+    t += (kmajor == 3 ? kReduceBothKmajorUs : kReduceUs) + kSecondLaunchUs +
+         kPartialUsPerMB * (double)p.ws_bytes / 1e6;
   return t;
 }
 
@@ -375,7 +381,7 @@ KmajorChoice choose_kmajor(int64_t M, int64_t N, int64_t K, bool a_kmajor, size_
   const Plan pr = choose_plan(M, N, K, false, ws_avail - bb);
   const double ck = linear_cost(c.plan, M, N, ksteps, false, 2);
   const double cr = linear_cost(pr, M, N, ksteps, false, 0) +
-                    2.0 * (double)N * K / kTransposeBytesPerUs + kTransposeLaunchUs;
+                    2.0 * (double)N * K / kTransposeBytesPerUs + kTransposeLaunchUs + kSecondLaunchUs;
   if (const char* d = std::getenv("BONGARD_FP8_GEMM_DEBUG"); d && d[0] == '1')
     std::fprintf(stderr, "bf8 kmajor M=%lld N=%lld K=%lld: K-major %.1f us, transposed B %.1f us\n",
                  (long long)M, (long long)N, (long long)K, ck, cr);
