@@ -232,22 +232,26 @@ __device__ __forceinline__ float mx_multiplier(uint32_t e) {
 constexpr int kWaveTilePitch = 17;  // dwords per staged row (odd: conflict-free row writes)
 constexpr int kWaveTileDwords = 64 * kWaveTilePitch;
 
-// Dword i of d holds 4 columns of row i: t[c] becomes column c of the 16 rows (byte i = row i).
+// Dword i of d holds 4 columns of row i: t[c] becomes column c of the 4 rows (byte i = row i).
+__device__ __forceinline__ void transpose_4x4(const uint32_t (&d)[4], uint32_t (&t)[4]) {
+  const uint32_t t0 = __byte_perm(d[0], d[1], 0x5140), t1 = __byte_perm(d[0], d[1], 0x7362);
+  const uint32_t t2 = __byte_perm(d[2], d[3], 0x5140), t3 = __byte_perm(d[2], d[3], 0x7362);
+  t[0] = __byte_perm(t0, t2, 0x5410);
+  t[1] = __byte_perm(t0, t2, 0x7632);
+  t[2] = __byte_perm(t1, t3, 0x5410);
+  t[3] = __byte_perm(t1, t3, 0x7632);
+}
+
+// The same for 16 rows.
 __device__ __forceinline__ void transpose_4x16(const uint32_t (&d)[16], uint4 (&t)[4]) {
-  uint32_t c[4][4];
+  uint32_t c[4][4];  // [rows 4k .. 4k + 3][column]
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {  // 4 x 4 byte transpose of rows 4k .. 4k+3
-    const uint32_t t0 = __byte_perm(d[4 * k], d[4 * k + 1], 0x5140);
-    const uint32_t t1 = __byte_perm(d[4 * k], d[4 * k + 1], 0x7362);
-    const uint32_t t2 = __byte_perm(d[4 * k + 2], d[4 * k + 3], 0x5140);
-    const uint32_t t3 = __byte_perm(d[4 * k + 2], d[4 * k + 3], 0x7362);
-    c[0][k] = __byte_perm(t0, t2, 0x5410);
-    c[1][k] = __byte_perm(t0, t2, 0x7632);
-    c[2][k] = __byte_perm(t1, t3, 0x5410);
-    c[3][k] = __byte_perm(t1, t3, 0x7632);
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t r[4] = {d[4 * k], d[4 * k + 1], d[4 * k + 2], d[4 * k + 3]};
+    transpose_4x4(r, c[k]);
   }
 #pragma unroll
-  for (int k = 0; k < 4; ++k) t[k] = make_uint4(c[k][0], c[k][1], c[k][2], c[k][3]);
+  for (int k = 0; k < 4; ++k) t[k] = make_uint4(c[0][k], c[1][k], c[2][k], c[3][k]);
 }
 
 // Transpose of a 64 x 64 byte tile that one wave has staged in its own LDS region (row r

@@ -357,41 +357,24 @@ __global__ __launch_bounds__(kBwdNT, 4) void geglu_bwd_mx_kernel(
   }
 }
 
-// Up to kMxMany tensors in one launch: tensor t owns blocks [first, next tensor's first), so
-// that a forward's small tensors fill the chip together and save launches.
-constexpr int kMxMany = 8;
-
-struct MxManyArgs {
-  MxTile t[kMxMany];
-  int64_t first[kMxMany + 1];
-  int count;
-};
-
-__global__ __launch_bounds__(kMxNT) void mx_tile_kernel(MxManyArgs a) {
+template <int FMT>
+__global__ __launch_bounds__(kMxNT) void mx_tile_kernel(MxTile p) {
   __shared__ uint32_t stage[kMT * kMPitch];
   __shared__ uint32_t erow[kMT], ecol[kMT];  // scale dwords of the tile's rows and columns
-  int i = 0;
-  for (int k = 1; k < a.count; ++k)
-    if ((int64_t)blockIdx.x >= a.first[k]) i = k;
-  const int64_t blk = (int64_t)blockIdx.x - a.first[i], nblk = a.first[i + 1] - a.first[i];
-  if (a.t[i].fmt == BF8_E4M3)
-    mx_tiles<BF8_E4M3>(a.t[i], blk, nblk, stage, erow, ecol);
-  else
-    mx_tiles<BF8_E5M2>(a.t[i], blk, nblk, stage, erow, ecol);
+  mx_tiles<FMT>(p, blockIdx.x, gridDim.x, stage, erow, ecol);
 }
 
-constexpr int kLR = 4;  // rows per lane of the rowwise kernel
-// Rowwise quantization of a wave's 16 rows x 128 columns: lane l holds columns 8 (l & 15) .. +7
-// of the rows 4 (l / 16) + k, k < 4 (rk: the maximum of its block of 32, a bf16 key).
-template <int FMT, bool FINITE>
+// Rowwise quantization of a wave's 4 LR rows x 128 columns: lane l holds columns 8 (l & 15) .. +7
+// of the rows LR (l / 16) + k, k < LR (rk: the maximum of its block of 32, a bf16 key).
+template <int FMT, bool FINITE, int LR>
 __device__ __forceinline__ void mx_rows_body(const MxTile& p, int64_t r0, int64_t c0,
-                                             const uint4 (&v)[kLR], const uint32_t (&rk)[kLR],
+                                             const uint4 (&v)[LR], const uint32_t (&rk)[LR],
                                              int lane) {
   const int cl = lane & 15;
-  const int64_t c = c0 + 8 * cl, rl = r0 + kLR * (lane >> 4);
-  uint32_t mine = 0;  // the scale dword of row rl + cl, in the lanes cl < kLR
+  const int64_t c = c0 + 8 * cl, rl = r0 + LR * (lane >> 4);
+  uint32_t mine = 0;  // the scale dword of row rl + cl, in the lanes cl < LR
 #pragma unroll
-  for (int k = 0; k < kLR; ++k) {
+  for (int k = 0; k < LR; ++k) {
     uint32_t e;
     if constexpr (FINITE)
       e = mx_exponent_finite_pk<FMT>(rk[k]) & 0xFFFFu;
@@ -409,33 +392,33 @@ __device__ __forceinline__ void mx_rows_body(const MxTile& p, int64_t r0, int64_
     if (cl == k) mine = e;
   }
   const int64_t r = rl + cl;
-  if (cl < kLR && r < p.rows) {
+  if (cl < LR && r < p.rows) {
     if (p.planes) p.planes[(c0 >> 7) * p.rows + r] = mine;
     if (p.sc) *reinterpret_cast<uint32_t*>(p.sc + r * p.ld_sc + (c0 >> 5)) = mine;
   }
 }
 
-template <int FMT>
+template <int FMT, int LR>
 __device__ __forceinline__ void mx_rows(const MxTile& p, int64_t blk, int64_t nblk) {
   const int lane = threadIdx.x & 63;
-  // wave-uniform 32-bit tile arithmetic (a tile is 2048 elements)
+  // wave-uniform 32-bit tile arithmetic (a tile is 512 LR elements)
   const uint32_t groups = (uint32_t)((p.cols + kMT - 1) / kMT);
-  const uint32_t ntiles = groups * (uint32_t)((p.rows + kLR * 4 - 1) / (kLR * 4));
+  const uint32_t ntiles = groups * (uint32_t)((p.rows + LR * 4 - 1) / (LR * 4));
   const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   for (uint32_t t = (uint32_t)blk * (kMxNT / 64) + wid; t < ntiles;
        t += (uint32_t)nblk * (kMxNT / 64)) {
-    const int64_t r0 = (int64_t)(t / groups) * (kLR * 4), c0 = (int64_t)(t % groups) * kMT;
-    const int64_t c = c0 + 8 * (lane & 15), rl = r0 + kLR * (lane >> 4);
-    uint4 v[kLR];
+    const int64_t r0 = (int64_t)(t / groups) * (LR * 4), c0 = (int64_t)(t % groups) * kMT;
+    const int64_t c = c0 + 8 * (lane & 15), rl = r0 + LR * (lane >> 4);
+    uint4 v[LR];
 #pragma unroll
-    for (int k = 0; k < kLR; ++k) {
+    for (int k = 0; k < LR; ++k) {
       v[k] = make_uint4(0u, 0u, 0u, 0u);
       if (rl + k < p.rows && c < p.cols)
         v[k] = *reinterpret_cast<const uint4*>(p.x + (rl + k) * p.cols + c);
     }
-    uint32_t rk[kLR], top = 0;
+    uint32_t rk[LR], top = 0;
 #pragma unroll
-    for (int k = 0; k < kLR; ++k) {
+    for (int k = 0; k < LR; ++k) {
       uint32_t m = pk_max_u16(pk_max_u16(v[k].x & 0x7FFF7FFFu, v[k].y & 0x7FFF7FFFu),
                               pk_max_u16(v[k].z & 0x7FFF7FFFu, v[k].w & 0x7FFF7FFFu));
       m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true));
@@ -444,52 +427,209 @@ __device__ __forceinline__ void mx_rows(const MxTile& p, int64_t blk, int64_t nb
       top = max(top, rk[k]);
     }
     if (__builtin_expect(__any(top >= 0x7F80u), 0))
-      mx_rows_body<FMT, false>(p, r0, c0, v, rk, lane);
+      mx_rows_body<FMT, false, LR>(p, r0, c0, v, rk, lane);
     else
-      mx_rows_body<FMT, true>(p, r0, c0, v, rk, lane);
+      mx_rows_body<FMT, true, LR>(p, r0, c0, v, rk, lane);
   }
 }
 
-// The rowwise copies alone, of up to kMxMany tensors. Memory-bound like the tile kernel, whose
-// registers and LDS for the columnwise copy hold it to 4 waves per SIMD; this one runs 8 (60
-// VGPRs, no LDS). Planes only, inputs repeated / rotated past the MALL, tile kernel -> this one:
-// [4096, 10240] 24.4 / 26.5 -> 20.8 / 22.3 us (5.7 TB/s), [20480, 2560] 27.9 / 29.7 -> 24.9 / 26.5,
-// [8192, 2560] 15.0 / 16.7 -> 11.5 / 13.1; with scale rows as well 27.9 / 29.4 -> 22.0 / 23.4.
-// Eight rows per lane (94 VGPRs) 22.8 / 24.7 us at [4096, 10240], two 20.1 / 23.0.
-__global__ __launch_bounds__(kMxNT) void mx_rows_kernel(MxManyArgs a) {
+// The rowwise copy alone. Memory-bound like the tile kernel, whose registers and LDS for the
+// columnwise copy hold it to 4 waves per SIMD; this one runs 8 (59 VGPRs, no LDS). Planes only,
+// inputs repeated / rotated past the MALL, tile kernel -> this one: [4096, 10240] 24.4 / 26.5 ->
+// 20.8 / 22.3 us (5.7 TB/s), [20480, 2560] 27.9 / 29.7 -> 24.9 / 26.5, [8192, 2560] 15.0 / 16.7 ->
+// 11.5 / 13.1; with scale rows as well 27.9 / 29.4 -> 22.0 / 23.4. Eight rows per lane (94 VGPRs)
+// 22.8 / 24.7 us at [4096, 10240], two 20.1 / 23.0.
+// Small tensors take one row per lane, four times the waves (kMxSmallRows).
+constexpr int kLR = 4;
+template <int FMT, int LR>
+__global__ __launch_bounds__(kMxNT) void mx_rows_kernel(MxTile p) {
+  mx_rows<FMT, LR>(p, blockIdx.x, gridDim.x);
+}
+
+// Both copies, or the columnwise one, of a small tensor: one wave per block takes 32 rows x 64
+// columns, so that the waves outnumber the CUs from 0.5M elements on, where the 128 x 128 tiles of
+// four waves leave most CUs idle. Lane l holds columns 8 (l & 7) .. +7 of the rows 8 k + l / 8,
+// k < 4; the wave holds whole blocks in both directions, and turns its bytes in its own LDS.
+// Latency-bound: scales leave as bytes and the columnwise copy in 32-byte pieces, which the L2
+// gathers while the tensor fits there.
+template <int FMT, bool FINITE>
+__device__ __forceinline__ void mx_wave_body(const MxTile& p, int64_t r0, int64_t c0,
+                                             const uint4 (&v)[4], const uint32_t (&rk)[4],
+                                             const uint32_t (&cm)[4], uint32_t* stage, int lane) {
+  const int cl = lane & 7, lr = lane >> 3;
+  const int64_t c = c0 + 8 * cl;
+  if (p.out && c < p.cols) {
+    const int64_t blk = c >> 5, nblk = p.cols >> 5;
+    // the block that ends a row also pads its last dword of scales
+    const int64_t end = blk == nblk - 1 ? (nblk + 3) & ~3LL : blk + 1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t r = r0 + 8 * k + lr;
+      uint32_t e;
+      if constexpr (FINITE)
+        e = mx_exponent_finite_pk<FMT>(rk[k]) & 0xFFFFu;
+      else
+        e = mx_exponent<FMT>(rk[k] << 16);
+      const float mult = mx_multiplier(e);
+      *reinterpret_cast<uint2*>(p.out + r * p.cols + c) =
+          FINITE ? quant8_bf16_finite<FMT, false>(v[k], mult) : quant8_bf16<FMT>(v[k], mult);
+      if ((cl & 3) == 0) {
+        for (int64_t b = blk; b < end; ++b) {
+          const uint8_t byte = b == blk ? (uint8_t)e : (uint8_t)kMxPadScale;
+          if (p.sc) p.sc[r * p.ld_sc + b] = byte;
+          if (p.planes) reinterpret_cast<uint8_t*>(p.planes + (b >> 2) * p.rows + r)[b & 3] = byte;
+        }
+      }
+    }
+  }
+  float s[8];
+  uint32_t ex[4];  // packed pairs of the lane's column exponents
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (FINITE)
+      ex[i] = mx_exponent_finite_pk<FMT>(cm[i]);
+    else
+      ex[i] = mx_exponent<FMT>(cm[i] << 16) | (mx_exponent<FMT>(cm[i] & 0xFFFF0000u) << 16);
+    s[2 * i] = mx_multiplier(ex[i] & 0xFFFFu);
+    s[2 * i + 1] = mx_multiplier(ex[i] >> 16);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint2 q = mx_quant8_vs<FMT, FINITE>(v[k], s);
+    uint32_t* d = stage + (8 * k + lr) * kWaveTilePitch + 2 * cl;
+    d[0] = q.x;
+    d[1] = q.y;
+  }
+  // lane (cl, lr) stores the scale of column c + lr, which its eight columns' lanes all hold
+  if (c + lr < p.cols) {
+    const uint32_t pair = lr < 4 ? (lr < 2 ? ex[0] : ex[1]) : (lr < 6 ? ex[2] : ex[3]);
+    const int64_t blk = r0 >> 5, nblk = p.rows >> 5;
+    const int64_t end = blk == nblk - 1 ? (nblk + 3) & ~3LL : blk + 1;
+    for (int64_t b = blk; b < end; ++b) {
+      const uint8_t byte = b == blk ? (uint8_t)(pair >> (16 * (lr & 1))) : (uint8_t)kMxPadScale;
+      if (p.sc_t) p.sc_t[(c + lr) * p.ld_sc_t + b] = byte;
+      if (p.planes_t)
+        reinterpret_cast<uint8_t*>(p.planes_t + (b >> 2) * p.cols + c + lr)[b & 3] = byte;
+    }
+  }
+}
+
+template <int FMT>
+__global__ __launch_bounds__(64) void mx_wave_kernel(MxTile p) {
+  __shared__ uint32_t stage[32 * kWaveTilePitch];
+  const int lane = threadIdx.x, cl = lane & 7, lr = lane >> 3;
+  const uint32_t tiles_c = (uint32_t)((p.cols + 63) / 64);
+  const int64_t r0 = (int64_t)(blockIdx.x / tiles_c) * 32, c0 = (int64_t)(blockIdx.x % tiles_c) * 64;
+  const int64_t c = c0 + 8 * cl;
+  uint4 v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)  // rows % 32 == 0: whole blocks of rows
+    v[k] = c < p.cols ? *reinterpret_cast<const uint4*>(p.x + (r0 + 8 * k + lr) * p.cols + c)
+                      : make_uint4(0u, 0u, 0u, 0u);
+  uint32_t rk[4], cm[4] = {}, top = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t a[4] = {v[k].x & 0x7FFF7FFFu, v[k].y & 0x7FFF7FFFu, v[k].z & 0x7FFF7FFFu,
+                           v[k].w & 0x7FFF7FFFu};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cm[i] = pk_max_u16(cm[i], a[i]);
+    uint32_t m = pk_max_u16(pk_max_u16(a[0], a[1]), pk_max_u16(a[2], a[3]));
+    m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true));
+    m = pk_max_u16(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, true));
+    rk[k] = max(m & 0xFFFFu, m >> 16);
+    top = max(top, rk[k]);
+  }
+#pragma unroll
+  for (int off = 8; off < 64; off <<= 1)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], off, 64));
+  if (__builtin_expect(__any(top >= 0x7F80u), 0))
+    mx_wave_body<FMT, false>(p, r0, c0, v, rk, cm, stage, lane);
+  else
+    mx_wave_body<FMT, true>(p, r0, c0, v, rk, cm, stage, lane);
+  __syncthreads();
+  // lane: 8 rows (lane & 3) x 4 columns (lane >> 2)
+  const int rg = (lane & 3) * 8, cg = lane >> 2;
+  uint32_t t[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint32_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = stage[(rg + 4 * h + i) * kWaveTilePitch + cg];
+    transpose_4x4(d, t[h]);
+  }
+#pragma unroll
+  for (int cc = 0; cc < 4; ++cc) {
+    const int64_t tr = c0 + 4 * cg + cc;  // row of out_t (a column of x)
+    if (tr < p.cols)
+      *reinterpret_cast<uint2*>(p.out_t + tr * p.rows + r0 + rg) = make_uint2(t[0][cc], t[1][cc]);
+  }
+}
+
+// Up to kMxMany tensors in one launch: tensor t owns blocks [first, next tensor's first), so
+// that a forward's small tensors fill the chip together and save launches. A single tensor runs
+// mx_rows_kernel: finding a tensor in the list is a chain of loads of the arguments, 1.1 us of the
+// 3.3 us that 32 x 2560 took in a list of one (2.2 us without).
+constexpr int kMxMany = 8;
+
+struct MxManyArgs {
+  MxTile t[kMxMany];
+  int64_t first[kMxMany + 1];
+  int count;
+};
+
+template <int LR>
+__global__ __launch_bounds__(kMxNT) void mx_rows_many_kernel(MxManyArgs a) {
   int i = 0;
   for (int k = 1; k < a.count; ++k)
     if ((int64_t)blockIdx.x >= a.first[k]) i = k;
   const int64_t blk = (int64_t)blockIdx.x - a.first[i], nblk = a.first[i + 1] - a.first[i];
   if (a.t[i].fmt == BF8_E4M3)
-    mx_rows<BF8_E4M3>(a.t[i], blk, nblk);
+    mx_rows<BF8_E4M3, LR>(a.t[i], blk, nblk);
   else
-    mx_rows<BF8_E5M2>(a.t[i], blk, nblk);
+    mx_rows<BF8_E5M2, LR>(a.t[i], blk, nblk);
 }
 
-// Adds a tensor to a launch (one with a columnwise copy is launched alone).
-void mx_add(MxManyArgs& a, const MxTile& t) {
-  const int64_t tiles_c = (t.cols + kMT - 1) / kMT;
-  // rowwise: a block's four waves take a tile of 4 kLR rows x 128 columns each
-  const int64_t blocks =
-      t.out_t ? std::min<int64_t>((t.rows + kMT - 1) / kMT * tiles_c, kMaxMxTileBlocks)
-              : std::min<int64_t>(((t.rows + 4 * kLR - 1) / (4 * kLR) * tiles_c + 3) / 4,
-                                  kMaxMxRowBlocks);
-  a.t[a.count] = t;
-  a.first[a.count + 1] = a.first[a.count] + blocks;
-  ++a.count;
+// Blocks of the rowwise kernel: four waves take a tile of 4 lr rows x 128 columns each.
+int64_t mx_row_blocks(const MxTile& t, int lr) {
+  const int64_t tiles = (t.rows + 4 * lr - 1) / (4 * lr) * ((t.cols + kMT - 1) / kMT);
+  return std::min<int64_t>((tiles + 3) / 4, kMaxMxRowBlocks);
 }
 
-int mx_launch(const MxManyArgs& a, void* stream) {
-  if (a.count == 0) return BF8_OK;
-  if (!a.t[0].out_t) {
-    hipLaunchKernelGGL(mx_rows_kernel, dim3((unsigned)a.first[a.count]), dim3(kMxNT), 0,
-                       as_stream(stream), a);
+// Elements up to which a tensor takes the small kernels. Large / small kernel, us, input not seen
+// before (repeated): rowwise 2.5M 5.1 / 4.1 (3.6 / 3.1), 5.6M 6.5 / 6.3 (4.8 / 4.9), 8.1M 7.9 / 7.8
+// (6.1 / 6.3), 10.4M 9.0 / 9.2; both copies 0.9M 7.8 / 5.0, 4.4M 10.8 / 8.5 (9.3 / 7.2), 8.1M 14.1 /
+// 11.2, 10.0M 14.5 / 13.7, 11.1M 15.2 / 16.3 (14.0 / 12.6), 30M 30.6 / 38.5 (29.2 / 26.6).
+constexpr int64_t kMxSmallRows = 6 << 20, kMxSmallTile = 8 << 20;
+
+template <int FMT>
+int mx_launch_one(const MxTile& t, hipStream_t s) {
+  const int64_t n = t.rows * t.cols;
+  if (!t.out_t) {
+    if (n <= kMxSmallRows)
+      hipLaunchKernelGGL((mx_rows_kernel<FMT, 1>), dim3((unsigned)mx_row_blocks(t, 1)), dim3(kMxNT),
+                         0, s, t);
+    else
+      hipLaunchKernelGGL((mx_rows_kernel<FMT, kLR>), dim3((unsigned)mx_row_blocks(t, kLR)),
+                         dim3(kMxNT), 0, s, t);
     return launch_status("mx_rows_kernel");
   }
-  hipLaunchKernelGGL(mx_tile_kernel, dim3((unsigned)a.first[a.count]), dim3(kMxNT), 0,
-                     as_stream(stream), a);
+  if (n <= kMxSmallTile) {
+    hipLaunchKernelGGL(mx_wave_kernel<FMT>, dim3((unsigned)(t.rows / 32 * ((t.cols + 63) / 64))),
+                       dim3(64), 0, s, t);
+    return launch_status("mx_wave_kernel");
+  }
+  const int64_t tiles = (t.rows + kMT - 1) / kMT * ((t.cols + kMT - 1) / kMT);
+  hipLaunchKernelGGL(mx_tile_kernel<FMT>,
+                     dim3((unsigned)std::min<int64_t>(tiles, kMaxMxTileBlocks)), dim3(kMxNT), 0, s,
+                     t);
   return launch_status("mx_tile_kernel");
+}
+
+int mx_launch(const MxTile& t, void* stream) {
+  return t.fmt == BF8_E4M3 ? mx_launch_one<BF8_E4M3>(t, as_stream(stream))
+                           : mx_launch_one<BF8_E5M2>(t, as_stream(stream));
 }
 
 }  // namespace
@@ -518,11 +658,10 @@ static int quantize_mx_entry(const char* who, const void* x, int64_t rows, int64
   BF8_CHECK(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 7) == 0 && ((uintptr_t)out_t & 15) == 0 &&
                 (((uintptr_t)out_scales | (uintptr_t)out_planes | (uintptr_t)out_t_planes) & 3) == 0,
             "%s: x, out_t 16-byte, out 8-byte, out_scales and scale planes 4-byte aligned", who);
-  MxManyArgs a{};
-  mx_add(a, MxTile{(const uint16_t*)x, rows, cols, out, out_scales, out_planes,
-                   out ? bf8_mx_scale_ld(cols) : 0, out_t, out_t_scales, out_t_planes,
-                   bf8_mx_scale_ld(rows), fmt});
-  return mx_launch(a, stream);
+  return mx_launch(MxTile{(const uint16_t*)x, rows, cols, out, out_scales, out_planes,
+                          out ? bf8_mx_scale_ld(cols) : 0, out_t, out_t_scales, out_t_planes,
+                          bf8_mx_scale_ld(rows), fmt},
+                   stream);
 }
 
 int bf8_quantize_mx_planes_bf16(const void* x, int64_t rows, int64_t cols, int fmt, uint8_t* out,
@@ -577,6 +716,7 @@ static int quantize_mx_many_entry(const char* who, int count, const void* const*
   BF8_CHECK(count >= 1 && count <= kMxMany, "%s: count %d outside [1, %d]", who, count, kMxMany);
   BF8_CHECK(x && rows && cols && fmt && out && out_scales, "%s: NULL array", who);
   MxManyArgs a{};
+  int64_t n = 0;
   for (int t = 0; t < count; ++t) {
     BF8_CHECK(fmt[t] == BF8_E4M3 || fmt[t] == BF8_E5M2, "%s: tensor %d: bad fmt %d", who, t, fmt[t]);
     BF8_CHECK(rows[t] >= 0 && cols[t] >= 0, "%s: tensor %d: negative shape", who, t);
@@ -590,10 +730,20 @@ static int quantize_mx_many_entry(const char* who, int count, const void* const*
     BF8_CHECK(((uintptr_t)x[t] & 15) == 0 && ((uintptr_t)out[t] & 7) == 0 &&
                   (((uintptr_t)out_scales[t] | (uintptr_t)planes) & 3) == 0,
               "%s: tensor %d: x 16-byte, out 8-byte, out_scales and scale planes 4-byte aligned", who, t);
-    mx_add(a, MxTile{(const uint16_t*)x[t], rows[t], cols[t], out[t], out_scales[t], planes,
-                     bf8_mx_scale_ld(cols[t]), nullptr, nullptr, nullptr, 0, fmt[t]});
+    a.t[a.count++] = MxTile{(const uint16_t*)x[t], rows[t], cols[t], out[t], out_scales[t], planes,
+                            bf8_mx_scale_ld(cols[t]), nullptr, nullptr, nullptr, 0, fmt[t]};
+    n += rows[t] * cols[t];
   }
-  return mx_launch(a, stream);
+  if (a.count == 0) return BF8_OK;
+  if (a.count == 1) return mx_launch(a.t[0], stream);
+  const int lr = n <= kMxSmallRows ? 1 : kLR;
+  for (int t = 0; t < a.count; ++t) a.first[t + 1] = a.first[t] + mx_row_blocks(a.t[t], lr);
+  const dim3 grid((unsigned)a.first[a.count]);
+  if (lr == 1)
+    hipLaunchKernelGGL(mx_rows_many_kernel<1>, grid, dim3(kMxNT), 0, as_stream(stream), a);
+  else
+    hipLaunchKernelGGL(mx_rows_many_kernel<kLR>, grid, dim3(kMxNT), 0, as_stream(stream), a);
+  return launch_status("mx_rows_many_kernel");
 }
 
 int bf8_quantize_mx_many_planes_bf16(int count, const void* const* x, const int64_t* rows,

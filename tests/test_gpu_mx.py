@@ -52,10 +52,12 @@ def test_quantize_mx_bit_exact(gpu, rows, cols, fmt):
     assert same_q and same_s
 
 
-@pytest.mark.parametrize("rows,cols", [(32, 32), (128, 128), (160, 96), (288, 416), (64, 144)])
+@pytest.mark.parametrize("rows,cols", [(32, 32), (128, 128), (160, 96), (288, 416), (64, 144),
+                                       (4128, 2144), (8352, 1040)])
 def test_quantize_mx_two_copies_edges(gpu, rows, cols):
-    """Both copies from one pass over 128 x 128 tiles: whole and partial tiles in either
-    direction (scale padding included), blocks holding inf, NaN and the largest and smallest
+    """Both copies from one pass over 32 x 64 tiles (small tensors) and 128 x 128 tiles (the last
+    two, past 8 x 2^20 elements): whole and partial tiles in either direction (scale padding
+    included), both layouts of the scales, blocks holding inf, NaN and the largest and smallest
     magnitudes, and the columnwise copy alone."""
     x = _x(rows, cols, 3 * rows + cols, spread=False).float()
     x[1, 3], x[rows - 1, cols - 1], x[rows // 2, cols // 2] = float("inf"), float("nan"), -float("inf")
@@ -70,10 +72,12 @@ def test_quantize_mx_two_copies_edges(gpu, rows, cols):
     for t in (q, only):
         assert torch.equal(t.data_t.view(torch.uint8).cpu(), cq)
         assert torch.equal(t.scales_t.cpu(), orc.mx_scale_rows(ce))
+        assert torch.equal(t.planes_t, _planes_of(t.scales_t))
     if rowwise:
         rq, re = orc.quantize_mx(x, ops.E4M3, -1)
         assert torch.equal(q.data.view(torch.uint8).cpu(), rq)
         assert torch.equal(q.scales.cpu(), orc.mx_scale_rows(re))
+        assert torch.equal(q.planes, _planes_of(q.scales))
 
 
 def test_quantize_mx_errors(gpu):
@@ -83,10 +87,11 @@ def test_quantize_mx_errors(gpu):
         ops.quantize_mx(torch.zeros(48, 64, dtype=torch.bfloat16, device=gpu), colwise=True)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 32), (33, 128), (95, 160), (128, 416), (300, 1056)])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (3, 96), (33, 128), (95, 160), (128, 416), (300, 1056),
+                                       (3001, 2112)])
 def test_quantize_mx_rows_alone(gpu, rows, cols):
-    """The rowwise copy alone: rows and columns that leave partial 32 x 128 wave tiles, with and
-    without inf, NaN and the largest and smallest magnitudes; bytes and both layouts of the scales,
+    """The rowwise copy alone: rows and columns that leave partial wave tiles of 4 x 128 (small
+    tensors) and 16 x 128 (the last, past 6 x 2^20 elements), with and without inf, NaN and the largest and smallest magnitudes; bytes and both layouts of the scales,
     one tensor or several, against the oracle."""
     x = _x(rows, cols, rows + cols, spread=False)
     y = x.float()
