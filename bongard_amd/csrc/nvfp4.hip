@@ -355,8 +355,8 @@ __global__ __launch_bounds__(kNT) void nvfp4_rows_kernel(const uint16_t* __restr
   }
 }
 
-// Columnwise quantization of a tensor whose rows are not whole 16-byte vectors (cols % 8 != 0),
-// which the tile kernel's loads need: one (column, 16-row block) per thread, consecutive
+// Columnwise quantization of a small tensor, or of one whose rows are not whole 16-byte vectors
+// (cols % 8 != 0), which the tile kernel's loads need: one (column, 16-row block) per thread, consecutive
 // threads on consecutive columns. out_t [cols, rows / 2], scales_t [cols, rows / 16].
 __global__ __launch_bounds__(kNT) void nvfp4_cols_kernel(const uint16_t* __restrict__ x,
                                                          int64_t rows, int64_t cols,
@@ -433,6 +433,12 @@ static int nvfp4_args(const char* who, const void* x, int64_t rows, int64_t cols
   return BF8_OK;
 }
 
+// Columnwise codes alone of at most this many elements take the columns kernel, one block of 16
+// values per thread: the tile kernel's 128 x 128 tiles leave most CUs idle and its code is long.
+// Tile / columns kernel, us, inputs not seen before: 64 x 640 5.3 / 3.4, 320 x 2048 5.9 / 4.0,
+// 1216 x 2048 6.7 / 5.9, 3584 x 2048 9.3 / 10.4, 2304 x 2560 9.1 / 11.1.
+constexpr int64_t kMaxColsKernel = 4 << 20;
+
 // The rowwise and/or columnwise casts, the per-tensor amax reduced from np partials (maxima
 // of |x| as fp32 bits) that are already written.
 static int nvfp4_casts(const void* x, const NvTile& p, const uint32_t* partials, int64_t np,
@@ -442,10 +448,10 @@ static int nvfp4_casts(const void* x, const NvTile& p, const uint32_t* partials,
                        (const uint16_t*)x, p, partials, np, meta);
     return launch_status("nvfp4_rows_kernel");
   }
-  if (p.cols % 8 != 0) {
-    // rows of broken vectors: only columnwise codes take these shapes
+  if (p.cols % 8 != 0)  // rows of broken vectors: only columnwise codes take these shapes
     BF8_CHECK(!p.deq_t, "nvfp4: a columnwise dequantization needs cols %% 8 == 0 (got %lld)",
               (long long)p.cols);
+  if (p.cols % 8 != 0 || (!p.out && !p.deq && !p.deq_t && p.rows * p.cols <= kMaxColsKernel)) {
     hipLaunchKernelGGL(nvfp4_cols_kernel, dim3(stream_grid(p.rows * p.cols / 16)), dim3(kNT), 0, s,
                        (const uint16_t*)x, p.rows, p.cols, partials, np, meta, p.out_t,
                        p.scales_t);
