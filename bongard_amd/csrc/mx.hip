@@ -465,6 +465,7 @@ __device__ __forceinline__ void mx_wave_body(const MxTile& p, int64_t r0, int64_
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int64_t r = r0 + 8 * k + lr;
+      if (r >= p.rows) break;
       uint32_t e;
       if constexpr (FINITE)
         e = mx_exponent_finite_pk<FMT>(rk[k]) & 0xFFFFu;
@@ -482,6 +483,7 @@ __device__ __forceinline__ void mx_wave_body(const MxTile& p, int64_t r0, int64_
       }
     }
   }
+  if (!p.out_t) return;
   float s[8];
   uint32_t ex[4];  // packed pairs of the lane's column exponents
 #pragma unroll
@@ -514,18 +516,11 @@ __device__ __forceinline__ void mx_wave_body(const MxTile& p, int64_t r0, int64_
   }
 }
 
+// The wave's loaded 32 x 64 tile at (r0, c0), v[k] the lane's vector of row 8 k + l / 8 (zeros past
+// p.rows or p.cols). Every wave of the block calls it alike, each with its own stage.
 template <int FMT>
-__global__ __launch_bounds__(64) void mx_wave_kernel(MxTile p) {
-  __shared__ uint32_t stage[32 * kWaveTilePitch];
-  const int lane = threadIdx.x, cl = lane & 7, lr = lane >> 3;
-  const uint32_t tiles_c = (uint32_t)((p.cols + 63) / 64);
-  const int64_t r0 = (int64_t)(blockIdx.x / tiles_c) * 32, c0 = (int64_t)(blockIdx.x % tiles_c) * 64;
-  const int64_t c = c0 + 8 * cl;
-  uint4 v[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k)  // rows % 32 == 0: whole blocks of rows
-    v[k] = c < p.cols ? *reinterpret_cast<const uint4*>(p.x + (r0 + 8 * k + lr) * p.cols + c)
-                      : make_uint4(0u, 0u, 0u, 0u);
+__device__ __forceinline__ void mx_wave_finish(const MxTile& p, int64_t r0, int64_t c0,
+                                               const uint4 (&v)[4], uint32_t* stage, int lane) {
   uint32_t rk[4], cm[4] = {}, top = 0;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -539,15 +534,18 @@ __global__ __launch_bounds__(64) void mx_wave_kernel(MxTile p) {
     rk[k] = max(m & 0xFFFFu, m >> 16);
     top = max(top, rk[k]);
   }
+  if (p.out_t) {
 #pragma unroll
-  for (int off = 8; off < 64; off <<= 1)
+    for (int off = 8; off < 64; off <<= 1)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], off, 64));
+      for (int i = 0; i < 4; ++i)
+        cm[i] = pk_max_u16(cm[i], (uint32_t)__shfl_xor((int)cm[i], off, 64));
+  }
   if (__builtin_expect(__any(top >= 0x7F80u), 0))
     mx_wave_body<FMT, false>(p, r0, c0, v, rk, cm, stage, lane);
   else
     mx_wave_body<FMT, true>(p, r0, c0, v, rk, cm, stage, lane);
+  if (!p.out_t) return;
   __syncthreads();
   // lane: 8 rows (lane & 3) x 4 columns (lane >> 2)
   const int rg = (lane & 3) * 8, cg = lane >> 2;
@@ -565,6 +563,69 @@ __global__ __launch_bounds__(64) void mx_wave_kernel(MxTile p) {
     if (tr < p.cols)
       *reinterpret_cast<uint2*>(p.out_t + tr * p.rows + r0 + rg) = make_uint2(t[0][cc], t[1][cc]);
   }
+}
+
+template <int FMT>
+__global__ __launch_bounds__(64) void mx_wave_kernel(MxTile p) {
+  __shared__ uint32_t stage[32 * kWaveTilePitch];
+  const int lane = threadIdx.x, cl = lane & 7, lr = lane >> 3;
+  const uint32_t tiles_c = (uint32_t)((p.cols + 63) / 64);
+  const int64_t r0 = (int64_t)(blockIdx.x / tiles_c) * 32, c0 = (int64_t)(blockIdx.x % tiles_c) * 64;
+  const int64_t c = c0 + 8 * cl;
+  uint4 v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)  // rows % 32 == 0: whole blocks of rows
+    v[k] = c < p.cols ? *reinterpret_cast<const uint4*>(p.x + (r0 + 8 * k + lr) * p.cols + c)
+                      : make_uint4(0u, 0u, 0u, 0u);
+  mx_wave_finish<FMT>(p, r0, c0, v, stage, lane);
+}
+
+// d_g (G) or d_u of the lane's four rows 8 k of a wave tile.
+template <bool G>
+__device__ __forceinline__ void geglu_bwd_wave_rows(const uint16_t* dp, const uint16_t* gp,
+                                                    int64_t I, int64_t rows_left,
+                                                    const uint16_t* ta, const uint32_t* tf,
+                                                    uint4 (&v)[4]) {
+  uint4 d[4], g[4], u[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    d[k] = g[k] = u[k] = make_uint4(0u, 0u, 0u, 0u);
+    if (8 * k < rows_left) {
+      d[k] = *reinterpret_cast<const uint4*>(dp + 8 * k * I);
+      g[k] = *reinterpret_cast<const uint4*>(gp + 16 * k * I);
+      if (G) u[k] = *reinterpret_cast<const uint4*>(gp + 16 * k * I + I);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = geglu_bwd8_half<G>(d[k], g[k], u[k], ta, tf);
+}
+
+// geglu_bwd_mx_kernel for small outputs: a block takes 32 rows x 128 columns of I, two waves their
+// d_g tiles and two their d_u tiles (as mx_wave_kernel), where a tile of 128 rows keeps one CU
+// busy for 12 us and leaves the others idle.
+template <int FMT>
+__global__ __launch_bounds__(kMxNT) void geglu_bwd_mx_wave_kernel(const uint16_t* __restrict__ dH,
+                                                                  const uint16_t* __restrict__ GU,
+                                                                  int64_t I, MxTile p) {
+  __shared__ __attribute__((aligned(16))) uint16_t ta[kGeluABytes / 2];
+  __shared__ __attribute__((aligned(16))) uint32_t tf[kGeluFBytes / 4];
+  __shared__ uint32_t stage[4][32 * kWaveTilePitch];
+  load_gelu_tables<kMxNT>(ta, tf);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wid >> 1;
+  const uint32_t tiles_c = (uint32_t)(I / kMT);
+  const int64_t r0 = (int64_t)(blockIdx.x / tiles_c) * 32;
+  const int64_t c0 = (int64_t)(blockIdx.x % tiles_c) * kMT + 64 * (wid & 1);
+  const int64_t rw = r0 + (lane >> 3);
+  const uint16_t* dp = dH + rw * I + c0 + 8 * (lane & 7);
+  const uint16_t* gp = GU + rw * 2 * I + c0 + 8 * (lane & 7);
+  uint4 v[4];
+  if (half == 0)
+    geglu_bwd_wave_rows<true>(dp, gp, I, p.rows - rw, ta, tf, v);
+  else
+    geglu_bwd_wave_rows<false>(dp, gp, I, p.rows - rw, ta, tf, v);
+  mx_wave_finish<FMT>(p, r0, half * I + c0, v, stage[wid], lane);
 }
 
 // Up to kMxMany tensors in one launch: tensor t owns blocks [first, next tensor's first), so
@@ -602,6 +663,10 @@ int64_t mx_row_blocks(const MxTile& t, int lr) {
 // (6.1 / 6.3), 10.4M 9.0 / 9.2; both copies 0.9M 7.8 / 5.0, 4.4M 10.8 / 8.5 (9.3 / 7.2), 8.1M 14.1 /
 // 11.2, 10.0M 14.5 / 13.7, 11.1M 15.2 / 16.3 (14.0 / 12.6), 30M 30.6 / 38.5 (29.2 / 26.6).
 constexpr int64_t kMxSmallRows = 6 << 20, kMxSmallTile = 8 << 20;
+// The same for the fused gated-GELU backward's dGU, us on gradients not seen before: both copies
+// 0.2M 15.0 / 7.4, 2.5M 16.0 / 9.8, 5.6M 17.5 / 13.3, 6.6M 18.1 / 19.1; rowwise alone 2.5M 13.1 /
+// 7.4, 8.8M 19.0 / 14.2, 12.8M 19.9 / 19.4.
+constexpr int64_t kBwdSmallRows = 12 << 20, kBwdSmall = 6 << 20;
 
 template <int FMT>
 int mx_launch_one(const MxTile& t, hipStream_t s) {
@@ -691,14 +756,23 @@ int bf8_geglu_bwd_mx_planes(const void* dH, const void* GU, int64_t M, int64_t I
             "%s: dH, GU, out_t 16-byte, out 8-byte, planes 4-byte aligned", who);
   const MxTile p{nullptr, M, 2 * I, out, nullptr, out_planes, 0, out_t, nullptr, out_t_planes, 0,
                  fmt};
+  const auto* d = (const uint16_t*)dH;
+  const auto* g = (const uint16_t*)GU;
+  hipStream_t s = as_stream(stream);
+  if (2 * M * I <= (out_t ? kBwdSmall : kBwdSmallRows)) {
+    const dim3 grid((unsigned)((M + 31) / 32 * (I / kMT)));
+    if (fmt == BF8_E4M3)
+      hipLaunchKernelGGL(geglu_bwd_mx_wave_kernel<BF8_E4M3>, grid, dim3(kMxNT), 0, s, d, g, I, p);
+    else
+      hipLaunchKernelGGL(geglu_bwd_mx_wave_kernel<BF8_E5M2>, grid, dim3(kMxNT), 0, s, d, g, I, p);
+    return launch_status("geglu_bwd_mx_wave_kernel");
+  }
   const int64_t tiles = ((M + kMT - 1) / kMT) * (I / kMT);
   const dim3 grid((unsigned)std::min<int64_t>(tiles, kMaxBwdBlocks));
   if (fmt == BF8_E4M3)
-    hipLaunchKernelGGL(geglu_bwd_mx_kernel<BF8_E4M3>, grid, dim3(kBwdNT), 0, as_stream(stream),
-                       (const uint16_t*)dH, (const uint16_t*)GU, I, p);
+    hipLaunchKernelGGL(geglu_bwd_mx_kernel<BF8_E4M3>, grid, dim3(kBwdNT), 0, s, d, g, I, p);
   else
-    hipLaunchKernelGGL(geglu_bwd_mx_kernel<BF8_E5M2>, grid, dim3(kBwdNT), 0, as_stream(stream),
-                       (const uint16_t*)dH, (const uint16_t*)GU, I, p);
+    hipLaunchKernelGGL(geglu_bwd_mx_kernel<BF8_E5M2>, grid, dim3(kBwdNT), 0, s, d, g, I, p);
   return launch_status("geglu_bwd_mx_kernel");
 }
 

@@ -282,11 +282,15 @@ def test_gemm_geglu_mx_quant_errors(gpu):
         ops.gemm_geglu_mx_quant(qx.data, qx.scales, qw.data, qw.scales, 256, colwise=True)
 
 
-@pytest.mark.parametrize("M,I", [(32, 128), (96, 384), (128, 256), (160, 128), (1056, 640)])
-@pytest.mark.parametrize("rowwise,colwise", [(True, True), (True, False), (False, True)])
+@pytest.mark.parametrize("M,I,rowwise,colwise", [
+    (M, I, *copies) for M, I in [(32, 128), (96, 384), (128, 256), (160, 128), (1056, 640),
+                                 (2080, 1536), (4128, 1536)]
+    for copies in [(True, True), (True, False), (False, True)]] + [
+    (M, I, True, False) for M, I in [(1, 128), (45, 256), (4131, 1536)]])
 def test_geglu_bwd_mx_equals_two_passes(gpu, M, I, rowwise, colwise):
-    """The fused gated-GELU backward and MX quantizer (one tile of I per half block, odd tile
-    counts, partial tile rows, an inf and a NaN gradient) against geglu_bwd and quantize_mx: the
+    """The fused gated-GELU backward and MX quantizer, by wave tiles of 32 x 64 and, past 6 x 2^20
+    elements of dGU (12 x 2^20 rowwise alone), tiles of 128 x 128: odd tile counts, partial tile
+    rows, an inf and a NaN gradient, against geglu_bwd and quantize_mx: the
     same bytes and scale planes."""
     g = torch.Generator().manual_seed(M + I)
     dH = torch.randn(M, I, generator=g)
