@@ -873,8 +873,19 @@ gemm_kernel(GemmParams p) {
   if constexpr (kLateTab) {
     if (niters >= 2)
       step(std::false_type{}, std::integral_constant<int, EXTRA_TABLE>{}, ls++);
-    else
-      load_table();  // no earlier step to load it behind: slot 0 holds no step
+    else {
+      // No earlier step to load it behind. Slot 0 holds no step, but its zero fill may be in flight.
+      // A wave's loads land in order, and both give 1 KB block b of the slot's tiles to wave b mod
+      // NW, so there the table lands last; where it reaches the scale dwords (the MX 64x128
+      // tile), which every wave fills a part of, the fill is waited for.
+      static_assert(kA == DA * NW * 1024 && BN * kBK == DB * NW * 1024,
+                    "the zero fill and the gelu table give a block of the tiles to one wave");
+      if constexpr (kData < kGeluA32Bytes) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+      }
+      load_table();
+    }
     step(std::false_type{}, none, ls);
   } else {
     for (; ls < niters; ++ls) step(std::false_type{}, none, ls);

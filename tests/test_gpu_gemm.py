@@ -347,6 +347,16 @@ def test_geglu_b_ahead_short_k(gpu, monkeypatch, K):
     _geglu_case(gpu, 300, 640, K, seed=K)
 
 
+@pytest.mark.parametrize("tile", ["256x256", "256x256w8"])
+@pytest.mark.parametrize("K", [64, 128, 256, 336, 512])
+def test_geglu_late_table_short_k(gpu, monkeypatch, tile, K):
+    """Gated-GELU tiles of two stages load the gelu table into a stage slot behind the last K
+    step: K loops of one step (the slot's zero fill may then still be in flight), two, three and
+    four, whole and partial, against the oracle."""
+    monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", tile)
+    _geglu_case(gpu, 300, 384, K, seed=K)
+
+
 def test_skinny_down_projection_auto_plan(gpu):
     """c4's down projection (M=512, K=10240): the automatic plan splits K."""
     assert ops._lib.lib().bf8_gemm_workspace(512, 2560, 10240) > 0
