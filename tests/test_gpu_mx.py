@@ -91,8 +91,9 @@ def test_quantize_mx_errors(gpu):
                                        (3001, 2112)])
 def test_quantize_mx_rows_alone(gpu, rows, cols):
     """The rowwise copy alone: rows and columns that leave partial wave tiles of 4 x 128 (small
-    tensors) and 16 x 128 (the last, past 6 x 2^20 elements), with and without inf, NaN and the largest and smallest magnitudes; bytes and both layouts of the scales,
-    one tensor or several, against the oracle."""
+    tensors) and 16 x 128 (the last, past 6 x 2^20 elements), with and without inf, NaN and the
+    largest and smallest magnitudes; bytes and both layouts of the scales, one tensor or several,
+    against the oracle."""
     x = _x(rows, cols, rows + cols, spread=False)
     y = x.float()
     y[0, :16], y[rows - 1, 16:32] = 3.38e38, 1e-39
@@ -136,10 +137,12 @@ def test_mx_scale_planes(gpu, rows, cols):
         ops.gemm_mx(q.data, None, qw.data, None, a_planes=qw.planes, b_planes=q.planes)
 
 
+@pytest.mark.parametrize("tile", ["", "256x256w8"])
 @pytest.mark.parametrize("M,I,K", [(32, 128, 96), (288, 384, 512), (512, 1280, 2560)])
-def test_gemm_geglu_mx_planes(gpu, M, I, K):
+def test_gemm_geglu_mx_planes(gpu, monkeypatch, tile, M, I, K):
     """The gated-GELU GEMM on planes: H's bytes, its planes (both copies) and GU equal those of
-    the GEMM on scale rows."""
+    the GEMM on scale rows (which test_gemm_geglu_mx_quant holds against the oracle)."""
+    monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", tile)
     x = _x(M, K, M, spread=False).to(gpu)
     w = (_x(2 * I, K, I, spread=False).float() * 0.02).to(torch.bfloat16).to(gpu)
     qx, qw = ops.quantize_mx(x), ops.quantize_mx(w)
@@ -165,7 +168,10 @@ def _mx_gemm_case(gpu, M, N, K, seed, bias=False):
     bias_g = bias_t.to(gpu) if bias else None
     y32 = ops.gemm_mx(qa.data, qa.scales, qb.data, qb.scales, out_dtype=torch.float32, bias=bias_g)
     y16 = ops.gemm_mx(qa.data, qa.scales, qb.data, qb.scales, bias=bias_g)
+    planes = ops.gemm_mx(qa.data, None, qb.data, None, a_planes=qa.planes, b_planes=qb.planes,
+                         bias=bias_g)
     torch.cuda.synchronize()
+    assert torch.equal(planes.view(torch.int16), y16.view(torch.int16))
     ra, ea = orc.quantize_mx(a, ops.E4M3)
     rb, eb = orc.quantize_mx(b, ops.E4M3)
     assert torch.equal(qa.data.view(torch.uint8).cpu(), ra)
@@ -192,10 +198,11 @@ def test_gemm_mx_bias(gpu):
     _mx_gemm_case(gpu, 200, 256, 512, seed=5, bias=True)
 
 
-def test_gemm_mx_tail_split(gpu, monkeypatch):
+@pytest.mark.parametrize("tile", ["256x256", "256x256w8"])
+def test_gemm_mx_tail_split(gpu, monkeypatch, tile):
     """MX operands under the tail split (272 tiles of 256x256, 16 of them split along K):
     the tail tiles' pieces are reduced with unit scales."""
-    monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", "256x256:t")
+    monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", tile + ":t")
     M, N, K = 4160, 3848, 4096
     assert ops._lib.lib().bf8_gemm_mx_workspace(M, N, K) % (16 * 256 * 256 * 4) == 0
     _mx_gemm_case(gpu, M, N, K, seed=63, bias=True)
@@ -228,11 +235,11 @@ def test_gemm_geglu_mx(gpu, M, I, K):
     assert (diff > 0).float().mean().item() <= 0.05
 
 
-GEGLU_TILES = ["256x256", "160x256", "192x256", "128x128", "64x128", "256x128"]
+GEGLU_TILES = ["256x256", "160x256", "192x256", "128x128", "64x128", "256x128", "256x256w8"]
 
 
 @pytest.mark.parametrize("tile", ["auto"] + GEGLU_TILES)
-@pytest.mark.parametrize("M,I,K", [(320, 384, 256), (100, 256, 128)])
+@pytest.mark.parametrize("M,I,K", [(320, 384, 256), (100, 256, 128), (288, 128, 352), (33, 128, 512)])
 def test_gemm_geglu_mx_quant(gpu, monkeypatch, tile, M, I, K):
     """H quantized in the GEGLU epilogue == bf8_quantize_mx_bf16 of the bf16 H of the
     unfused kernel, byte for byte (fp8 payloads, E8M0 scales, the transposed copy and its
@@ -436,12 +443,55 @@ def test_fused_mlp_mxfp8_fwd_bwd(gpu):
 
 
 @pytest.mark.parametrize("tile", ["256x256", "256x160", "160x256", "128x128", "192x256",
-                                  "128x64", "64x128", "256x128"])
-def test_gemm_mx_every_tile(gpu, monkeypatch, tile):
+                                  "128x64", "64x128", "256x128", "256x256w8", "128x128o2"])
+@pytest.mark.parametrize("M,N,K", [(300, 392, 544), (100, 264, 96), (520, 264, 256), (257, 520, 352)])
+def test_gemm_mx_every_tile(gpu, monkeypatch, tile, M, N, K):
     """Every block tile's MX variant (those whose stages would overflow the LDS with the
-    scale dwords run with one stage fewer), forced through the tuning override."""
+    scale dwords run with one stage fewer), forced through the tuning override: partial tiles in M
+    and N, K of one, two, three and five steps with whole and partial last steps, bf16 and fp32
+    out, scale rows and planes."""
     monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", tile)
-    _mx_gemm_case(gpu, 300, 392, 544, seed=17)
+    _mx_gemm_case(gpu, M, N, K, seed=17 + K, bias=K == 352)
+
+
+def test_gemm_mx_eight_wave_split_k(gpu, monkeypatch):
+    """Three K pieces (7, 7 and 6 steps, the last with a partial one) of the eight-wave tile."""
+    monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", "256x256w8:3")
+    M, N, K = 300, 520, 2528
+    assert ops._lib.lib().bf8_gemm_mx_workspace(M, N, K) == 3 * M * N * 4
+    _mx_gemm_case(gpu, M, N, K, seed=23, bias=True)
+
+
+@pytest.mark.parametrize("tile", ["128x128", "256x256w8"])
+def test_gemm_mx_inf_and_nan(gpu, monkeypatch, tile):
+    """NaN bytes, NaN scales and scales of 2^127 stay in their own row and column of the output,
+    and every other element is the oracle's."""
+    monkeypatch.setenv("BONGARD_FP8_GEMM_TILE", tile)
+    M, N, K = 300, 264, 416
+    g = torch.Generator().manual_seed(31)
+    qa = ops.quantize_mx(torch.randn(M, K, generator=g).to(torch.bfloat16).to(gpu))
+    qb = ops.quantize_mx(torch.randn(N, K, generator=g).to(torch.bfloat16).to(gpu))
+    qa.data.view(torch.uint8)[9, K - 1] = 0x7F      # an e4m3 NaN in the partial last step
+    qa.scales[258, 1] = 0xFF                        # an E8M0 NaN block
+    qb.scales[261, 0] = 254                         # 2^127 against 2^127
+    qa.scales[5, 0] = 254
+    planes = [_planes_of(q.scales) for q in (qa, qb)]
+    y = ops.gemm_mx(qa.data, qa.scales, qb.data, qb.scales)
+    yp = ops.gemm_mx(qa.data, None, qb.data, None, a_planes=planes[0], b_planes=planes[1])
+    torch.cuda.synchronize()
+    y, yp = y.float().cpu(), yp.float().cpu()
+    assert torch.equal(y.isnan(), yp.isnan()) and torch.equal(y.nan_to_num(), yp.nan_to_num())
+    assert y[[9, 258]].isnan().all() and not y[5, 261].isfinite()
+    keep_m, keep_n = torch.ones(M, dtype=torch.bool), torch.ones(N, dtype=torch.bool)
+    keep_m[[5, 9, 258]] = False
+    keep_n[261] = False
+    a8, ae = qa.data.view(torch.uint8).cpu()[keep_m], qa.scales.cpu()[keep_m][:, :K // 32].int()
+    b8, be = qb.data.view(torch.uint8).cpu()[keep_n], qb.scales.cpu()[keep_n][:, :K // 32].int()
+    ref = orc.scaled_mm_mx(a8, ae, b8, be)
+    got = y[keep_m][:, keep_n]
+    assert got.isfinite().all()
+    excess = ((got - ref).abs() - 0.5 * orc.bf16_ulp(ref)).max().item()
+    assert excess <= 0.01 * _rms(ref)
 
 
 def test_quantize_mx_many_equals_quantize_mx(gpu, monkeypatch):
