@@ -126,7 +126,7 @@ _linear_op.register_autograd(_linear_grad, setup_context=_linear_setup)
 
 def fp8_linear(x, weight, bias, recipe):
     """y = x @ weight^T (+ bias) in FP8 under a torchao recipe, as one custom op (x: bf16
-    [M, K], M % 16 == 0 when x or weight needs a gradient)."""
+    [M, K]; under 'rowwise' M % 16 == 0 when the weight needs a gradient)."""
     grad = torch.is_grad_enabled()
     need_dx = grad and x.requires_grad
     need_dw = grad and weight.requires_grad

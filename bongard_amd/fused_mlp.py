@@ -3,9 +3,11 @@
 Drop-in for bongard/fused_mlp.py (TransformerEngine te.LayerNormMLP path): same
 ``RECIPES``, ``FusedMLP(mlp, norm, recipe)`` with parameters ``layer_norm_weight``
 [hidden], ``fc1_weight`` [2I, hidden] (= [gate; up]), ``fc2_weight`` [hidden, I] and an
-``_extra_state`` (empty for 'fp8'; the amax histories for 'fp8_delayed'); HF eval views (``_hf_mlp``, ``_hf_norm``) sharing storage and
-refreshed by ``_apply``; counters ``weight_quantizations`` / ``cached_weights`` /
-``real_tokens`` / ``kernel_tokens``; ``enable_fused_mlp(model, recipe) -> int``; and
+``_extra_state`` (empty for 'fp8'; the amax histories for 'fp8_delayed'); HF eval views
+(``_hf_mlp``, ``_hf_norm``) sharing storage and refreshed by ``_apply``; counters
+``weight_quantizations`` / ``cached_weights`` / ``real_tokens`` / ``kernel_tokens`` (the
+reference's: rows rounded up to 32, bongard/fused_mlp.py:73-74; a nominal count, since only the
+block-scaled recipes run padded rows here); ``enable_fused_mlp(model, recipe) -> int``; and
 ``hf_state_dict(backbone)`` for export.
 
 Training forward: RMSNorm with zero-centred gamma (``x * rsqrt(mean(x^2) + eps) *
@@ -130,8 +132,8 @@ class FusedMLP(_ScalingExtraState, torch.nn.Module):
         self._cached_weight_versions = versions
         self.counts['weight_quantizations' if first else 'cached_weights'] += 1
         length = flat.shape[0]
-        # the token count of the 32-row granularity the reference pads to; only the
-        # block-scaled recipes' kernels need the padded rows themselves
+        # kernel_tokens is nominal, the reference's 32-row granularity: only the block-scaled
+        # recipes' kernels need the padded rows themselves
         self.counts['real_tokens'] += length
         self.counts['kernel_tokens'] += (length + 31) // 32 * 32
         if _is_blocked(self.recipe):

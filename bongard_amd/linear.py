@@ -211,8 +211,8 @@ def linear_axiswise_backward(dy, saved, recipe, need_dx, need_dw):
 
 
 class Fp8LinearAxiswiseFunction(_Fp8Function):
-    """y = x @ W^T (+ b) under torchao's axiswise recipes; x: bf16 [M, K], M % 16 == 0 when
-    grads are needed. Every cast is e4m3 with power-of-2 scales (torchao 0.17.0
+    """y = x @ W^T (+ b) under torchao's axiswise recipes; x: bf16 [M, K] (under 'rowwise'
+    M % 16 == 0 when the weight needs a gradient). Every cast is e4m3 with power-of-2 scales (torchao 0.17.0
     Float8LinearConfig.from_recipe_name, round_scales_to_power_of_2=True):
 
       forward              y  = X8[per row] . W8[per row]^T

@@ -519,36 +519,59 @@ def test_inference_forward_shares_quantize_launches(gpu, monkeypatch):
     assert torch.equal(y_train.detach(), y_inf)
 
 
-
 @pytest.mark.parametrize("rows", [1, 15, 77, 301])
 @pytest.mark.parametrize("kind", ["te_fp8", "te_delayed", "tensorwise", "gw_hp"])
 def test_ragged_rows_equal_padded_rows(gpu, rows, kind):
-    """Row counts that are not multiples of 16 or 32 run without padded copies: the gradients
-    and outputs are those of the zero-padded rows (fp32 sums of the same products; the K split
-    may differ), also for an input view off 16-byte alignment and an expanded gradient."""
-    from bongard_amd import linear, scaling
-    K, N, pad = 512, 384, (rows + 31) // 32 * 32
+    """Row counts that are not multiples of 16 or 32 run without padded copies: a module's
+    gradients and outputs are those of rows that the caller padded with zeros (fp32 sums of the
+    same products; the K split may differ), over two micro-batches (a TELinear's second uses its
+    cached weight), for an input view off 16-byte alignment and an expanded gradient."""
+    F = torch.nn.functional
+    K, N, pad = 512, 384, (rows + 31) // 32 * 32 - rows
     g = torch.Generator().manual_seed(rows)
     buf = torch.randn(rows * K + 3, generator=g).to(torch.bfloat16).to(gpu)
     x = buf[3:].view(rows, K)                       # 6 bytes past the allocation's alignment
     w = (torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
     dy = torch.full((1, N), 1e-3, dtype=torch.bfloat16, device=gpu).expand(rows, N)
 
-    def run(x, dy):
-        xg, wg = x.detach().requires_grad_(True), w.detach().clone().requires_grad_(True)
-        if kind == "gw_hp":
-            y = linear.Fp8LinearAxiswiseFunction.apply(xg, wg, None, "rowwise_with_gw_hp")
-        else:
-            sc = scaling.LinearScaling(16) if kind == "te_delayed" else None
-            y = linear.Fp8LinearFunction.apply(xg, wg, None, None, sc)
-        return (y, *torch.autograd.grad(y, [xg, wg], dy))
+    def module():
+        lin = nn.Linear(K, N, bias=False, dtype=torch.bfloat16, device=gpu)
+        with torch.no_grad():
+            lin.weight.copy_(w)
+        if kind.startswith("te_"):
+            return te_linear.TELinear([lin], "fp8" if kind == "te_fp8" else "fp8_delayed").train()
+        recipe = "tensorwise" if kind == "tensorwise" else "rowwise_with_gw_hp"
+        config = float8_training.Float8LinearConfig.from_recipe_name(recipe)
+        return float8_training.Float8Linear.from_float(lin, config).train()
 
-    F = torch.nn.functional
-    y, dx, dw = run(x, dy)
-    py, pdx, pdw = run(F.pad(x, (0, 0, 0, pad - rows)), F.pad(dy, (0, 0, 0, pad - rows)))
+    ragged, padded = module(), module()
+    for step in range(2):
+        out = []
+        for m, xi, di in ((ragged, x, dy), (padded, F.pad(x, (0, 0, 0, pad)), F.pad(dy, (0, 0, 0, pad)))):
+            xg = xi.detach().requires_grad_(True)
+            y = m(xg)
+            out.append((y, *torch.autograd.grad(y, [xg, m.weight], di)))
+        torch.cuda.synchronize()
+        for what, a, b in zip(("y", "dx", "dw"), *out):
+            _close(a, b if what == "dw" else b[:rows], f"ragged {kind} {rows} {what} {step}", tol=1e-3)
+    if kind.startswith("te_"):
+        assert ragged.counts == {"weight_quantizations": 1, "cached_weights": 1}
+
+
+@pytest.mark.parametrize("recipe,run_rows", [("fp8", 150), ("fp8_delayed", 150), ("mxfp8", 160),
+                                             ("nvfp4", 160)])
+def test_fused_mlp_rows_run(gpu, monkeypatch, recipe, run_rows):
+    """Only the block-scaled recipes run padded rows; ``kernel_tokens`` stays the nominal count, of
+    rows rounded up to 32, for every recipe."""
+    seen = []
+    real = ops.rmsnorm
+    monkeypatch.setattr(ops, "rmsnorm", lambda x, *a, **k: seen.append(x.shape[0]) or real(x, *a, **k))
+    norm = T5Gemma2RMSNorm(256, eps=1e-6).to(torch.bfloat16).to(gpu)
+    f = fused_mlp.FusedMLP(_mlp(256, 512, 3, gpu), norm, recipe).train()
+    y = f(torch.randn(150, 256, device=gpu).to(torch.bfloat16))
     torch.cuda.synchronize()
-    for what, a, b in (("y", y, py[:rows]), ("dx", dx, pdx[:rows]), ("dw", dw, pdw)):
-        _close(a, b, f"ragged {kind} {rows} {what}", tol=1e-3)
+    assert y.shape == (150, 256) and seen == [run_rows]
+    assert f.counts["real_tokens"] == 150 and f.counts["kernel_tokens"] == 160
 
 
 @pytest.mark.parametrize("recipe", ["fp8", "fp8_delayed"])
