@@ -606,9 +606,9 @@ def _bench_state_kv(torch, workloads, dev, steps=20):
 
 def _bench_c2_mx(torch, ops, workloads, dev, steps=30):
     """The c2 MLP forward under TE's 'mxfp8' recipe: X, [W_gate; W_up], W_down quantized in
-    32-element blocks (E8M0 scales), gated-GELU GEMM on the block-scaled MFMA with H
-    quantized in blocks in its epilogue, down GEMM (and, for comparison, the same step with
-    a separate bf16 H and quantize pass)."""
+    32-element blocks (E8M0 scales, as planes), gated-GELU GEMM on the block-scaled MFMA with H
+    quantized in blocks in its epilogue, down GEMM: the calls of the layers' own forward (and, for
+    comparison, the same step on scale rows with a separate bf16 H and quantize pass)."""
     c = workloads.config2()
     x = c["x"].to(dev)
     w_gu = torch.cat([c["w_gate"], c["w_up"]]).to(dev)
@@ -617,12 +617,14 @@ def _bench_c2_mx(torch, ops, workloads, dev, steps=30):
     I = c["w_gate"].shape[0]
 
     def step(fused=True):
-        xq, gq, dq = ops.quantize_mx_many([x, w_gu, w_d])   # one launch, as the MX forward
+        # one launch, as the MX forward
+        xq, gq, dq = ops.quantize_mx_many([x, w_gu, w_d], scale_rows=not fused)
         if fused:  # H quantized in the gate/up GEMM's epilogue (the product path)
-            hq, _, _ = ops.gemm_geglu_mx_quant(xq.data, xq.scales, gq.data, gq.scales, I)
-        else:
-            H, _ = ops.gemm_geglu_mx(xq.data, xq.scales, gq.data, gq.scales, I)
-            hq = ops.quantize_mx(H)
+            hq, _ = ops.gemm_geglu_mx_planes(xq.data, xq.planes, gq.data, gq.planes, I)
+            return ops.gemm_mx(hq.data, None, dq.data, None, a_planes=hq.planes,
+                               b_planes=dq.planes)
+        H, _ = ops.gemm_geglu_mx(xq.data, xq.scales, gq.data, gq.scales, I)
+        hq = ops.quantize_mx(H)
         return ops.gemm_mx(hq.data, hq.scales, dq.data, dq.scales)
 
     for _ in range(PREWARM_STEPS):
@@ -636,12 +638,14 @@ def _bench_c2_mx(torch, ops, workloads, dev, steps=30):
     hq = ops.quantize_mx(H)
     g_s = _ev_time(torch, lambda: ops.gemm_geglu_mx(xq.data, xq.scales, gq.data, gq.scales, I),
                    steps)
-    gq_s = _ev_time(torch, lambda: ops.gemm_geglu_mx_quant(xq.data, xq.scales, gq.data,
-                                                           gq.scales, I), steps)
-    d_s = _ev_time(torch, lambda: ops.gemm_mx(hq.data, hq.scales, dq.data, dq.scales), steps)
-    h_s = _ev_time(torch, lambda: ops.quantize_mx(H), steps)
-    qm_s = _ev_time(torch, lambda: ops.quantize_mx_many([x, w_gu, w_d]), steps)
-    qs_s = _ev_time(torch, lambda: [ops.quantize_mx(t) for t in (x, w_gu, w_d)], steps)
+    gq_s = _ev_time(torch, lambda: ops.gemm_geglu_mx_planes(xq.data, xq.planes, gq.data,
+                                                            gq.planes, I), steps)
+    d_s = _ev_time(torch, lambda: ops.gemm_mx(hq.data, None, dq.data, None, a_planes=hq.planes,
+                                              b_planes=dq.planes), steps)
+    h_s = _ev_time(torch, lambda: ops.quantize_mx(H, scale_rows=False), steps)
+    qm_s = _ev_time(torch, lambda: ops.quantize_mx_many([x, w_gu, w_d], scale_rows=False), steps)
+    qs_s = _ev_time(torch, lambda: [ops.quantize_mx(t, scale_rows=False) for t in (x, w_gu, w_d)],
+                    steps)
     flop = 2.0 * M * (2 * I * K + K * I)
     return {"workload": f"c2 MLP forward [{M},{K}] x [2*{I},{K}] -> [{M},{I}] x [{K},{I}], MXFP8",
             "us_per_step": round(s * 1e6, 2), "tflops": round(flop / s / 1e12, 1),

@@ -13,7 +13,8 @@ the fused norm: the config-2 MLP forward under MXFP8 (block quantize, MX gated-G
 quantized in its epilogue, MX down GEMM), the axiswise (torchao rowwise) quantization of a [8192, 2560] activation
 per row and per column, the fused RMSNorm of the same activation, and the config-2 MLP
 forward under NVFP4 (block quantize, exact dequantization, bf16 MFMA GEMMs, elementwise
-gated GELU). ``c5``: the
+gated GELU). ``recipes_train``: training steps of that MLP under MXFP8 and NVFP4, and two
+products on the two-stage tiles. ``c5``: the
 config-5 training step (the c2 MLP at M = 8192, forward and backward, delayed scaling with
 an amax history of 16). ``vs_hipblaslt``: this library's FP8 GEMM and hipBLASLt's (through
 ``torch._scaled_mm``) on the c2 / c4 / square shapes, each captured as a HIP graph of 20
@@ -38,8 +39,8 @@ def main():
     p = argparse.ArgumentParser()
     p.add_argument("--iters", type=int, default=5)
     p.add_argument("--rows", type=int, default=4096)
-    p.add_argument("--case", choices=("c2", "square", "recipes", "c5", "vs_hipblaslt", "c4",
-                                      "vs_hipblaslt_eager"),
+    p.add_argument("--case", choices=("c2", "square", "recipes", "recipes_train", "c5",
+                                      "vs_hipblaslt", "c4", "vs_hipblaslt_eager"),
                    default="c2")
     args = p.parse_args()
     dev = torch.device("cuda:0")
@@ -55,6 +56,9 @@ def main():
         return
     if args.case == "recipes":
         _recipes(dev, args.iters)
+        return
+    if args.case == "recipes_train":
+        _recipes_train(dev, args.iters)
         return
     if args.case == "c5":
         _c5(dev, args.iters)
@@ -220,9 +224,10 @@ def _recipes(dev, iters):
     dst = torch.empty_like(src)
     for _ in range(iters):
         dst.copy_(src)
-        xq, gq, dq = ops.quantize_mx(x), ops.quantize_mx(w_gu), ops.quantize_mx(w_d)
-        hq, _, _ = ops.gemm_geglu_mx_quant(xq.data, xq.scales, gq.data, gq.scales, I)
-        ops.gemm_mx(hq.data, hq.scales, dq.data, dq.scales)
+        # MXFP8 as the modules run it: scales as planes, H quantized in the gate/up epilogue
+        xq, gq, dq = ops.quantize_mx_many([x, w_gu, w_d], scale_rows=False)
+        hq, _ = ops.gemm_geglu_mx_planes(xq.data, xq.planes, gq.data, gq.planes, I)
+        ops.gemm_mx(hq.data, None, dq.data, None, a_planes=hq.planes, b_planes=dq.planes)
         ops.quantize_axiswise(a, ops.E4M3, rowwise=True, colwise=True)
         ops.rmsnorm(a, gamma, 1e-6)
         # NVFP4 as the modules run it: X and H written as their bf16 dequantization, H's
@@ -236,6 +241,33 @@ def _recipes(dev, iters):
                        a_deq=ops.nvfp4_dequant(hn))
     torch.cuda.synchronize()
     print(f"profile_target done: {iters} iterations (recipes), copy {COPY_BYTES} bytes", flush=True)
+
+
+def _recipes_train(dev, iters):
+    """Training steps (forward and backward, weights quantized in the step) of the config-2 MLP
+    under MXFP8 and NVFP4, and two products that the planner runs on the two-stage tiles."""
+    from . import linear
+
+    c = workloads.config2()
+    I = workloads.INTERMEDIATE
+    x = c["x"].to(dev).requires_grad_(True)
+    w_gu = torch.cat([c["w_gate"], c["w_up"]], 0).to(dev).requires_grad_(True)
+    w_d = c["w_down"].to(dev).requires_grad_(True)
+    dy = (torch.randn(x.shape[0], w_d.shape[0], device=dev) * 1e-3).to(torch.bfloat16)
+    aq = ops.quantize(torch.randn(2001, 4096, device=dev).to(torch.bfloat16))
+    bq = ops.quantize(torch.randn(2560, 4096, device=dev).to(torch.bfloat16))
+    cq = ops.quantize(torch.randn(20480, 1024, device=dev).to(torch.bfloat16))
+    dq = ops.quantize(torch.randn(2560, 1024, device=dev).to(torch.bfloat16))
+    for _ in range(iters):
+        y = linear.Fp8GegluMlpMxFunction.apply(x, w_gu, w_d, None, None, I)
+        torch.autograd.grad(y, [x, w_gu, w_d], dy)
+        h, parts = linear.GegluGateUpNvfp4Function.apply(x, w_gu, None, I, None)
+        y = linear.Fp8LinearNvfp4Function.apply(h, w_d, None, parts)
+        torch.autograd.grad(y, [x, w_gu, w_d], dy)
+        ops.gemm(aq.data, ops.E4M3, aq.meta, bq.data, ops.E4M3, bq.meta)
+        ops.gemm(cq.data, ops.E4M3, cq.meta, dq.data, ops.E4M3, dq.meta)
+    torch.cuda.synchronize()
+    print(f"profile_target done: {iters} iterations (recipes_train)", flush=True)
 
 
 if __name__ == "__main__":
