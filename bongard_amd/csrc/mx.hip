@@ -81,7 +81,7 @@ __device__ __forceinline__ uint2 mx_quant8_vs(uint4 v, const float* s) {
 // the MALL: [4096, 20480] 133.1 us in two passes, 78.4 us in one (4.3 TB/s); [20480, 2560]
 // 72.9 -> 45.4 us (4.7 TB/s); one pass over 64 x 64 tiles per wave, whose stores are half
 // lines, 99.7 and 56.3 us. With planes in place of the scale rows' scattered dwords 75.2 and
-// 43.0 us. The rowwise copy alone is mx_rows_kernel's.
+// 43.0 us. The rowwise copy alone is mx_rows_kernel's, a small tensor's copies mx_wave_kernel's.
 struct MxTile {
   const uint16_t* x;
   int64_t rows, cols;
