@@ -765,9 +765,15 @@ int bf8_cast_delayed_bf16(const void* x, int64_t rows, int64_t cols, float* stat
                      "bf8_cast_delayed_bf16");
 }
 
+// Whether work on s is captured. Where the runtime can't tell, its error is taken back, so that
+// the launches that follow don't report it, and the answer is yes (the general path).
 static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
 }
 
 // keep_partials: the caller may read the partials afterwards (they are not mere scratch).

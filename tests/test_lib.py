@@ -6,6 +6,7 @@ import re
 from pathlib import Path
 
 import pytest
+import torch
 
 from bongard_amd import _lib
 
@@ -269,3 +270,16 @@ def test_errors_name_the_entry_called():
         assert message.startswith(name + ":"), message
         if "planes" in name:
             assert "planes" in message, message
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="launches on host memory")
+@pytest.mark.parametrize("cols, first", [(1024, b"quantize_small_kernel"),
+                                         (8192, b"amax_partials_kernel")])
+def test_quantize_without_a_known_capture_state(cols, first):
+    """Where the runtime can't tell whether the stream is captured (here: no device), sizes whose
+    one-launch form is for eager calls alone take the general path."""
+    L = _lib.lib()
+    buf = ctypes.create_string_buffer(1 << 20)
+    p = ctypes.c_void_p((ctypes.addressof(buf) + 255) // 256 * 256)
+    assert L.bf8_quantize_bf16(p, 16, cols, 0, p, None, p, p, None) != 0
+    assert L.bf8_last_error().startswith(first)
