@@ -308,25 +308,18 @@ __global__ __launch_bounds__(kNT) void nvfp4_tile_kernel(const uint16_t* __restr
   }
 }
 
-// The rowwise copy alone: one 16-block per thread (grid-stride), so codes and scale bytes leave
-// in whole lines; the tile kernel's 128-column rows would write the codes in half lines. Codes of
-// [4096, 20480]: 40.5 us (5.3 TB/s; 56.3 us on the tile kernel, 54.6 us with the rounding by
-// comparisons).
-__global__ __launch_bounds__(kNT) void nvfp4_rows_kernel(const uint16_t* __restrict__ x, NvTile p,
-                                                         const uint32_t* __restrict__ partials,
-                                                         int64_t np, float* __restrict__ meta) {
-  __shared__ float mult_of[128];
-  const float s_enc = scale_from_partials_block<kNT>(partials, np, kNvfp4Global, meta, false,
-                                                     blockIdx.x == 0);
+// The rowwise copy by blocks 0 .. nblk - 1: one 16-block per thread (grid-stride).
+__device__ __forceinline__ void nv_rows_body(const uint16_t* __restrict__ x, const NvTile& p,
+                                             float s_enc, float* mult_of, int64_t blk,
+                                             int64_t nblk) {
   if (threadIdx.x < 128) {
     const float s = e4m3_value(threadIdx.x);
     mult_of[threadIdx.x] = s == 0.0f ? 0.0f : s_enc / s;
   }
   __syncthreads();
   const bool s_finite = fabsf(s_enc) < INFINITY;
-  const int64_t nblk = p.rows * (p.cols / 16);
-  for (int64_t b = (int64_t)blockIdx.x * kNT + threadIdx.x; b < nblk;
-       b += (int64_t)gridDim.x * kNT) {
+  const int64_t items = p.rows * (p.cols / 16);
+  for (int64_t b = blk * kNT + threadIdx.x; b < items; b += nblk * kNT) {
     const uint4* src = reinterpret_cast<const uint4*>(x + b * 16);
     const uint4 v0 = src[0], v1 = src[1];
     const uint32_t key = max(absmax_key8(v0), absmax_key8(v1));
@@ -355,21 +348,28 @@ __global__ __launch_bounds__(kNT) void nvfp4_rows_kernel(const uint16_t* __restr
   }
 }
 
-// Columnwise quantization of a small tensor, or of one whose rows are not whole 16-byte vectors
-// (cols % 8 != 0), which the tile kernel's loads need: one (column, 16-row block) per thread, consecutive
-// threads on consecutive columns. out_t [cols, rows / 2], scales_t [cols, rows / 16].
-__global__ __launch_bounds__(kNT) void nvfp4_cols_kernel(const uint16_t* __restrict__ x,
-                                                         int64_t rows, int64_t cols,
+// The rowwise copy alone: codes and scale bytes leave in whole lines, where the tile kernel's
+// 128-column rows would write the codes in half lines. Codes of [4096, 20480]: 40.5 us (5.3 TB/s;
+// 56.3 us on the tile kernel, 54.6 us with the rounding by comparisons).
+__global__ __launch_bounds__(kNT) void nvfp4_rows_kernel(const uint16_t* __restrict__ x, NvTile p,
                                                          const uint32_t* __restrict__ partials,
-                                                         int64_t np, float* __restrict__ meta,
-                                                         uint8_t* __restrict__ out_t,
-                                                         uint8_t* __restrict__ scales_t) {
+                                                         int64_t np, float* __restrict__ meta) {
+  __shared__ float mult_of[128];
   const float s_enc = scale_from_partials_block<kNT>(partials, np, kNvfp4Global, meta, false,
                                                      blockIdx.x == 0);
+  nv_rows_body(x, p, s_enc, mult_of, blockIdx.x, gridDim.x);
+}
+
+// The columnwise copy by blocks 0 .. nblk - 1: one (column, 16-row block) per thread, consecutive
+// threads on consecutive columns. out_t [cols, rows / 2], scales_t [cols, rows / 16].
+__device__ __forceinline__ void nv_cols_body(const uint16_t* __restrict__ x, int64_t rows,
+                                             int64_t cols, float s_enc,
+                                             uint8_t* __restrict__ out_t,
+                                             uint8_t* __restrict__ scales_t, int64_t blk,
+                                             int64_t nblk) {
   const int64_t rblocks = rows / 16;
   const int64_t nitems = cols * rblocks;
-  for (int64_t it = (int64_t)blockIdx.x * kNT + threadIdx.x; it < nitems;
-       it += (int64_t)gridDim.x * kNT) {
+  for (int64_t it = blk * kNT + threadIdx.x; it < nitems; it += nblk * kNT) {
     const int64_t rb = it / cols, c = it - rb * cols;
     uint32_t w[8];
     uint32_t key = 0;
@@ -386,6 +386,35 @@ __global__ __launch_bounds__(kNT) void nvfp4_cols_kernel(const uint16_t* __restr
     *reinterpret_cast<uint2*>(out_t + c * (rows / 2) + rb * 8) = pack16(w, mult);
     scales_t[c * rblocks + rb] = (uint8_t)sbyte;
   }
+}
+
+// Columnwise quantization of a small tensor, or of one whose rows are not whole 16-byte vectors
+// (cols % 8 != 0), which the tile kernel's loads need.
+__global__ __launch_bounds__(kNT) void nvfp4_cols_kernel(const uint16_t* __restrict__ x,
+                                                         int64_t rows, int64_t cols,
+                                                         const uint32_t* __restrict__ partials,
+                                                         int64_t np, float* __restrict__ meta,
+                                                         uint8_t* __restrict__ out_t,
+                                                         uint8_t* __restrict__ scales_t) {
+  const float s_enc = scale_from_partials_block<kNT>(partials, np, kNvfp4Global, meta, false,
+                                                     blockIdx.x == 0);
+  nv_cols_body(x, rows, cols, s_enc, out_t, scales_t, blockIdx.x, gridDim.x);
+}
+
+// Both copies of a small tensor: the first row_blocks blocks take the rowwise copy, the others the
+// columnwise codes, each reading x for itself (the second time from a cache).
+__global__ __launch_bounds__(kNT) void nvfp4_pair_kernel(const uint16_t* __restrict__ x, NvTile p,
+                                                         const uint32_t* __restrict__ partials,
+                                                         int64_t np, float* __restrict__ meta,
+                                                         int row_blocks) {
+  __shared__ float mult_of[128];
+  const float s_enc = scale_from_partials_block<kNT>(partials, np, kNvfp4Global, meta, false,
+                                                     blockIdx.x == 0);
+  if ((int)blockIdx.x < row_blocks)
+    nv_rows_body(x, p, s_enc, mult_of, blockIdx.x, row_blocks);
+  else
+    nv_cols_body(x, p.rows, p.cols, s_enc, p.out_t, p.scales_t, blockIdx.x - row_blocks,
+                 gridDim.x - row_blocks);
 }
 
 // bf16 [rows, cols] = e2m1(q) * s for every block (exact); S_dec is left to the GEMM.
@@ -438,6 +467,11 @@ static int nvfp4_args(const char* who, const void* x, int64_t rows, int64_t cols
 // Tile / columns kernel, us, inputs not seen before: 64 x 640 5.3 / 3.4, 320 x 2048 5.9 / 4.0,
 // 1216 x 2048 6.7 / 5.9, 3584 x 2048 9.3 / 10.4, 2304 x 2560 9.1 / 11.1.
 constexpr int64_t kMaxColsKernel = 4 << 20;
+// Both copies, the columnwise one as codes: the same with the rows kernel's work beside it, where
+// the second read of x costs less than the idle CUs. Tile / pair kernel, us, likewise: 32 x 2560
+// 7.2 / 3.6, 736 x 1024 7.5 / 4.4, 800 x 2560 8.0 / 6.2, 1792 x 2048 8.9 / 8.2, 256 x 16384 9.2 /
+// 8.2, 1312 x 3584 11.2 / 12.6, 1664 x 3584 11.5 / 14.4. (One launch a copy at 32 x 2560: 6.7.)
+constexpr int64_t kMaxPairKernel = kMaxColsKernel;
 
 // The rowwise and/or columnwise casts, the per-tensor amax reduced from np partials (maxima
 // of |x| as fp32 bits) that are already written.
@@ -456,6 +490,12 @@ static int nvfp4_casts(const void* x, const NvTile& p, const uint32_t* partials,
                        (const uint16_t*)x, p.rows, p.cols, partials, np, meta, p.out_t,
                        p.scales_t);
     return launch_status("nvfp4_cols_kernel");
+  }
+  if ((p.out || p.deq) && !p.deq_t && p.rows * p.cols <= kMaxPairKernel) {
+    const unsigned half = stream_grid(p.rows * p.cols / 16);
+    hipLaunchKernelGGL(nvfp4_pair_kernel, dim3(2 * half), dim3(kNT), 0, s, (const uint16_t*)x, p,
+                       partials, np, meta, (int)half);
+    return launch_status("nvfp4_pair_kernel");
   }
   const int64_t tiles = ((p.rows + kNT4 - 1) / kNT4) * ((p.cols + kNT4 - 1) / kNT4);
   const unsigned grid = (unsigned)(tiles < kMaxNvTileBlocks ? tiles : kMaxNvTileBlocks);

@@ -68,7 +68,8 @@ def test_quantize_nvfp4_bit_exact(gpu, rows, cols):
     assert torch.equal(deq.cpu().float(), ref)        # e2m1 x e4m3 is exact in bf16
 
 
-@pytest.mark.parametrize("rows,cols", [(16, 128), (128, 128), (144, 272), (272, 48), (400, 2560)])
+@pytest.mark.parametrize("rows,cols", [(16, 128), (128, 128), (144, 272), (272, 48), (400, 2560),
+                                       (1648, 2640)])
 def test_quantize_nvfp4_tile_edges(gpu, rows, cols):
     """Whole and partial 128 x 128 tiles in either direction: codes and scales of both copies
     against the oracle, and both copies written as their bf16 dequantization."""
@@ -91,9 +92,9 @@ def test_quantize_nvfp4_tile_edges(gpu, rows, cols):
 
 @pytest.mark.parametrize("special", [None, float("inf"), float("nan")])
 def test_quantize_nvfp4_broken_rows_and_non_finite(gpu, special):
-    """Columns that do not fill 16-byte vectors take the per-column kernel: the same bytes as the
-    tile kernel gives for those columns of a padded tensor under the same tensor amax, also
-    where the tensor or some of its blocks hold inf or NaN."""
+    """Columns that do not fill 16-byte vectors: the same bytes as for those columns of a padded
+    tensor under the same tensor amax, also where the tensor or some of its blocks hold inf or
+    NaN."""
     x = _inputs(160, 24, 5)
     if special is not None:
         x[3, 4], x[100, 7] = special, -special
@@ -107,6 +108,32 @@ def test_quantize_nvfp4_broken_rows_and_non_finite(gpu, special):
         assert torch.equal(a.data_t[:20], b.data_t) and torch.equal(a.scales_t[:20], b.scales_t)
     with pytest.raises(Exception, match="cols"):
         ops.quantize_nvfp4(x[:, :20].contiguous(), rowwise=False, colwise=True, dequant_cols=True)
+
+
+@pytest.mark.parametrize("special", [None, float("inf"), float("nan")])
+@pytest.mark.parametrize("rows", [16, 144, 1024])
+def test_quantize_nvfp4_small_and_large_kernels(gpu, rows, special):
+    """Tensors of up to 4M elements take kernels of their own: the first rows of a larger tensor
+    quantized by themselves, under its amax, give the bytes that they have within it."""
+    x = torch.randn(1040, 4096, generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16)
+    if special is not None:
+        x[3, 4], x[rows - 1, 700] = special, -special
+    x = x.to(gpu)
+    assert x.numel() > 4 << 20 >= x[:rows].numel()
+    for parts in (ops.amax(x), ops.amax(torch.full((16, 8), 3.0, dtype=torch.bfloat16, device=gpu))):
+        big = ops.quantize_nvfp4(x, colwise=True, partials=parts)
+        for args in (dict(), dict(dequant_rows=True), dict(rowwise=False)):
+            small = ops.quantize_nvfp4(x[:rows], colwise=True, partials=parts, **args)
+            torch.cuda.synchronize()
+            if "dequant_rows" in args:
+                want = ops.nvfp4_dequant(big)[:rows]
+                assert torch.equal(ops.nvfp4_dequant(small).view(torch.int16), want.view(torch.int16))
+            elif not args:
+                assert torch.equal(small.data, big.data[:rows])
+                assert torch.equal(small.scales, big.scales[:rows])
+            assert torch.equal(small.data_t, big.data_t[:, :rows // 2])
+            assert torch.equal(small.scales_t, big.scales_t[:, :rows // 16])
+            assert torch.equal(small.meta.view(torch.int32), big.meta.view(torch.int32))
 
 
 def test_quantize_nvfp4_zero_tensor_and_columnwise_only(gpu):
